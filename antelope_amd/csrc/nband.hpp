@@ -182,6 +182,35 @@ constexpr int64_t kNb32VelMaxK = 1024;
 hipError_t nb32_launch_vel_fused(const NbArgs &a, const NbVelFused &f, const double2 *P, const double *Eocc,
                                  double2 *rho, double *partials, hipStream_t s);
 
+// Time-fused LengthWannier steps of the analytic classes with N <= 8
+// (nb_evolve_kernel): steps [s0, s1) in one launch, one partial row per block and step.
+constexpr int kEvolveMaxTerms = 9;
+struct EvolveTerms {  // analytic_terms.hpp
+    int T;
+    double vec[kEvolveMaxTerms][3], grad[kEvolveMaxTerms][3];
+};
+struct NbEvolve {
+    EvolveTerms terms;
+    const double2 *coef;   // [1 + 2 T + 1][N][N]: m0, (p_t, q_t) per term, the current's element factors
+    const double *table;   // [nt + 1][row]: cos / sin(A.v_t) at the step's distinct times
+    int jz;                // any z current
+    int64_t nt, s0, s1;
+    double dt;
+    int nblocks;
+    double *lam;           // [nk_stride][8] band energies at the stored eigenvectors' time
+    int lam_valid;         // the stored eigenvectors and lam belong to t_{s0}
+};
+// distinct stage times of a step (t_n first, t_n + dt being the next step's), the padded
+// number of terms of the kernels, doubles per table row and blocks of a launch
+inline int evolve_times(int rk_order) { return rk_order == 4 ? 2 : 5; }
+inline int evolve_padded_terms(int T) { return T <= 3 ? 3 : (T <= 6 ? 6 : 9); }
+inline int evolve_row_len(int rk_order, int T) { return (6 + 2 * evolve_times(rk_order)) * evolve_padded_terms(T); }
+int evolve_blocks(int N, int64_t nk);
+// the table of rows n in [0, rows) from A at the distinct times, [rows][times][3]
+hipError_t launch_evolve_table(const double *A, const EvolveTerms &t, int rk_order, int64_t rows, double *tab, hipStream_t s);
+hipError_t launch_evolve(const NbArgs &a, const NbEvolve &e, int rk_order, double2 *rho, double2 *U, double *partials,
+                         hipStream_t s);
+
 // One time step of the VelocityHamiltonian gauge: A at the stage times and
 // the tableau (coefficients already multiplied by dt).
 struct NbVelStep {

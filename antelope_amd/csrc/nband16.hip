@@ -43,182 +43,13 @@
 #include <mutex>
 
 #include "nband.hpp"
-#include "tile16.hpp"
+#include "tile_eig.hpp"
 
 namespace sbe {
 namespace {
 
 using namespace tile;
 
-
-// U <- U (3I - U^dag U) / 2 (Newton-Schulz: unitarity error e -> ~e^2);
-// returns e = max |U^dag U - I| before the step (over the wave)
-__device__ __forceinline__ double orthonormalize(Tile &U, Tile &Ut, cd *buf)
-{
-    const int c = lane_c(), g = lane_g();
-    const Tile G = cmm(U, true, U);
-    Tile S;
-    double e = 0.0;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const double dr = G.re[r] - (g + 4 * r == c ? 1.0 : 0.0);
-        e = fmax(e, fmax(fabs(dr), fabs(G.im[r])));
-        S.re[r] = (g + 4 * r == c ? 1.5 : 0.0) - 0.5 * G.re[r];
-        S.im[r] = -0.5 * G.im[r];
-    }
-    U = cmm(Ut, false, S);
-    Ut = transpose(U, buf);
-    return wave_max(e);
-}
-
-// Warm-started eigenvectors of the Hermitian part of H (as zheevr, which
-// reads one triangle; H from FP16-split sums is Hermitian only to their
-// error): U (and its transpose Ut) in, refined U, Ut out.
-// small: max|K| below which the last round is U (I + K) (its neglected K^2/2 and the
-// next round's O(K^2) residual are the eigenvectors' error); ortho: end with a
-// Newton-Schulz step (U unitary to rounding rather than to O(small^2))
-// herm: Hin is Hermitian to rounding already (FP64 sums), no symmetrization; lam_out:
-// this lane's column of diag(U^dag H U) before the last rotation (the band energies to
-// O(max|K|^2), for ranking)
-__device__ void eig_refine(const Tile &Hin, Tile &U, Tile &Ut, int N, cd *buf, double small_tol = 1e-8,
-                           bool ortho = true, bool herm = false, double *lam_out = nullptr)
-{
-    const int c = lane_c(), g = lane_g();
-    Tile H = Hin;
-    if (!herm) {
-        const Tile T = transpose(Hin, buf);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            H.re[r] = 0.5 * (Hin.re[r] + T.re[r]);
-            H.im[r] = 0.5 * (Hin.im[r] - T.im[r]);
-        }
-    }
-    Tile W = cmm(U, true, cmm(H, true, U));  // U^dag (H U)
-    double lam_last = 0.0;
-    for (int it = 0; it < 30; ++it) {
-        double lam_r[4], lam_c;
-        diag_bcast(W, lam_r, lam_c);
-        lam_last = lam_c;
-        Tile K;
-        double kmax = 0.0;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int i = g + 4 * r;
-            K.re[r] = 0.0;
-            K.im[r] = 0.0;
-            const double w2 = W.re[r] * W.re[r] + W.im[r] * W.im[r];
-            if (i != c && i < N && c < N && w2 > 0.0) {
-                const double D = lam_c - lam_r[r];
-                const double s = (D > 0.0 || (D == 0.0 && i < c)) ? 1.0 : -1.0;
-                const double inv = 1.0 / (0.5 * D + s * sqrt(0.25 * D * D + w2));
-                K.re[r] = W.re[r] * inv;
-                K.im[r] = W.im[r] * inv;
-                kmax = fmax(kmax, K.re[r] * K.re[r] + K.im[r] * K.im[r]);  // |K|^2 here, the root once below
-            }
-        }
-        kmax = sqrt(wave_max(kmax));
-        if (kmax == 0.0) break;
-        if (kmax > 0.5) {  // far from converged (a cold-like start): damped rotations
-            const double f = 0.5 / kmax;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                K.re[r] *= f;
-                K.im[r] *= f;
-            }
-        }
-        Tile V;
-        const bool small = kmax < small_tol;
-        if (small) {  // I + K: the neglected K^2 / 2 is below 1e-16
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                V.re[r] = K.re[r] + (g + 4 * r == c ? 1.0 : 0.0);
-                V.im[r] = K.im[r];
-            }
-        } else {  // I + K + K^2/2, unitary to |K|^4 / 4; K^T's tile is -conj(K)
-            Tile Kn;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                Kn.re[r] = -K.re[r];
-                Kn.im[r] = -K.im[r];
-            }
-            const Tile K2 = cmm(Kn, true, K);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                V.re[r] = K.re[r] + 0.5 * K2.re[r] + (g + 4 * r == c ? 1.0 : 0.0);
-                V.im[r] = K.im[r] + 0.5 * K2.im[r];
-            }
-        }
-        U = cmm(Ut, false, V);  // U V
-        Ut = transpose(U, buf);
-        if (small) break;
-        if (kmax > 1e-3) {  // V far from unitary: restore U fully, then W from H itself
-            for (int q = 0; q < 8; ++q)
-                if (orthonormalize(U, Ut, buf) < 1e-8) break;
-            W = cmm(U, true, cmm(H, true, U));
-        } else {
-            W = cmm(V, true, cmm(W, true, V));  // V^dag (W V)
-        }
-    }
-    if (ortho) orthonormalize(U, Ut, buf);
-    if (lam_out) *lam_out = lam_last;
-}
-
-// ------------------------------------------------------------- RK stage --
-// The band-diagonal part of y, U diag(U^dag y U) U^dag, and this lane's column
-// of its diagonal d = (U^dag y U)_cc (two products)
-__device__ __forceinline__ Tile band_diag(const Tile &Y, const Tile &U, const Tile &Ut, double &d)
-{
-    const int g = lane_g();
-    const Tile G = cmm(Y, true, U);  // y U
-    d = col_dot(U, G);               // (U^dag y U)_cc
-    Tile Ud;  // (U diag(d))^T's tile: U^T[4kb + g][c] d_{4kb+g}
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const double dr = __shfl(d, 4 * r + g, 64);
-        Ud.re[r] = Ut.re[r] * dr;
-        Ud.im[r] = Ut.im[r] * dr;
-    }
-    return cmm(Ud, false, Ut, true);  // U diag(d) U^dag (B = U^dag: tile conj(U^T))
-}
-
-// The stage derivative at y given H~^T's tile (HERM: H~'s own tile, H~ Hermitian, so
-// that H~^T's tile is its conjugate) and (dephasing on) y's band-diagonal part M:
-// -i(H~ y - (H~ y)^dag) - g2 y - (g1 - g2) M.
-template <bool HERM = false>
-__device__ __forceinline__ Tile stage_derivative_m(const NbArgs &a, const Tile &Y, const Tile &HtT, const Tile &M,
-                                                   cd *buf)
-{
-    const Tile T = cmm(HtT, HERM, Y);  // H~ y
-    const Tile Tt = transpose(T, buf);
-    Tile X;  // -i (T - T^dag)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const double dr = T.re[r] - Tt.re[r], di = T.im[r] + Tt.im[r];
-        X.re[r] = di;
-        X.im[r] = -dr;
-    }
-    if (a.deph) {
-        const double g2 = a.gam2, g12 = a.gam1 - a.gam2;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            X.re[r] -= g2 * Y.re[r] + g12 * M.re[r];
-            X.im[r] -= g2 * Y.im[r] + g12 * M.im[r];
-        }
-    }
-    return X;
-}
-
-// The same with U, U^T given (M formed here when dephasing)
-__device__ __forceinline__ Tile stage_derivative(const NbArgs &a, const Tile &Y, const Tile &HtT, const Tile &U,
-                                                 const Tile &Ut, cd *buf)
-{
-    Tile M{};
-    if (a.deph) {
-        double d;
-        M = band_diag(Y, U, Ut, d);
-    }
-    return stage_derivative_m(a, Y, HtT, M, buf);
-}
 
 // Stage i: y = rho + sum_j dt a_ij k_j; k_i = f(y); after the last stage
 // rho += sum_i dt b_i k_i. PAIR: stage sg and the next stage sg2 at the same
@@ -588,15 +419,6 @@ __device__ __forceinline__ double lane_value(double x, int j)
     const int lo = __builtin_amdgcn_readlane(__double2loint(x), j);
     const int hi = __builtin_amdgcn_readlane(__double2hiint(x), j);
     return __hiloint2double(hi, lo);
-}
-
-__device__ __forceinline__ void axpy_tile(Tile &Y, const Tile &X, double s, const Tile &B)
-{  // Y = B + s X
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        Y.re[r] = fma(s, X.re[r], B.re[r]);
-        Y.im[r] = fma(s, X.im[r], B.im[r]);
-    }
 }
 
 // the refinements' last-round threshold: eigenvector error O(1e-12), one rotation

@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "analytic.hpp"
+#include "analytic_terms.hpp"
 #include "nband.hpp"
 #include "sbe_internal.hpp"
 
@@ -195,6 +196,24 @@ bool nb32_eligible(const sbe_config &cfg, const sbe_model &m)
 // separable passes cost more in launches than they save in arithmetic.
 bool nb32_dense_multi_n(int nr, int64_t nk) { return nr >= 1 && nr <= kNbDenseMultiMaxR && nk <= 1024; }
 
+// The time-fused steps of the analytic classes (nb_evolve_kernel): FP64 LengthWannier, RK4 or
+// RK5, N <= 8, a class that is a short trigonometric sum. ANTELOPE_NB_FUSED=0 and
+// ANTELOPE_NB_LDS=1 keep the separate kernels.
+bool evolve_eligible(const sbe_config &cfg, const sbe_model &m, int64_t nk, AnalyticTerms &t)
+{
+    if (const char *e = std::getenv("ANTELOPE_NB_FUSED"))
+        if (std::atoi(e) == 0) return false;
+    if (const char *e = std::getenv("ANTELOPE_NB_LDS"))
+        if (std::atoi(e) == 1) return false;
+    if (cfg.gauge != SBE_GAUGE_LENGTH_WANNIER || cfg.precision != SBE_PREC_FP64 ||
+        (cfg.rk_order != SBE_RK4 && cfg.rk_order != SBE_RK5_FEHLBERG) || !am::is_analytic(m.kind))
+        return false;
+    sbe_tuning tu{};
+    if (tuning_lookup(cfg, m, nk, tu) && tu.nb_kernels == 2) return false;
+    static_assert(kMaxTerms == kEvolveMaxTerms, "one limit");
+    return analytic_terms(m.kind, m.nband, m.params, t);
+}
+
 // Steps whose Fourier evaluations one batch of launches covers (the fused RK4 steps):
 // at most kNbEvalSteps (a few launches per hundred steps) and about kNbEvalBytes of outputs
 // and scratch, at least one, at most the pulse; ANTELOPE_NB_EVAL_STEPS sets it (the results
@@ -252,6 +271,7 @@ struct NbPlan {
     size_t bytes_box;
     size_t bytes_fused;  // fused steps: four second-pass outputs and the band energies
     size_t bytes_vel;    // time-fused velocity steps: A at the stage times of the whole pulse
+    size_t bytes_evolve; // time-fused analytic steps: coefficients, energies, A and the table of the pulse
     // offsets inside the box buffer: B, T1, T2, E_1..E_3, R map, k map
     size_t off_t1, off_t2, off_e[3], off_r, off_kinv;
 };
@@ -259,7 +279,7 @@ struct NbPlan {
 size_t align256(size_t x) { return (x + 255) / 256 * 256; }
 
 NbPlan nb_plan(int N, int nr, int64_t nk, int64_t nt, int nstage, bool split16, const BoxShape &bx, bool fused,
-               bool vel_fused = false, bool nb32 = false)
+               bool vel_fused = false, bool nb32 = false, int evolve_terms = -1)
 {
     NbPlan p{};
     p.nk_stride = (nk + 63) / 64 * 64;
@@ -270,6 +290,15 @@ NbPlan nb_plan(int N, int nr, int64_t nk, int64_t nt, int nstage, bool split16, 
     int64_t rows = fused ? std::max<int64_t>(p.sample_waves, fused_blocks(bx, g1)) : p.sample_waves;
     if (vel_fused) rows = std::max<int64_t>(rows, N > 16 ? nk : (nk + vel_waves(nk) - 1) / vel_waves(nk));
     p.bytes_vel = vel_fused ? align256(static_cast<size_t>(nt) * 12 * sizeof(double)) : 0;
+    p.bytes_evolve = 0;
+    if (evolve_terms >= 0) {
+        rows = evolve_blocks(N, nk);
+        const int rk = nstage == 4 ? SBE_RK4 : SBE_RK5_FEHLBERG;
+        p.bytes_evolve = align256((2 + 2 * static_cast<size_t>(evolve_terms)) * nn * sizeof(double2)) +
+                         align256(static_cast<size_t>(p.nk_stride) * 8 * sizeof(double)) +
+                         align256(static_cast<size_t>(nt + 1) * evolve_times(rk) * 3 * sizeof(double)) +
+                         align256(static_cast<size_t>(nt + 1) * evolve_row_len(rk, evolve_terms) * sizeof(double));
+    }
     const size_t row = static_cast<size_t>(rows) * p.nv * sizeof(double);
     p.chunk = std::max<int64_t>(1, std::min<int64_t>(nt, static_cast<int64_t>(kNbPartialBytes / row)));
     // e^{ik.R} for the dense sums (also the N <= 32 fused step's one-launch sums); the
@@ -390,6 +419,54 @@ bool box_tables(const sbe_model &m, const std::vector<double> &hk, int64_t nk, c
     return true;
 }
 
+// Device tables of the time-fused analytic steps: the class's coefficients, the energies, A at
+// the distinct times of every step and the table of phases formed from it
+int setup_evolve(sbe_ctx *ctx, const AnalyticTerms &t, char *buf, int nblocks)
+{
+    const NbArgs &a = ctx->nargs;
+    const size_t nn = static_cast<size_t>(a.N) * a.N;
+    const int64_t nt = ctx->laser.nt;
+    const int rk = ctx->cfg.rk_order, times = evolve_times(rk);
+    NbEvolve &e = ctx->evolve;
+    e = NbEvolve{};
+    e.terms.T = t.T;
+    std::memcpy(e.terms.vec, t.vec, sizeof t.vec);
+    std::memcpy(e.terms.grad, t.grad, sizeof t.grad);
+    for (int i = 0; i < t.T; ++i) e.jz = e.jz || t.grad[i][2] != 0.0;
+    std::vector<double> c(t.m0);
+    for (int i = 0; i < t.T; ++i) {
+        c.insert(c.end(), t.p.begin() + 2 * nn * i, t.p.begin() + 2 * nn * (i + 1));
+        c.insert(c.end(), t.q.begin() + 2 * nn * i, t.q.begin() + 2 * nn * (i + 1));
+    }
+    c.insert(c.end(), t.scale.begin(), t.scale.end());
+    const double mid[2][4] = {{ctx->tab.c[1]}, {ctx->tab.c[1], ctx->tab.c[2], ctx->tab.c[3], ctx->tab.c[5]}};
+    std::vector<double> A(static_cast<size_t>(nt + 1) * times * 3);
+    for (int64_t n = 0; n <= nt; ++n) {
+        const double tn = ctx->laser.atmin + ctx->laser.dt * static_cast<double>(n);  // antelope.cpp:299
+        for (int u = 0; u < times; ++u) {
+            double E[3];
+            ctx->laser.eval(u == 0 ? tn : tn + mid[rk == SBE_RK4 ? 0 : 1][u - 1] * ctx->laser.dt,
+                            A.data() + (static_cast<size_t>(n) * times + u) * 3, E);
+        }
+    }
+    char *q = buf;
+    auto take = [&](size_t bytes) { char *r = q; q += align256(bytes); return r; };
+    char *dc = take(c.size() * sizeof(double));
+    e.lam = reinterpret_cast<double *>(take(static_cast<size_t>(a.nk_stride) * 8 * sizeof(double)));
+    double *dA = reinterpret_cast<double *>(take(A.size() * sizeof(double)));
+    double *dtab = reinterpret_cast<double *>(take(static_cast<size_t>(nt + 1) * evolve_row_len(rk, t.T) * sizeof(double)));
+    int rc = hipc(ctx, hipMemcpy(dc, c.data(), c.size() * sizeof(double), hipMemcpyHostToDevice), "upload terms");
+    if (!rc) rc = hipc(ctx, hipMemcpy(dA, A.data(), A.size() * sizeof(double), hipMemcpyHostToDevice), "upload A");
+    if (!rc) rc = hipc(ctx, launch_evolve_table(dA, e.terms, rk, nt + 1, dtab, ctx->stream), "phase table kernel");
+    e.coef = reinterpret_cast<const double2 *>(dc);
+    e.table = dtab;
+    e.nt = nt;
+    e.dt = ctx->laser.dt;
+    e.nblocks = nblocks;
+    ctx->nbe = rc == SBE_OK;
+    return rc;
+}
+
 }  // namespace
 
 size_t nb_footprint(const sbe_config &cfg, const sbe_model &m, int64_t nk, int64_t nt, int nstage)
@@ -399,9 +476,11 @@ size_t nb_footprint(const sbe_config &cfg, const sbe_model &m, int64_t nk, int64
     const bool fused = fused_eligible(cfg, m, nk, bx);
     const bool vfused = vel_fused_eligible(cfg, m, nk);
     const bool f32 = nb32_eligible(cfg, m);
+    AnalyticTerms terms;
+    const int nterms = evolve_eligible(cfg, m, nk, terms) ? terms.T : -1;
     const NbPlan p =
-        nb_plan(m.nband, am::is_analytic(m.kind) ? 0 : m.nrpts, nk, nt, nstage, split16, bx, fused, vfused, f32);
-    return p.bytes_P + p.bytes_rho + p.bytes_mats + p.bytes_k + p.bytes_tab + p.bytes_partials + p.bytes_series +
+        nb_plan(m.nband, am::is_analytic(m.kind) ? 0 : m.nrpts, nk, nt, nstage, split16, bx, fused, vfused, f32, nterms);
+    return p.bytes_evolve + p.bytes_P + p.bytes_rho + p.bytes_mats + p.bytes_k + p.bytes_tab + p.bytes_partials + p.bytes_series +
            p.bytes_split + p.bytes_b64 + p.bytes_box + p.bytes_fused + p.bytes_vel;
 }
 
@@ -474,7 +553,10 @@ int nb_setup(sbe_ctx *ctx)
     const bool fused = fused_eligible(ctx->cfg, m, nk, bx);
     const bool vfused = vel_fused_eligible(ctx->cfg, m, nk);
     const bool f32 = nb32_eligible(ctx->cfg, m);
-    const NbPlan p = nb_plan(N, nr, nk, ctx->laser.nt, ctx->tab.nstage, split16, bx, fused, vfused, f32);
+    AnalyticTerms terms;
+    const bool evolve = evolve_eligible(ctx->cfg, m, nk, terms);
+    const NbPlan p =
+        nb_plan(N, nr, nk, ctx->laser.nt, ctx->tab.nstage, split16, bx, fused, vfused, f32, evolve ? terms.T : -1);
     const size_t nn = static_cast<size_t>(N) * N;
     ctx->nk = nk;
     ctx->nk_stride = p.nk_stride;
@@ -494,6 +576,7 @@ int nb_setup(sbe_ctx *ctx)
     char *boxbuf = p.bytes_box ? nalloc<char>(ctx, p.bytes_box, rc) : nullptr;
     char *fbuf = p.bytes_fused ? nalloc<char>(ctx, p.bytes_fused, rc) : nullptr;
     double *vtab = p.bytes_vel ? nalloc<double>(ctx, p.bytes_vel, rc) : nullptr;
+    char *ebuf = p.bytes_evolve ? nalloc<char>(ctx, p.bytes_evolve, rc) : nullptr;
     if (rc) return rc;
 
     // host copies of the tables: k [nk_stride][3], w, R cartesian, weights, H, r
@@ -692,6 +775,10 @@ int nb_setup(sbe_ctx *ctx)
         ctx->nb32_blocks = static_cast<int>(std::min<int64_t>(nk, kNb32MaxBlocks));
         ctx->nb32 = true;
     }
+
+    ctx->nbe = false;
+    if (ebuf) rc = setup_evolve(ctx, terms, ebuf, evolve_blocks(N, nk));
+    if (rc) return rc;
 
     a.velocity = ctx->velocity ? 1 : 0;
     // e^{ik.R}, then rho(k) from H(k) (A(atmin) = 0)
@@ -1039,8 +1126,31 @@ int nb_run_fused32(sbe_ctx *ctx, int64_t step_begin, int64_t step_end)
 
 }  // namespace
 
+// Analytic classes, N <= 8: the steps of a chunk in one launch
+static int nb_run_evolve(sbe_ctx *ctx, int64_t step_begin, int64_t step_end)
+{
+    const NbArgs &a = ctx->nargs;
+    NbEvolve &e = ctx->evolve;
+    int rc = SBE_OK;
+    for (int64_t c0 = step_begin; c0 < step_end && !rc; c0 += ctx->chunk_steps) {
+        const int64_t n = std::min<int64_t>(ctx->chunk_steps, step_end - c0);
+        e.s0 = c0;
+        e.s1 = c0 + n;
+        rc = hipc(ctx, launch_evolve(a, e, ctx->cfg.rk_order, ctx->nb_rho, ctx->nb_U, ctx->d_partials, ctx->stream),
+                  "step kernel");
+        e.lam_valid = 1;  // the launch leaves the eigenvectors and energies at t_{s1}
+        if (!rc)
+            rc = hipc(ctx, launch_series_reduce(ctx->d_partials, n, e.nblocks, a.nv, ctx->d_series + c0 * a.nv,
+                                                ctx->stream, ctx->nonfinite_d, kNbReduceGroup),
+                      "series kernel");
+        if (!rc) ctx->steps_done = c0 + n;
+    }
+    return rc;
+}
+
 int nb_run(sbe_ctx *ctx, int64_t step_begin, int64_t step_end)
 {
+    if (ctx->nbe) return nb_run_evolve(ctx, step_begin, step_end);
     if (ctx->velocity) return nb_run_velocity(ctx, step_begin, step_end);
     if (ctx->nbf) return nb_run_fused(ctx, step_begin, step_end);
     if (ctx->nb32) return nb_run_fused32(ctx, step_begin, step_end);

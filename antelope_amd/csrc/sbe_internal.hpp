@@ -211,6 +211,9 @@ struct sbe_ctx {
     bool nbv = false;
     const double *nbv_A = nullptr;  // [nt][4][3] A at the RK4 stage times
     int nbv_nblocks = 0, nbv_waves = 8;
+    // time-fused length-gauge steps of the analytic classes (nb_evolve_kernel)
+    bool nbe = false;
+    sbe::NbEvolve evolve{};
     std::string err;
 
     // optional kernel timing: (start, stop) event pairs per kernel class

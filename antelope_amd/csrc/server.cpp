@@ -358,7 +358,7 @@ int sbe_server_step(sbe_server *s)
                     r.status = SBE_ERR_HIP, r.err = "hipEventCreate failed";
             r.slice = std::min(s->slice, r.ctx->chunk_steps);
         } else {
-            if (r.ctx->path == sbe::PathKind::NBand && !(r.ctx->nbf || r.ctx->nb32 || r.ctx->nbv)) {
+            if (r.ctx->path == sbe::PathKind::NBand && !(r.ctx->nbf || r.ctx->nb32 || r.ctx->nbv || r.ctx->nbe)) {
                 // every N-band step on the separate kernels is a dozen small launches: short
                 // slices keep the hardware queue this request shares with others from filling
                 // with thousands of them (the fused steps take one or two launches per step)

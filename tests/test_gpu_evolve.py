@@ -1,0 +1,83 @@
+"""Time-fused steps of the analytic classes (nb_evolve_kernel) where its tiling can go wrong: one to
+eight bands, k counts around the four-per-wave and block limits, RK4 and RK5, each decay setting, a
+Fermi start, k blocks and runs split into parts. Against the oracle within 1e-10 (the bar of the
+N-band paths) and the same against the separate kernels; split runs give the same bits. The grids keep
+off points where two bands meet exactly (Gamma for the transition-metal and Kane-Mele classes, the line k_x = 0 with
+spin-orbit, planes through Gamma for WDSM_TaAs): there the band basis, and so the dephasing and the band populations,
+is the eigensolver's choice and the two paths differ with rounding / gap."""
+import numpy as np
+import pytest
+
+from antelope_amd import AnalyticModel, SBESolver, query_footprint, tmdc
+from tests.cases import rel_l2, small_config
+
+pytestmark = pytest.mark.gpu
+
+
+def _models():
+    return {
+        "wilson": AnalyticModel.from_reference("WilsonMass", t=0.02, delta=0.03, mu=-0.015, a0=4.0, a1=5.5),
+        "mos2": tmdc("MoS2"),
+        "kanemele": AnalyticModel.from_reference("KaneMele", t1=0.075, t2=0.025, tR=0.01, Mt2=1.5, phi0=0.9, a0=1.42),
+        "wdsm": AnalyticModel.from_reference("WDSM_TaAs", t=0.02, delta=0.5, my=0.8, mz=0.9, a0=3.4),
+        "wse2_soc": tmdc("WSe2", soc=True),
+    }
+
+
+def _run(cfg, m, cuts=(), **kw):
+    with SBESolver(cfg, m, **kw) as s:
+        for c in cuts:
+            s.run(s.info.steps_done, c)
+        s.run()
+        out = s.series()
+        out["state"] = s.state()
+        return out
+
+
+CASES = [
+    # name, k grid, tableau, T1, T2, init
+    ("wilson", (1, 1), 4, 0.0, 0.0, "uniform"),
+    ("wilson", (3, 1), 5, 120.0, 90.0, "uniform"),
+    ("mos2", (5, 2), 4, 0.0, 150.0, "uniform"),
+    ("mos2", (17, 2), 5, 200.0, 0.0, "fermi"),
+    ("kanemele", (4, 4), 5, 150.0, 150.0, "uniform"),
+    ("kanemele", (9, 8), 4, 300.0, 150.0, "uniform"),
+    ("wdsm", (4, 4, 2), 5, 0.0, 150.0, "uniform"),
+    ("wse2_soc", (2, 1), 5, 0.0, 0.0, "uniform"),
+    ("wse2_soc", (4, 2), 4, 200.0, 100.0, "fermi"),
+    ("wse2_soc", (6, 1), 5, 0.0, 100.0, "uniform"),
+]
+
+
+@pytest.mark.parametrize("name,n,rk,T1,T2,init", CASES)
+def test_evolve(oracle, monkeypatch, name, n, rk, T1, T2, init):
+    m = _models()[name]
+    cfg = small_config(n=n, ncycles=0.5, ellip=0.3, rk=rk, T1=T1, T2=T2, grid="mp", init=init, fermi_energy=0.02)
+    print(name, n, rk, flush=True)
+    ref = oracle.run(cfg, m, nthreads=8, want_state=True)
+    got = _run(cfg, m)
+    split = _run(cfg, m, cuts=(1, 2, 130))
+    with monkeypatch.context() as mp:
+        mp.setenv("ANTELOPE_NB_FUSED", "0")
+        sep = _run(cfg, m)
+        foot_sep = query_footprint(cfg, m)
+    for key in ("j_inter", "j_intra", "band_pop", "rho_bar", "state"):
+        assert np.array_equal(got[key], split[key]), key
+        if np.linalg.norm(ref[key]) == 0.0:
+            continue
+        e, es = rel_l2(got[key], ref[key]), rel_l2(got[key], sep[key])
+        print(f"  {key}: oracle {e:.1e}, separate kernels {es:.1e}", flush=True)
+        assert e < 1e-10 and es < 1e-10, key
+    assert query_footprint(cfg, m) != foot_sep
+    with SBESolver(cfg, m) as s:
+        assert s.info.device_bytes == query_footprint(cfg, m)
+
+
+def test_evolve_k_blocks(oracle):
+    """Two k blocks' sums add up to the whole grid's."""
+    m = _models()["kanemele"]
+    cfg = small_config(n=(5, 6), ncycles=0.5, ellip=0.3, rk=5, T2=150.0, grid="mp")
+    whole = _run(cfg, m)
+    a, b = _run(cfg, m, k_begin=0, k_end=11), _run(cfg, m, k_begin=11, k_end=30)
+    for key in ("j_inter", "j_intra", "band_pop", "rho_bar"):
+        assert rel_l2(a[key] + b[key], whole[key]) < 1e-11, key
