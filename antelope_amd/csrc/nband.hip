@@ -328,13 +328,13 @@ __global__ __launch_bounds__(256) void nb_box_pass_multi_kernel(const NbArgs a, 
     (void)K1;
 }
 
-// evaluation e of a run of RK4 steps (NbBoxSteps): its A, E, matrices and outputs
+// evaluation e of a run of RK steps (NbBoxSteps): its A, E, matrices and outputs
 __device__ __forceinline__ NbEval box_step_eval(const NbBoxSteps &d, int e, cd *&t2)
 {
-    const int sl = e / 3, typ = e - 3 * sl;
+    const int ntyp = d.mids + 2, sl = e / ntyp, typ = e - ntyp * sl;
     const int64_t step = d.s0 + sl;
     NbEval ev{};
-    const double *lt = d.laser + (step * 3 + typ) * 6;
+    const double *lt = d.laser + (step * ntyp + typ) * 6;
     for (int i = 0; i < 3; ++i) {
         ev.A[i] = lt[i];
         ev.E[i] = lt[3 + i];
@@ -349,7 +349,8 @@ __device__ __forceinline__ NbEval box_step_eval(const NbBoxSteps &d, int e, cd *
         ev.nmat = 2;
         ev.mats[0] = kMatHtilde;
         ev.mats[1] = kMatH0;
-        t2 = typ == 1 ? d.th + sl * d.t2_stride : d.ring + (step % d.nring) * d.t2_stride;
+        t2 = typ <= d.mids ? d.th + (static_cast<int64_t>(sl) * d.mids + typ - 1) * d.t2_stride
+                           : d.ring + (step % d.nring) * d.t2_stride;
     }
     return ev;
 }
@@ -1734,7 +1735,7 @@ static void box_steps_pass(const NbArgs &a, const NbBoxSteps &d, int64_t maxcols
     const int M1 = a.boxM[0], M2 = a.boxM[1], K2 = a.boxK[1], K3 = a.boxK[2];
     const int K = PASS == 0 ? K3 : K2;
     const int64_t outer = PASS == 0 ? static_cast<int64_t>(M1) * M2 : M1, inner = PASS == 0 ? 1 : K3;
-    const int64_t nev = 3 * static_cast<int64_t>(d.ns);
+    const int64_t nev = (d.mids + 2) * static_cast<int64_t>(d.ns);
     const int64_t xy = outer * inner * ((maxcols + 255) / 256) * nev;
     const int kc = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(K, K * xy / 2048)));
     const int nz = (K + kc - 1) / kc;
@@ -1755,12 +1756,13 @@ static void box_steps_pass_m(const NbArgs &a, const NbBoxSteps &d, int64_t maxco
 
 hipError_t nb_launch_box_steps(const NbArgs &a, const NbBoxSteps &d, hipStream_t s)
 {
-    if (!a.box || a.split16 || a.dzero || d.ns < 1 || d.nring < 1 || d.s0 < 0 || 3 * static_cast<int64_t>(d.ns) > 65535)
+    if (!a.box || a.split16 || a.dzero || d.ns < 1 || d.nring < 1 || d.s0 < 0 || d.mids < 1 ||
+        (d.mids + 2) * static_cast<int64_t>(d.ns) > 65535)
         return hipErrorInvalidValue;
     const int64_t maxcols = 3 * static_cast<int64_t>(a.N) * a.N;
     const int64_t ncells = static_cast<int64_t>(a.boxM[0]) * a.boxM[1] * a.boxM[2];
     nb_box_steps_bform_kernel<<<dim3(static_cast<unsigned>((ncells * maxcols + 255) / 256), 1,
-                                     static_cast<unsigned>(3 * d.ns)),
+                                     static_cast<unsigned>((d.mids + 2) * d.ns)),
                                 256, 0, s>>>(a, d, ncells);
     box_steps_pass_m<0>(a, d, maxcols, s);
     box_steps_pass_m<1>(a, d, maxcols, s);

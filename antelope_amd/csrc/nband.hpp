@@ -107,16 +107,17 @@ hipError_t nb_launch_box_t2(const NbArgs &a, const NbEval &ev, double2 *t2, hipS
 // [cells][bcols], t1 [M1][M2][K3][bcols] and output t2
 hipError_t nb_launch_box_t2_multi(const NbArgs &a, int nev, const NbEval *evs, double2 *const *b, double2 *const *t1,
                                   double2 *const *t2, hipStream_t s);
-// The separable sums up to the second pass for a run of RK4 steps [s0, s0 + ns) in three
-// launches (bform, the passes along a3 and a2), evaluation e = 3 sl + typ: typ 0 J at t_n
-// into tj + sl t2_stride, typ 1 H~ H at t_n + dt/2 into th + sl t2_stride, typ 2 H~ H at
-// t_n + dt into ring + (step mod nring) t2_stride (the pair of the step before s0 stays in the
-// ring when nring > ns); per evaluation scratch b + e b_stride, t1 + e t1_stride. laser:
-// [nt][3][6], A and E at t_n, t_n + dt/2, t_n + dt.
+// The separable sums up to the second pass for a run of RK steps [s0, s0 + ns) in three
+// launches (bform, the passes along a3 and a2), evaluation e = (mids + 2) sl + typ: typ 0 J at
+// t_n into tj + sl t2_stride, typ 1..mids H~ H at the tableau's times between t_n and t_n + dt
+// (RK4: dt/2; RK5: dt/4, 3dt/8, 12dt/13, dt/2) into th + (mids sl + typ - 1) t2_stride, the last
+// H~ H at t_n + dt into ring + (step mod nring) t2_stride (the pair of the step before s0 stays
+// in the ring when nring > ns); per evaluation scratch b + e b_stride, t1 + e t1_stride. laser:
+// [nt][mids + 2][6], A and E at t_n, the times between and t_n + dt.
 struct NbBoxSteps {
     const double *laser;
     int64_t s0;
-    int ns, nring;
+    int ns, nring, mids;
     double2 *b, *t1, *tj, *th, *ring;
     int64_t b_stride, t1_stride, t2_stride;  // elements
 };
@@ -210,6 +211,23 @@ int evolve_blocks(int N, int64_t nk);
 hipError_t launch_evolve_table(const double *A, const EvolveTerms &t, int rk_order, int64_t rows, double *tab, hipStream_t s);
 hipError_t launch_evolve(const NbArgs &a, const NbEvolve &e, int rk_order, double2 *rho, double2 *U, double *partials,
                          hipStream_t s);
+
+// The same for Wannier models with N <= 8 on the separable Fourier sums: steps [s0, s0 + ns),
+// whose second-pass outputs are in place (NbBoxSteps), one partial row per block and step.
+struct NbBoxRun {
+    const double2 *tj, *th, *ring;
+    int64_t t2_stride;
+    int nring, ns;
+    int64_t s0, row0;      // row0: the first step's row of the partial sums
+    int jz;                // any z current
+    double dt;
+    int nblocks;
+    double *lam;           // [nk_stride][16]
+    int lam_valid;
+};
+int box_evolve_blocks(int N, const int K[3]);
+hipError_t launch_box_evolve(const NbArgs &a, const NbBoxRun &e, int rk_order, double2 *rho, double2 *U, double *partials,
+                             hipStream_t s);
 
 // One time step of the VelocityHamiltonian gauge: A at the stage times and
 // the tableau (coefficients already multiplied by dt).

@@ -1,19 +1,25 @@
-// nband_evolve.hip - time-fused LengthWannier steps of the analytic classes
-// (N <= 8), classical RK4 and fixed-step RK5: one launch runs every step of a
-// chunk with rho, the eigenvectors and the model in registers.
+// nband_evolve.hip - time-fused LengthWannier steps for N <= 8, classical RK4 and
+// fixed-step RK5: one launch runs every step it has matrices for, with rho and
+// the eigenvectors in registers.
 //
 // The reference's step (SBEs.h:596-624, stage right-hand side :762-861, sample
 // :694-760) on the register tiles of tile_small.hpp: N <= 4 takes four k points
-// per wave, N <= 8 one, one matrix element per lane. H(k + A(t)) and J are
-// trigonometric sums (analytic_terms.hpp): a lane keeps its element's
-// coefficients p_t, q_t turned by e^{ik.v_t} once per launch, so a stage's H is
-// 4 FMAs per term against the k-independent cos / sin(A.v_t) of a table row, and
-// nothing of a step touches HBM but the row of k sums.
+// per wave, N <= 8 one, one matrix element per lane. The matrices come from a
+// source:
+//  * AnalyticSource: H(k + A(t)) and J are trigonometric sums (analytic_terms.hpp).
+//    A lane keeps its element's coefficients p_t, q_t turned by e^{ik.v_t} once per
+//    launch, so a stage's H is 4 FMAs per term against the k-independent
+//    cos / sin(A.v_t) of a table row; a launch covers a chunk of the pulse.
+//  * BoxSource: the second-pass outputs of the separable Fourier sums of a run of
+//    steps (nb_launch_box_steps); the last pass, X = sum_m E1[k1][m] T2[m], is
+//    M1 complex multiply-adds per element here, its rows loaded one evaluation
+//    ahead into registers.
 //
 // Bound by latency: a wave's step is one serial chain of small products (the
 // eigenvector refinements above all), so the split that pays is many waves with
-// little in each. 64 x 48 k points, bilayer Haldane (4 bands), RK5, 502 steps:
-// see the figures at launch_evolve.
+// little in each. Measured over 502 steps: bilayer Haldane (4 bands), 64 x 48 k,
+// RK5: 5.2 ms in one launch against 123 ms in 7,000 launches of the 16x16-tile stage,
+// sample and model kernels; MoS2 (3 bands), 72 x 72 k, RK4: 4.6 ms against 103 ms.
 #include <cmath>
 
 #include "haldane_dev.hpp"
@@ -26,6 +32,15 @@ using namespace tile;
 using dev::Coef;
 
 constexpr int kWaves = 4;  // waves per block: one partial row per block and step
+
+// what the step loop needs beside the source: steps [s0, s1), the first step's row of the partial
+// sums, the energies [k][lam_pitch]
+struct EvolveRun {
+    int64_t s0, s1, row0;
+    double dt;
+    double *lam;
+    int lam_pitch, lam_valid;
+};
 
 // doubles per table row: at t_n H's (cos, sin) pairs and, times the gradients,
 // those of J_x, J_y, J_z; then H's pairs at the tableau's other distinct times
@@ -99,50 +114,59 @@ __device__ __forceinline__ double ranked_population(double lam, double p, int N)
     return out;
 }
 
+// ------------------------------------------------------------ sources --
+// Per wave: which k point and element a lane works for, and the matrices of the
+// current step. herm(): H~ is Hermitian and equal to H. pair(u): H~^T's tile (the
+// commutator's A operand) and H at the u-th of the tableau's later distinct times
+// (the last, u = mids, is t_n + dt); issue(u) / issue_j() start the loads the next
+// pair / currents will need.
 template <int Q, int RK, int NT>
-__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))) void nb_evolve_kernel(
-    const NbArgs a, const NbEvolve e, cd *__restrict__ rho, cd *__restrict__ Ust, double *__restrict__ partials)
-{
+struct AnalyticSource {
     using T = SmallTile<Q>;
-    constexpr int KW = Q == 1 ? 4 : 1;  // k points per wave
-    constexpr int R = row_len<RK, NT>();
+    static constexpr bool kHerm = true;
+    static constexpr int R = row_len<RK, NT>(), kMids = mid_times<RK>();
     static_assert(R <= 64 * kWaves, "a row is fetched by one thread per value");
-    extern __shared__ double evolve_lds[];
-    double *rows = evolve_lds;                  // [3][R]: table rows n, n + 1, n + 2 by n mod 3
-    double *sums = evolve_lds + 3 * R;          // [2][kWaves][nv]
-    const int N = a.N, nn = N * N, nv = a.nv;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int i = Shape<T>::row(0), c = Shape<T>::col(), b = (lane >> 2) & 3;
-    const int64_t k = (static_cast<int64_t>(blockIdx.x) * kWaves + w) * KW + (KW == 4 ? b : 0);
-    const bool valid = k < a.nk;  // lanes past the block's k points repeat the last one with weight 0
-    const int64_t kk = valid ? k : a.nk - 1;
-    const double wk = valid ? a.weight[kk] : 0.0;
-    const bool in = i < N && c < N;
-    const int el = in ? i * N + c : 0;
-
-    // this element's coefficients, turned by the phases of k
+    const NbEvolve &e;
+    double *rows;  // LDS [3][R]: table rows n, n + 1, n + 2 by n mod 3
     double pr[NT], pi[NT], qr[NT], qi[NT];
-    const double kx = a.kpts[3 * kk], ky = a.kpts[3 * kk + 1], kz = a.kpts[3 * kk + 2];
-    const cd zero = make_double2(0.0, 0.0);
+    cd m0, sc;
+    int sl, sn, sf;  // slots of this step's row and the next two
+    bool fetch = false;
+    double ahead = 0.0;
+
+    __device__ AnalyticSource(const NbArgs &a, const NbEvolve &ev, double *lds, int64_t kk, bool in, int el)
+        : e(ev), rows(lds)
+    {
+        const double kx = a.kpts[3 * kk], ky = a.kpts[3 * kk + 1], kz = a.kpts[3 * kk + 2];
+        const int nn = a.N * a.N;
+        const cd zero = make_double2(0.0, 0.0);
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        double s = 0.0, co = 0.0;
-        cd p = zero, q = zero;
-        if (t < e.terms.T) {
-            sincos(kx * e.terms.vec[t][0] + ky * e.terms.vec[t][1] + kz * e.terms.vec[t][2], &s, &co);
-            if (in) {
-                p = e.coef[(1 + 2 * t) * nn + el];
-                q = e.coef[(2 + 2 * t) * nn + el];
+        for (int t = 0; t < NT; ++t) {
+            double s = 0.0, co = 0.0;
+            cd p = zero, q = zero;
+            if (t < e.terms.T) {
+                sincos(kx * e.terms.vec[t][0] + ky * e.terms.vec[t][1] + kz * e.terms.vec[t][2], &s, &co);
+                if (in) {
+                    p = e.coef[(1 + 2 * t) * nn + el];
+                    q = e.coef[(2 + 2 * t) * nn + el];
+                }
             }
+            pr[t] = p.x * co + q.x * s;
+            pi[t] = p.y * co + q.y * s;
+            qr[t] = q.x * co - p.x * s;
+            qi[t] = q.y * co - p.y * s;
         }
-        pr[t] = p.x * co + q.x * s;
-        pi[t] = p.y * co + q.y * s;
-        qr[t] = q.x * co - p.x * s;
-        qi[t] = q.y * co - p.y * s;
+        m0 = in ? e.coef[el] : zero;
+        sc = in ? e.coef[(1 + 2 * e.terms.T) * nn + el] : zero;
+        for (int x = threadIdx.x; x < 2 * R; x += 64 * kWaves)
+            rows[((e.s0 + x / R) % 3) * R + x % R] = e.table[e.s0 * R + x];
+        __syncthreads();
+        sl = static_cast<int>(e.s0 % 3);
+        sn = sl == 2 ? 0 : sl + 1;
+        sf = sn == 2 ? 0 : sn + 1;
     }
-    const cd m0 = in ? e.coef[el] : zero, sc = in ? e.coef[(1 + 2 * e.terms.T) * nn + el] : zero;
-    auto hmat = [&](const double *r) {
+    __device__ T hmat(const double *r) const
+    {
         T H;
         double x = m0.x, y = m0.y;
 #pragma unroll
@@ -154,8 +178,18 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
         H.re[0] = x;
         H.im[0] = y;
         return H;
-    };
-    auto jmat = [&](const double *r, double &jr, double &ji) {  // r: the axis's gradient pairs
+    }
+    __device__ void start(T &Ht, T &H) { Ht = H = hmat(rows + sl * R); }
+    __device__ void begin(int64_t step)
+    {
+        fetch = threadIdx.x < R && step + 2 <= e.nt;
+        ahead = fetch ? e.table[(step + 2) * R + threadIdx.x] : 0.0;
+    }
+    __device__ void current(int ax, double &jr, double &ji) const
+    {
+        jr = ji = 0.0;
+        if (ax == 2 && !e.jz) return;
+        const double *r = rows + sl * R + (2 + 2 * ax) * NT;
         double x = 0.0, y = 0.0;
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
@@ -165,43 +199,152 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
         }
         jr = sc.x * x - sc.y * y;
         ji = sc.x * y + sc.y * x;
-    };
-
-    T Rh, U, Ut;
+    }
+    // past the step's barrier every wave has left step n - 1, whose slot takes row n + 2
+    __device__ void after_barrier()
     {
-        const cd v = in ? rho[kk * nn + el] : zero;
-        const cd u = in ? Ust[kk * nn + el] : make_double2(i == c ? 1.0 : 0.0, 0.0);
+        if (fetch) rows[sf * R + threadIdx.x] = ahead;
+    }
+    __device__ void issue(int) {}
+    __device__ void issue_j(int64_t) {}
+    __device__ void pair(int u, T &Ht, T &H) { Ht = H = hmat(u < kMids ? rows + sl * R + (8 + 2 * u) * NT : rows + sn * R); }
+    __device__ void advance()
+    {
+        sl = sn;
+        sn = sf;
+        sf = sn == 2 ? 0 : sn + 1;
+    }
+};
+
+template <int Q, int RK, int MM>
+struct BoxSource {
+    using T = SmallTile<Q>;
+    static constexpr bool kHerm = false;
+    static constexpr int kMids = mid_times<RK>();
+    const NbBoxRun &e;
+    const bool jz;
+    int64_t off, nn, mstride;  // this lane's element in a second-pass output, per matrix and per row m
+    int M1;
+    cd w[MM];                  // E1[k1][m], 0 past M1, off the matrix and for holes of the k box
+    cd raw[3 * MM];
+    int64_t step = 0;
+
+    __device__ BoxSource(const NbArgs &a, const NbBoxRun &ev, int k1, int64_t col, bool on, int el)
+        : e(ev), jz(ev.jz != 0), nn(a.N * a.N), M1(a.boxM[0])
+    {
+        mstride = static_cast<int64_t>(a.boxK[1]) * a.boxK[2] * a.bcols;
+        off = col * a.bcols + el;
+#pragma unroll
+        for (int m = 0; m < MM; ++m)
+            w[m] = on && m < M1 ? a.boxE[0][static_cast<int64_t>(k1) * M1 + m] : make_double2(0.0, 0.0);
+    }
+    __device__ const cd *ring(int64_t s) const
+    {
+        return e.ring + ((s % e.nring + e.nring) % e.nring) * e.t2_stride;
+    }
+    __device__ void load(const cd *src, int n)
+    {
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+            if (j < n)
+#pragma unroll
+                for (int m = 0; m < MM; ++m) raw[j * MM + m] = src[off + j * nn + (m < M1 ? m : 0) * mstride];
+    }
+    __device__ cd form(int j) const
+    {
+        double re = 0.0, im = 0.0;
+#pragma unroll
+        for (int m = 0; m < MM; ++m) {
+            const cd x = raw[j * MM + m];
+            re = fma(w[m].x, x.x, fma(-w[m].y, x.y, re));
+            im = fma(w[m].x, x.y, fma(w[m].y, x.x, im));
+        }
+        return make_double2(re, im);
+    }
+    __device__ void take(T &Ht, T &H)
+    {
+        const cd t = form(0), h = form(1);
+        T X;
+        X.re[0] = t.x, X.im[0] = t.y;
+        H.re[0] = h.x, H.im[0] = h.y;
+        Ht = transpose(X, nullptr);  // H~ need not be Hermitian: its transpose, not its conjugate
+    }
+    __device__ void start(T &Ht, T &H)
+    {
+        load(ring(e.s0 - 1), 2);
+        take(Ht, H);
+        step = e.s0;
+        issue_j(step);
+    }
+    __device__ void begin(int64_t s) { step = s; }
+    __device__ void issue_j(int64_t s)
+    {
+        if (s < e.s0 + e.ns) load(e.tj + (s - e.s0) * e.t2_stride, jz ? 3 : 2);
+    }
+    __device__ void current(int ax, double &jr, double &ji) const
+    {
+        jr = ji = 0.0;
+        if (ax == 2 && !jz) return;
+        const cd v = form(ax);
+        jr = v.x;
+        ji = v.y;
+    }
+    __device__ void after_barrier() {}
+    __device__ void issue(int u)
+    {
+        load(u < kMids ? e.th + ((step - e.s0) * kMids + u) * e.t2_stride : ring(step), 2);
+    }
+    __device__ void pair(int, T &Ht, T &H) { take(Ht, H); }
+    __device__ void advance() {}
+};
+
+// ---------------------------------------------------------------- steps --
+// Steps [s0, s1) of the lane's k point kk (valid: the block's, else a stand-in of
+// weight 0 that is not stored): rho, the eigenvectors and the energies in, and out.
+// on: the element is inside the N x N matrix. sums: LDS [2][kWaves][nv].
+template <int Q, int RK, class SRC>
+__device__ __forceinline__ void evolve_steps(const NbArgs &a, SRC &src, const EvolveRun &e, int64_t kk, bool valid, bool in,
+                                             bool load, double *sums, cd *__restrict__ rho, cd *__restrict__ Ust,
+                                             double *__restrict__ partials)
+{
+    using T = SmallTile<Q>;
+    constexpr int KW = Q == 1 ? 4 : 1, kMids = mid_times<RK>();
+    const int N = a.N, nn = N * N, nv = a.nv;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i = Shape<T>::row(0), c = Shape<T>::col(), b = (lane >> 2) & 3;
+    const int el = in ? i * N + c : 0;
+    const double wk = valid ? a.weight[kk] : 0.0;
+    cd *const none = nullptr;
+
+    T Rh, U, Ut, Ht, H;
+    {
+        const cd v = in && load ? rho[kk * nn + el] : make_double2(0.0, 0.0);
+        const cd u = in && load ? Ust[kk * nn + el] : make_double2(i == c ? 1.0 : 0.0, 0.0);
         Rh.re[0] = v.x, Rh.im[0] = v.y;
         U.re[0] = u.x, U.im[0] = u.y;
-        Ut = transpose(U, nullptr);
+        Ut = transpose(U, none);
     }
-    for (int x = tid; x < 2 * R; x += 64 * kWaves) rows[((e.s0 + x / R) % 3) * R + x % R] = e.table[e.s0 * R + x];
-    __syncthreads();
-    int sl = static_cast<int>(e.s0 % 3);  // this step's row slot
-    T H = hmat(rows + sl * R);            // at t_n, carried from step to step
+    src.start(Ht, H);  // at t_n; carried from step to step
     double lam = 0.0;
-    if (e.lam_valid) lam = e.lam[kk * 8 + c];
-    else eig_refine(H, U, Ut, N, static_cast<cd *>(nullptr), 1e-8, true, true, &lam);
+    if (e.lam_valid) lam = load ? e.lam[kk * e.lam_pitch + c] : 0.0;
+    else eig_refine(H, U, Ut, N, none, 1e-8, true, SRC::kHerm, &lam);
 
     const double dt = e.dt, g12 = a.gam1 - a.gam2;
     const bool deph = a.deph != 0;
     // the band-diagonal part enters the dephasing only where T1 and T2 differ
-    auto deriv = [&](const T &Y, const T &Hs, const T &V, const T &Vt) {
+    auto deriv = [&](const T &Y, const T &Hc, const T &V, const T &Vt) {
         T M{};
         double d;
         if (deph && g12 != 0.0) M = band_diag(Y, V, Vt, d);
-        return stage_derivative_m<true>(a, Y, Hs, M, static_cast<cd *>(nullptr));
+        return stage_derivative_m<SRC::kHerm>(a, Y, Hc, M, none);
     };
     auto refine = [&](const T &Hs, T &V, T &Vt) {
-        if (deph && g12 != 0.0) eig_refine(Hs, V, Vt, N, static_cast<cd *>(nullptr), 1e-8, true, true);
+        if (deph && g12 != 0.0) eig_refine(Hs, V, Vt, N, none, 1e-8, true, SRC::kHerm);
     };
 
     for (int64_t step = e.s0; step < e.s1; ++step) {
-        const double *row = rows + sl * R;
-        const int sn = sl == 2 ? 0 : sl + 1, sf = sn == 2 ? 0 : sn + 1;  // slots of the next two rows
-        const double *next = rows + sn * R;
-        const bool fetch = tid < R && step + 2 <= e.nt;
-        const double ahead = fetch ? e.table[(step + 2) * R + tid] : 0.0;
+        src.begin(step);
         // ---- sample at t_n
         double pc;
         const T M = band_diag(Rh, U, Ut, pc);
@@ -209,14 +352,15 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
         v[6] = v[7] = 0.0;
 #pragma unroll
         for (int ax = 0; ax < 3; ++ax) {
-            double jr = 0.0, ji = 0.0;
-            if (ax < 2 || e.jz) jmat(row + (2 + 2 * ax) * NT, jr, ji);
+            double jr, ji;
+            src.current(ax, jr, ji);
             // Re Tr(rho J) = Re sum conj(rho_ij) J_ij and the same with rho's band-diagonal part
             const double tot = Rh.re[0] * jr + Rh.im[0] * ji;
             const double intra = a.inter_intra ? M.re[0] * jr + M.im[0] * ji : 0.0;
-            v[ax] = (tot - intra) * wk;
-            v[3 + ax] = intra * wk;
+            v[ax] = in ? (tot - intra) * wk : 0.0;
+            v[3 + ax] = in ? intra * wk : 0.0;
         }
+        src.issue(0);
         double *mine = sums + ((step & 1) * kWaves + w) * nv;
         {
             const double cur = dev::wave_reduce8(v);
@@ -238,38 +382,41 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
                 mine[6 + N + 2 * el + 1] = ri;
             }
         }
-        // one barrier a step: past it every wave has left step n - 1, whose row slot takes row n + 2,
-        // and the sums written before it are added below while the other buffer takes step n + 1's
+        // one barrier a step: the sums written before it are added below while the other buffer
+        // takes the next step's
         __syncthreads();
-        if (fetch) rows[sf * R + tid] = ahead;
+        src.after_barrier();
         {
-            double *out = partials + ((step - e.s0) * gridDim.x + blockIdx.x) * static_cast<int64_t>(nv);
+            double *out = partials + (e.row0 + step - e.s0) * static_cast<int64_t>(gridDim.x) * nv +
+                          static_cast<int64_t>(blockIdx.x) * nv;
             const double *s = sums + (step & 1) * kWaves * nv;
             for (int x = tid; x < nv; x += 64 * kWaves) out[x] = ((s[x] + s[nv + x]) + s[2 * nv + x]) + s[3 * nv + x];
         }
         // ---- stages
-        T X = stage_derivative_m<true>(a, Rh, H, M, static_cast<cd *>(nullptr));
+        T X = stage_derivative_m<SRC::kHerm>(a, Rh, Ht, M, none);
         if constexpr (RK == 4) {
             T Acc, Y;
             axpy_tile(Acc, X, dt / 6.0, Rh);
             axpy_tile(Y, X, 0.5 * dt, Rh);
-            H = hmat(row + 8 * NT);
+            src.pair(0, Ht, H);
+            src.issue(kMids);
             refine(H, U, Ut);
-            X = deriv(Y, H, U, Ut);
+            X = deriv(Y, Ht, U, Ut);
             axpy_tile(Acc, X, dt / 3.0, Acc);
             axpy_tile(Y, X, 0.5 * dt, Rh);
-            X = deriv(Y, H, U, Ut);
+            X = deriv(Y, Ht, U, Ut);
             axpy_tile(Acc, X, dt / 3.0, Acc);
             axpy_tile(Y, X, dt, Rh);
-            H = hmat(next);
-            eig_refine(H, U, Ut, N, static_cast<cd *>(nullptr), 1e-8, true, true, &lam);
-            X = deriv(Y, H, U, Ut);
+            src.pair(kMids, Ht, H);
+            src.issue_j(step + 1);
+            eig_refine(H, U, Ut, N, none, 1e-8, true, SRC::kHerm, &lam);
+            X = deriv(Y, Ht, U, Ut);
             axpy_tile(Rh, X, dt / 6.0, Acc);
         } else {
             // c = 0, 1/4, 3/8, 12/13, 1, 1/2: the last stage starts its eigenvectors from those at
             // 3/8, the step's own go on to the next sample
             using C = Coef<5>;
-            T Kd[6], Vm, Vmt, Hs;
+            T Kd[6], Vm, Vmt, Hc;
             Kd[0] = X;
             auto input = [&](int s) {
                 T Y = Rh;
@@ -278,34 +425,84 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))
                     if (j < s && C::a[s][j] != 0.0) axpy_tile(Y, Kd[j], dt * C::a[s][j], Y);
                 return Y;
             };
-            Hs = hmat(row + 8 * NT);
-            refine(Hs, U, Ut);
-            Kd[1] = deriv(input(1), Hs, U, Ut);
-            Hs = hmat(row + 10 * NT);
-            refine(Hs, U, Ut);
-            Kd[2] = deriv(input(2), Hs, U, Ut);
+            src.pair(0, Hc, H);
+            src.issue(1);
+            refine(H, U, Ut);
+            Kd[1] = deriv(input(1), Hc, U, Ut);
+            src.pair(1, Hc, H);
+            src.issue(2);
+            refine(H, U, Ut);
+            Kd[2] = deriv(input(2), Hc, U, Ut);
             Vm = U;
             Vmt = Ut;
-            Hs = hmat(row + 12 * NT);
-            refine(Hs, U, Ut);
-            Kd[3] = deriv(input(3), Hs, U, Ut);
-            H = hmat(next);
-            eig_refine(H, U, Ut, N, static_cast<cd *>(nullptr), 1e-8, true, true, &lam);
-            Kd[4] = deriv(input(4), H, U, Ut);
-            Hs = hmat(row + 14 * NT);
-            refine(Hs, Vm, Vmt);
-            Kd[5] = deriv(input(5), Hs, Vm, Vmt);
+            src.pair(2, Hc, H);
+            src.issue(kMids);
+            refine(H, U, Ut);
+            Kd[3] = deriv(input(3), Hc, U, Ut);
+            src.pair(kMids, Ht, H);
+            src.issue(3);
+            eig_refine(H, U, Ut, N, none, 1e-8, true, SRC::kHerm, &lam);
+            Kd[4] = deriv(input(4), Ht, U, Ut);
+            src.pair(3, Hc, H);
+            src.issue_j(step + 1);
+            refine(H, Vm, Vmt);
+            Kd[5] = deriv(input(5), Hc, Vm, Vmt);
 #pragma unroll
             for (int j = 0; j < 6; ++j)
                 if (C::b[j] != 0.0) axpy_tile(Rh, Kd[j], dt * C::b[j], Rh);
         }
-        sl = sn;
+        src.advance();
     }
     if (valid && in) {
-        rho[k * nn + el] = make_double2(Rh.re[0], Rh.im[0]);
-        Ust[k * nn + el] = make_double2(U.re[0], U.im[0]);
+        rho[kk * nn + el] = make_double2(Rh.re[0], Rh.im[0]);
+        Ust[kk * nn + el] = make_double2(U.re[0], U.im[0]);
     }
-    if (valid && i == 0) e.lam[k * 8 + c] = lam;
+    if (valid && i == 0) e.lam[kk * e.lam_pitch + c] = lam;
+}
+
+template <int Q, int RK, int NT>
+__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))) void nb_evolve_kernel(
+    const NbArgs a, const NbEvolve e, cd *__restrict__ rho, cd *__restrict__ Ust, double *__restrict__ partials)
+{
+    using T = SmallTile<Q>;
+    extern __shared__ double evolve_lds[];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int64_t unit = static_cast<int64_t>(blockIdx.x) * kWaves + w;
+    const int64_t k = Q == 1 ? unit * 4 + ((lane >> 2) & 3) : unit;
+    const bool valid = k < a.nk;  // lanes past the last k point repeat it with weight 0
+    const int64_t kk = valid ? k : a.nk - 1;
+    const int i = Shape<T>::row(0), c = Shape<T>::col();
+    const bool in = i < a.N && c < a.N;
+    AnalyticSource<Q, RK, NT> src(a, e, evolve_lds, kk, in, in ? i * a.N + c : 0);
+    const EvolveRun run{e.s0, e.s1, 0, e.dt, e.lam, 8, e.lam_valid};
+    evolve_steps<Q, RK>(a, src, run, kk, valid, in, true, evolve_lds + 3 * row_len<RK, NT>(), rho, Ust, partials);
+}
+
+// Wannier models on a product k grid: a wave's k points differ along a1 (one (k2, k3)
+// column, so its second-pass rows are shared), neighbouring units run along a1 too
+template <int Q, int RK, int MM>
+__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2))) void nb_box_evolve_kernel(
+    const NbArgs a, const NbBoxRun e, cd *__restrict__ rho, cd *__restrict__ Ust, double *__restrict__ partials)
+{
+    using T = SmallTile<Q>;
+    extern __shared__ double evolve_lds[];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int K1 = a.boxK[0], K2 = a.boxK[1], K3 = a.boxK[2];
+    const int g1 = Q == 1 ? (K1 + 3) / 4 : K1;  // units per column
+    const int64_t unit = static_cast<int64_t>(blockIdx.x) * kWaves + w;
+    const int64_t ncol = static_cast<int64_t>(K2) * K3;
+    const bool there = unit < g1 * ncol;
+    const int64_t col = there ? unit / g1 : 0;
+    const int g = there ? static_cast<int>(unit - col * g1) : 0;
+    const int k1 = Q == 1 ? 4 * g + ((lane >> 2) & 3) : g;
+    // a k block of the grid leaves holes in its box (k map -1): zero matrices, nothing stored
+    const int64_t kmap = there && k1 < K1 ? a.box_kinv[(static_cast<int64_t>(k1) * K2 * K3) + col] : -1;
+    const bool valid = kmap >= 0;
+    const int i = Shape<T>::row(0), c = Shape<T>::col();
+    const bool in = i < a.N && c < a.N;
+    BoxSource<Q, RK, MM> src(a, e, valid ? k1 : 0, col, valid && in, in ? i * a.N + c : 0);
+    const EvolveRun run{e.s0, e.s0 + e.ns, e.row0, e.dt, e.lam, 16, e.lam_valid};
+    evolve_steps<Q, RK>(a, src, run, valid ? kmap : 0, valid, in, valid, evolve_lds, rho, Ust, partials);
 }
 
 template <int Q, int RK, int NT>
@@ -332,7 +529,37 @@ hipError_t launch_rk(const NbArgs &a, const NbEvolve &e, double2 *rho, double2 *
     }
 }
 
+template <int Q, int RK>
+hipError_t launch_box(const NbArgs &a, const NbBoxRun &e, double2 *rho, double2 *U, double *partials, hipStream_t s)
+{
+    const size_t lds = sizeof(double) * 2 * kWaves * a.nv;
+    const dim3 grid(static_cast<unsigned>(e.nblocks));
+    if (a.boxM[0] <= 3) nb_box_evolve_kernel<Q, RK, 3><<<grid, 64 * kWaves, lds, s>>>(a, e, rho, U, partials);
+    else if (a.boxM[0] <= 5) nb_box_evolve_kernel<Q, RK, 5><<<grid, 64 * kWaves, lds, s>>>(a, e, rho, U, partials);
+    else nb_box_evolve_kernel<Q, RK, 7><<<grid, 64 * kWaves, lds, s>>>(a, e, rho, U, partials);
+    return hipGetLastError();
+}
+
 }  // namespace
+
+int box_evolve_blocks(int N, const int K[3])
+{
+    const int64_t units = static_cast<int64_t>(N <= 4 ? (K[0] + 3) / 4 : K[0]) * K[1] * K[2];
+    return static_cast<int>((units + kWaves - 1) / kWaves);
+}
+
+hipError_t launch_box_evolve(const NbArgs &a, const NbBoxRun &e, int rk_order, double2 *rho, double2 *U, double *partials,
+                             hipStream_t s)
+{
+    if (!a.box || a.N < 1 || a.N > 8 || a.boxM[0] > kNbFusedMaxM1 || e.ns < 1 || e.nring < 1 || e.s0 < 0 ||
+        e.nblocks != box_evolve_blocks(a.N, a.boxK))
+        return hipErrorInvalidValue;
+    if (rk_order == SBE_RK4)
+        return a.N <= 4 ? launch_box<1, 4>(a, e, rho, U, partials, s) : launch_box<2, 4>(a, e, rho, U, partials, s);
+    if (rk_order == SBE_RK5_FEHLBERG)
+        return a.N <= 4 ? launch_box<1, 5>(a, e, rho, U, partials, s) : launch_box<2, 5>(a, e, rho, U, partials, s);
+    return hipErrorInvalidValue;
+}
 
 int evolve_blocks(int N, int64_t nk)
 {

@@ -163,6 +163,18 @@ bool fused_eligible(const sbe_config &cfg, const sbe_model &m, int64_t nk, const
     return true;  // the whole grid, or a k block of it (holes in the box are idle waves)
 }
 
+// RK5 (Fehlberg) steps of small Wannier models (nb_box_evolve_kernel): as fused_eligible with
+// N <= 8. The plan does not depend on ANTELOPE_NB_FUSED, which only selects the kernels that run.
+bool rk5_small_eligible(const sbe_config &cfg, const sbe_model &m, int64_t nk, const BoxShape &bx)
+{
+    if (!bx.ok || cfg.rk_order != SBE_RK5_FEHLBERG || cfg.gauge != SBE_GAUGE_LENGTH_WANNIER ||
+        cfg.precision != SBE_PREC_FP64 || am::is_analytic(m.kind) || m.is_dipole_zero || m.nband > 8 ||
+        bx.M[0] > kNbFusedMaxM1)
+        return false;
+    sbe_tuning tu{};
+    return !(tuning_lookup(cfg, m, nk, tu) && tu.nb_kernels == 2);
+}
+
 // The time-fused velocity-gauge steps (nb16_vel_fused_kernel for N <= 16 on the
 // register-tile kernels, nb32_vel_fused_kernel for 16 < N <= 32 up to kNb32VelMaxK k
 // points, one block per k point): FP64 with the classical RK4 tableau; any model (the step
@@ -228,11 +240,40 @@ int64_t eval_steps(size_t bytes_per_step, int64_t nt)
     return std::max<int64_t>(1, std::min<int64_t>(nt, S));
 }
 
-// N <= 16: the separable passes up to the second of three evaluations per step (at most
-// 21845 steps: three evaluations a step in one grid dimension)
-int nb16_steps_per_eval(size_t t2, size_t b, size_t t1, int64_t nt)
+// N <= 16: the separable passes up to the second of a step's evaluations (RK4 three, RK5 six),
+// all in one grid dimension of at most 65535. RK4 keeps them in a buffer of its own; RK5, whose
+// plan also holds the separate kernels' stage derivatives, puts them there where that holds at
+// least kNbEvalInK steps, else in a buffer of at most kNbEvalBytes5, else there again, so that
+// its footprint grows by no more than that (0 steps: neither holds one).
+constexpr int64_t kNbEvalInK = 8;
+constexpr size_t kNbEvalBytes5 = size_t(64) << 20;
+struct FusedEval {
+    int S = 0;            // steps per batch of launches
+    int mids = 1;         // evaluation times between t_n and t_n + dt
+    bool in_k = false;    // RK5: the outputs and scratch live in the stage-derivative slots
+    size_t t2 = 0, b = 0, t1 = 0;  // bytes per evaluation: second-pass output, B, first-pass output
+    size_t bytes() const { return (static_cast<size_t>(mids + 2) * S + 1) * t2 + static_cast<size_t>(mids + 2) * S * (b + t1); }
+};
+FusedEval fused_eval(const BoxShape &bx, int64_t bcols, int64_t nt, int nstage, size_t bytes_rho)
 {
-    return static_cast<int>(std::min<int64_t>(eval_steps(3 * (t2 + b + t1), nt), 21845));
+    FusedEval f;
+    const size_t col = sizeof(double2) * static_cast<size_t>(bcols);
+    f.t2 = (col * bx.M[0] * bx.K[1] * bx.K[2] + 255) / 256 * 256;
+    f.b = (col * static_cast<size_t>(bx.cells()) + 255) / 256 * 256;
+    f.t1 = (col * bx.M[0] * bx.M[1] * bx.K[2] + 255) / 256 * 256;
+    const size_t per = f.t2 + f.b + f.t1;
+    if (nstage == 4) {
+        f.S = static_cast<int>(std::min<int64_t>(eval_steps(3 * per, nt), 21845));
+        return f;
+    }
+    f.mids = 4;
+    const int64_t want = std::min<int64_t>(eval_steps(1, nt), 10922);  // the switch or the step limit alone
+    const size_t k_bytes = static_cast<size_t>(nstage) * bytes_rho;
+    const int64_t in_k = k_bytes > f.t2 ? static_cast<int64_t>((k_bytes - f.t2) / (6 * per)) : 0;
+    const int64_t own = static_cast<int64_t>(kNbEvalBytes5 / (6 * per));
+    f.in_k = in_k >= std::min(want, kNbEvalInK) || own < 1;
+    f.S = static_cast<int>(std::min(want, f.in_k ? in_k : own));
+    return f;
 }
 
 // 16 < N <= 32, one dense launch: seven N x N matrices per k point and step
@@ -269,7 +310,8 @@ struct NbPlan {
     int64_t bcols;
     size_t bytes_P, bytes_rho, bytes_mats, bytes_k, bytes_tab, bytes_partials, bytes_series, bytes_split, bytes_b64;
     size_t bytes_box;
-    size_t bytes_fused;  // fused steps: four second-pass outputs and the band energies
+    size_t bytes_fused;  // fused steps: second-pass outputs, scratch, band energies, A and E
+    FusedEval fe;
     size_t bytes_vel;    // time-fused velocity steps: A at the stage times of the whole pulse
     size_t bytes_evolve; // time-fused analytic steps: coefficients, energies, A and the table of the pulse
     // offsets inside the box buffer: B, T1, T2, E_1..E_3, R map, k map
@@ -288,6 +330,7 @@ NbPlan nb_plan(int N, int nr, int64_t nk, int64_t nt, int nstage, bool split16, 
     const size_t nn = static_cast<size_t>(N) * N;
     int g1 = 0;
     int64_t rows = fused ? std::max<int64_t>(p.sample_waves, fused_blocks(bx, g1)) : p.sample_waves;
+    if (fused && N <= 8) rows = std::max<int64_t>(p.sample_waves, box_evolve_blocks(N, bx.K));
     if (vel_fused) rows = std::max<int64_t>(rows, N > 16 ? nk : (nk + vel_waves(nk) - 1) / vel_waves(nk));
     p.bytes_vel = vel_fused ? align256(static_cast<size_t>(nt) * 12 * sizeof(double)) : 0;
     p.bytes_evolve = 0;
@@ -339,15 +382,12 @@ NbPlan nb_plan(int N, int nr, int64_t nk, int64_t nt, int nstage, bool split16, 
         p.bytes_box = o;
     }
     p.bytes_fused = 0;
-    if (fused) {  // second-pass outputs of S steps (J, the midpoint pair, the end pairs in a ring
-        // of S + 1), the energies, per evaluation B and the first pass, A and E of the pulse
-        const size_t col = sizeof(double2) * static_cast<size_t>(p.bcols);
-        const size_t t2 = align256(col * bx.M[0] * bx.K[1] * bx.K[2]);
-        const size_t b = align256(col * static_cast<size_t>(bx.cells()));
-        const size_t t1 = align256(col * bx.M[0] * bx.M[1] * bx.K[2]);
-        const size_t S = static_cast<size_t>(nb16_steps_per_eval(t2, b, t1, nt));
-        p.bytes_fused = (3 * S + 1) * t2 + align256(static_cast<size_t>(p.nk_stride) * 16 * sizeof(double)) +
-                        3 * S * (b + t1) + align256(static_cast<size_t>(nt) * 18 * sizeof(double));
+    if (fused) {  // per batch of S steps J, the pairs between and the end pairs in a ring of S + 1,
+        // per evaluation B and the first pass; the energies; A and E of the pulse
+        p.fe = fused_eval(bx, p.bcols, nt, nstage, p.bytes_rho);
+        if (p.fe.S >= 1)
+            p.bytes_fused = (p.fe.in_k ? 0 : p.fe.bytes()) + align256(static_cast<size_t>(p.nk_stride) * 16 * sizeof(double)) +
+                            align256(static_cast<size_t>(nt) * (p.fe.mids + 2) * 6 * sizeof(double));
     }
     if (nb32) {  // the energies, and with the separable sums per evaluation B and both passes
         p.bytes_fused = align256(static_cast<size_t>(p.nk_stride) * 32 * sizeof(double));
@@ -473,7 +513,7 @@ size_t nb_footprint(const sbe_config &cfg, const sbe_model &m, int64_t nk, int64
 {
     const bool split16 = cfg.precision == SBE_PREC_SPLIT16;
     const BoxShape bx = box_shape(cfg, m, nk, split16);
-    const bool fused = fused_eligible(cfg, m, nk, bx);
+    const bool fused = fused_eligible(cfg, m, nk, bx) || rk5_small_eligible(cfg, m, nk, bx);
     const bool vfused = vel_fused_eligible(cfg, m, nk);
     const bool f32 = nb32_eligible(cfg, m);
     AnalyticTerms terms;
@@ -550,7 +590,7 @@ int nb_setup(sbe_ctx *ctx)
     const int64_t nk = ctx->grid.k_end - ctx->grid.k_begin;
     const bool split16 = ctx->cfg.precision == SBE_PREC_SPLIT16;
     const BoxShape bx = box_shape(ctx->cfg, m, nk, split16);
-    const bool fused = fused_eligible(ctx->cfg, m, nk, bx);
+    const bool fused = fused_eligible(ctx->cfg, m, nk, bx) || rk5_small_eligible(ctx->cfg, m, nk, bx);
     const bool vfused = vel_fused_eligible(ctx->cfg, m, nk);
     const bool f32 = nb32_eligible(ctx->cfg, m);
     AnalyticTerms terms;
@@ -688,36 +728,43 @@ int nb_setup(sbe_ctx *ctx)
         }
     }
 
-    // fused RK4 steps: the planned grid must have grouped into the whole box (every node one k point)
+    // fused RK steps: the planned grid must have grouped into the whole box (every node one k point)
     ctx->nbf = false;
-    if (fbuf && a.box && a.tile16 && nb16_step_lds_bytes(N, bx.M[0], a.nv, fused_waves(bx)) <= (size_t(160) << 10)) {
-        const size_t col = sizeof(double2) * static_cast<size_t>(p.bcols);
-        const size_t t2 = align256(col * bx.M[0] * bx.K[1] * bx.K[2]);
-        const size_t b = align256(col * static_cast<size_t>(bx.cells()));
-        const size_t t1 = align256(col * bx.M[0] * bx.M[1] * bx.K[2]);
+    ctx->nbf_small = fused && N <= 8;
+    const char *sw = std::getenv("ANTELOPE_NB_FUSED");
+    const bool off = sw && std::atoi(sw) == 0;
+    if (fbuf && fused && p.fe.S >= 1 && !off && a.box && a.tile16 &&
+        (ctx->nbf_small || nb16_step_lds_bytes(N, bx.M[0], a.nv, fused_waves(bx)) <= (size_t(160) << 10))) {
+        const FusedEval &fe = p.fe;
         const int64_t nt = ctx->laser.nt;
-        const int S = nb16_steps_per_eval(t2, b, t1, nt);
-        char *q = fbuf;
-        ctx->nbf_S = S;
-        ctx->nbf_t2_stride = static_cast<int64_t>(t2 / sizeof(double2));
+        const size_t S = static_cast<size_t>(fe.S), types = static_cast<size_t>(fe.mids) + 2;
+        char *q = fe.in_k ? reinterpret_cast<char *>(ctx->nb_k) : fbuf;
+        ctx->nbf_S = fe.S;
+        ctx->nbf_mids = fe.mids;
+        ctx->nbf_t2_stride = static_cast<int64_t>(fe.t2 / sizeof(double2));
         ctx->nbf_tj = reinterpret_cast<double2 *>(q);
-        ctx->nbf_th = reinterpret_cast<double2 *>(q + S * t2);
-        ctx->nbf_ring = reinterpret_cast<double2 *>(q + 2 * S * t2);
-        q += (3 * static_cast<size_t>(S) + 1) * t2;
+        ctx->nbf_th = reinterpret_cast<double2 *>(q + S * fe.t2);
+        ctx->nbf_ring = reinterpret_cast<double2 *>(q + (1 + fe.mids) * S * fe.t2);
+        q += (types * S + 1) * fe.t2;
+        ctx->nbf_bs = reinterpret_cast<double2 *>(q);
+        ctx->nbf_b_stride = static_cast<int64_t>(fe.b / sizeof(double2));
+        q += types * S * fe.b;
+        ctx->nbf_t1s = reinterpret_cast<double2 *>(q);
+        ctx->nbf_t1_stride = static_cast<int64_t>(fe.t1 / sizeof(double2));
+        q += types * S * fe.t1;
+        if (fe.in_k) q = fbuf;
         ctx->nbf_lam = reinterpret_cast<double *>(q);
         q += align256(static_cast<size_t>(p.nk_stride) * 16 * sizeof(double));
-        ctx->nbf_bs = reinterpret_cast<double2 *>(q);
-        ctx->nbf_b_stride = static_cast<int64_t>(b / sizeof(double2));
-        q += 3 * static_cast<size_t>(S) * b;
-        ctx->nbf_t1s = reinterpret_cast<double2 *>(q);
-        ctx->nbf_t1_stride = static_cast<int64_t>(t1 / sizeof(double2));
-        q += 3 * static_cast<size_t>(S) * t1;
         double *lt = reinterpret_cast<double *>(q);
-        std::vector<double> hl(static_cast<size_t>(nt) * 18);
+        std::vector<double> hl(static_cast<size_t>(nt) * types * 6);
+        const double mid5[4] = {ctx->tab.c[1], ctx->tab.c[2], ctx->tab.c[3], ctx->tab.c[5]};
         for (int64_t n = 0; n < nt; ++n) {  // the times of the step loop's evaluations
             const double tn = ctx->laser.atmin + ctx->laser.dt * static_cast<double>(n);  // antelope.cpp:299
-            const double ts[3] = {tn, tn + 0.5 * ctx->laser.dt, tn + ctx->laser.dt};
-            for (int j = 0; j < 3; ++j) ctx->laser.eval(ts[j], hl.data() + 18 * n + 6 * j, hl.data() + 18 * n + 6 * j + 3);
+            for (size_t j = 0; j < types; ++j) {
+                const double c = j == 0 ? 0.0 : (j == types - 1 ? 1.0 : (fe.mids == 1 ? 0.5 : mid5[j - 1]));
+                double *o = hl.data() + 6 * (types * n + j);
+                ctx->laser.eval(tn + c * ctx->laser.dt, o, o + 3);
+            }
         }
         rc = hipc(ctx, hipMemcpy(lt, hl.data(), hl.size() * sizeof(double), hipMemcpyHostToDevice), "upload laser");
         if (rc) return rc;
@@ -725,7 +772,8 @@ int nb_setup(sbe_ctx *ctx)
         // blocks over the k points' own box (a k block of the grid may span fewer k1, k2, k3)
         ctx->nbf_waves = fused_waves(bx);
         ctx->nbf_g1 = (a.boxK[0] + ctx->nbf_waves - 1) / ctx->nbf_waves;
-        ctx->nbf_nblocks = ctx->nbf_g1 * a.boxK[1] * a.boxK[2];
+        ctx->nbf_nblocks = ctx->nbf_small ? box_evolve_blocks(N, a.boxK) : ctx->nbf_g1 * a.boxK[1] * a.boxK[2];
+        for (int r = 0; r < nr; ++r) ctx->nbf_jz = ctx->nbf_jz || hr[3 * r + 2] != 0.0;
         ctx->nbf = true;
     }
     ctx->nbf_prev_valid = false;
@@ -907,8 +955,8 @@ int nb_run_velocity(sbe_ctx *ctx, int64_t step_begin, int64_t step_end)
 
 namespace {
 
-// LengthWannier RK4 steps as one nb16_step_kernel launch each (after the
-// Fourier passes of the step's times)
+// LengthWannier RK steps after the Fourier passes of a batch of steps' times: N <= 8 one launch
+// for the batch (nb_box_evolve_kernel), N <= 16 one nb16_step_kernel launch per step
 int nb_run_fused(sbe_ctx *ctx, int64_t step_begin, int64_t step_end)
 {
     const NbArgs &a = ctx->nargs;
@@ -940,6 +988,7 @@ int nb_run_fused(sbe_ctx *ctx, int64_t step_begin, int64_t step_end)
             d.s0 = step0;
             d.ns = ns;
             d.nring = nring;
+            d.mids = ctx->nbf_mids;
             d.b = ctx->nbf_bs;
             d.t1 = ctx->nbf_t1s;
             d.tj = ctx->nbf_tj;
@@ -949,6 +998,30 @@ int nb_run_fused(sbe_ctx *ctx, int64_t step_begin, int64_t step_end)
             d.t1_stride = ctx->nbf_t1_stride;
             d.t2_stride = t2s;
             if (!rc) rc = hipc(ctx, nb_launch_box_steps(a, d, ctx->stream), "fourier passes");
+            if (ctx->nbf_small && !rc) {  // every step of the batch in one launch
+                NbBoxRun f{};
+                f.tj = ctx->nbf_tj;
+                f.th = ctx->nbf_th;
+                f.ring = ctx->nbf_ring;
+                f.t2_stride = t2s;
+                f.nring = nring;
+                f.ns = ns;
+                f.s0 = step0;
+                f.row0 = s;
+                f.jz = ctx->nbf_jz ? 1 : 0;
+                f.dt = dt;
+                f.nblocks = ctx->nbf_nblocks;
+                f.lam = ctx->nbf_lam;
+                f.lam_valid = same_time(ctx->nb_u_time, t0, dt) && ctx->nbf_lam_valid && same_time(ctx->nbf_lam_time, t0, dt);
+                rc = hipc(ctx, launch_box_evolve(a, f, ctx->cfg.rk_order, ctx->nb_rho, ctx->nb_U, ctx->d_partials, ctx->stream),
+                          "step kernel");
+                const double t1 = ctx->laser.atmin + dt * static_cast<double>(step0 + ns - 1) + dt;
+                ctx->nbf_prev_time = ctx->nb_u_time = ctx->nbf_lam_time = t1;
+                ctx->nbf_prev_valid = ctx->nbf_lam_valid = true;
+                ctx->nb_ht_valid = ctx->nb_h_valid = false;
+                s += ns;
+                continue;
+            }
             for (int i = 0; i < ns && !rc; ++i) {
                 const int64_t step = step0 + i;
                 const double tn = ctx->laser.atmin + dt * static_cast<double>(step);

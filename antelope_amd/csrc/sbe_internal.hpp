@@ -178,6 +178,9 @@ struct sbe_ctx {
     bool nb_vel_p_lds = false;   // velocity gauge: pMatrix of the k point staged in LDS
     // fused RK4 steps (nb16_step_kernel): second-pass outputs of the separable sums
     bool nbf = false;
+    bool nbf_small = false;  // N <= 8: nb_box_evolve_kernel
+    bool nbf_jz = false;     // any lattice vector with a z component
+    int nbf_mids = 1;        // evaluation times between t_n and t_n + dt
     // second-pass outputs of up to nbf_S steps: J at t_n and H~ H at t_n + dt/2 per step, the
     // end pairs H~ H at t_n + dt in a ring of nbf_S + 1 (step mod ring)
     int nbf_S = 0;

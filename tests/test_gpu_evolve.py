@@ -8,7 +8,8 @@ is the eigensolver's choice and the two paths differ with rounding / gap."""
 import numpy as np
 import pytest
 
-from antelope_amd import AnalyticModel, SBESolver, query_footprint, tmdc
+from antelope_amd import AnalyticModel, Pulse, RunConfig, SBESolver, query_footprint, tmdc
+from antelope_amd.models import synthetic_wannier
 from tests.cases import rel_l2, small_config
 
 pytestmark = pytest.mark.gpu
@@ -81,3 +82,50 @@ def test_evolve_k_blocks(oracle):
     a, b = _run(cfg, m, k_begin=0, k_end=11), _run(cfg, m, k_begin=11, k_end=30)
     for key in ("j_inter", "j_intra", "band_pop", "rho_bar"):
         assert rel_l2(a[key] + b[key], whole[key]) < 1e-11, key
+
+
+BOX_CASES = [
+    # bands, R range, k grid, tableau, T1, T2, InterIntra
+    (1, (1, 1, 0), (7, 6, 1), 4, 0.0, 80.0, True),
+    (2, (1, 1, 0), (512, 2, 1), 5, 150.0, 80.0, True),  # RK5 scratch in the stage-derivative slots
+    (3, (2, 2, 1), (5, 4, 3), 5, 0.0, 80.0, True),
+    (4, (3, 1, 0), (13, 6, 1), 4, 120.0, 60.0, True),
+    (4, (1, 2, 1), (4, 7, 4), 5, 0.0, 0.0, False),
+    (5, (3, 2, 0), (9, 11, 1), 5, 90.0, 90.0, True),
+    (7, (2, 1, 1), (6, 5, 3), 4, 0.0, 0.0, True),
+    (8, (2, 2, 0), (14, 11, 1), 5, 200.0, 80.0, True),
+]
+
+
+@pytest.mark.parametrize("N,nmax,npts,rk,T1,T2,ii", BOX_CASES)
+def test_box_evolve(oracle, monkeypatch, N, nmax, npts, rk, T1, T2, ii):
+    """Wannier models with N <= 8 (nb_box_evolve_kernel), positions not Hermitian (H~ = H + E.D is
+    used as a general matrix), against the oracle, the separate kernels, split runs and k blocks."""
+    m = synthetic_wannier(N, nmax=nmax, seed=70 + N)
+    m.pos = m.pos * (1.0 + 0.3j)
+    cfg = RunConfig(npoints=list(npts), pulses=[Pulse(E0=0.01, w0=0.05, ncycles=0.25, ellip=0.4, envelope="sin2")],
+                    dt=0.5, T1=T1, T2=T2, rk_order=rk, inter_intra=ii)
+    print(N, nmax, npts, rk, flush=True)
+    ref = oracle.run(cfg, m, nthreads=8, want_state=True)
+    got = _run(cfg, m)
+    split = _run(cfg, m, cuts=(1, 2, 40))
+    nk = int(np.prod(npts))
+    cut = nk // 2 + 1
+    blocks = [_run(cfg, m, k_begin=a, k_end=b) for a, b in ((0, cut), (cut, nk))]
+    with monkeypatch.context() as mp:
+        mp.setenv("ANTELOPE_NB_EVAL_STEPS", "3")
+        three = _run(cfg, m)
+        mp.setenv("ANTELOPE_NB_FUSED", "0")
+        sep = _run(cfg, m)
+    for key in ("j_inter", "j_intra", "band_pop", "rho_bar", "state"):
+        assert np.array_equal(got[key], split[key]), key
+        assert np.array_equal(got[key], three[key]), key
+        if np.linalg.norm(ref[key]) == 0.0:
+            continue
+        e, es = rel_l2(got[key], ref[key]), rel_l2(got[key], sep[key])
+        print(f"  {key}: oracle {e:.1e}, separate kernels {es:.1e}", flush=True)
+        assert e < 1e-10 and es < 1e-10, key
+        if key != "state":
+            assert rel_l2(blocks[0][key] + blocks[1][key], ref[key]) < 1e-10, key
+    with SBESolver(cfg, m) as s:
+        assert s.info.device_bytes == query_footprint(cfg, m)
