@@ -165,20 +165,20 @@ struct NbStep32 {
 hipError_t nb32_launch_step(const NbArgs &a, const NbStep32 &f, int nblocks, double2 *rho, double2 *U, double *partials,
                             hipStream_t s);
 
-// Time-fused VelocityHamiltonian steps for N <= 16 with the classical RK4 tableau
-// (nb16_vel_fused_kernel): one wave per k point for steps [s0, s1), one partial row
-// per block of kNbFusedWaves k points and step.
+// Time-fused VelocityHamiltonian steps for N <= 16, RK4 or RK5 (nb_vel_fused_kernel):
+// steps [s0, s1) in one launch, one partial row per block and step.
 struct NbVelFused {
-    const double *A;  // [nt][4][3]: A(t_n + c_s dt)
+    const double *A;  // [nt][stages][3]: A(t_n + c_s dt)
     int64_t s0, s1;
     double dt;
-    int nblocks;      // partial rows per step: ceil(nk / waves) for N <= 16, nk above
-    int waves;        // N <= 16: k points per block, 8, or 4 where 8 gives fewer blocks than CUs
+    int nblocks;      // partial rows per step: vel_fused_blocks for N <= 16, nk above
+    int waves;        // N <= 16: vel_fused_waves
 };
-size_t nb16_vel_fused_lds_bytes(int nv, int waves);
-hipError_t nb16_launch_vel_fused(const NbArgs &a, const NbVelFused &f, const double2 *P, const double *Eocc,
-                                 double2 *rho, double *partials, hipStream_t s);
-// the same for 16 < N <= 32: one block of four waves per k point (nblocks = nk)
+int vel_fused_waves(int N, int64_t nk);
+int64_t vel_fused_blocks(int N, int64_t nk);
+hipError_t nb_launch_vel_fused(const NbArgs &a, const NbVelFused &f, int rk_order, const double2 *P, const double *Eocc,
+                               double2 *rho, double *partials, hipStream_t s);
+// the same for 16 < N <= 32, RK4: one block of four waves per k point (nblocks = nk)
 constexpr int64_t kNb32VelMaxK = 1024;
 hipError_t nb32_launch_vel_fused(const NbArgs &a, const NbVelFused &f, const double2 *P, const double *Eocc,
                                  double2 *rho, double *partials, hipStream_t s);

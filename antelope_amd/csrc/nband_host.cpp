@@ -175,17 +175,17 @@ bool rk5_small_eligible(const sbe_config &cfg, const sbe_model &m, int64_t nk, c
     return !(tuning_lookup(cfg, m, nk, tu) && tu.nb_kernels == 2);
 }
 
-// The time-fused velocity-gauge steps (nb16_vel_fused_kernel for N <= 16 on the
-// register-tile kernels, nb32_vel_fused_kernel for 16 < N <= 32 up to kNb32VelMaxK k
-// points, one block per k point): FP64 with the classical RK4 tableau; any model (the step
-// has no Fourier sums). ANTELOPE_NB_FUSED=0 keeps one launch per step.
+// The time-fused velocity-gauge steps (nb_vel_fused_kernel for N <= 16, RK4 and RK5;
+// nb32_vel_fused_kernel for 16 < N <= 32, RK4, up to kNb32VelMaxK k points, one block per k
+// point): FP64; any model (the step has no Fourier sums). ANTELOPE_NB_FUSED=0 keeps one
+// launch per step.
 bool vel_fused_eligible(const sbe_config &cfg, const sbe_model &m, int64_t nk)
 {
     if (const char *e = std::getenv("ANTELOPE_NB_FUSED"))
         if (std::atoi(e) == 0) return false;
-    if (cfg.gauge != SBE_GAUGE_VELOCITY_HAMILTONIAN || cfg.rk_order != SBE_RK4 || cfg.precision != SBE_PREC_FP64 ||
-        m.nband > 32 || (m.nband > 16 && nk > kNb32VelMaxK))
-        return false;
+    if (cfg.gauge != SBE_GAUGE_VELOCITY_HAMILTONIAN || cfg.precision != SBE_PREC_FP64 || m.nband > 32) return false;
+    if (cfg.rk_order != SBE_RK4 && !(cfg.rk_order == SBE_RK5_FEHLBERG && m.nband <= 16)) return false;
+    if (m.nband > 16 && nk > kNb32VelMaxK) return false;
     if (const char *e = std::getenv("ANTELOPE_NB_LDS"))
         if (std::atoi(e) == 1) return false;
     sbe_tuning tu{};
@@ -292,9 +292,6 @@ int fused_waves(const BoxShape &bx)
     return b8 < kNbCUs ? 4 : 8;
 }
 
-// the same rule for the time-fused velocity steps (one k point per wave, k in order)
-int vel_waves(int64_t nk) { return (nk + 7) / 8 < kNbCUs ? 4 : 8; }
-
 int fused_blocks(const BoxShape &bx, int &g1)
 {
     const int w = fused_waves(bx);
@@ -331,8 +328,8 @@ NbPlan nb_plan(int N, int nr, int64_t nk, int64_t nt, int nstage, bool split16, 
     int g1 = 0;
     int64_t rows = fused ? std::max<int64_t>(p.sample_waves, fused_blocks(bx, g1)) : p.sample_waves;
     if (fused && N <= 8) rows = std::max<int64_t>(p.sample_waves, box_evolve_blocks(N, bx.K));
-    if (vel_fused) rows = std::max<int64_t>(rows, N > 16 ? nk : (nk + vel_waves(nk) - 1) / vel_waves(nk));
-    p.bytes_vel = vel_fused ? align256(static_cast<size_t>(nt) * 12 * sizeof(double)) : 0;
+    if (vel_fused) rows = std::max<int64_t>(rows, N > 16 ? nk : vel_fused_blocks(N, nk));
+    p.bytes_vel = vel_fused ? align256(static_cast<size_t>(nt) * nstage * 3 * sizeof(double)) : 0;
     p.bytes_evolve = 0;
     if (evolve_terms >= 0) {
         rows = evolve_blocks(N, nk);
@@ -859,20 +856,21 @@ int nb_setup(sbe_ctx *ctx)
         const size_t lds_p = nb_vel_lds_bytes(N, ctx->tab.nstage, true);
         ctx->nb_vel_p_lds = lds_p <= (size_t(64) << 10);
         ctx->nbv = false;
-        if (vtab && (a.tile16 || N > 16)) {  // A at the four RK4 stage times of every step, as the host evaluates them
+        if (vtab && (a.tile16 || N > 16)) {  // A at the stage times of every step, as the host evaluates them
             const int64_t nt = ctx->laser.nt;
-            std::vector<double> hv(static_cast<size_t>(nt) * 12);
+            const int ns = ctx->tab.nstage;
+            std::vector<double> hv(static_cast<size_t>(nt) * ns * 3);
             for (int64_t n = 0; n < nt; ++n) {
                 const double tn = ctx->laser.atmin + ctx->laser.dt * static_cast<double>(n);  // antelope.cpp:299
-                for (int st = 0; st < 4; ++st) {
+                for (int st = 0; st < ns; ++st) {
                     double E[3];
-                    ctx->laser.eval(tn + ctx->tab.c[st] * ctx->laser.dt, hv.data() + 12 * n + 3 * st, E);  // SBEs.h:612
+                    ctx->laser.eval(tn + ctx->tab.c[st] * ctx->laser.dt, hv.data() + 3 * (n * ns + st), E);  // SBEs.h:612
                 }
             }
             if (!rc) rc = hipc(ctx, hipMemcpy(vtab, hv.data(), hv.size() * sizeof(double), hipMemcpyHostToDevice), "upload A");
             ctx->nbv_A = vtab;
-            ctx->nbv_waves = vel_waves(nk);
-            ctx->nbv_nblocks = static_cast<int>(N > 16 ? nk : (nk + ctx->nbv_waves - 1) / ctx->nbv_waves);
+            ctx->nbv_waves = vel_fused_waves(N, nk);
+            ctx->nbv_nblocks = static_cast<int>(N > 16 ? nk : vel_fused_blocks(N, nk));
             ctx->nbv = true;
         }
         if (!rc) rc = hipc(ctx, hipStreamSynchronize(ctx->stream), "init sync");
@@ -914,7 +912,8 @@ int nb_run_velocity(sbe_ctx *ctx, int64_t step_begin, int64_t step_end)
             f.waves = ctx->nbv_waves;
             rc = hipc(ctx,
                       a.N > 16 ? nb32_launch_vel_fused(a, f, Pv, Eocc, ctx->nb_rho, ctx->d_partials, ctx->stream)
-                               : nb16_launch_vel_fused(a, f, Pv, Eocc, ctx->nb_rho, ctx->d_partials, ctx->stream),
+                               : nb_launch_vel_fused(a, f, ctx->cfg.rk_order, Pv, Eocc, ctx->nb_rho, ctx->d_partials,
+                                                     ctx->stream),
                       "velocity step kernel");
             if (!rc)
                 rc = hipc(ctx, launch_series_reduce(ctx->d_partials, n, ctx->nbv_nblocks, a.nv, ctx->d_series + c0 * a.nv,

@@ -210,9 +210,9 @@ struct sbe_ctx {
     int nb32_S = 0;
     double2 *nb32_j = nullptr, *nb32_half = nullptr, *nb32_ring = nullptr;
     const double *nb32_laser = nullptr;  // [nt][3][6] A, E at t_n, t_n + dt/2, t_n + dt
-    // time-fused velocity-gauge steps (nb16_vel_fused_kernel)
+    // time-fused velocity-gauge steps (nb_vel_fused_kernel, nb32_vel_fused_kernel)
     bool nbv = false;
-    const double *nbv_A = nullptr;  // [nt][4][3] A at the RK4 stage times
+    const double *nbv_A = nullptr;  // [nt][stages][3] A at the stage times
     int nbv_nblocks = 0, nbv_waves = 8;
     // time-fused length-gauge steps of the analytic classes (nb_evolve_kernel)
     bool nbe = false;

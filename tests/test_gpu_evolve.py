@@ -129,3 +129,30 @@ def test_box_evolve(oracle, monkeypatch, N, nmax, npts, rk, T1, T2, ii):
             assert rel_l2(blocks[0][key] + blocks[1][key], ref[key]) < 1e-10, key
     with SBESolver(cfg, m) as s:
         assert s.info.device_bytes == query_footprint(cfg, m)
+
+
+@pytest.mark.parametrize("N,npts,rk,T1,T2,ii", [
+    (1, (5, 1, 1), 5, 0.0, 80.0, True),
+    (3, (3, 3, 1), 4, 120.0, 80.0, False),
+    (4, (17, 1, 1), 5, 120.0, 80.0, True),
+    (5, (3, 1, 1), 4, 0.0, 0.0, True),
+    (8, (3, 3, 1), 5, 0.0, 80.0, True),
+    (9, (5, 1, 1), 5, 120.0, 80.0, False),
+    (16, (3, 3, 1), 5, 0.0, 80.0, True),
+])
+def test_velocity_evolve(oracle, monkeypatch, N, npts, rk, T1, T2, ii):
+    """Time-fused velocity-gauge steps (nb_vel_fused_kernel) on each tile size and tableau."""
+    m = synthetic_wannier(N, nmax=(1, 1, 0), seed=50 + N)
+    cfg = RunConfig(npoints=list(npts), pulses=[Pulse(E0=0.01, w0=0.05, ncycles=0.5, ellip=0.4, envelope="sin2")],
+                    dt=0.5, T1=T1, T2=T2, rk_order=rk, inter_intra=ii, gauge="VelocityHamiltonian")
+    print(N, npts, rk, flush=True)
+    ref = oracle.run(cfg, m, nthreads=8)
+    got, split = _run(cfg, m), _run(cfg, m, cuts=(1, 2, 40))
+    with monkeypatch.context() as mp:
+        mp.setenv("ANTELOPE_NB_FUSED", "0")
+        sep = _run(cfg, m)
+    for key in ("j_inter", "j_intra", "band_pop", "rho_bar", "state"):
+        assert np.array_equal(got[key], split[key]), key
+        assert rel_l2(got[key], sep[key]) < 1e-12, key
+        if key != "state":
+            assert rel_l2(got[key], ref[key]) < 1e-10, key
