@@ -28,7 +28,7 @@ ARCH = os.environ.get("ANTELOPE_OFFLOAD_ARCH", "gfx950")
 LIB_SOURCES = [
     "host_setup.cpp", "sbe_api.cpp", "nband_host.cpp", "frontend.cpp", "server.cpp", "wannier_tb.cpp", "atl.cpp", "spectrum.cpp", "tuner.cpp", "material.cpp",
     "analytic_terms.cpp",
-    "haldane.hip", "haldane_velocity.hip", "haldane_adaptive.hip", "nband.hip", "nband16.hip", "nband32.hip", "nband_evolve.hip", "nband_velocity.hip", "analytic.hip", "series.hip", "noalloc.hip",
+    "haldane.hip", "haldane_table.hip", "haldane_velocity.hip", "haldane_adaptive.hip", "nband.hip", "nband16.hip", "nband32.hip", "nband_evolve.hip", "nband_velocity.hip", "analytic.hip", "series.hip", "noalloc.hip",
 ]
 DRIVER = "antelope_mi355x"
 

@@ -88,18 +88,20 @@ bool analytic_terms(int kind, int N, const double *params, AnalyticTerms &out)
                 smp.push_back(std::move(H));
             }
     if (!std::isfinite(hmax)) return false;
+    // e^{-2 pi i m / L} by index modulo L
+    std::vector<cplx> root[3];
+    for (int d = 0; d < 3; ++d)
+        for (int m = 0; m < Ld[d]; ++m)
+            root[d].push_back(std::polar(1.0, -kTwoPi * m / Ld[d]));
     auto coef = [&](int nx, int ny, int nz, int e) {
         cplx s = 0.0;
         size_t q = 0;
+        auto at = [&](int d, int n, int x) { return root[d][((n * x) % Ld[d] + Ld[d]) % Ld[d]]; };
         for (int x = 0; x < Ld[0]; ++x)
-            for (int y = 0; y < Ld[1]; ++y)
-                for (int z = 0; z < Ld[2]; ++z, ++q) {
-                    // the phase index modulo the period: exact multiples of the step angle
-                    const double ph = kTwoPi * ((nx * x % Ld[0]) / static_cast<double>(Ld[0]) +
-                                                (ny * y % Ld[1]) / static_cast<double>(Ld[1]) +
-                                                (nz * z % Ld[2]) / static_cast<double>(Ld[2]));
-                    s += smp[q][e] * cplx(std::cos(ph), -std::sin(ph));
-                }
+            for (int y = 0; y < Ld[1]; ++y) {
+                const cplx xy = at(0, nx, x) * at(1, ny, y);
+                for (int z = 0; z < Ld[2]; ++z, ++q) s += smp[q][e] * (xy * at(2, nz, z));
+            }
         return s / static_cast<double>(smp.size());
     };
     auto clean = [&](cplx v) {  // rounding residue of the transform

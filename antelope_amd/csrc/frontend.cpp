@@ -420,6 +420,8 @@ int sbe_write_snapshot(const char *dir, const sbe_config *cfg, const sbe_model *
     const bool ok = f1 && fn && fp && fl;
     if (ok) {
         const int n0 = g.n[0], n1 = g.n[1], n2 = g.n[2];
+        const sbe::GridArgs ga = g.args();
+        double kp[3];
         const size_t nn = static_cast<size_t>(N) * N;
         std::vector<double> occ1d(2 * static_cast<size_t>(n0), 0.0), nc(g.ntotal);
         std::vector<double> pi(2 * static_cast<size_t>(g.ntotal));
@@ -428,8 +430,9 @@ int sbe_write_snapshot(const char *dir, const sbe_config *cfg, const sbe_model *
             const double *cc = r + 2 * (static_cast<size_t>(nv) * N + nv);      // rho_H[Nval][Nval]
             const double *co = r + 2 * (static_cast<size_t>(nv) * N + nv - 1);  // rho_H[Nval][Nval-1]
             const int64_t i0 = k / (static_cast<int64_t>(n1) * n2);             // momaxis.h:87-91
-            occ1d[2 * i0] += cc[0] * g.w[k];
-            occ1d[2 * i0 + 1] += cc[1] * g.w[k];
+            const double wk = sbe::grid_point(ga, k, kp);
+            occ1d[2 * i0] += cc[0] * wk;
+            occ1d[2 * i0 + 1] += cc[1] * wk;
             nc[k] = cc[0];
             pi[2 * k] = co[0];
             pi[2 * k + 1] = co[1];

@@ -209,33 +209,38 @@ int Grid::build(const sbe_config &cfg, const sbe_model &m, int64_t kb, int64_t k
     }
     dV = std::fabs(vol) / static_cast<double>(ntotal);
 
-    const int64_t nk = ke - kb;
-    k.assign(static_cast<size_t>(nk) * 3, 0.0);
-    w.assign(static_cast<size_t>(nk), 1.0);
-    total_weight = 0.0;
-    const bool mp = cfg.grid == SBE_GRID_MP;
-    for (int64_t g = kb; g < ke; ++g) {
-        const int64_t plane = static_cast<int64_t>(n[1]) * n[2];
-        const int idx[3] = {static_cast<int>(g / plane), static_cast<int>((g / n[2]) % n[1]),
-                            static_cast<int>(g % n[2])};
-        double frac[3], wt = 1.0;
-        for (int d = 0; d < 3; ++d) {
-            if (mp) {
-                frac[d] = (idx[d] + 0.5) / n[d] - 0.5;
-            } else if (n[d] == 1) {
-                frac[d] = 0.0;
-            } else {
-                frac[d] = static_cast<double>(idx[d]) / (n[d] - 1) - 0.5;
-                if (idx[d] == 0 || idx[d] == n[d] - 1) wt *= 0.5;  // trapezoid ends
-            }
-        }
-        const int64_t o = g - kb;
-        for (int c = 0; c < 3; ++c)
-            k[3 * o + c] = origin[c] + frac[0] * axes[c] + frac[1] * axes[3 + c] + frac[2] * axes[6 + c];
-        w[o] = wt;
-        total_weight += wt;
-    }
+    mp = cfg.grid == SBE_GRID_MP;
+    total_weight = weight_before(ke) - weight_before(kb);
     return SBE_OK;
+}
+
+// Sum of the weights of the flattened indices below g, axis by axis: multiples
+// of 1/8, so exact in any order.
+double Grid::weight_before(int64_t g) const
+{
+    auto cum = [&](int d, int64_t i) {  // weights of the first i points of axis d
+        const double ends = mp || n[d] == 1 ? 0.0 : 0.5 * ((i > 0) + (i >= n[d]));
+        return static_cast<double>(i) - ends;
+    };
+    auto one = [&](int d, int64_t i) { return cum(d, i + 1) - cum(d, i); };
+    const int64_t plane = static_cast<int64_t>(n[1]) * n[2];
+    const int64_t i = g / plane, j = (g / n[2]) % n[1], l = g % n[2];
+    const double t2 = cum(2, n[2]), t1 = cum(1, n[1]) * t2;
+    double s = cum(0, i) * t1;
+    if (i < n[0]) s += one(0, i) * (cum(1, j) * t2 + one(1, j) * cum(2, l));
+    return s;
+}
+
+GridArgs Grid::args() const
+{
+    GridArgs a{};
+    for (int d = 0; d < 3; ++d) {
+        a.n[d] = n[d];
+        a.origin[d] = origin[d];
+    }
+    std::memcpy(a.axes, axes, sizeof axes);
+    a.mp = mp;
+    return a;
 }
 
 // -------------------------------------------------------------- tableau --

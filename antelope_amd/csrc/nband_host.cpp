@@ -599,6 +599,7 @@ int nb_setup(sbe_ctx *ctx)
     ctx->nk_stride = p.nk_stride;
     ctx->nv = p.nv;
     ctx->chunk_steps = p.chunk;
+    ctx->partial_bytes = static_cast<int64_t>(p.bytes_partials);
     int rc = SBE_OK;
     ctx->nb_P = p.bytes_P ? nalloc<double2>(ctx, p.bytes_P, rc) : nullptr;
     ctx->nb_rho = nalloc<double2>(ctx, p.bytes_rho, rc);
@@ -618,10 +619,8 @@ int nb_setup(sbe_ctx *ctx)
 
     // host copies of the tables: k [nk_stride][3], w, R cartesian, weights, H, r
     std::vector<double> hk(static_cast<size_t>(p.nk_stride) * 4, 0.0);
-    for (int64_t k = 0; k < nk; ++k) {
-        for (int c = 0; c < 3; ++c) hk[3 * k + c] = ctx->grid.k[3 * k + c];
-        hk[3 * p.nk_stride + k] = ctx->grid.w[k];
-    }
+    const GridArgs ga = ctx->grid.args();
+    for (int64_t k = 0; k < nk; ++k) hk[3 * p.nk_stride + k] = grid_point(ga, ctx->grid.k_begin + k, &hk[3 * k]);
     std::vector<double> hr(static_cast<size_t>(nr) * 4, 0.0);
     for (int r = 0; r < nr; ++r) {
         const int32_t *n = m.rvec + 3 * r;  // R = n1 a1 + n2 a2 + n3 a3 (Wannier90.h:193-204)
@@ -1322,17 +1321,40 @@ int nb_run(sbe_ctx *ctx, int64_t step_begin, int64_t step_end)
 
 int nb_series(sbe_ctx *ctx, double *j_inter, double *j_intra, double *rho_bar, double *band_pop)
 {
-    const int N = ctx->N, nv = ctx->nv;
+    const int N = ctx->N, nv = ctx->nv, nh = 6 + N;
     const int64_t nt = ctx->laser.nt;
-    std::vector<double> s(static_cast<size_t>(nt) * nv);
-    int rc = hipc(ctx, hipMemcpyAsync(s.data(), ctx->d_series, s.size() * sizeof(double), hipMemcpyDeviceToHost, ctx->stream), "copy series");
+    const size_t nr = 2 * static_cast<size_t>(N) * N;
+    // rho's sums are nearly all of the series: the device parts the rows into [nt][6 + N] and
+    // [nt][2 N^2] (in the idle partial-row buffer), and each goes to the host in one copy, rho's
+    // into the caller's array. Small series, and partial-row buffers that cannot hold it, come as
+    // whole rows.
+    const size_t bytes = static_cast<size_t>(nt) * nv * sizeof(double);
+    const bool parted = rho_bar && bytes >= (size_t(1) << 20) &&
+                        bytes <= static_cast<size_t>(ctx->partial_bytes);
+    std::vector<double> s(static_cast<size_t>(nt) * (parted ? nh : nv));
+    const size_t pitch = parted ? nh : nv;
+    const double *src = ctx->d_series;
+    int rc = SBE_OK;
+    if (parted) {
+        rc = hipc(ctx, launch_part_rows(ctx->d_series, nt, nv, nh, ctx->d_partials, ctx->stream), "series kernel");
+        src = ctx->d_partials;
+        if (!rc)
+            rc = hipc(ctx, hipMemcpyAsync(rho_bar, ctx->d_partials + static_cast<size_t>(nt) * nh, nt * nr * sizeof(double),
+                                          hipMemcpyDeviceToHost, ctx->stream), "copy series");
+    }
+    if (!rc) rc = hipc(ctx, hipMemcpyAsync(s.data(), src, s.size() * sizeof(double), hipMemcpyDeviceToHost, ctx->stream), "copy series");
     if (!rc) rc = hipc(ctx, hipStreamSynchronize(ctx->stream), "sync series");
     if (rc) return rc;
     bool finite = true;
     for (int64_t n = 0; n < nt; ++n) {
-        const double *r = s.data() + n * nv;
-        if (n < ctx->steps_done)
-            for (int i = 0; i < nv; ++i) finite = finite && std::isfinite(r[i]);
+        const double *r = s.data() + n * pitch;
+        const double *rb = parted ? rho_bar + n * nr : r + nh;
+        if (n < ctx->steps_done) {
+            double sum = 0.0;  // x - x is 0, or NaN where x is not finite
+            for (int i = 0; i < nh; ++i) sum += r[i] - r[i];
+            for (size_t i = 0; i < nr; ++i) sum += rb[i] - rb[i];
+            finite = finite && sum == 0.0;
+        }
         double dia[3] = {0.0, 0.0, 0.0};  // velocity gauge: sum_k w_k Nval A(t_n) (SBEs.h:683-690,750-757)
         if (ctx->velocity && n < ctx->steps_done) {
             double A[3], E[3];
@@ -1345,7 +1367,7 @@ int nb_series(sbe_ctx *ctx, double *j_inter, double *j_intra, double *rho_bar, d
         }
         if (band_pop)
             for (int m = 0; m < N; ++m) band_pop[n * N + m] = r[6 + m];
-        if (rho_bar) std::memcpy(rho_bar + n * 2 * N * N, r + 6 + N, sizeof(double) * 2 * N * N);
+        if (rho_bar && !parted) std::memcpy(rho_bar + n * nr, rb, sizeof(double) * nr);
     }
     if (!finite) {
         ctx->err = "non-finite value in the propagated state";

@@ -59,54 +59,6 @@ int scratch_address(int dev, void **out, std::string &err)
     return SBE_OK;
 }
 
-// Everything the table kernel needs, by value (about 1.4 KB of kernel
-// arguments): the pulses and the stage times of the tableau.
-struct TableArgs {
-    PulseConst pulses[kMaxDevicePulses];
-    int32_t npulses;
-    int32_t consistent;
-    int32_t nstage;
-    double A_at_min[3];
-    double atmin, dt, t1;
-    double c[7];
-    double va[3][2], vb[3][2];
-    int64_t step0, nsteps;
-};
-
-// Row (step, stage) of the per-stage phase table, the same quantities the
-// host writes for a context: t1 e^{iA.a_j} (j < 3) and e^{iA.b_j} as (re, im)
-// pairs, at t_n + c_s dt (the stage at c = 1 at t_{n+1} itself), A the sum of
-// the pulses less its value at atmin.
-__global__ __launch_bounds__(256) void noalloc_table_kernel(const TableArgs a, double *__restrict__ tab)
-{
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= a.nsteps * a.nstage) return;
-    const int64_t n = a.step0 + i / a.nstage;
-    const int s = static_cast<int>(i % a.nstage);
-    const double tn = a.atmin + a.dt * static_cast<double>(n);
-    const double tn1 = a.atmin + a.dt * static_cast<double>(n + 1);
-    const double t = a.c[s] == 1.0 ? tn1 : tn + a.c[s] * a.dt;
-    double A[3] = {0.0, 0.0, 0.0};
-    for (int p = 0; p < a.npulses; ++p) {
-        double pa[3], pe[3];
-        pulse_field(a.pulses[p], t, a.consistent != 0, pa, pe);
-        for (int j = 0; j < 3; ++j) A[j] += pa[j];
-    }
-    for (int j = 0; j < 3; ++j) A[j] -= a.A_at_min[j];
-    double *row = tab + i * 12;
-    for (int j = 0; j < 3; ++j) {
-        const double pa = A[0] * a.va[j][0] + A[1] * a.va[j][1];
-        const double pb = A[0] * a.vb[j][0] + A[1] * a.vb[j][1];
-        double sa, ca, sb, cb;
-        sincos(pa, &sa, &ca);
-        sincos(pb, &sb, &cb);
-        row[2 * j] = a.t1 * ca;
-        row[2 * j + 1] = a.t1 * sa;
-        row[6 + 2 * j] = cb;
-        row[7 + 2 * j] = sb;
-    }
-}
-
 int fail(int code, const std::string &msg) { return set_thread_error(code, msg); }
 
 int hip_fail(hipError_t e, const char *what)
@@ -191,18 +143,7 @@ extern "C" int sbe_run_haldane_noalloc(const sbe_config *cfg, const sbe_model *m
         if (e != hipSuccess) return hip_fail(e, "init kernel");
     }
 
-    TableArgs ta{};
-    for (size_t p = 0; p < laser.pulses.size(); ++p) ta.pulses[p] = laser.pulses[p];
-    ta.npulses = static_cast<int32_t>(laser.pulses.size());
-    ta.consistent = laser.consistent ? 1 : 0;
-    ta.nstage = tab.nstage;
-    for (int j = 0; j < 3; ++j) ta.A_at_min[j] = laser.A_at_min[j];
-    ta.atmin = laser.atmin;
-    ta.dt = laser.dt;
-    ta.t1 = model->t1;
-    for (int i = 0; i < 7; ++i) ta.c[i] = tab.c[i];
-    std::memcpy(ta.va, va, sizeof va);
-    std::memcpy(ta.vb, vb, sizeof vb);
+    TableArgs ta = table_args(laser, tab, tab.nstage, model->t1, va, vb);
 
     // scratch: [chunk][nstage][12] table rows, then [chunk][nwaves][8] partial rows
     double *d_tab = static_cast<double *>(base);
@@ -212,9 +153,7 @@ extern "C" int sbe_run_haldane_noalloc(const sbe_config *cfg, const sbe_model *m
         const int64_t n = std::min<int64_t>(chunk, step_end - s0);
         ta.step0 = s0;
         ta.nsteps = n;
-        const int64_t rows = n * tab.nstage;
-        noalloc_table_kernel<<<static_cast<unsigned>((rows + 255) / 256), 256, 0, s>>>(ta, d_tab);
-        if ((e = hipGetLastError()) != hipSuccess) return hip_fail(e, "table kernel");
+        if ((e = launch_haldane_table(ta, d_tab, nullptr, s)) != hipSuccess) return hip_fail(e, "table kernel");
         HaldaneArgs a = h;
         a.phase_tab = d_tab;
         a.step0 = 0;  // the table starts at this launch's first step

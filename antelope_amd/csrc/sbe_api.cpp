@@ -270,6 +270,43 @@ int reset_2band(sbe_ctx *ctx, hipStream_t s)
                      "init kernel");
 }
 
+// The laser table of a 2-band fixed-step context, evaluated on the host (any number of pulses).
+int host_table(sbe_ctx *ctx, const double va[3][2], const double vb[3][2], int S, float *d32)
+{
+    const int64_t nt = ctx->laser.nt;
+    const size_t n64 = static_cast<size_t>(nt) * S * 12;
+    std::vector<double> tab(n64);
+    std::vector<float> tab32(n64);
+    for (int64_t n = 0; n < nt; ++n) {
+        const double tn = ctx->laser.atmin + ctx->laser.dt * static_cast<double>(n);  // antelope.cpp:299
+        const double tn1 = ctx->laser.atmin + ctx->laser.dt * static_cast<double>(n + 1);
+        for (int s = 0; s < S; ++s) {
+            double A[3], E[3];
+            // SBEs.h:612; the stage at c = 1 is taken at t_{n+1} itself
+            ctx->laser.eval(ctx->tab.c[s] == 1.0 ? tn1 : tn + ctx->tab.c[s] * ctx->laser.dt, A, E);
+            if (ctx->velocity) {  // A at the stage times, [nt][S][2]
+                double *row = tab.data() + (static_cast<size_t>(n) * S + s) * 2;
+                row[0] = A[0];
+                row[1] = A[1];
+                continue;
+            }
+            double *row = tab.data() + (static_cast<size_t>(n) * S + s) * 12;
+            for (int j = 0; j < 3; ++j) {
+                const double pa = A[0] * va[j][0] + A[1] * va[j][1];
+                const double pb = A[0] * vb[j][0] + A[1] * vb[j][1];
+                row[2 * j] = ctx->model.t1 * std::cos(pa);  // NN part carries t1
+                row[2 * j + 1] = ctx->model.t1 * std::sin(pa);
+                row[6 + 2 * j] = std::cos(pb);
+                row[6 + 2 * j + 1] = std::sin(pb);
+            }
+        }
+    }
+    for (size_t i = 0; i < n64; ++i) tab32[i] = static_cast<float>(tab[i]);
+    int rc = hip_check(ctx, hipMemcpy(ctx->d_phase_tab, tab.data(), n64 * sizeof(double), hipMemcpyHostToDevice), "upload table");
+    if (!rc) rc = hip_check(ctx, hipMemcpy(d32, tab32.data(), n64 * sizeof(float), hipMemcpyHostToDevice), "upload table");
+    return rc;
+}
+
 }  // namespace
 
 namespace sbe {
@@ -565,14 +602,8 @@ int sbe_create(const sbe_config *cfg, const sbe_model *model, int64_t k_begin, i
     ctx->d_weight = ctx->d_kpts + 3 * ctx->nk_stride;
 
     // k points (SoA, zero-padded) and weights
-    {
-        std::vector<double> hk(static_cast<size_t>(ctx->nk_stride) * 4, 0.0);
-        for (int64_t k = 0; k < nk; ++k) {
-            for (int c = 0; c < 3; ++c) hk[c * ctx->nk_stride + k] = ctx->grid.k[3 * k + c];
-            hk[3 * ctx->nk_stride + k] = ctx->grid.w[k];
-        }
-        rc = hip_check(ctx, hipMemcpy(ctx->d_kpts, hk.data(), p.bytes_kpts, hipMemcpyHostToDevice), "upload k");
-    }
+    rc = hip_check(ctx, sbe::launch_kgrid(ctx->grid.args(), ctx->grid.k_begin, nk, ctx->nk_stride, ctx->d_kpts, ctx->stream),
+                   "k grid kernel");
 
     // Haldane geometry (Haldane.h:134-143) and per-stage laser phase tables
     sbe::HaldaneArgs &h = ctx->hargs;
@@ -606,61 +637,22 @@ int sbe_create(const sbe_config *cfg, const sbe_model *model, int64_t k_begin, i
         const int S = ctx->adaptive ? 1 : ctx->tab.nstage;  // adaptive: rows at the sample times t_n
         const int64_t nt = ctx->laser.nt;
         const size_t n64 = static_cast<size_t>(nt) * S * 12;
-        std::vector<double> tab(n64);
-        std::vector<float> tab32(n64);
-        for (int64_t n = 0; n < nt; ++n) {
-            const double tn = ctx->laser.atmin + ctx->laser.dt * static_cast<double>(n);  // antelope.cpp:299
-            const double tn1 = ctx->laser.atmin + ctx->laser.dt * static_cast<double>(n + 1);
-            for (int s = 0; s < S; ++s) {
-                double A[3], E[3];
-                // SBEs.h:612; the stage at c = 1 is taken at t_{n+1} itself, so its row is the
-                // next step's first row bit for bit (the step kernels carry it across steps)
-                ctx->laser.eval(ctx->tab.c[s] == 1.0 ? tn1 : tn + ctx->tab.c[s] * ctx->laser.dt, A, E);
-                if (ctx->velocity) {  // A at the stage times, [nt][S][2]
-                    double *row = tab.data() + (static_cast<size_t>(n) * S + s) * 2;
-                    row[0] = A[0];
-                    row[1] = A[1];
-                    continue;
-                }
-                double *row = tab.data() + (static_cast<size_t>(n) * S + s) * 12;
-                for (int j = 0; j < 3; ++j) {
-                    const double pa = A[0] * va[j][0] + A[1] * va[j][1];
-                    const double pb = A[0] * vb[j][0] + A[1] * vb[j][1];
-                    row[2 * j] = model->t1 * std::cos(pa);  // NN part carries t1
-                    row[2 * j + 1] = model->t1 * std::sin(pa);
-                    row[6 + 2 * j] = std::cos(pb);
-                    row[6 + 2 * j + 1] = std::sin(pb);
-                }
-            }
-        }
-        for (size_t i = 0; i < n64; ++i) tab32[i] = static_cast<float>(tab[i]);
         float *d32 = reinterpret_cast<float *>(ctx->d_phase_tab + n64);
-        if (!rc) rc = hip_check(ctx, hipMemcpy(ctx->d_phase_tab, tab.data(), n64 * sizeof(double), hipMemcpyHostToDevice), "upload table");
-        if (!rc) rc = hip_check(ctx, hipMemcpy(d32, tab32.data(), n64 * sizeof(float), hipMemcpyHostToDevice), "upload table");
+        double *d_at = reinterpret_cast<double *>(d32 + n64);  // adaptive: A, dA/dt at t_n
+        const bool f32 = ctx->cfg.precision == SBE_PREC_FP32;
         h.phase_tab = ctx->d_phase_tab;
         h.phase_tab32 = d32;
-        if (ctx->adaptive && !rc) {  // A - A(t_min) and the consistent dA/dt = -E at t_n, summed in pulse order
-            const int64_t na = std::max<int64_t>(nt, 2);  // an interval to interpolate in
-            std::vector<double> at(static_cast<size_t>(na) * 4);
-            for (int64_t n = 0; n < na; ++n) {
-                const double tn = ctx->laser.atmin + ctx->laser.dt * static_cast<double>(n);
-                double sx = 0.0, sy = 0.0, gx = 0.0, gy = 0.0;
-                for (const sbe::PulseConst &pc : ctx->laser.pulses) {
-                    double pa[3], pe[3];
-                    sbe::pulse_field(pc, tn, true, pa, pe);
-                    sx += pa[0];
-                    sy += pa[1];
-                    gx -= pe[0];
-                    gy -= pe[1];
-                }
-                at[4 * n] = sx - ctx->laser.A_at_min[0];
-                at[4 * n + 1] = sy - ctx->laser.A_at_min[1];
-                at[4 * n + 2] = gx;
-                at[4 * n + 3] = gy;
-            }
-            double *d_at = reinterpret_cast<double *>(d32 + n64);
-            rc = hip_check(ctx, hipMemcpy(d_at, at.data(), at.size() * sizeof(double), hipMemcpyHostToDevice), "upload table");
-            ctx->aargs.a_tab = d_at;
+        if (ctx->adaptive) ctx->aargs.a_tab = d_at;
+        const int64_t na = std::max<int64_t>(nt, 2);  // an interval to interpolate in
+        if (ctx->laser.pulses.size() <= static_cast<size_t>(sbe::kMaxDevicePulses)) {
+            sbe::TableArgs ta = sbe::table_args(ctx->laser, ctx->tab, S, model->t1, va, vb);
+            ta.plain = ctx->velocity ? 1 : 0;
+            if (!rc)
+                rc = hip_check(ctx, sbe::launch_haldane_table(ta, ctx->d_phase_tab, f32 ? d32 : nullptr,
+                                                              ctx->stream), "table kernel");
+            if (!rc && ctx->adaptive) rc = hip_check(ctx, sbe::launch_field_table(ta, na, d_at, ctx->stream), "table kernel");
+        } else if (!rc) {  // more pulses than the kernels' arguments hold: rows from the host
+            rc = host_table(ctx, va, vb, S, d32);
         }
     }
     if (ctx->adaptive && !rc) {
@@ -865,8 +857,11 @@ int sbe_get_state(sbe_ctx *ctx, int32_t basis, double *rho)
         // the state is band-basis at k (phases of band_frame.hpp); orbital: s_orb = sum_i s_i f_i
         if (basis == SBE_BASIS_ORBITAL) {
             const sbe::HaldaneArgs &h = ctx->hargs;
+            const sbe::GridArgs ga = ctx->grid.args();
             for (int64_t k = 0; k < ctx->nk; ++k) {
-                const double kx = ctx->grid.k[3 * k], ky = ctx->grid.k[3 * k + 1];
+                double kp[3];
+                sbe::grid_point(ga, ctx->grid.k_begin + k, kp);
+                const double kx = kp[0], ky = kp[1];
                 double ca = 0, sa = 0, sb = 0;
                 for (int j = 0; j < 3; ++j) {
                     ca += std::cos(kx * h.va[j][0] + ky * h.va[j][1]);
@@ -894,8 +889,11 @@ int sbe_get_state(sbe_ctx *ctx, int32_t basis, double *rho)
         double A[3], E[3];
         ctx->laser.eval(t, A, E);
         const sbe::HaldaneArgs &h = ctx->hargs;
+        const sbe::GridArgs ga = ctx->grid.args();
         for (int64_t k = 0; k < ctx->nk; ++k) {
-            const double kx = ctx->grid.k[3 * k] + A[0], ky = ctx->grid.k[3 * k + 1] + A[1];
+            double kp[3];
+            sbe::grid_point(ga, ctx->grid.k_begin + k, kp);
+            const double kx = kp[0] + A[0], ky = kp[1] + A[1];
             double sa = 0, ca = 0, sb = 0;
             for (int j = 0; j < 3; ++j) {
                 ca += std::cos(kx * h.va[j][0] + ky * h.va[j][1]);

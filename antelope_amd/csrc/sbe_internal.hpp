@@ -31,17 +31,47 @@ struct Laser {
 };
 
 // ----------------------------------------------------------------- grid --
-// Block [k_begin,k_end) of the flattened k grid (momaxis.h) on the host.
+// The flattened k grid (momaxis.h:147-186,349-383): point g and its weight, the
+// same operations on the host and the device (no contraction), so the same bits.
+struct GridArgs {
+    int n[3];
+    int mp;
+    double axes[9], origin[3];
+};
+__host__ __device__ inline double grid_point(const GridArgs &a, int64_t g, double k[3])
+{
+#pragma clang fp contract(off)
+    const int64_t plane = static_cast<int64_t>(a.n[1]) * a.n[2];
+    const int idx[3] = {static_cast<int>(g / plane), static_cast<int>((g / a.n[2]) % a.n[1]),
+                        static_cast<int>(g % a.n[2])};
+    double frac[3], wt = 1.0;
+    for (int d = 0; d < 3; ++d) {
+        if (a.mp) {
+            frac[d] = (idx[d] + 0.5) / a.n[d] - 0.5;
+        } else if (a.n[d] == 1) {
+            frac[d] = 0.0;
+        } else {
+            frac[d] = static_cast<double>(idx[d]) / (a.n[d] - 1) - 0.5;
+            if (idx[d] == 0 || idx[d] == a.n[d] - 1) wt *= 0.5;  // trapezoid ends
+        }
+    }
+    for (int c = 0; c < 3; ++c)
+        k[c] = a.origin[c] + frac[0] * a.axes[c] + frac[1] * a.axes[3 + c] + frac[2] * a.axes[6 + c];
+    return wt;
+}
+
+// Block [k_begin,k_end) of the flattened k grid (momaxis.h).
 struct Grid {
     int n[3] = {1, 1, 1};
+    bool mp = false;
     int64_t ntotal = 0, k_begin = 0, k_end = 0;
     double axes[9] = {0}, origin[3] = {0};
     double dV = 0, total_weight = 0;
-    std::vector<double> k;  // [nk][3]
-    std::vector<double> w;  // [nk]
 
     int build(const sbe_config &cfg, const sbe_model &m, int64_t kb, int64_t ke,
               std::string &err);
+    double weight_before(int64_t g) const;
+    GridArgs args() const;
 };
 
 // Explicit Runge-Kutta tableau (SBEs.h:395-416; Cash-Karp 1990 for the
@@ -110,6 +140,19 @@ struct AdaptiveArgs {
     int32_t *fail;             // set when a wave exhausts its attempts or its step falls below hmin
 };
 
+// What the rows of a 2-band laser table are made of (haldane_table.hip): the pulses and the stage
+// times, passed by value (about 1.4 KB). Row (step, stage): t1 e^{iA.a_j} (j < 3) and e^{iA.b_j} as
+// (re, im) pairs at t_n + c_s dt (the stage at c = 1 at t_{n+1} itself), or A_x, A_y when plain.
+struct TableArgs {
+    PulseConst pulses[kMaxDevicePulses];
+    int32_t npulses, consistent, nstage, plain;
+    double A_at_min[3];
+    double atmin, dt, t1;
+    double c[7];
+    double va[3][2], vb[3][2];
+    int64_t step0, nsteps;
+};
+
 // ------------------------------------------------------------------ ctx --
 enum class PathKind { Haldane2 = 0, NBand = 1 };
 
@@ -143,6 +186,7 @@ struct sbe_ctx {
     double *d_phase_tab = nullptr;  // per-stage laser phase table
     void *d_state = nullptr;
     double *d_partials = nullptr;   // [chunk][nwaves][nv]
+    int64_t partial_bytes = 0;      // N-band: its size
     double *d_series = nullptr;     // [nt][nv]
     // set to 1 by the series reductions when a k sum is not finite (pinned
     // host memory mapped for the device: readable without a copy once the
@@ -225,6 +269,13 @@ struct sbe_ctx {
 };
 
 namespace sbe {
+// haldane_table.hip: set-up on the device. tab rows [nsteps][nstage][12] (plain: [2]), tab32 (may
+// be null) the same rounded to FP32; A - A(t_min) and the consistent dA/dt at t_n, [n][4]; the k
+// points and weights of a block, SoA [4][nk_stride] (zeros past nk)
+TableArgs table_args(const Laser &L, const Tableau &t, int nstage, double t1, const double va[3][2], const double vb[3][2]);
+hipError_t launch_haldane_table(const TableArgs &a, double *tab, float *tab32, hipStream_t s);
+hipError_t launch_field_table(const TableArgs &a, int64_t rows, double *at, hipStream_t s);
+hipError_t launch_kgrid(const GridArgs &g, int64_t k_begin, int64_t nk, int64_t nk_stride, double *kpts, hipStream_t s);
 // Launchers (haldane.hip, series.hip).
 hipError_t launch_haldane_init(const HaldaneArgs &a, int init_type, double ef, hipStream_t s);
 hipError_t launch_haldane_steps(const HaldaneArgs &a, int rk_order, bool t1_on, hipStream_t s);
@@ -232,6 +283,8 @@ hipError_t launch_haldane_steps(const HaldaneArgs &a, int rk_order, bool t1_on, 
 // (0: the default) is the first pass's group size for steps of many rows
 hipError_t launch_series_reduce(double *partials, int64_t nsteps, int32_t nrows, int nv,
                                 double *series, hipStream_t s, int32_t *flag = nullptr, int32_t group_rows = 0);
+// the first nh values of each row of series [nt][nv] into out [nt][nh], the rest behind them [nt][nv - nh]
+hipError_t launch_part_rows(const double *series, int64_t nt, int nv, int nh, double *out, hipStream_t s);
 // One k block's share of a multi-block reduction: steps [first, first +
 // nsteps) of the launch grid sum partials[nsteps][nrows][nv] into series.
 struct SeriesJob {

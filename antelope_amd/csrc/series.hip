@@ -99,7 +99,23 @@ __global__ __launch_bounds__(kReduceThreads) void series_reduce_multi_kernel(con
                 j.series + step * nv + blockIdx.y * vl, j.flag);
 }
 
+__global__ __launch_bounds__(256) void part_rows_kernel(const double *__restrict__ series, int64_t nt, int nv, int nh,
+                                                        double *__restrict__ out)
+{
+    const int64_t id = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (id >= nt * nv) return;
+    const int64_t n = id / nv;
+    const int v = static_cast<int>(id - n * nv);
+    out[v < nh ? n * nh + v : nt * nh + n * (nv - nh) + v - nh] = series[id];
+}
+
 }  // namespace
+
+hipError_t launch_part_rows(const double *series, int64_t nt, int nv, int nh, double *out, hipStream_t s)
+{
+    part_rows_kernel<<<dim3(static_cast<unsigned>((nt * nv + 255) / 256)), 256, 0, s>>>(series, nt, nv, nh, out);
+    return hipGetLastError();
+}
 
 bool series_multi_ok(int32_t nrows) { return nrows <= 2 * kGroupRows; }
 

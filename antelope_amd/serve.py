@@ -73,7 +73,7 @@ class SBEServer:
         self._chk(self._lib.sbe_server_get_series(self._h, rid, _ptr(out["j_inter"]), _ptr(out["j_intra"]),
                                                   _ptr(out["rho_bar"]), _ptr(out["band_pop"])))
         rb = out.pop("rho_bar")
-        out["rho_bar"] = rb[..., 0] + 1j * rb[..., 1]
+        out["rho_bar"] = rb.view(np.complex128)[..., 0]  # [re, im] pairs as they are
         return out
 
     def release(self, rid: int) -> None:

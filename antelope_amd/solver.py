@@ -176,7 +176,7 @@ class SBESolver:
                                       _ptr(out["rho_bar"]), _ptr(out["band_pop"]))
         _check(self._lib, self._ctx, rc)
         rb = out.pop("rho_bar")
-        out["rho_bar"] = rb[..., 0] + 1j * rb[..., 1]
+        out["rho_bar"] = rb.view(np.complex128)[..., 0]  # [re, im] pairs as they are
         return out
 
     def state(self, basis: str = "orbital") -> np.ndarray:
@@ -185,7 +185,7 @@ class SBESolver:
         buf = np.zeros((nk, self.nband, self.nband, 2))
         b = {"orbital": A.SBE_BASIS_ORBITAL, "band": A.SBE_BASIS_BAND}[basis]
         _check(self._lib, self._ctx, self._lib.sbe_get_state(self._ctx, b, _ptr(buf)))
-        return buf[..., 0] + 1j * buf[..., 1]
+        return buf.view(np.complex128)[..., 0]
 
     def set_timing(self, enable: bool = True) -> None:
         _check(self._lib, self._ctx, self._lib.sbe_set_timing(self._ctx, int(enable)))
@@ -271,7 +271,7 @@ class SBEBatch:
         self._chk(self._lib.sbe_batch_get_series(self._h, i, _ptr(out["j_inter"]), _ptr(out["j_intra"]),
                                                  _ptr(out["rho_bar"]), _ptr(out["band_pop"])))
         rb = out.pop("rho_bar")
-        out["rho_bar"] = rb[..., 0] + 1j * rb[..., 1]
+        out["rho_bar"] = rb.view(np.complex128)[..., 0]  # [re, im] pairs as they are
         return out
 
     def step_stats(self, i: int) -> A.sbe_step_stats:
