@@ -421,10 +421,6 @@ __device__ __forceinline__ double lane_value(double x, int j)
     return __hiloint2double(hi, lo);
 }
 
-// the refinements' last-round threshold: eigenvector error O(1e-12), one rotation
-// round fewer than 1e-8 where the first round turns by ~1e-4
-constexpr double kFusedSmallK = 1e-6;
-
 template <int W>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) void nb16_step_kernel(
     const NbArgs a, const NbFused f, cd *__restrict__ rho, cd *__restrict__ Ust, double *__restrict__ partials)
@@ -565,9 +561,9 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) voi
     stage_async<W>(a, step_lds, 1, f.t2_end, 0, f.t2_end, 1, col, w, lane);
     if (active) {
         Ht = form_tile(fused_slot<W>(step_lds, 0, 0), e1, M1, N);
-        // within the step only: the last round at max|K| < 1e-6 and no final Newton-Schulz step
+        // (within the step only: the columns' unitarity is left to the refinement at its end)
         if (a.deph)
-            eig_refine(form_tile(fused_slot<W>(step_lds, 0, 1), e1, M1, N), U, Ut, N, buf, kFusedSmallK, false, true);
+            eig_refine(form_tile(fused_slot<W>(step_lds, 0, 1), e1, M1, N), U, Ut, N, buf, false, true);
         Tile Mh{};
         double dd;
         if (a.deph) Mh = band_diag(Y, U, Ut, dd);
@@ -592,7 +588,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) voi
     if (active) {
         Ht = form_tile(fused_slot<W>(step_lds, 1, 0), e1, M1, N);
         const Tile H = form_tile(fused_slot<W>(step_lds, 1, 1), e1, M1, N);
-        eig_refine(H, U, Ut, N, buf, kFusedSmallK, true, true, &lam);
+        eig_refine(H, U, Ut, N, buf, true, true, &lam);
         Tile Me{};
         double dd;
         if (a.deph) Me = band_diag(Y, U, Ut, dd);

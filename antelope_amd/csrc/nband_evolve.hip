@@ -328,7 +328,7 @@ __device__ __forceinline__ void evolve_steps(const NbArgs &a, SRC &src, const Ev
     src.start(Ht, H);  // at t_n; carried from step to step
     double lam = 0.0;
     if (e.lam_valid) lam = load ? e.lam[kk * e.lam_pitch + c] : 0.0;
-    else eig_refine(H, U, Ut, N, none, 1e-8, true, SRC::kHerm, &lam);
+    else eig_refine(H, U, Ut, N, none, true, SRC::kHerm, &lam);
 
     const double dt = e.dt, g12 = a.gam1 - a.gam2;
     const bool deph = a.deph != 0;
@@ -340,7 +340,7 @@ __device__ __forceinline__ void evolve_steps(const NbArgs &a, SRC &src, const Ev
         return stage_derivative_m<SRC::kHerm>(a, Y, Hc, M, none);
     };
     auto refine = [&](const T &Hs, T &V, T &Vt) {
-        if (deph && g12 != 0.0) eig_refine(Hs, V, Vt, N, none, 1e-8, true, SRC::kHerm);
+        if (deph && g12 != 0.0) eig_refine(Hs, V, Vt, N, none, true, SRC::kHerm);
     };
 
     for (int64_t step = e.s0; step < e.s1; ++step) {
@@ -409,7 +409,7 @@ __device__ __forceinline__ void evolve_steps(const NbArgs &a, SRC &src, const Ev
             axpy_tile(Y, X, dt, Rh);
             src.pair(kMids, Ht, H);
             src.issue_j(step + 1);
-            eig_refine(H, U, Ut, N, none, 1e-8, true, SRC::kHerm, &lam);
+            eig_refine(H, U, Ut, N, none, true, SRC::kHerm, &lam);
             X = deriv(Y, Ht, U, Ut);
             axpy_tile(Rh, X, dt / 6.0, Acc);
         } else {
@@ -441,7 +441,7 @@ __device__ __forceinline__ void evolve_steps(const NbArgs &a, SRC &src, const Ev
             Kd[3] = deriv(input(3), Hc, U, Ut);
             src.pair(kMids, Ht, H);
             src.issue(3);
-            eig_refine(H, U, Ut, N, none, 1e-8, true, SRC::kHerm, &lam);
+            eig_refine(H, U, Ut, N, none, true, SRC::kHerm, &lam);
             Kd[4] = deriv(input(4), Ht, U, Ut);
             src.pair(3, Hc, H);
             src.issue_j(step + 1);

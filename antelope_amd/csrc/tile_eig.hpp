@@ -32,14 +32,12 @@ __device__ __forceinline__ double orthonormalize(T &U, T &Ut, cd *buf)
     return wave_max_dpp(e);
 }
 
-// 1 / (D/2 + s sqrt(D^2/4 + w2)), s = the sign of D (sgn). 16x16 tiles divide and
-// take the root; small tiles take the hardware estimates with one Newton step
-// each (1e-15 relative): an angle's own error is second order in the eigenvectors.
-template <class T>
+// 1 / (D/2 + s sqrt(D^2/4 + w2)), s = the sign of D, from the hardware estimates with
+// one Newton step each (1e-15 relative): an angle's own error is second order in
+// the eigenvectors.
 __device__ __forceinline__ double inv_angle(double D, double w2, double s)
 {
-    const double x = 0.25 * D * D + w2;
-    if (Shape<T>::E > 1) return 1.0 / (0.5 * D + s * sqrt(x));
+    const double x = fma(0.25 * D, D, w2);
     double q = __builtin_amdgcn_rsq(x);
     q = q * fma(-0.5 * x * q, q, 1.5);
     const double y = fma(s * x, q, 0.5 * D);
@@ -47,20 +45,62 @@ __device__ __forceinline__ double inv_angle(double D, double w2, double s)
     return v * fma(-y, v, 2.0);
 }
 
+// K_ij = W_ij / (D/2 + s sqrt(D^2/4 + |W_ij|^2)), D = W_jj - W_ii: the 2x2 Jacobi angles
+// of a nearly diagonal W, 0 on the diagonal and outside N x N. Elements below the
+// rounding of W (1e-16 of its diagonal) count as zero: their angle would be noise
+// where two bands meet. Returns max |K|^2 over the wave.
+template <class T>
+__device__ __forceinline__ double angles(const T &W, T &K, int N, double &lam_c)
+{
+    constexpr int E = Shape<T>::E;
+    const int c = Shape<T>::col();
+    double lam_r[E], k2 = 0.0;
+    diag_bcast(W, lam_r, lam_c);
+#pragma unroll
+    for (int r = 0; r < E; ++r) {
+        const int i = Shape<T>::row(r);
+        const double w2 = W.re[r] * W.re[r] + W.im[r] * W.im[r];
+        const double D = lam_c - lam_r[r];
+        const double s = (D > 0.0 || (D == 0.0 && i < c)) ? 1.0 : -1.0;
+        // (1e-280: below it the root's estimate would leave its range)
+        const bool on = i != c && i < N && c < N && w2 > fmax(1e-280, 1e-32 * (lam_c * lam_c + lam_r[r] * lam_r[r]));
+        const double inv = on ? inv_angle(D, on ? w2 : 1.0, s) : 0.0;
+        K.re[r] = W.re[r] * inv;
+        K.im[r] = W.im[r] * inv;
+        k2 = fmax(k2, K.re[r] * K.re[r] + K.im[r] * K.im[r]);
+    }
+    k2 = wave_max_dpp(k2);
+    // the same in every lane: a scalar, so that the branches on it are
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(k2)),
+                            __builtin_amdgcn_readfirstlane(__double2loint(k2)));
+}
+
 // Warm-started eigenvectors of the Hermitian part of H (as zheevr, which
 // reads one triangle; H from FP16-split sums is Hermitian only to their
 // error): U (and its transpose Ut) in, refined U, Ut out.
-// small: max|K| below which the last round is U (I + K) (its neglected K^2/2 and the
-// next round's O(K^2) residual are the eigenvectors' error); ortho: end with a
-// Newton-Schulz step (U unitary to rounding rather than to O(small^2))
+//
+// W = U^dag H U is nearly diagonal, W = L + E. One round takes the angles to second
+// order: with K the angles of W, the angles X of W + [E, K] / 2 (the part of the
+// rotated W that K leaves at second order), U <- U (I + X + X^2/2). What is left off
+// the diagonal is then of third order: a round that starts at max|K| < 1e-5 is the
+// last (eigenvector error 1e-15), one that starts below 1e-7 needs K alone. Three
+// products a round against four of a first-order round, and no second round where a
+// first-order scheme would need one. Later rounds take W from H again with
+// G = U^dag U = I + e: W - e (W_ii + W_jj) / 2 is W in orthonormal columns, and
+// - e / 2 in the rotation makes the columns so (unitarity error ~e^2); ortho asks for
+// that in the last round also when it is the first. Between RK stages of the 16-band
+// workload (max|K| ~ 2e-2) 9 products against 14, of weak fields 5 against 9.
+// Far starts (max|K| > 0.3) take damped first-order rotations with Newton-Schulz
+// steps until they are near. The columns keep the order of the warm start.
 // herm: Hin is Hermitian to rounding already (FP64 sums), no symmetrization; lam_out:
-// this lane's column of diag(U^dag H U) before the last rotation (the band energies to
-// O(max|K|^2), for ranking)
+// this lane's column of diag W before the last rotation (the band energies, for
+// ranking: off by the squares of the last angles).
 template <class T>
-__device__ void eig_refine(const T &Hin, T &U, T &Ut, int N, cd *buf, double small_tol = 1e-8, bool ortho = true,
-                           bool herm = false, double *lam_out = nullptr)
+__device__ __forceinline__ void eig_refine(const T &Hin, T &U, T &Ut, int N, cd *buf, bool ortho = true, bool herm = false,
+                           double *lam_out = nullptr)
 {
     constexpr int E = Shape<T>::E;
+    constexpr double kFar = 0.09, kLast2 = 1e-10, kLast1 = 1e-14;  // squares of 0.3, 1e-5, 1e-7
     const int c = Shape<T>::col();
     T H = Hin;
     if (!herm) {
@@ -72,73 +112,101 @@ __device__ void eig_refine(const T &Hin, T &U, T &Ut, int N, cd *buf, double sma
         }
     }
     T W = cmm(U, true, cmm(H, true, U));  // U^dag (H U)
+    T G;                                  // e = U^dag U - I, where formed
+    bool have_e = false;
+    auto form_e = [&]() {
+        G = cmm(U, true, U);
+#pragma unroll
+        for (int r = 0; r < E; ++r) G.re[r] -= Shape<T>::row(r) == c ? 1.0 : 0.0;
+        have_e = true;
+    };
     double lam_last = 0.0;
     for (int it = 0; it < 30; ++it) {
-        double lam_r[E], lam_c;
-        diag_bcast(W, lam_r, lam_c);
-        lam_last = lam_c;
-        T K;
-        double kmax = 0.0;
+        T K, V;
+        const double k2 = angles(W, K, N, lam_last);
+        if (!(k2 > kFar)) {  // (a NaN ends here, in the state it makes non-finite)
+            const bool last = !(k2 >= kLast2);
+            if (k2 >= kLast1) {
+                T F;  // E K, then W + (E K + (E K)^dag) / 2
+                {
+                    T Eo;
+#pragma unroll
+                    for (int r = 0; r < E; ++r) {
+                        const bool dg = Shape<T>::row(r) == c;
+                        Eo.re[r] = dg ? 0.0 : W.re[r];
+                        Eo.im[r] = dg ? 0.0 : W.im[r];
+                    }
+                    F = cmm(Eo, true, K);
+                }
+                const T Ft = transpose(F, buf);
+#pragma unroll
+                for (int r = 0; r < E; ++r) {
+                    F.re[r] = fma(0.5, F.re[r] + Ft.re[r], W.re[r]);
+                    F.im[r] = fma(0.5, F.im[r] - Ft.im[r], W.im[r]);
+                }
+                (void)angles(F, K, N, lam_last);
+                T Kn;  // K^T's tile is -conj(K)
+#pragma unroll
+                for (int r = 0; r < E; ++r) {
+                    Kn.re[r] = -K.re[r];
+                    Kn.im[r] = -K.im[r];
+                }
+                const T K2 = cmm(Kn, true, K);
+#pragma unroll
+                for (int r = 0; r < E; ++r) {
+                    V.re[r] = fma(0.5, K2.re[r], K.re[r]);
+                    V.im[r] = fma(0.5, K2.im[r], K.im[r]);
+                }
+            } else {
+                V = K;
+            }
+            if (last && ortho && !have_e) form_e();
+#pragma unroll
+            for (int r = 0; r < E; ++r) {
+                V.re[r] += Shape<T>::row(r) == c ? 1.0 : 0.0;
+                if (have_e) {
+                    V.re[r] = fma(-0.5, G.re[r], V.re[r]);
+                    V.im[r] = fma(-0.5, G.im[r], V.im[r]);
+                }
+            }
+            U = cmm(Ut, false, V);  // U V
+            Ut = transpose(U, buf);
+            if (last) break;
+            W = cmm(U, true, cmm(H, true, U));
+            form_e();
+            double lr[E], lc;
+            diag_bcast(W, lr, lc);
+#pragma unroll
+            for (int r = 0; r < E; ++r) {
+                const double h = -0.5 * (lr[r] + lc);
+                W.re[r] = fma(h, G.re[r], W.re[r]);
+                W.im[r] = fma(h, G.im[r], W.im[r]);
+            }
+            continue;
+        }
+        // far from converged (a cold-like start): damped rotations
+        const double f = k2 > 0.25 ? 0.5 / sqrt(k2) : 1.0;
+        T Kn;
 #pragma unroll
         for (int r = 0; r < E; ++r) {
-            const int i = Shape<T>::row(r);
-            K.re[r] = 0.0;
-            K.im[r] = 0.0;
-            const double w2 = W.re[r] * W.re[r] + W.im[r] * W.im[r];
-            // (small tiles: squares below 1e-280 would leave the root's estimate's range)
-            if (i != c && i < N && c < N && w2 > (E > 1 ? 0.0 : 1e-280)) {
-                const double D = lam_c - lam_r[r];
-                const double s = (D > 0.0 || (D == 0.0 && i < c)) ? 1.0 : -1.0;
-                const double inv = inv_angle<T>(D, w2, s);
-                K.re[r] = W.re[r] * inv;
-                K.im[r] = W.im[r] * inv;
-                kmax = fmax(kmax, K.re[r] * K.re[r] + K.im[r] * K.im[r]);  // |K|^2 here, the root once below
-            }
+            K.re[r] *= f;
+            K.im[r] *= f;
+            Kn.re[r] = -K.re[r];
+            Kn.im[r] = -K.im[r];
         }
-        kmax = sqrt(wave_max_dpp(kmax));
-        if (kmax == 0.0) break;
-        if (kmax > 0.5) {  // far from converged (a cold-like start): damped rotations
-            const double f = 0.5 / kmax;
+        const T K2 = cmm(Kn, true, K);
 #pragma unroll
-            for (int r = 0; r < E; ++r) {
-                K.re[r] *= f;
-                K.im[r] *= f;
-            }
+        for (int r = 0; r < E; ++r) {
+            V.re[r] = K.re[r] + 0.5 * K2.re[r] + (Shape<T>::row(r) == c ? 1.0 : 0.0);
+            V.im[r] = K.im[r] + 0.5 * K2.im[r];
         }
-        T V;
-        const bool small = kmax < small_tol;
-        if (small) {  // I + K: the neglected K^2 / 2 is below 1e-16
-#pragma unroll
-            for (int r = 0; r < E; ++r) {
-                V.re[r] = K.re[r] + (Shape<T>::row(r) == c ? 1.0 : 0.0);
-                V.im[r] = K.im[r];
-            }
-        } else {  // I + K + K^2/2, unitary to |K|^4 / 4; K^T's tile is -conj(K)
-            T Kn;
-#pragma unroll
-            for (int r = 0; r < E; ++r) {
-                Kn.re[r] = -K.re[r];
-                Kn.im[r] = -K.im[r];
-            }
-            const T K2 = cmm(Kn, true, K);
-#pragma unroll
-            for (int r = 0; r < E; ++r) {
-                V.re[r] = K.re[r] + 0.5 * K2.re[r] + (Shape<T>::row(r) == c ? 1.0 : 0.0);
-                V.im[r] = K.im[r] + 0.5 * K2.im[r];
-            }
-        }
-        U = cmm(Ut, false, V);  // U V
+        U = cmm(Ut, false, V);
         Ut = transpose(U, buf);
-        if (small) break;
-        if (kmax > 1e-3) {  // V far from unitary: restore U fully, then W from H itself
-            for (int q = 0; q < 8; ++q)
-                if (orthonormalize(U, Ut, buf) < 1e-8) break;
-            W = cmm(U, true, cmm(H, true, U));
-        } else {
-            W = cmm(V, true, cmm(W, true, V));  // V^dag (W V)
-        }
+        for (int q = 0; q < 8; ++q)
+            if (orthonormalize(U, Ut, buf) < 1e-8) break;
+        W = cmm(U, true, cmm(H, true, U));
+        have_e = false;
     }
-    if (ortho) orthonormalize(U, Ut, buf);
     if (lam_out) *lam_out = lam_last;
 }
 

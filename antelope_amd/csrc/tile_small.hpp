@@ -44,7 +44,7 @@ constexpr int kXor1 = 0xB1, kXor2 = 0x4E;  // quad_perm [1,0,3,2], [2,3,0,1]
 constexpr int kHalfMirror = 0x141;         // lane l <-> l ^ 7
 constexpr int kMirror = 0x140;             // lane l <-> l ^ 15
 constexpr int kRor4 = 0x124, kRor8 = 0x128;
-constexpr int kShl4 = 0x104, kShl8 = 0x108, kShr4 = 0x114, kShr8 = 0x118;
+constexpr int kShl4 = 0x104, kShr4 = 0x114;
 
 // ---- element of this lane: row(r), col()
 template <class T>
@@ -90,20 +90,18 @@ __device__ __forceinline__ SmallTile<1> cmm_t(const SmallTile<1> &A, const Small
     return C;
 }
 
-// the A operand of quadrant row r for every output block (p, q): A^T's quadrant
-// (r, p), i.e. blocks [0,0,1,1] (r = 0) and [2,2,3,3] (r = 1)
-__device__ __forceinline__ double quad_a0(double x) { return bank_move<kShr8, 0x8>(bank_move<kShr4, 0x6>(x, x), x); }
-__device__ __forceinline__ double quad_a1(double x) { return bank_move<kShl8, 0x1>(bank_move<kShl4, 0x6>(x, x), x); }
-// the B operand, B's quadrant (r, q): blocks [0,1,0,1] and [2,3,2,3]
-__device__ __forceinline__ double quad_b0(double x) { return bank_move<kShr8, 0xc>(x, x); }
-__device__ __forceinline__ double quad_b1(double x) { return bank_move<kShl8, 0x3>(x, x); }
+// C_pq = A_pp B_pq + A_p(1-p) B_(1-p)q: the first term takes B where it lies, the
+// second B's rows of quadrants exchanged (one DPP move per word). A^T's tile holds
+// A_pr^T in block (r, p): the A operands are its blocks [0,0,3,3] and [2,2,1,1].
+__device__ __forceinline__ double quad_diag(double x) { return bank_move<kShl4, 0x4>(bank_move<kShr4, 0x2>(x, x), x); }
 
 template <bool CA, bool CB>
 __device__ __forceinline__ SmallTile<2> cmm_t(const SmallTile<2> &A, const SmallTile<2> &B)
 {
     constexpr int kNegRe2 = (CA != CB) ? 0 : 1, kNegIm1 = CB ? 2 : 0, kNegIm2 = CA ? 1 : 0;
-    const double ar0 = quad_a0(A.re[0]), ai0 = quad_a0(A.im[0]), br0 = quad_b0(B.re[0]), bi0 = quad_b0(B.im[0]);
-    const double ar1 = quad_a1(A.re[0]), ai1 = quad_a1(A.im[0]), br1 = quad_b1(B.re[0]), bi1 = quad_b1(B.im[0]);
+    const double ar0 = quad_diag(A.re[0]), ai0 = quad_diag(A.im[0]), br0 = B.re[0], bi0 = B.im[0];
+    const double ar1 = quad_diag(lane_move<kRor8>(A.re[0])), ai1 = quad_diag(lane_move<kRor8>(A.im[0]));
+    const double br1 = lane_move<kRor8>(B.re[0]), bi1 = lane_move<kRor8>(B.im[0]);
     SmallTile<2> C;
     C.re[0] = mfma4(ar0, br0, 0.0);
     C.im[0] = mfma4n<kNegIm1>(ar0, bi0, 0.0);
