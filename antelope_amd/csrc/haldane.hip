@@ -17,10 +17,15 @@
 // never leaves registers inside a launch, so HBM sees the state once per
 // chunk. H(k+A) uses e^{i(k+A).v} = e^{ik.v} e^{iA.v}: the six e^{ik.v} are
 // computed once per launch, the k-independent e^{iA(t).v} come from a
-// per-stage table read with uniform (scalar) loads. Every time sample is
-// reduced over the 64 lanes of a wave with gfx950 permlane swaps and DPP,
-// and one row of 8 FP64 partial sums per wave and step goes to HBM; a second
-// kernel (series.hip) sums the rows in a fixed order.
+// per-stage table staged in LDS. Every time sample is reduced over the 64
+// lanes of a wave on the matrix pipe, and one row of 8 FP64 partial sums per
+// wave and step goes to HBM; a second kernel (series.hip) sums the rows in a
+// fixed order.
+//
+// Bound by the VALU: a wave alone on its SIMD (fewer than 65536 k points) issues its
+// FP64 chain at 4 cycles an instruction, about 240 of them for an RK4 step of a k point
+// (316 before the k sums moved to the matrix pipe and the sample and the right-hand side
+// were factored; 465 for RK5 with T1), so fewer instructions are what there is to gain.
 #include "haldane_dev.hpp"
 
 namespace sbe {
@@ -93,8 +98,9 @@ __device__ __forceinline__ void steps_body(const HaldaneArgs &a, const R *__rest
     const R c3 = static_cast<R>(a.c3), M0 = static_cast<R>(a.M0);
     const R gh1 = static_cast<R>(0.5 * a.gam1), gh2 = static_cast<R>(0.5 * a.gam2);
     const R gh12 = static_cast<R>(0.5 * (a.gam1 - a.gam2));
-    const R ii = a.inter_intra ? R(1) : R(0);
     const int lane = __lane_id();
+    const double scale = sum8_scale(a, lane);
+    const bool ii = a.inter_intra != 0;
 
     // The k-independent phase rows of kTile steps are staged in LDS (double
     // buffered): every lane reads the same row, so LDS broadcasts replace a
@@ -146,12 +152,10 @@ __device__ __forceinline__ void steps_body(const HaldaneArgs &a, const R *__rest
         // ---- time sample at t_n from the state before the step
         double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-        for (int q = 0; q < KPT; ++q) time_sample<R>(p[q], ph[q], a, ii, v);
-        {
-            const double r = wave_reduce8(v);
-            // lanes 8q..8q+7 all hold value q: duplicate stores of equal data keep the step branch-free
-            partials[(static_cast<int64_t>(step) * a.nwaves + wave) * kHaldaneNV + (lane >> 3)] = r;
-        }
+        for (int q = 0; q < KPT; ++q) time_sample<R>(p[q], ph[q], a, v);
+        // eight lanes hold each value: duplicate stores of equal data keep the step branch-free
+        partials[(static_cast<int64_t>(step) * a.nwaves + wave) * kHaldaneNV + sum8_value(lane)] =
+            sample_sums(v, scale, ii, lane);
 
         // ---- one RK step (SBEs.h:596-624), stage RHS halved (see above)
 #pragma unroll
@@ -159,7 +163,7 @@ __device__ __forceinline__ void steps_body(const HaldaneArgs &a, const R *__rest
             R kn[S];
             Vec3<R> kv[S];
             Vec3<R> ds_[S];  // d at each stage time
-            R inv_[S];       // 1/|d|^2 at each stage time
+            R kap_[S];       // -(g1 - g2)/2 / |d|^2 at each stage time
 #pragma unroll
             for (int i = 0; i < S; ++i) {
                 R yn = p[q].n;
@@ -175,18 +179,18 @@ __device__ __forceinline__ void steps_body(const HaldaneArgs &a, const R *__rest
                     }
                 }
                 Vec3<R> d;
-                R inv;
+                R kap;
                 const int same = same_time_stage<RK>(i);
                 if (i == 0) {
                     d = ph[q].d;
-                    inv = ph[q].inv;
+                    kap = -gh12 * ph[q].inv;
                 } else if (same > 0) {
                     d = ds_[same];
-                    inv = inv_[same];
+                    kap = kap_[same];
                 } else if (kCarry && i == kOne) {
                     ph[q] = phases_at(p[q], tr + i * 12, c3, M0);  // the next step's t_n
                     d = ph[q].d;
-                    inv = ph[q].inv;
+                    kap = -gh12 * ph[q].inv;
                 } else {
                     const R *row = tr + i * 12;
                     R dx = 0, dy = 0, sb = 0;
@@ -198,21 +202,12 @@ __device__ __forceinline__ void steps_body(const HaldaneArgs &a, const R *__rest
                     }
                     d = {dx, dy, M0 - c3 * sb};
                     const R dd = d.x * d.x + d.y * d.y + d.z * d.z;
-                    inv = dd > R(0) ? rcp_nr(dd) : R(0);
+                    // a gap closing gives a finite inverse and a zero projection
+                    kap = DEPH ? -gh12 * rcp_nr(dd > smallest<R>() ? dd : smallest<R>()) : R(0);
                 }
                 ds_[i] = d;
-                inv_[i] = inv;
-                // f/2 = d x y - (g2/2) y + ((g2-g1)/2) (y.d / |d|^2) d
-                Vec3<R> f;
-                f.x = d.y * y.z - d.z * y.y;
-                f.y = d.z * y.x - d.x * y.z;
-                f.z = d.x * y.y - d.y * y.x;
-                if (DEPH) {
-                    const R c = -gh12 * (y.x * d.x + y.y * d.y + y.z * d.z) * inv;
-                    f.x += c * d.x - gh2 * y.x;
-                    f.y += c * d.y - gh2 * y.y;
-                    f.z += c * d.z - gh2 * y.z;
-                }
+                kap_[i] = kap;
+                const Vec3<R> f = half_rhs<DEPH>(d, kap, y, gh2);
                 kv[i] = f;
                 kn[i] = T1ON ? -gh1 * yn : R(0);
             }

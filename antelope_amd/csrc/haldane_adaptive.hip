@@ -499,7 +499,7 @@ __device__ __forceinline__ void kahan(R &sum, R &c, R inc)
 // updates them in place, D'_0 = f_new, D'_k = (D'_k-1 - D_k-1) / (t_new - t_n+1-k),
 // and the oldest node drops out of the stencil by itself. The node times are
 // uniform (in the wave's LDS slice); each lane keeps the differences of its
-// wave-summed observable (value lane >> 3).
+// wave-summed observable (sum8_value).
 struct SampleRing {
     double D[6];  // divided differences of this lane's value, newest node first
     double *t;    // [6] node times, newest first (LDS)
@@ -545,8 +545,8 @@ struct SampleRing {
 
     // Writes the samples mi, mi + 1, ... (below mend) whose times
     // atmin + n dt_out do not exceed t_hi, and returns the next one. The eight
-    // lanes of a group hold the same value's ring, so lane l evaluates sample
-    // mi + (l & 7) of value l >> 3: eight samples per pass, each with the
+    // lanes of a value hold the same ring, so a lane evaluates sample
+    // mi + sum8_member of it: eight samples per pass, each with the
     // arithmetic of a single evaluation. part points at this lane's value
     // column of sample row out0.
     __device__ __forceinline__ int emit(int mi, int mend, double atmin, double dt_out, double t_hi, double *part,
@@ -555,14 +555,14 @@ struct SampleRing {
         double tk[6];  // the node times, from LDS once per call
 #pragma unroll
         for (int k = 0; k < 6; ++k) tk[k] = t[k];
-        const int j = __lane_id() & 7;
+        const int j = sum8_member(__lane_id());
         while (mi < mend) {
             const bool in = j < mend - mi;
             const int mj = in ? mi + j : mi;
             const double tm = atmin + dt_out * static_cast<double>(mj);
             const bool ok = in && !(tm > t_hi);
-            // the times grow with j, so the lanes that write are a prefix of each group
-            const int n = __popcll(__ballot(ok) & 0xffull);
+            // the times grow with j, so the members that write are a prefix of each value's
+            const int n = __popcll(__ballot(ok) & kSum8First);
             if (ok) part[(static_cast<int64_t>(mj) - out0) * row_stride] = at(tm, tk);
             mi += n;
             if (n < 8) break;
@@ -635,8 +635,8 @@ __device__ void adaptive_body(const AdaptiveArgs &A, int64_t blk, const int64_t 
     // T1 is off on this path (the host rejects it): g1 = 0
     const R gh2 = static_cast<R>(0.5 * a.gam2), gh12 = static_cast<R>(-0.5 * a.gam2);
     const R ii = a.inter_intra ? R(1) : R(0);
-    // this lane writes value (lane >> 3) of the wave's partial row of each sample
-    double *part = a.partials + static_cast<int64_t>(wave) * kHaldaneNV + (lane >> 3);
+    // this lane writes value sum8_value of the wave's partial row of each sample
+    double *part = a.partials + static_cast<int64_t>(wave) * kHaldaneNV + sum8_value(lane);
     const int64_t row_stride = static_cast<int64_t>(a.nwaves) * kHaldaneNV;
 
     __shared__ R lds_rows[kAdaptiveBlock / 64][6 * kRow];
@@ -700,7 +700,7 @@ __device__ void adaptive_body(const AdaptiveArgs &A, int64_t blk, const int64_t 
     bool failed = false;
 
     // Step ends carry the wave sums of the observables (this lane: value
-    // lane >> 3) into the six-node ring; samples are its Lagrange
+    // sum8_value) into the six-node ring; samples are its Lagrange
     // interpolants. At the window start: the sample itself, and the first
     // stage.
     Vec3<R> k1[KPT];
@@ -736,7 +736,7 @@ __device__ void adaptive_body(const AdaptiveArgs &A, int64_t blk, const int64_t 
                            Vec3<R>{2 * k1[q].x, 2 * k1[q].y, 2 * k1[q].z}, row, a, ii, o, od);
             }
         }
-        const double O0 = wave_reduce8(o);
+        const double O0 = wave_sum8(o);
         part[(m - out0) * row_stride] = O0;
         ring.push(t, O0);
         ++m;
@@ -836,7 +836,7 @@ __device__ void adaptive_body(const AdaptiveArgs &A, int64_t blk, const int64_t 
                 else observe<R>(p[q], p[q].n - p[q].cn, Vec3<R>{p[q].sx - p[q].cx, p[q].sy - p[q].cy, p[q].sz - p[q].cz},
                                 Vec3<R>{2 * k1[q].x, 2 * k1[q].y, 2 * k1[q].z}, row7, a, ii, o, od);
             }
-            ring.push(tn, wave_reduce8(o));
+            ring.push(tn, wave_sum8(o));
             if (ring.cnt >= 6) emit(ring.t[2]);  // samples up to node c - 2
             t = tn;
             ++nacc;
@@ -881,14 +881,14 @@ __device__ void adaptive_body(const AdaptiveArgs &A, int64_t blk, const int64_t 
     }
 }
 
-// f/2 of the Bloch equation at d (1/|d|^2 = inv): d x y - (g2/2) y + ((g2 - g1)/2) (y.d/|d|^2) d
-// d(k + A) and 1/|d|^2 at a stage time: the sums of
+// d(k + A) and |d|^2 at a stage time (and the sum sb of the b phases' sines): the sums of
 // phases_at, each component formed as one FMA chain (a stage needs no single
 // phase, only d)
-__device__ __forceinline__ void stage_d_inv(const KPoint<double> &p, const double *row, double c3, double M0,
-                                            Vec3<double> &d, double &inv, double &dd)
+__device__ __forceinline__ void stage_d(const KPoint<double> &p, const double *row, double c3, double M0,
+                                        Vec3<double> &d, double &dd, double &sb)
 {
-    double dx = p.er[0] * row[0], dy = p.er[0] * row[1], sb = p.er[3] * row[7];
+    double dx = p.er[0] * row[0], dy = p.er[0] * row[1];
+    sb = p.er[3] * row[7];
     dx = fma(-p.ei[0], row[1], dx);
     dy = fma(p.ei[0], row[0], dy);
     sb = fma(p.ei[3], row[6], sb);
@@ -903,8 +903,6 @@ __device__ __forceinline__ void stage_d_inv(const KPoint<double> &p, const doubl
     }
     d = Vec3<double>{dx, dy, fma(-c3, sb, M0)};
     dd = fma(d.x, d.x, fma(d.y, d.y, d.z * d.z));
-    // d = 0 (a gap closing) gives a finite inv and a zero dephasing projection
-    inv = rcp_nr(fmax(dd, 1e-300));
 }
 
 // The single phases t1 e^{i(k+A).a_j} and e^{i(k+A).b_j} of a row (the
@@ -918,23 +916,6 @@ __device__ __forceinline__ void step_end_phases(const KPoint<double> &p, const d
         e.br[j] = fma(p.er[j + 3], row[6 + 2 * j], -(p.ei[j + 3] * row[7 + 2 * j]));
         e.bi[j] = fma(p.er[j + 3], row[7 + 2 * j], p.ei[j + 3] * row[6 + 2 * j]);
     }
-}
-
-template <bool DEPH>
-__device__ __forceinline__ Vec3<double> half_f_at(const Vec3<double> &d, double inv, const Vec3<double> &y, double gh2,
-                                                  double gh12)
-{
-    Vec3<double> f;
-    f.x = d.y * y.z - d.z * y.y;
-    f.y = d.z * y.x - d.x * y.z;
-    f.z = d.x * y.y - d.y * y.x;
-    if (DEPH) {
-        const double c = -gh12 * (y.x * d.x + y.y * d.y + y.z * d.z) * inv;
-        f.x += c * d.x - gh2 * y.x;
-        f.y += c * d.y - gh2 * y.y;
-        f.z += c * d.z - gh2 * y.z;
-    }
-    return f;
 }
 
 // The FP64 stepper. Per accepted step of a wave: five new stage times (the
@@ -972,8 +953,9 @@ __device__ void adaptive_body64(const AdaptiveArgs &A, int64_t blk, const int64_
     }
     const double c3 = a.c3, M0 = a.M0;
     const double gh2 = 0.5 * a.gam2, gh12 = -0.5 * a.gam2;  // T1 off on this path
-    const double ii = a.inter_intra ? 1.0 : 0.0;
-    double *part = a.partials + static_cast<int64_t>(wave) * kHaldaneNV + (lane >> 3);
+    const bool ii = a.inter_intra != 0;
+    const double scale = sum8_scale(a, lane);
+    double *part = a.partials + static_cast<int64_t>(wave) * kHaldaneNV + sum8_value(lane);
     const int64_t row_stride = static_cast<int64_t>(a.nwaves) * kHaldaneNV;
     __shared__ double lds_rows[kAdaptiveBlock / 64][6 * kRow];
     double *rows = lds_rows[threadIdx.x >> 6];
@@ -1008,10 +990,10 @@ __device__ void adaptive_body64(const AdaptiveArgs &A, int64_t blk, const int64_
         for (int q = 0; q < KPT; ++q) {
             const Phases<double> e = phases_at(p[q], rows + 5 * kRow, c3, M0);
             const Vec3<double> y{p[q].sx, p[q].sy, p[q].sz};
-            k1[q] = half_f_at<DEPH>(e.d, e.inv, y, gh2, gh12);
-            sample_state(e, p[q].w, p[q].n, y.x, y.y, y.z, a, ii, v);
+            k1[q] = half_rhs<DEPH>(e.d, -gh12 * e.inv, y, gh2);
+            sample_state(e, p[q].w, p[q].n, y.x, y.y, y.z, a, v);
         }
-        const double val = wave_reduce8(v);
+        const double val = sample_sums(v, scale, ii, lane);
         part[0] = val;
         ring.push(t, val);
         ++m;
@@ -1031,7 +1013,7 @@ __device__ void adaptive_body64(const AdaptiveArgs &A, int64_t blk, const int64_
 
         Vec3<double> inc[KPT];
         Vec3<double> d_end[KPT];  // d, 1/|d|^2 and |d|^2 at the step end (the stage at c = 1)
-        double inv_end[KPT], dd_end[KPT];
+        double inv_end[KPT], dd_end[KPT], q_end[KPT], sb_end[KPT];
         double err_k = 0.0;
 #pragma unroll
         for (int q = 0; q < KPT; ++q) {
@@ -1051,13 +1033,17 @@ __device__ void adaptive_body64(const AdaptiveArgs &A, int64_t blk, const int64_
                     }
                 }
                 Vec3<double> d;
-                double inv, dd;
-                stage_d_inv(p[q], rows + (i - 1) * kRow, c3, M0, d, inv, dd);
-                kv[i] = half_f_at<DEPH>(d, inv, y, gh2, gh12);
+                double inv, dd, sb;
+                stage_d(p[q], rows + (i - 1) * kRow, c3, M0, d, dd, sb);
+                // d = 0 (a gap closing) gives finite inverses and a zero dephasing projection
+                if (CK::c[i] == 1.0) rsqrt_rcp(fmax(dd, smallest<double>()), q_end[q], inv);
+                else inv = rcp_nr(fmax(dd, smallest<double>()));
+                kv[i] = half_rhs<DEPH>(d, -gh12 * inv, y, gh2);
                 if (CK::c[i] == 1.0) {
                     d_end[q] = d;
                     inv_end[q] = inv;
                     dd_end[q] = dd;
+                    sb_end[q] = sb;
                 }
             }
             inc[q] = Vec3<double>{0, 0, 0};
@@ -1107,10 +1093,12 @@ __device__ void adaptive_body64(const AdaptiveArgs &A, int64_t blk, const int64_
                 e1.d = d_end[q];
                 e1.dd = dd_end[q];
                 e1.inv = inv_end[q];
-                k1[q] = half_f_at<DEPH>(e1.d, e1.inv, y, gh2, gh12);  // f(t + h, y5)
-                sample_state(e1, p[q].w, p[q].n, y.x, y.y, y.z, a, ii, v);
+                e1.q = q_end[q];
+                e1.sb = sb_end[q];
+                k1[q] = half_rhs<DEPH>(e1.d, -gh12 * e1.inv, y, gh2);  // f(t + h, y5)
+                sample_state(e1, p[q].w, p[q].n, y.x, y.y, y.z, a, v);
             }
-            ring.push(tn, wave_reduce8(v));
+            ring.push(tn, sample_sums(v, scale, ii, lane));
             if (ring.cnt >= 6) emit(ring.t[2]);  // samples up to node c - 2
             t = tn;
             ++nacc;

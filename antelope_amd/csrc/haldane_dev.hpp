@@ -73,37 +73,36 @@ __device__ __forceinline__ void swap16(double &a, double &b)
     b = __hiloint2double(hi[1], lo[1]);
 }
 
-// Sum each of v[0..7] over the 64 lanes of the wave (reduce-scatter):
-// lane l ends with the total of v[(l >> 3) & 7]. Requires all 64 lanes.
-__device__ __forceinline__ double wave_reduce8(double v[8])
+// The sums of v[0..7] over the 64 lanes of the wave, each in eight lanes: lane l ends with
+// the total of v[sum8_value(l)], and the lanes of a value are numbered 0..7 by sum8_member.
+// Requires all 64 lanes.
+__device__ __forceinline__ int sum8_value(int lane) { return (lane & 3) | ((lane >> 2) & 4); }
+__device__ __forceinline__ int sum8_member(int lane) { return ((lane >> 2) & 3) | ((lane >> 3) & 4); }
+constexpr unsigned long long kSum8First = 0x0000111100001111ull;  // the lanes of value 0
+
+// On the matrix pipe, which these kernels leave idle: the 4x4x4 FP64 MFMA of four blocks
+// (lane l = j + 4 b + 16 i) with A = v_q and B = ones in column q adds v_q's four rows of
+// lanes into column q, so four values share one accumulator; a second one with A = ones
+// adds the rows of that. The four blocks of a row are added with DPP. 10 MFMAs and 8 VALU
+// additions and moves, against 45 VALU instructions of a reduce-scatter by permlane swaps
+// and DPP (316 -> 280 instructions of an RK4 step of the 2-band kernel).
+__device__ __forceinline__ double wave_sum8(const double v[8])
 {
     const int lane = __lane_id();
-    // lane bit 5: permlane32 swap + add
+    double s[2] = {0.0, 0.0};
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        double a = v[j], b = v[j + 4];
-        swap32(a, b);
-        v[j] = a + b;  // lanes 0-31: v[j], lanes 32-63: v[j+4]
+    for (int q = 0; q < 4; ++q) {
+        const double e = (lane & 3) == q ? 1.0 : 0.0;
+        s[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(v[q], e, s[0], 0, 0, 0);
+        s[1] = __builtin_amdgcn_mfma_f64_4x4x4f64(v[4 + q], e, s[1], 0, 0, 0);
     }
-    // lane bit 4: permlane16 swap + add
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        double a = v[j], b = v[j + 2];
-        swap16(a, b);
-        v[j] = a + b;  // even rows: v[j], odd rows: v[j+2]
-    }
-    // lane bit 3: rotate by 8 inside each 16-lane row (= lane ^ 8)
-    const bool hi = (lane & 8) != 0;
-    const double keep = hi ? v[1] : v[0];
-    const double send = hi ? v[0] : v[1];
-    double x = keep + dpp_f64<0x128>(send);  // row_ror:8
-    // lanes 8q..8q+7 now share value index q: all-reduce over the low 3 bits
-    x += dpp_f64<0x141>(x);  // row_half_mirror (i <-> 7-i)
-    x += dpp_f64<0x4E>(x);   // quad_perm [2,3,0,1]
-    x += dpp_f64<0xB1>(x);   // quad_perm [1,0,3,2]
+    s[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(1.0, s[0], 0.0, 0, 0, 0);
+    s[1] = __builtin_amdgcn_mfma_f64_4x4x4f64(1.0, s[1], 0.0, 0, 0, 0);
+    double x = (lane & 16) != 0 ? s[1] : s[0];
+    x += dpp_f64<0x128>(x);  // row_ror:8
+    x += dpp_f64<0x124>(x);  // row_ror:4
     return x;
 }
-
 // -------------------------------------------------------- model kernels
 template <typename R>
 struct Vec3 {
@@ -136,21 +135,34 @@ template <> struct StateT<float> {
 __device__ __forceinline__ float fmar(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ double fmar(double a, double b, double c) { return __builtin_fma(a, b, c); }
 
-// 1/x from the hardware reciprocal with Newton steps (two in FP64, one in FP32)
+// 1/x from the hardware reciprocal: FP64 with one cubic step (residual e: r (1 + e + e^2),
+// the estimate's error cubed), FP32 with a Newton step
 __device__ __forceinline__ double rcp_nr(double x)
 {
-    double r = __builtin_amdgcn_rcp(x);
-    r = fmar(r, fmar(-x, r, 1.0), r);
-    return fmar(r, fmar(-x, r, 1.0), r);
+    const double r = __builtin_amdgcn_rcp(x);
+    const double e = fmar(-x, r, 1.0);
+    return fmar(r, fmar(e, e, e), r);
 }
 __device__ __forceinline__ float rcp_nr(float x)
 {
     const float r = __builtin_amdgcn_rcpf(x);
     return fmar(r, fmar(-x, r, 1.0f), r);
 }
-// 1/sqrt(x): the FP32 hardware rsqrt (1 ulp), the library one in FP64
-__device__ __forceinline__ double rsqrt_r(double x) { return rsqrt(x); }
-__device__ __forceinline__ float rsqrt_r(float x) { return __builtin_amdgcn_rsqf(x); }
+// 1/sqrt(x) and 1/x together: FP64 the hardware root with a cubic step, its square corrected by
+// one residual; FP32 the hardware root (1 ulp) and rcp_nr
+__device__ __forceinline__ void rsqrt_rcp(double x, double &q, double &inv)
+{
+    const double q0 = __builtin_amdgcn_rsq(x);
+    const double e = fmar(-(x * q0), q0, 1.0);
+    q = fmar(q0 * e, fmar(0.375, e, 0.5), q0);
+    const double i0 = q * q;
+    inv = fmar(i0, fmar(-x, i0, 1.0), i0);
+}
+__device__ __forceinline__ void rsqrt_rcp(float x, float &q, float &inv)
+{
+    q = __builtin_amdgcn_rsqf(x);
+    inv = rcp_nr(x);
+}
 
 // complex product (a + ib)(c + id)
 template <typename R>
@@ -170,15 +182,21 @@ struct KPoint {
 };
 
 // Everything a k point needs at one time t: the phases e^{i(k+A(t)).v_j},
-// d(k+A), |d|^2 and 1/|d|^2 (0 at a gap closing). One function computes it
-// wherever it is needed, with explicit FMAs, so equal inputs give equal bits.
+// d(k+A), |d|^2, 1/|d|^2 and 1/|d|. One function computes it wherever it is
+// needed, with explicit FMAs, so equal inputs give equal bits. At a gap closing
+// (d = 0) the inverses are finite and meet d = 0 in every product.
 template <typename R>
 struct Phases {
     R ar[3], ai[3];  // t1 e^{i(k+A).a_j}
     R br[3], bi[3];  // e^{i(k+A).b_j}
     Vec3<R> d;
-    R dd, inv;
+    R sb;            // sum of bi
+    R dd, inv, q;
 };
+
+template <typename R> __device__ __forceinline__ R smallest();  // far below any |d|^2 but invertible
+template <> __device__ __forceinline__ double smallest<double>() { return 1e-300; }
+template <> __device__ __forceinline__ float smallest<float>() { return 1e-36f; }
 
 template <typename R>
 __device__ __forceinline__ Phases<R> phases_at(const KPoint<R> &p, const R *row, R c3, R M0)
@@ -193,67 +211,96 @@ __device__ __forceinline__ Phases<R> phases_at(const KPoint<R> &p, const R *row,
     }
     e.d.x = e.ar[0] + e.ar[1] + e.ar[2];
     e.d.y = e.ai[0] + e.ai[1] + e.ai[2];
-    e.d.z = fmar(-c3, e.bi[0] + e.bi[1] + e.bi[2], M0);
+    e.sb = e.bi[0] + e.bi[1] + e.bi[2];
+    e.d.z = fmar(-c3, e.sb, M0);
     e.dd = fmar(e.d.x, e.d.x, fmar(e.d.y, e.d.y, e.d.z * e.d.z));
-    e.inv = e.dd > R(0) ? rcp_nr(e.dd) : R(0);
+    rsqrt_rcp(e.dd > smallest<R>() ? e.dd : smallest<R>(), e.q, e.inv);
     return e;
+}
+
+// Half of the stage right-hand side at d (kap = -(g1 - g2)/2 / |d|^2):
+// f/2 = d x y - (g2/2) y + ((g2 - g1)/2) (y.d / |d|^2) d, each component one FMA chain.
+template <bool DEPH, typename R>
+__device__ __forceinline__ Vec3<R> half_rhs(const Vec3<R> &d, R kap, const Vec3<R> &y, R gh2)
+{
+    Vec3<R> f;
+    if (DEPH) {
+        const R c = kap * fmar(y.x, d.x, fmar(y.y, d.y, y.z * d.z));
+        f.x = fmar(c, d.x, fmar(d.y, y.z, fmar(-d.z, y.y, -(gh2 * y.x))));
+        f.y = fmar(c, d.y, fmar(d.z, y.x, fmar(-d.x, y.z, -(gh2 * y.y))));
+        f.z = fmar(c, d.z, fmar(d.x, y.y, fmar(-d.y, y.x, -(gh2 * y.z))));
+    } else {
+        f.x = fmar(d.y, y.z, -(d.z * y.y));
+        f.y = fmar(d.z, y.x, -(d.x * y.z));
+        f.z = fmar(d.x, y.y, -(d.y * y.x));
+    }
+    return f;
 }
 
 // Time sample of one k point at t_n (antelope.cpp:307-333 with
 // SBEs.h:694-760), from the state nn, s and the phases at t_n: adds
-// w x (inter_x, inter_y, intra_x, intra_y, s_x, s_y, s_z, s.dhat) to v (FP64).
+// w x (inter_x, inter_y, intra_x, intra_y, s_x, s_y, s_z, s.dhat) to v (FP64), the
+// currents without the factor sum8_scale applies to the k sums. Every value is linear in the
+// state, so the weight multiplies the four components once; the honeycomb vectors
+// (Haldane.h:134-143) turn the derivatives of d0 and d into differences of phases,
+//   d/dkx = a0 sqrt3/2 (-(ai3 - ai2), ar3 - ar2, -c3 (2 br1 - br2 - br3)), d0: -c0 (2 bi1 - bi2 - bi3)
+//   d/dky = a0/2 (dy - 3 ai1, 3 ar1 - dx, -3 c3 (br2 - br3)),              d0: -3 c0 (bi2 - bi3)
 // Evaluated in the state precision R; the k sum is always FP64. Branch-free
 // so the scheduler can interleave it with the RK chain.
 template <typename R>
-__device__ __forceinline__ void sample_state(const Phases<R> &e, double w, R nn, R s_x, R s_y, R s_z,
-                                             const HaldaneArgs &a, R ii, double v[8])
+__device__ __forceinline__ void sample_state(const Phases<R> &e, double wk, R n, R x, R y, R z, const HaldaneArgs &a,
+                                             double v[8])
 {
-    const R c3 = static_cast<R>(a.c3);
+    const R c3 = static_cast<R>(a.c3), c0 = static_cast<R>(a.c0), w = static_cast<R>(wk);
     const Vec3<R> &d = e.d;
-    // derivatives d/dk_x, d/dk_y of (d0, dx, dy, dz)
-    R xx = 0, xy = 0, yx = 0, yy = 0, zx = 0, zy = 0, ox = 0, oy = 0;
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-        const R ax = static_cast<R>(a.va[j][0]), ay = static_cast<R>(a.va[j][1]);
-        const R bx = static_cast<R>(a.vb[j][0]), by = static_cast<R>(a.vb[j][1]);
-        xx -= ax * e.ai[j];
-        xy -= ay * e.ai[j];
-        yx += ax * e.ar[j];
-        yy += ay * e.ar[j];
-        zx += bx * e.br[j];
-        zy += by * e.br[j];
-        ox += bx * e.bi[j];
-        oy += by * e.bi[j];
+    const R nn = n * w, s_x = x * w, s_y = y * w, s_z = z * w;
+    const R xx = e.ai[1] - e.ai[2], yx = e.ar[2] - e.ar[1];
+    const R zx = -c3 * fmar(R(2), e.br[0], -(e.br[1] + e.br[2]));
+    const R ox = -c0 * fmar(R(3), e.bi[0], -e.sb);
+    const R xy = fmar(R(-3), e.ai[0], d.y), yy = fmar(R(3), e.ar[0], -d.x);
+    const R zy = R(-3) * c3 * (e.br[1] - e.br[2]), oy = R(-3) * c0 * (e.bi[1] - e.bi[2]);
+    const R sd = fmar(s_x, d.x, fmar(s_y, d.y, s_z * d.z));
+    const R g = sd * e.inv;
+    const R tx = fmar(s_x, xx, fmar(s_y, yx, s_z * zx));  // s . d_x d
+    const R ty = fmar(s_x, xy, fmar(s_y, yy, s_z * zy));
+    const R px = g * fmar(d.x, xx, fmar(d.y, yx, d.z * zx));  // (s.dh)(dh.d_x d)
+    const R py = g * fmar(d.x, xy, fmar(d.y, yy, d.z * zy));
+    // inter = -(s.d_a d - px), intra = -(n d_a d0 + px)
+    v[0] += static_cast<double>(tx - px);
+    v[1] += static_cast<double>(ty - py);
+    v[2] += static_cast<double>(fmar(nn, ox, px));
+    v[3] += static_cast<double>(fmar(nn, oy, py));
+    v[4] += static_cast<double>(s_x);
+    v[5] += static_cast<double>(s_y);
+    v[6] += static_cast<double>(s_z);
+    v[7] += static_cast<double>(e.dd > R(0) ? sd * e.q : -s_z);
+}
+
+// the factor of this lane's value in the k sums of sample_state
+__device__ __forceinline__ double sum8_scale(const HaldaneArgs &a, int lane)
+{
+    const int v = sum8_value(lane);
+    if (v > 3) return 1.0;
+    return (v & 1 ? -0.5 : -0.86602540378443864676) * a.va[0][1];  // va[0] = (0, a0)
+}
+
+// The k sums of a sample in this lane's value: inter and intra as they are, or (GenCurrent) the
+// total current in the first pair and nothing in the second.
+__device__ __forceinline__ double sample_sums(const double v[8], double scale, bool inter_intra, int lane)
+{
+    double r = wave_sum8(v) * scale;
+    if (!inter_intra) {  // uniform
+        const double o = dpp_f64<0x4E>(r);  // values 0 <-> 2, 1 <-> 3
+        const int q = sum8_value(lane);
+        r = q > 3 ? r : (q < 2 ? r + o : 0.0);
     }
-    zx *= -c3;
-    zy *= -c3;
-    const R c0 = static_cast<R>(a.c0);
-    ox *= -c0;
-    oy *= -c0;
-    const R inv = e.inv;
-    const R sd = s_x * d.x + s_y * d.y + s_z * d.z;
-    const R tx = s_x * xx + s_y * yx + s_z * zx;  // s . d_x d
-    const R ty = s_x * xy + s_y * yy + s_z * zy;
-    const R px = sd * (d.x * xx + d.y * yx + d.z * zx) * inv;  // (s.dh)(dh.d_x d)
-    const R py = sd * (d.x * xy + d.y * yy + d.z * zy) * inv;
-    // InterIntra (ii = 1): inter = -(s.d_a d - px), intra = -(n d_a d0 + px)
-    // GenCurrent  (ii = 0): inter = -(n d_a d0 + s.d_a d), intra = 0
-    const R ni = R(1) - ii;
-    v[0] -= static_cast<double>(tx - ii * px + ni * nn * ox) * w;
-    v[1] -= static_cast<double>(ty - ii * py + ni * nn * oy) * w;
-    v[2] -= static_cast<double>(ii * (nn * ox + px)) * w;
-    v[3] -= static_cast<double>(ii * (nn * oy + py)) * w;
-    v[4] += static_cast<double>(s_x) * w;
-    v[5] += static_cast<double>(s_y) * w;
-    v[6] += static_cast<double>(s_z) * w;
-    v[7] += static_cast<double>(e.dd > R(0) ? sd * rsqrt_r(e.dd) : -s_z) * w;
+    return r;
 }
 
 template <typename R>
-__device__ __forceinline__ void time_sample(const KPoint<R> &p, const Phases<R> &e, const HaldaneArgs &a, R ii,
-                                            double v[8])
+__device__ __forceinline__ void time_sample(const KPoint<R> &p, const Phases<R> &e, const HaldaneArgs &a, double v[8])
 {
-    sample_state(e, p.w, p.n - p.cn, p.sx - p.cx, p.sy - p.cy, p.sz - p.cz, a, ii, v);
+    sample_state(e, p.w, p.n - p.cn, p.sx - p.cx, p.sy - p.cy, p.sz - p.cz, a, v);
 }
 
 }  // namespace dev

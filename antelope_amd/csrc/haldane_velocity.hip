@@ -195,10 +195,7 @@ __device__ __forceinline__ void vel_body(const HaldaneArgs &a, const R *__restri
             v[6] += static_cast<double>(z) * w;
             v[7] -= static_cast<double>(z) * w;  // band populations (n -+ v7)/2 as in the length gauge
         }
-        {
-            const double r = wave_reduce8(v);
-            partials[(static_cast<int64_t>(step) * a.nwaves + wave) * kHaldaneNV + (lane >> 3)] = r;
-        }
+        partials[(static_cast<int64_t>(step) * a.nwaves + wave) * kHaldaneNV + sum8_value(lane)] = wave_sum8(v);
 
         // ---- one RK step (SBEs.h:596-624)
 #pragma unroll

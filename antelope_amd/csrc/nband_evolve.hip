@@ -363,8 +363,8 @@ __device__ __forceinline__ void evolve_steps(const NbArgs &a, SRC &src, const Ev
         src.issue(0);
         double *mine = sums + ((step & 1) * kWaves + w) * nv;
         {
-            const double cur = dev::wave_reduce8(v);
-            if ((lane & 7) == 0 && (lane >> 3) < 6) mine[lane >> 3] = cur;
+            const double cur = dev::wave_sum8(v);
+            if (dev::sum8_value(lane) < 6) mine[dev::sum8_value(lane)] = cur;  // eight lanes hold each
             double pop = ranked_population<Q>(lam, pc, N) * wk;
             double rr = Rh.re[0] * wk, ri = Rh.im[0] * wk;
             if (KW == 4) {  // over the wave's four k points

@@ -92,9 +92,9 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) voi
             v[ax] = inter * wk;
             v[3 + ax] = intra * wk;
         }
-        const double cur = dev::wave_reduce8(v);
+        const double cur = dev::wave_sum8(v);
         double *mine = red + ((step & 1) * W + w) * nv;
-        if ((lane & 7) == 0 && (lane >> 3) < 6) mine[lane >> 3] = cur;
+        if (dev::sum8_value(lane) < 6) mine[dev::sum8_value(lane)] = cur;  // eight lanes hold each
 #pragma unroll
         for (int r = 0; r < E; ++r) {
             const int i = Shape<T>::row(r);
