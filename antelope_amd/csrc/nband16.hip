@@ -14,20 +14,10 @@
 //    movement; a transpose (U^T, T^dag) goes through a padded 16x17 LDS
 //    buffer of the wave, conflict-free.
 //  * Eigenvectors U(k + A(t)) are refined from the stored ones (warm start)
-//    by simultaneous Jacobi rotations written as matrix products: with
-//    W = U^dag H U nearly diagonal, K_ij = W_ij / (D/2 + s sqrt(D^2/4 +
-//    |W_ij|^2)), D = W_jj - W_ii (the 2x2 Jacobi angle; W_ij / D for small
-//    W_ij, bounded for near-degenerate pairs), K anti-Hermitian;
-//    U <- U (I + K + K^2/2), W <- V^dag W V until max|K| < 1e-8, then a last
-//    U (I + K) and one Newton-Schulz step U (3I - U^dag U)/2 to keep U
-//    unitary to rounding. After a round with max|K| > 1e-3 (V unitary only to
-//    |K|^4 / 4) U is made unitary again by Newton-Schulz steps until
-//    |U^dag U - I| < 1e-8 and W is rebuilt from H; rounds with max|K| > 0.5
-//    are damped to 0.5 (a cold-like start converges in ~10 rounds).
-//    Convergence is quadratic; between RK stages two or three rounds reach
-//    machine precision. The columns keep the order of
-//    the warm start (bands are followed continuously); the sample kernel
-//    ranks them by eigenvalue, as the reference's ascending zheevr order.
+//    by rotations written as matrix products, second order in the Jacobi
+//    angles (eig_refine). The columns keep the order of the warm start (bands
+//    are followed continuously); the sample kernel ranks them by eigenvalue,
+//    as the reference's ascending zheevr order.
 //  * The dephasing U (Gamma o (U^dag y U)) U^dag is g2 y + (g1 - g2)
 //    U diag(U^dag y U) U^dag (Gamma = g1 on the diagonal, g2 off it): one
 //    product y U, a column reduction and one product U diag(d) U^dag.
@@ -42,6 +32,7 @@
 #include <map>
 #include <mutex>
 
+#include "haldane_dev.hpp"
 #include "nband.hpp"
 #include "tile_eig.hpp"
 
@@ -319,9 +310,8 @@ __global__ __launch_bounds__(64) void nb16_vel_step_kernel(const NbArgs a, const
 // ------------------------------------------------- fused RK4 step ----
 // One RK4 step per launch (SBEs.h:596-624 with the stage right-hand side of
 // SBEs.h:762-861 and the sample of SBEs.h:694-760), for a product k grid with
-// separable Fourier sums. Block = W k points that share (k2, k3) and differ
-// along a1, one wave each (W = 8; W = 4 where the grid has fewer blocks than
-// CUs, so each wave has a SIMD of its own). The sums' last pass (along a1),
+// separable Fourier sums. Block = four k points that share (k2, k3) and differ
+// along a1, one wave each. The sums' last pass (along a1),
 //   X(k1, k2, k3) = sum_m E1[k1][m] T2[m][k2][k3],
 // runs here: the block stages T2's M1 rows of its column for two matrices at a
 // time in LDS and every wave forms its own tiles from them, so H~, H and J of
@@ -330,43 +320,54 @@ __global__ __launch_bounds__(64) void nb16_vel_step_kernel(const NbArgs a, const
 // band energies from the last step), stage 1 at t_n, stages 2 and 3 at
 // t_n + dt/2 (eigenvectors refined there), stage 4 at t_n + dt (eigenvectors
 // refined for the next sample); rho, U and the energies are the only per-k
-// HBM traffic. The W waves' sample sums are added in LDS in wave order into
+// HBM traffic. The waves' sample sums are added in LDS in wave order into
 // one partial row per block.
-// dynamic LDS of a block: the waves' transpose buffers, then two buffers of two
-// staging slots of kNbFusedMaxM1 x 256 complex each (row m of the second-pass output
-// at m * 256, so the m offsets are immediates). While a block computes from one
-// buffer, the other fills straight from global memory (global_load_lds); a buffer
-// also holds the block's sample sums (W nv doubles) once read.
+//
+// Bound by the FP64 pipe, which MFMA and VALU share: per k point 31 thousand cycles of
+// MFMA (30 products), about 16 of VALU, and 30 of waits for LDS, barriers and MFMA results that
+// the second wave of the SIMD covers in part. Two staging slots instead of four let two
+// blocks of four waves share a CU (one of eight before): while one waits at a barrier the
+// other has products to do. That and one fixed chunk of every staged row per wave, in place of a chunk
+// list with a division per load (3800 scalar instructions per k point), took 48x48x8 with 16
+// bands from 371 to 328 ms, 628 steps; six wave sums in one (wave_sum8) are part of it.
+// dynamic LDS of a block: the waves' transpose buffers (which also hold a wave's sample
+// sums once), then two staging slots of kNbFusedMaxM1 x 256 complex each (row m of the
+// second-pass output at m * 256, so the m offsets are immediates). The slots fill straight from global memory (global_load_lds); their tiles are
+// formed into registers first, so they fill again while the block computes.
+constexpr int kFusedW = kNbFusedWaves;
 constexpr int kFusedPitch = 256;
-constexpr int64_t kFusedSlot = static_cast<int64_t>(kNbFusedMaxM1) * kFusedPitch;  // complex per slot
-template <int W>
-constexpr int64_t fused_tb() { return static_cast<int64_t>(W) * 16 * kTpad; }  // complex of the tb
+constexpr int kFusedBuf = 16 * kTpad;  // complex per wave
+static_assert(2 * kFusedBuf >= 6 + 16 + 2 * 256, "a wave's sample sums fit its transpose buffer");
 
-template <int W>
-__device__ __forceinline__ cd *fused_slot(cd *lds, int buf, int slot) { return lds + fused_tb<W>() + (2 * buf + slot) * kFusedSlot; }
+__device__ __forceinline__ cd *fused_slot(cd *lds, int slot)
+{
+    return lds + kFusedW * kFusedBuf + slot * (kNbFusedMaxM1 * kFusedPitch);
+}
 
-// This wave's share of filling buffer buf with matrix j0 of src0 and j1 of src1 (src1
-// may be null), rows m < M1 of column col: chunks of 64 complex go straight to LDS,
-// each lane one element; their completion is counted by vmcnt (fused_wait).
-template <int W>
-__device__ __forceinline__ void stage_async(const NbArgs &a, cd *lds, int buf, const cd *src0, int j0, const cd *src1,
-                                            int j1, int64_t col, int w, int lane)
+// This wave's share of filling slot 0 with matrix j0 of src0 and slot 1 with j1 of src1
+// (src1 may be null), rows m < M1 of column col: wave w takes chunk w of 64 complex of
+// every row (N N <= 256), each lane one element straight to LDS; their completion is
+// counted by vmcnt (fused_wait).
+__device__ __forceinline__ void stage_async(const NbArgs &a, cd *lds, const cd *src0, int j0, const cd *src1, int j1,
+                                            int64_t col, int w, int lane)
 {
     const int nn = a.N * a.N, M1 = a.boxM[0];
-    const int Q = (nn + 63) >> 6;  // chunks per row
     const int64_t mstride = static_cast<int64_t>(a.boxK[1]) * a.boxK[2] * a.bcols;
-    const int64_t cbase = col * a.bcols;
-    const int per = M1 * Q;
-    const int total = src1 ? 2 * per : per;
-    for (int ch = w; ch < total; ch += W) {  // uniform over the wave
-        const int slot = ch >= per ? 1 : 0;
-        const int rem = ch - slot * per;
-        const int m = rem / Q, q = rem - m * Q;
-        const cd *src = slot ? src1 : src0;
-        const int j = slot ? j1 : j0;
-        const int ij = q * 64 + lane;
-        cd *dst = lds + fused_tb<W>() + (2 * buf + slot) * kFusedSlot + m * kFusedPitch + q * 64;
-        if (ij < nn) __builtin_amdgcn_global_load_lds(src + m * mstride + cbase + j * nn + ij, dst, 16, 0, 0);
+    const int ij = w * 64 + lane;
+    if (ij < nn) {
+#pragma unroll
+        for (int slot = 0; slot < 2; ++slot) {
+            if (slot && !src1) break;
+            const cd *src = (slot ? src1 : src0) + col * a.bcols + (slot ? j1 : j0) * nn + ij;
+            cd *dst = fused_slot(lds, slot) + w * 64;
+#pragma unroll
+            for (int m = 0; m < kNbFusedMaxM1; ++m) {
+                if (m < M1) {
+                    __builtin_amdgcn_global_load_lds(src, dst + m * kFusedPitch, 16, 0, 0);
+                    src += mstride;
+                }
+            }
+        }
     }
 }
 
@@ -378,8 +379,10 @@ __device__ __forceinline__ void fused_wait()
 }
 
 // this lane's elements of X = sum_m E1[m] Y[m] from a staging slot, in the order of
-// operations of the a1 pass of the separable sums
-__device__ __forceinline__ Tile form_tile(const cd *ys, const cd *__restrict__ e1, int M1, int N)
+// operations of the a1 pass of the separable sums. The row loop keeps its branch at M1:
+// without it (rows clamped, factors 0) the reads of a whole tile are in flight at once and
+// their registers spill (48x48x8, 16 bands: 329 ms against 357).
+__device__ __forceinline__ Tile form_tile(const cd *ys, const cd *e1, int M1, int N)
 {
     const int c = lane_c(), g = lane_g();
     int off[4];
@@ -421,8 +424,7 @@ __device__ __forceinline__ double lane_value(double x, int j)
     return __hiloint2double(hi, lo);
 }
 
-template <int W>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) void nb16_step_kernel(
+__global__ __launch_bounds__(64 * kFusedW) __attribute__((amdgpu_waves_per_eu(2))) void nb16_step_kernel(
     const NbArgs a, const NbFused f, cd *__restrict__ rho, cd *__restrict__ Ust, double *__restrict__ partials)
 {
     extern __shared__ cd step_lds[];
@@ -436,28 +438,25 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) voi
     const int lin = nb % 8 == 0 ? (b % 8) * (nb / 8) + b / 8 : b;
     const int col = lin / f.g1, grp = lin - col * f.g1;
     const int k2 = col / K3, k3 = col - k2 * K3;
-    const int k1 = grp * W + w;
+    const int k1 = grp * kFusedW + w;
     // a k block of the grid leaves holes in its box (k map -1): those waves only stage
     const int64_t kmap = k1 < K1 ? a.box_kinv[(static_cast<int64_t>(k1) * K2 + k2) * K3 + k3] : -1;
     const bool active = kmap >= 0;
     const int64_t k = active ? kmap : 0;
-    cd *buf = step_lds + w * 16 * kTpad;
+    cd *buf = step_lds + w * kFusedBuf;
     const double dt = f.dt;
     // this wave's a1 factors E1[k1][m] in LDS (read as broadcasts by every tile formed)
-    cd *e1 = step_lds + fused_tb<W>() + 4 * kFusedSlot + w * kNbFusedMaxM1;
+    cd *e1 = fused_slot(step_lds, 2) + w * kNbFusedMaxM1;
     if (lane < M1) e1[lane] = a.boxE[0][static_cast<int64_t>(active ? k1 : 0) * M1 + lane];
 
     Tile R, U, Ut, Y, Acc, Ht, X;
     double lam = 0.0, p = 0.0;
-    double cur[6] = {0, 0, 0, 0, 0, 0};
     double pop = 0.0;
-    double racc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     const double wk = active ? a.weight[k] : 0.0;
     const bool need_h = !f.u_valid || !f.lam_valid;
-    // staging order: [H(t_n) if needed] [J_x J_y] [J_z H~(t_n)] [H~ H at t + dt/2] [H~ H at t + dt],
-    // buffers alternating, each filled while the previous one is read
-    if (need_h) stage_async<W>(a, step_lds, 1, f.t2_prev, 1, nullptr, 0, col, w, lane);
-    stage_async<W>(a, step_lds, 0, f.t2_j, 0, f.t2_j, 1, col, w, lane);
+    // staging order: [H(t_n) if needed] [J_x J_y] [J_z H~(t_n)] [H~ H at t + dt/2] [H~ H at t + dt]
+    if (need_h) stage_async(a, step_lds, f.t2_prev, 1, nullptr, 0, col, w, lane);
+    else stage_async(a, step_lds, f.t2_j, 0, f.t2_j, 1, col, w, lane);
     if (active) {
         R = load_tile(rho + k * nn, N);
         U = load_tile(Ust + k * nn, N, true);
@@ -467,10 +466,12 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) voi
     if (need_h) {  // eigenvectors / energies at t_n from H(t_n)
         fused_wait();
         if (active) {
-            const Tile H = form_tile(fused_slot<W>(step_lds, 1, 0), e1, M1, N);
+            const Tile H = form_tile(fused_slot(step_lds, 0), e1, M1, N);
             if (!f.u_valid) eig_refine(H, U, Ut, N, buf);
             lam = col_dot(U, cmm(H, true, U));
         }
+        __syncthreads();  // slots read
+        stage_async(a, step_lds, f.t2_j, 0, f.t2_j, 1, col, w, lane);
     } else if (active) {
         lam = f.lam[k * 16 + c];
     }
@@ -489,16 +490,13 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) voi
             const int dst = (lane < N ? rank : lane) * 4;  // byte address of the receiving lane
             const int lo = __builtin_amdgcn_ds_permute(dst, __double2loint(p));
             const int hi = __builtin_amdgcn_ds_permute(dst, __double2hiint(p));
-            if (lane < N) pop += __hiloint2double(hi, lo) * wk;
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            racc[2 * r] = R.re[r] * wk;
-            racc[2 * r + 1] = R.im[r] * wk;
+            if (lane < N) pop = __hiloint2double(hi, lo) * wk;
         }
     }
     // Re Tr(rho J_a) = Re sum_ij conj(rho_ij) J_ij (rho Hermitian; J need not be) and
-    // Re Tr(M J_a) = sum_c p_c Re (U^dag J_a U)_cc the same way, elementwise on J's tile
+    // Re Tr(M J_a) = sum_c p_c Re (U^dag J_a U)_cc the same way, elementwise on J's tile:
+    // this lane's part of the inter and intra sums, summed over the wave together
+    double cur[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     auto current = [&](int ax, const Tile &J) {
         double tot = 0.0, intra = 0.0;
 #pragma unroll
@@ -506,64 +504,67 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) voi
             tot += R.re[r] * J.re[r] + R.im[r] * J.im[r];
             intra += M.re[r] * J.re[r] + M.im[r] * J.im[r];
         }
-        tot = wave_sum(tot);
-        intra = a.inter_intra ? wave_sum(intra) : 0.0;
-        cur[ax] += (tot - intra) * wk;
-        cur[3 + ax] += intra * wk;
+        if (!a.inter_intra) intra = 0.0;
+        cur[ax] = (tot - intra) * wk;
+        cur[3 + ax] = intra * wk;
     };
-    fused_wait();  // [J_x J_y] in buffer 0; buffer 1 read (H(t_n))
-    stage_async<W>(a, step_lds, 1, f.t2_j, 2, f.t2_prev, 0, col, w, lane);
+    fused_wait();  // [J_x J_y]
     if (active) {
-        current(0, form_tile(fused_slot<W>(step_lds, 0, 0), e1, M1, N));
-        current(1, form_tile(fused_slot<W>(step_lds, 0, 1), e1, M1, N));
+        current(0, form_tile(fused_slot(step_lds, 0), e1, M1, N));
+        current(1, form_tile(fused_slot(step_lds, 1), e1, M1, N));
     }
-    // ---- stage 1 at t_n (H~ of t_n), with J_z
-    fused_wait();  // [J_z H~] in buffer 1; buffer 0 read
-    stage_async<W>(a, step_lds, 0, f.t2_half, 0, f.t2_half, 1, col, w, lane);
+    __syncthreads();  // slots read
+    stage_async(a, step_lds, f.t2_j, 2, f.t2_prev, 0, col, w, lane);
+    fused_wait();  // [J_z H~]
     if (active) {
-        current(2, form_tile(fused_slot<W>(step_lds, 1, 0), e1, M1, N));
-        Ht = form_tile(fused_slot<W>(step_lds, 1, 1), e1, M1, N);  // H~ (Hermitian: its conjugate is H~^T's tile)
-        X = stage_derivative_m<true>(a, R, Ht, M, buf);
-        axpy_tile(Acc, X, dt / 6.0, R);
-        axpy_tile(Y, X, 0.5 * dt, R);
+        current(2, form_tile(fused_slot(step_lds, 0), e1, M1, N));
+        Ht = form_tile(fused_slot(step_lds, 1), e1, M1, N);  // H~ (Hermitian: its conjugate is H~^T's tile)
     }
-    // ---- the block's sample sums in buffer 1 (read): one partial row, waves added in order
-    __syncthreads();
+    // ---- the block's sample sums: one partial row, waves added in order
     {
-        double *red = reinterpret_cast<double *>(fused_slot<W>(step_lds, 1, 0));  // [W][nv]
-        double *mine = red + w * a.nv;
-        if (lane < 6) {
-            double v = 0.0;
-#pragma unroll
-            for (int q = 0; q < 6; ++q)
-                if (lane == q) v = cur[q];
-            mine[lane] = v;
-        }
+        double *red = reinterpret_cast<double *>(step_lds);  // a transpose buffer per wave
+        double *mine = reinterpret_cast<double *>(buf);
+        const double v = dev::wave_sum8(cur);
+        const int q = dev::sum8_value(lane);
+        if (q < 6) mine[q] = v;  // eight lanes hold each
         if (lane < N) mine[6 + lane] = pop;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int i = g + 4 * r;
             if (i < N && c < N) {
-                mine[6 + N + 2 * (i * N + c)] = racc[2 * r];
-                mine[6 + N + 2 * (i * N + c) + 1] = racc[2 * r + 1];
+                mine[6 + N + 2 * (i * N + c)] = active ? R.re[r] * wk : 0.0;
+                mine[6 + N + 2 * (i * N + c) + 1] = active ? R.im[r] * wk : 0.0;
             }
         }
-        __syncthreads();
+        __syncthreads();  // slots read, sums written
+        stage_async(a, step_lds, f.t2_half, 0, f.t2_half, 1, col, w, lane);
         double *row = partials + (f.step_local * nb + b) * static_cast<int64_t>(a.nv);
-        for (int v = threadIdx.x; v < a.nv; v += blockDim.x) {
+        for (int u = threadIdx.x; u < a.nv; u += blockDim.x) {
             double sum = 0.0;
-            for (int q = 0; q < W; ++q) sum += red[q * a.nv + v];
-            row[v] = sum;
+#pragma unroll
+            for (int j = 0; j < kFusedW; ++j) sum += red[j * 2 * kFusedBuf + u];
+            row[u] = sum;
         }
+        __syncthreads();  // sums read: the transpose buffers are free
+    }
+    // ---- stage 1 at t_n
+    if (active) {
+        X = stage_derivative_m<true>(a, R, Ht, M, buf);
+        axpy_tile(Acc, X, dt / 6.0, R);
+        axpy_tile(Y, X, 0.5 * dt, R);
     }
     // ---- stages 2 and 3 at t_n + dt/2
-    fused_wait();  // [H~ H at t + dt/2] in buffer 0; buffer 1 read (sample sums)
-    stage_async<W>(a, step_lds, 1, f.t2_end, 0, f.t2_end, 1, col, w, lane);
+    fused_wait();  // [H~ H at t + dt/2]
+    Tile H;
     if (active) {
-        Ht = form_tile(fused_slot<W>(step_lds, 0, 0), e1, M1, N);
+        Ht = form_tile(fused_slot(step_lds, 0), e1, M1, N);
+        if (a.deph) H = form_tile(fused_slot(step_lds, 1), e1, M1, N);
+    }
+    __syncthreads();  // slots read
+    stage_async(a, step_lds, f.t2_end, 0, f.t2_end, 1, col, w, lane);
+    if (active) {
         // (within the step only: the columns' unitarity is left to the refinement at its end)
-        if (a.deph)
-            eig_refine(form_tile(fused_slot<W>(step_lds, 0, 1), e1, M1, N), U, Ut, N, buf, false, true);
+        if (a.deph) eig_refine(H, U, Ut, N, buf, false, true);
         Tile Mh{};
         double dd;
         if (a.deph) Mh = band_diag(Y, U, Ut, dd);
@@ -584,10 +585,10 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) voi
         axpy_tile(Y, X, dt, R);
     }
     // ---- stage 4 at t_n + dt; eigenvectors and energies for the next sample
-    fused_wait();  // [H~ H at t + dt] in buffer 1
+    fused_wait();  // [H~ H at t + dt]
     if (active) {
-        Ht = form_tile(fused_slot<W>(step_lds, 1, 0), e1, M1, N);
-        const Tile H = form_tile(fused_slot<W>(step_lds, 1, 1), e1, M1, N);
+        Ht = form_tile(fused_slot(step_lds, 0), e1, M1, N);
+        H = form_tile(fused_slot(step_lds, 1), e1, M1, N);
         eig_refine(H, U, Ut, N, buf, true, true, &lam);
         Tile Me{};
         double dd;
@@ -658,33 +659,16 @@ static hipError_t allow_lds(const void *kernel, size_t lds)
     return hipSuccess;
 }
 
-size_t nb16_step_lds_bytes(int N, int M1, int nv, int waves)
-{
-    (void)N;
-    (void)M1;
-    // the sample sums must fit in one buffer (two slots)
-    if (static_cast<int64_t>(waves) * nv > 2 * kFusedSlot * 2) return ~size_t(0);
-    return sizeof(double2) * static_cast<size_t>(static_cast<int64_t>(waves) * 16 * kTpad + 4 * kFusedSlot +
-                                                 static_cast<int64_t>(waves) * kNbFusedMaxM1);
-}
-
-template <int W>
-static hipError_t launch_step_w(const NbArgs &a, const NbFused &f, double2 *rho, double2 *U, double *partials,
-                                hipStream_t s)
-{
-    const size_t lds = nb16_step_lds_bytes(a.N, a.boxM[0], a.nv, W);
-    const hipError_t e = allow_lds(reinterpret_cast<const void *>(&nb16_step_kernel<W>), lds);
-    if (e != hipSuccess) return e;
-    nb16_step_kernel<W><<<dim3(static_cast<unsigned>(f.nblocks)), 64 * W, lds, s>>>(a, f, rho, U, partials);
-    return hipGetLastError();
-}
-
 hipError_t nb16_launch_step(const NbArgs &a, const NbFused &f, double2 *rho, double2 *U, double *partials,
                             hipStream_t s)
 {
-    if (a.N > 16 || !a.box || a.boxM[0] > kNbFusedMaxM1 || f.nblocks < 1 || (f.waves != 4 && f.waves != 8))
-        return hipErrorInvalidValue;
-    return f.waves == 4 ? launch_step_w<4>(a, f, rho, U, partials, s) : launch_step_w<8>(a, f, rho, U, partials, s);
+    if (a.N > 16 || !a.box || a.boxM[0] < 1 || a.boxM[0] > kNbFusedMaxM1 || f.nblocks < 1) return hipErrorInvalidValue;
+    constexpr size_t lds = sizeof(double2) * static_cast<size_t>(
+        kFusedW * kFusedBuf + 2 * kNbFusedMaxM1 * kFusedPitch + kFusedW * kNbFusedMaxM1);
+    const hipError_t e = allow_lds(reinterpret_cast<const void *>(&nb16_step_kernel), lds);
+    if (e != hipSuccess) return e;
+    nb16_step_kernel<<<dim3(static_cast<unsigned>(f.nblocks)), 64 * kFusedW, lds, s>>>(a, f, rho, U, partials);
+    return hipGetLastError();
 }
 
 }  // namespace sbe

@@ -282,20 +282,10 @@ int nb32_steps_per_eval(int64_t nk_stride, int N, int64_t nt)
     return static_cast<int>(eval_steps(7 * static_cast<size_t>(nk_stride) * N * N * sizeof(double2), nt));
 }
 
-// k points along a1 per block of the fused N <= 16 step: 8, or 4 where 8 would give fewer
-// blocks than the GPU has CUs (small grids: a wave per SIMD shortens the step, whose time is
-// then one k point's chain of products)
-constexpr int kNbCUs = 256;
-int fused_waves(const BoxShape &bx)
-{
-    const int64_t b8 = static_cast<int64_t>((bx.K[0] + 7) / 8) * bx.K[1] * bx.K[2];
-    return b8 < kNbCUs ? 4 : 8;
-}
-
+// blocks of the fused N <= 16 step
 int fused_blocks(const BoxShape &bx, int &g1)
 {
-    const int w = fused_waves(bx);
-    g1 = (bx.K[0] + w - 1) / w;
+    g1 = (bx.K[0] + kNbFusedWaves - 1) / kNbFusedWaves;
     return g1 * bx.K[1] * bx.K[2];
 }
 
@@ -729,8 +719,7 @@ int nb_setup(sbe_ctx *ctx)
     ctx->nbf_small = fused && N <= 8;
     const char *sw = std::getenv("ANTELOPE_NB_FUSED");
     const bool off = sw && std::atoi(sw) == 0;
-    if (fbuf && fused && p.fe.S >= 1 && !off && a.box && a.tile16 &&
-        (ctx->nbf_small || nb16_step_lds_bytes(N, bx.M[0], a.nv, fused_waves(bx)) <= (size_t(160) << 10))) {
+    if (fbuf && fused && p.fe.S >= 1 && !off && a.box && a.tile16) {
         const FusedEval &fe = p.fe;
         const int64_t nt = ctx->laser.nt;
         const size_t S = static_cast<size_t>(fe.S), types = static_cast<size_t>(fe.mids) + 2;
@@ -766,8 +755,7 @@ int nb_setup(sbe_ctx *ctx)
         if (rc) return rc;
         ctx->nbf_laser = lt;
         // blocks over the k points' own box (a k block of the grid may span fewer k1, k2, k3)
-        ctx->nbf_waves = fused_waves(bx);
-        ctx->nbf_g1 = (a.boxK[0] + ctx->nbf_waves - 1) / ctx->nbf_waves;
+        ctx->nbf_g1 = (a.boxK[0] + kNbFusedWaves - 1) / kNbFusedWaves;
         ctx->nbf_nblocks = ctx->nbf_small ? box_evolve_blocks(N, a.boxK) : ctx->nbf_g1 * a.boxK[1] * a.boxK[2];
         for (int r = 0; r < nr; ++r) ctx->nbf_jz = ctx->nbf_jz || hr[3 * r + 2] != 0.0;
         ctx->nbf = true;
@@ -1035,7 +1023,6 @@ int nb_run_fused(sbe_ctx *ctx, int64_t step_begin, int64_t step_end)
                 f.step_local = s + i;
                 f.g1 = ctx->nbf_g1;
                 f.nblocks = ctx->nbf_nblocks;
-                f.waves = ctx->nbf_waves;
                 rc = hipc(ctx, nb16_launch_step(a, f, ctx->nb_rho, ctx->nb_U, ctx->d_partials, ctx->stream), "step kernel");
                 // the end of this step is the start of the next: its H~, H serve there
                 ctx->nbf_prev_time = tn + dt;

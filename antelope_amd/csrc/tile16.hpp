@@ -40,8 +40,8 @@ __device__ __forceinline__ Tile cmm_t(const Tile &Aop, const Tile &B)
     for (int kb = 0; kb < 4; ++kb) {
         const double ar = Aop.re[kb], ai = Aop.im[kb], br = B.re[kb], bi = B.im[kb];
         re = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, br, re, 0, 0, 0);
-        re = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, bi, re, 0, 0, kNegRe2);
         im = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, bi, im, 0, 0, kNegIm1);
+        re = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, bi, re, 0, 0, kNegRe2);
         im = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, br, im, 0, 0, kNegIm2);
     }
     Tile C;
@@ -66,20 +66,23 @@ __device__ __forceinline__ void wave_lds_order()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// X^T through the wave's LDS buffer (16 x kTpad complex)
+// X^T through the wave's LDS buffer (16 x kTpad complex), real and imaginary parts as two
+// planes of pitch kTpad: both are register pairs already, so nothing is packed (16 moves
+// less than writing complex elements), and column reads stay free of bank conflicts
 __device__ __forceinline__ Tile transpose(const Tile &X, cd *buf)
 {
     const int c = lane_c(), g = lane_g();
+    double *re = reinterpret_cast<double *>(buf), *im = re + 16 * kTpad;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) buf[(g + 4 * r) * kTpad + c] = make_double2(X.re[r], X.im[r]);
+    for (int r = 0; r < 4; ++r) re[(g + 4 * r) * kTpad + c] = X.re[r];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) im[(g + 4 * r) * kTpad + c] = X.im[r];
     wave_lds_order();
     Tile T;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const cd v = buf[c * kTpad + g + 4 * r];
-        T.re[r] = v.x;
-        T.im[r] = v.y;
-    }
+    for (int r = 0; r < 4; ++r) T.re[r] = re[c * kTpad + g + 4 * r];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) T.im[r] = im[c * kTpad + g + 4 * r];
     wave_lds_order();  // the next transpose overwrites the buffer
     return T;
 }

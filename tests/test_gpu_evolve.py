@@ -131,6 +131,29 @@ def test_box_evolve(oracle, monkeypatch, N, nmax, npts, rk, T1, T2, ii):
         assert s.info.device_bytes == query_footprint(cfg, m)
 
 
+@pytest.mark.parametrize("N,nmax,npts,T2,ii", [
+    (9, (0, 1, 0), (3, 5, 1), 80.0, True),     # one lattice vector along a1, a block not full
+    (12, (1, 1, 0), (4, 4, 1), 80.0, False),
+    (13, (2, 0, 1), (5, 2, 2), 0.0, True),     # three chunks of a staged row
+    (16, (3, 1, 0), (9, 3, 1), 80.0, True),    # seven lattice vectors, three blocks a column
+])
+def test_step_blocks(oracle, monkeypatch, N, nmax, npts, T2, ii):
+    """Blocks of four k points and the staged rows of the 9..16-band step (nb16_step_kernel), against the
+    oracle and the separate kernels."""
+    m = synthetic_wannier(N, nmax=nmax, seed=90 + N)
+    cfg = RunConfig(npoints=list(npts), pulses=[Pulse(E0=0.01, w0=0.05, ncycles=0.25, ellip=0.4, envelope="sin2")],
+                    dt=0.5, T2=T2, rk_order=4, inter_intra=ii)
+    print(N, nmax, npts, flush=True)
+    ref = oracle.run(cfg, m, nthreads=8, want_state=True)
+    got = _run(cfg, m)
+    with monkeypatch.context() as mp:
+        mp.setenv("ANTELOPE_NB_FUSED", "0")
+        sep = _run(cfg, m)
+    for key in ("j_inter", "j_intra", "band_pop", "rho_bar", "state"):
+        if np.linalg.norm(ref[key]) > 0.0:
+            assert rel_l2(got[key], ref[key]) < 1e-10 and rel_l2(got[key], sep[key]) < 1e-10, key
+
+
 @pytest.mark.parametrize("N,npts,rk,T1,T2,ii", [
     (1, (5, 1, 1), 5, 0.0, 80.0, True),
     (3, (3, 3, 1), 4, 120.0, 80.0, False),
