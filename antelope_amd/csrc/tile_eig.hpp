@@ -82,8 +82,10 @@ __device__ __forceinline__ double angles(const T &W, T &K, int N, double &lam_c)
 // W = U^dag H U is nearly diagonal, W = L + E. One round takes the angles to second
 // order: with K the angles of W, the angles X of W + [E, K] / 2 (the part of the
 // rotated W that K leaves at second order), U <- U (I + X + X^2/2). What is left off
-// the diagonal is then of third order: a round that starts at max|K| < 1e-5 is the
-// last (eigenvector error 1e-15), one that starts below 1e-7 needs K alone. Three
+// the diagonal is then of third order, times the ratio of the largest gap to the
+// smallest: a round that starts at max|K| < 1e-6 is the last, one that starts below 1e-7 needs
+// K alone. (From 1e-5 on as the last, 16 bands took 1.5% less time, but their intraband current,
+// nearly cancelled over k, was off the oracle by 2e-13 instead of 6e-15.) Three
 // products a round against four of a first-order round, and no second round where a
 // first-order scheme would need one. Later rounds take W from H again with
 // G = U^dag U = I + e: W - e (W_ii + W_jj) / 2 is W in orthonormal columns, and
@@ -100,7 +102,7 @@ __device__ __forceinline__ void eig_refine(const T &Hin, T &U, T &Ut, int N, cd 
                            double *lam_out = nullptr)
 {
     constexpr int E = Shape<T>::E;
-    constexpr double kFar = 0.09, kLast2 = 1e-10, kLast1 = 1e-14;  // squares of 0.3, 1e-5, 1e-7
+    constexpr double kFar = 0.09, kLast2 = 1e-12, kLast1 = 1e-14;  // squares of 0.3, 1e-6, 1e-7
     const int c = Shape<T>::col();
     T H = Hin;
     if (!herm) {

@@ -154,6 +154,23 @@ def test_step_blocks(oracle, monkeypatch, N, nmax, npts, T2, ii):
             assert rel_l2(got[key], ref[key]) < 1e-10 and rel_l2(got[key], sep[key]) < 1e-10, key
 
 
+@pytest.mark.parametrize("N,npts,nmax", [(8, (5, 5, 3), (1, 1, 1)), (16, (6, 5, 1), (2, 2, 0))])
+def test_refined_eigenvectors_hold_rounding(oracle, N, npts, nmax):
+    """The refinement may end only where what it leaves off the diagonal is below rounding also between
+    bands whose gap is a hundredth of the largest: the intraband current, which the k sum nearly cancels and
+    which is first order in the eigenvectors' error, within 200 roundings (4.5e-14; 6e-15 reached, 2e-13 where a
+    round from max|K| = 1e-5 was the last)."""
+    m = synthetic_wannier(N, nmax=nmax, seed=40 + N)
+    cfg = RunConfig(npoints=list(npts), pulses=[Pulse(E0=0.01, w0=0.05, ncycles=0.5, ellip=0.4, envelope="sin2")],
+                    dt=0.5, T2=80.0, rk_order=4, inter_intra=True)
+    print(N, npts, flush=True)
+    ref = oracle.run(cfg, m, nthreads=8)
+    got = _run(cfg, m)
+    e = {key: rel_l2(got[key], ref[key]) for key in ("j_inter", "j_intra", "band_pop", "rho_bar")}
+    print({k: f"{v:.1e}" for k, v in e.items()}, flush=True)
+    assert all(v < 200 * 2.0**-52 for v in e.values()), e
+
+
 @pytest.mark.parametrize("N,npts,rk,T1,T2,ii", [
     (1, (5, 1, 1), 5, 0.0, 80.0, True),
     (3, (3, 3, 1), 4, 120.0, 80.0, False),
