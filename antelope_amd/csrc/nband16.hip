@@ -307,8 +307,8 @@ __global__ __launch_bounds__(64) void nb16_vel_step_kernel(const NbArgs a, const
 }
 
 
-// ------------------------------------------------- fused RK4 step ----
-// One RK4 step per launch (SBEs.h:596-624 with the stage right-hand side of
+// ------------------------------------------------- fused RK step -----
+// One RK4 or RK5 step per launch (SBEs.h:596-624 with the stage right-hand side of
 // SBEs.h:762-861 and the sample of SBEs.h:694-760), for a product k grid with
 // separable Fourier sums. Block = four k points that share (k2, k3) and differ
 // along a1, one wave each. The sums' last pass (along a1),
@@ -324,19 +324,28 @@ __global__ __launch_bounds__(64) void nb16_vel_step_kernel(const NbArgs a, const
 // one partial row per block.
 //
 // Bound by the FP64 pipe, which MFMA and VALU share: per k point 31 thousand cycles of
-// MFMA (30 products), about 16 of VALU, and 30 of waits for LDS, barriers and MFMA results that
-// the second wave of the SIMD covers in part. Two staging slots instead of four let two
+// MFMA (30 products), about 16 of VALU, and 30 of waits for LDS, barriers and MFMA results
+// that the second wave of the SIMD covers in part. Two staging slots instead of four let two
 // blocks of four waves share a CU (one of eight before): while one waits at a barrier the
-// other has products to do. That and one fixed chunk of every staged row per wave, in place of a chunk
-// list with a division per load (3800 scalar instructions per k point), took 48x48x8 with 16
-// bands from 371 to 328 ms, 628 steps; six wave sums in one (wave_sum8) are part of it.
+// other has products to do. That and one fixed chunk of every staged row per wave, in place
+// of a chunk list with a division per load (3800 scalar instructions per k point), took
+// 48x48x8 with 16 bands from 371 to 329 ms, 628 steps; six wave sums in one (wave_sum8) are
+// part of it.
+//
+// RK5 (Fehlberg): the same blocks and staging over five later times; the six stage
+// derivatives stay in registers, so one wave has a SIMD to itself (512 registers). One launch
+// instead of fourteen: 247 -> 105 us a step on 24x24 k points, 2162 -> 1600 on 48x48x8,
+// 16 bands; 207 -> 83 on 14x14, 12 bands.
+
 // dynamic LDS of a block: the waves' transpose buffers (which also hold a wave's sample
 // sums once), then two staging slots of kNbFusedMaxM1 x 256 complex each (row m of the
-// second-pass output at m * 256, so the m offsets are immediates). The slots fill straight from global memory (global_load_lds); their tiles are
-// formed into registers first, so they fill again while the block computes.
+// second-pass output at m * 256, so the m offsets are immediates). The slots fill straight
+// from global memory (global_load_lds); their tiles are formed into registers first, so they
+// fill again while the block computes.
 constexpr int kFusedW = kNbFusedWaves;
 constexpr int kFusedPitch = 256;
 constexpr int kFusedBuf = 16 * kTpad;  // complex per wave
+static_assert(64 * kFusedW >= 256, "a wave per chunk of a 16 x 16 matrix");
 static_assert(2 * kFusedBuf >= 6 + 16 + 2 * 256, "a wave's sample sums fit its transpose buffer");
 
 __device__ __forceinline__ cd *fused_slot(cd *lds, int slot)
@@ -424,7 +433,8 @@ __device__ __forceinline__ double lane_value(double x, int j)
     return __hiloint2double(hi, lo);
 }
 
-__global__ __launch_bounds__(64 * kFusedW) __attribute__((amdgpu_waves_per_eu(2))) void nb16_step_kernel(
+template <int RK>
+__global__ __launch_bounds__(64 * kFusedW) __attribute__((amdgpu_waves_per_eu(RK == 4 ? 2 : 1))) void nb16_step_kernel(
     const NbArgs a, const NbFused f, cd *__restrict__ rho, cd *__restrict__ Ust, double *__restrict__ partials)
 {
     extern __shared__ cd step_lds[];
@@ -449,6 +459,12 @@ __global__ __launch_bounds__(64 * kFusedW) __attribute__((amdgpu_waves_per_eu(2)
     cd *e1 = fused_slot(step_lds, 2) + w * kNbFusedMaxM1;
     if (lane < M1) e1[lane] = a.boxE[0][static_cast<int64_t>(active ? k1 : 0) * M1 + lane];
 
+    // RK4: H~ is Hermitian (its conjugate is H~^T's tile); RK5 takes it as a general matrix
+    constexpr bool kHerm = RK == 4;
+    auto form_ht = [&](int slot) {
+        const Tile T = form_tile(fused_slot(step_lds, slot), e1, M1, N);
+        return kHerm ? T : transpose(T, buf);
+    };
     Tile R, U, Ut, Y, Acc, Ht, X;
     double lam = 0.0, p = 0.0;
     double pop = 0.0;
@@ -518,7 +534,7 @@ __global__ __launch_bounds__(64 * kFusedW) __attribute__((amdgpu_waves_per_eu(2)
     fused_wait();  // [J_z H~]
     if (active) {
         current(2, form_tile(fused_slot(step_lds, 0), e1, M1, N));
-        Ht = form_tile(fused_slot(step_lds, 1), e1, M1, N);  // H~ (Hermitian: its conjugate is H~^T's tile)
+        Ht = form_ht(1);
     }
     // ---- the block's sample sums: one partial row, waves added in order
     {
@@ -548,8 +564,9 @@ __global__ __launch_bounds__(64 * kFusedW) __attribute__((amdgpu_waves_per_eu(2)
         __syncthreads();  // sums read: the transpose buffers are free
     }
     // ---- stage 1 at t_n
+    if (active) X = stage_derivative_m<kHerm>(a, R, Ht, M, buf);
+    if constexpr (RK == 4) {
     if (active) {
-        X = stage_derivative_m<true>(a, R, Ht, M, buf);
         axpy_tile(Acc, X, dt / 6.0, R);
         axpy_tile(Y, X, 0.5 * dt, R);
     }
@@ -595,6 +612,65 @@ __global__ __launch_bounds__(64 * kFusedW) __attribute__((amdgpu_waves_per_eu(2)
         if (a.deph) Me = band_diag(Y, U, Ut, dd);
         X = stage_derivative_m<true>(a, Y, Ht, Me, buf);
         axpy_tile(R, X, dt / 6.0, Acc);
+    }
+    } else {
+        // c = 0, 1/4, 3/8, 12/13, 1, 1/2: the last stage starts its eigenvectors from those at 3/8,
+        // the step's own go on to the next sample
+        using C = dev::Coef<5>;
+        Tile Kd[6], Vm, Vmt, H;
+        Kd[0] = X;
+        auto input = [&](int st) {
+            Tile Yi = R;
+#pragma unroll
+            for (int j = 0; j < 5; ++j)
+                if (j < st && C::a[st][j] != 0.0) axpy_tile(Yi, Kd[j], dt * C::a[st][j], Yi);
+            return Yi;
+        };
+        // H~, H of the time staged last; the slots then take those of src (if given)
+        auto pair = [&](const cd *src) {
+            fused_wait();
+            if (active) {
+                Ht = form_ht(0);
+                H = form_tile(fused_slot(step_lds, 1), e1, M1, N);
+            }
+            __syncthreads();  // slots read
+            if (src) stage_async(a, step_lds, src, 0, src, 1, col, w, lane);
+        };
+        auto deriv = [&](int st, const Tile &V, const Tile &Vt) {
+            const Tile Yi = input(st);
+            Tile Md{};
+            double dd;
+            if (a.deph) Md = band_diag(Yi, V, Vt, dd);
+            Kd[st] = stage_derivative_m<false>(a, Yi, Ht, Md, buf);
+        };
+        const cd *mid = f.t2_half;
+#pragma unroll
+        for (int st = 1; st <= 3; ++st) {  // 1/4, 3/8, 12/13
+            pair(st < 3 ? mid + st * f.mid_stride : f.t2_end);
+            if (active) {
+                if (a.deph) eig_refine(H, U, Ut, N, buf, true, false);
+                deriv(st, U, Ut);
+                if (st == 2) {
+                    Vm = U;
+                    Vmt = Ut;
+                }
+            }
+        }
+        pair(mid + 3 * f.mid_stride);
+        if (active) {
+            eig_refine(H, U, Ut, N, buf, true, false, &lam);
+            deriv(4, U, Ut);
+        }
+        pair(nullptr);
+        if (active) {
+            if (a.deph) eig_refine(H, Vm, Vmt, N, buf, true, false);
+            deriv(5, Vm, Vmt);
+#pragma unroll
+            for (int j = 0; j < 6; ++j)
+                if (C::b[j] != 0.0) axpy_tile(R, Kd[j], dt * C::b[j], R);
+        }
+    }
+    if (active) {
         store_tile(rho + k * nn, R, N);
         store_tile(Ust + k * nn, U, N);
         if (lane < 16) f.lam[k * 16 + c] = lam;
@@ -659,16 +735,25 @@ static hipError_t allow_lds(const void *kernel, size_t lds)
     return hipSuccess;
 }
 
-hipError_t nb16_launch_step(const NbArgs &a, const NbFused &f, double2 *rho, double2 *U, double *partials,
+template <int RK>
+static hipError_t launch_step(const NbArgs &a, const NbFused &f, double2 *rho, double2 *U, double *partials,
+                              hipStream_t s)
+{
+    constexpr size_t lds = sizeof(double2) * static_cast<size_t>(
+        kFusedW * kFusedBuf + 2 * kNbFusedMaxM1 * kFusedPitch + kFusedW * kNbFusedMaxM1);
+    const hipError_t e = allow_lds(reinterpret_cast<const void *>(&nb16_step_kernel<RK>), lds);
+    if (e != hipSuccess) return e;
+    nb16_step_kernel<RK><<<dim3(static_cast<unsigned>(f.nblocks)), 64 * kFusedW, lds, s>>>(a, f, rho, U, partials);
+    return hipGetLastError();
+}
+
+hipError_t nb16_launch_step(const NbArgs &a, const NbFused &f, int rk_order, double2 *rho, double2 *U, double *partials,
                             hipStream_t s)
 {
     if (a.N > 16 || !a.box || a.boxM[0] < 1 || a.boxM[0] > kNbFusedMaxM1 || f.nblocks < 1) return hipErrorInvalidValue;
-    constexpr size_t lds = sizeof(double2) * static_cast<size_t>(
-        kFusedW * kFusedBuf + 2 * kNbFusedMaxM1 * kFusedPitch + kFusedW * kNbFusedMaxM1);
-    const hipError_t e = allow_lds(reinterpret_cast<const void *>(&nb16_step_kernel), lds);
-    if (e != hipSuccess) return e;
-    nb16_step_kernel<<<dim3(static_cast<unsigned>(f.nblocks)), 64 * kFusedW, lds, s>>>(a, f, rho, U, partials);
-    return hipGetLastError();
+    if (rk_order == SBE_RK4) return launch_step<4>(a, f, rho, U, partials, s);
+    if (rk_order == SBE_RK5_FEHLBERG) return launch_step<5>(a, f, rho, U, partials, s);
+    return hipErrorInvalidValue;
 }
 
 }  // namespace sbe

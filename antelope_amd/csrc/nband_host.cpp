@@ -163,12 +163,12 @@ bool fused_eligible(const sbe_config &cfg, const sbe_model &m, int64_t nk, const
     return true;  // the whole grid, or a k block of it (holes in the box are idle waves)
 }
 
-// RK5 (Fehlberg) steps of small Wannier models (nb_box_evolve_kernel): as fused_eligible with
-// N <= 8. The plan does not depend on ANTELOPE_NB_FUSED, which only selects the kernels that run.
-bool rk5_small_eligible(const sbe_config &cfg, const sbe_model &m, int64_t nk, const BoxShape &bx)
+// RK5 (Fehlberg) steps of Wannier models with N <= 16 (nb_box_evolve_kernel, nb16_step_kernel): as
+// fused_eligible. The plan does not depend on ANTELOPE_NB_FUSED, which only selects the kernels that run.
+bool rk5_eligible(const sbe_config &cfg, const sbe_model &m, int64_t nk, const BoxShape &bx)
 {
     if (!bx.ok || cfg.rk_order != SBE_RK5_FEHLBERG || cfg.gauge != SBE_GAUGE_LENGTH_WANNIER ||
-        cfg.precision != SBE_PREC_FP64 || am::is_analytic(m.kind) || m.is_dipole_zero || m.nband > 8 ||
+        cfg.precision != SBE_PREC_FP64 || am::is_analytic(m.kind) || m.is_dipole_zero || m.nband > 16 ||
         bx.M[0] > kNbFusedMaxM1)
         return false;
     sbe_tuning tu{};
@@ -500,7 +500,7 @@ size_t nb_footprint(const sbe_config &cfg, const sbe_model &m, int64_t nk, int64
 {
     const bool split16 = cfg.precision == SBE_PREC_SPLIT16;
     const BoxShape bx = box_shape(cfg, m, nk, split16);
-    const bool fused = fused_eligible(cfg, m, nk, bx) || rk5_small_eligible(cfg, m, nk, bx);
+    const bool fused = fused_eligible(cfg, m, nk, bx) || rk5_eligible(cfg, m, nk, bx);
     const bool vfused = vel_fused_eligible(cfg, m, nk);
     const bool f32 = nb32_eligible(cfg, m);
     AnalyticTerms terms;
@@ -577,7 +577,7 @@ int nb_setup(sbe_ctx *ctx)
     const int64_t nk = ctx->grid.k_end - ctx->grid.k_begin;
     const bool split16 = ctx->cfg.precision == SBE_PREC_SPLIT16;
     const BoxShape bx = box_shape(ctx->cfg, m, nk, split16);
-    const bool fused = fused_eligible(ctx->cfg, m, nk, bx) || rk5_small_eligible(ctx->cfg, m, nk, bx);
+    const bool fused = fused_eligible(ctx->cfg, m, nk, bx) || rk5_eligible(ctx->cfg, m, nk, bx);
     const bool vfused = vel_fused_eligible(ctx->cfg, m, nk);
     const bool f32 = nb32_eligible(ctx->cfg, m);
     AnalyticTerms terms;
@@ -1014,7 +1014,8 @@ int nb_run_fused(sbe_ctx *ctx, int64_t step_begin, int64_t step_end)
                 NbFused f{};
                 f.t2_prev = pair(step - 1);
                 f.t2_j = ctx->nbf_tj + i * t2s;
-                f.t2_half = ctx->nbf_th + i * t2s;
+                f.t2_half = ctx->nbf_th + i * ctx->nbf_mids * t2s;
+                f.mid_stride = t2s;
                 f.t2_end = pair(step);
                 f.lam = ctx->nbf_lam;
                 f.u_valid = same_time(ctx->nb_u_time, tn, dt) ? 1 : 0;
@@ -1023,7 +1024,8 @@ int nb_run_fused(sbe_ctx *ctx, int64_t step_begin, int64_t step_end)
                 f.step_local = s + i;
                 f.g1 = ctx->nbf_g1;
                 f.nblocks = ctx->nbf_nblocks;
-                rc = hipc(ctx, nb16_launch_step(a, f, ctx->nb_rho, ctx->nb_U, ctx->d_partials, ctx->stream), "step kernel");
+                rc = hipc(ctx, nb16_launch_step(a, f, ctx->cfg.rk_order, ctx->nb_rho, ctx->nb_U, ctx->d_partials, ctx->stream),
+                          "step kernel");
                 // the end of this step is the start of the next: its H~, H serve there
                 ctx->nbf_prev_time = tn + dt;
                 ctx->nbf_prev_valid = true;

@@ -154,6 +154,46 @@ def test_step_blocks(oracle, monkeypatch, N, nmax, npts, T2, ii):
             assert rel_l2(got[key], ref[key]) < 1e-10 and rel_l2(got[key], sep[key]) < 1e-10, key
 
 
+@pytest.mark.parametrize("N,nmax,npts,T1,T2,ii", [
+    (9, (0, 1, 0), (3, 5, 1), 0.0, 80.0, True),
+    (12, (1, 1, 0), (4, 4, 1), 120.0, 80.0, False),
+    (13, (2, 0, 1), (5, 2, 2), 0.0, 0.0, True),
+    (16, (3, 1, 0), (9, 3, 1), 150.0, 80.0, True),
+    (16, (1, 1, 0), (64, 8, 1), 0.0, 80.0, True),  # scratch in the stage-derivative slots
+])
+def test_step_rk5(oracle, monkeypatch, N, nmax, npts, T1, T2, ii):
+    """RK5 steps of 9 to 16 bands (nb16_step_kernel<5>), positions not Hermitian (H~ = H + E.D is used as a
+    general matrix), against the oracle, the separate kernels, split runs and k blocks."""
+    m = synthetic_wannier(N, nmax=nmax, seed=110 + N)
+    m.pos = m.pos * (1.0 + 0.3j)
+    cfg = RunConfig(npoints=list(npts), pulses=[Pulse(E0=0.01, w0=0.05, ncycles=0.125, ellip=0.4, envelope="sin2")],
+                    dt=0.5, T1=T1, T2=T2, rk_order=5, inter_intra=ii)
+    print(N, nmax, npts, flush=True)
+    ref = oracle.run(cfg, m, nthreads=8, want_state=True)
+    got = _run(cfg, m)
+    split = _run(cfg, m, cuts=(1, 2, 17))
+    nk = int(np.prod(npts))
+    cut = nk // 2 + 1
+    blocks = [_run(cfg, m, k_begin=a, k_end=b) for a, b in ((0, cut), (cut, nk))]
+    with monkeypatch.context() as mp:
+        mp.setenv("ANTELOPE_NB_EVAL_STEPS", "3")
+        three = _run(cfg, m)
+        mp.setenv("ANTELOPE_NB_FUSED", "0")
+        sep = _run(cfg, m)
+    for key in ("j_inter", "j_intra", "band_pop", "rho_bar", "state"):
+        assert np.array_equal(got[key], split[key]), key
+        assert np.array_equal(got[key], three[key]), key
+        if np.linalg.norm(ref[key]) == 0.0:
+            continue
+        e, es = rel_l2(got[key], ref[key]), rel_l2(got[key], sep[key])
+        print(f"  {key}: oracle {e:.1e}, separate kernels {es:.1e}", flush=True)
+        assert e < 1e-10 and es < 1e-10, key
+        if key != "state":
+            assert rel_l2(blocks[0][key] + blocks[1][key], ref[key]) < 1e-10, key
+    with SBESolver(cfg, m) as s:
+        assert s.info.device_bytes == query_footprint(cfg, m)
+
+
 @pytest.mark.parametrize("N,npts,nmax", [(8, (5, 5, 3), (1, 1, 1)), (16, (6, 5, 1), (2, 2, 0))])
 def test_refined_eigenvectors_hold_rounding(oracle, N, npts, nmax):
     """The refinement may end only where what it leaves off the diagonal is below rounding also between
