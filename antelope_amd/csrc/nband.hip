@@ -824,8 +824,9 @@ __device__ void weigh(cd *A, cd *U, double *ev, cd *work, int N, double4 *rot, b
     wcopy(U, work, nn);
 }
 
-// Warm-started eigenvectors for the LDS kernels: the simultaneous-rotation
-// refinement of nband16.hip's eig_refine on LDS matrices and wmm products.
+// Warm-started eigenvectors for the LDS kernels: simultaneous Jacobi rotations
+// written as wmm products on LDS matrices (first order in the angles; the register
+// tiles' eig_refine takes them to second order).
 // In: A = H (overwritten; its Hermitian part is used), U = eigenvectors of a
 // nearby H; Hsrc = H in memory (reloaded when W is rebuilt). Out: U refined,
 // columns in the warm start's order. W, T, X: scratch. Pointers are swapped

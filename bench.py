@@ -51,8 +51,9 @@ PEAK_HBM_GBS = 8000.0
 ALGO_BYTES_PER_KSTEP = {"fp64": 128.0, "fp32": 64.0, "adaptive_fp64": 128.0}
 # Executed flops per k-point RK4 step of the step kernel, from the rocprofv3
 # counters SQ_INSTS_VALU_{FMA,MUL,ADD}_{F64,F32} (FMA = 2) on this workload:
-# FP64 385; FP32 state 365 FP32 + 26 FP64 (the k sums).
-FLOPS_PER_KSTEP = {"fp64": 385.0, "fp32": 391.0}
+# FP64 337; FP32 state 326 FP32 + 11 FP64 (the k sums run on the matrix pipe and are not
+# counted).
+FLOPS_PER_KSTEP = {"fp64": 337.2, "fp32": 336.8}
 KERNEL_NAME = {"fp64": "haldane_steps_kernel<double, 4, false, true, 2>",
                "fp32": "haldane_steps_kernel<float, 4, false, true, 1>",
                "adaptive_fp64": "haldane_adaptive_kernel<double, true, 1>"}
@@ -66,7 +67,7 @@ VEL_FLOPS_PER_KSTEP = {"fp64": 181.0, "fp32": 181.0}
 # on the 64 x 200^2 batch (profiles/haldane_batch_64x200x200_traffic.json);
 # includes rejected attempts and the per-wave laser, controller, reduction and
 # sample work counted on all 64 lanes
-ADAPT_FLOPS_PER_KSTEP = {"fp64": 929.8}
+ADAPT_FLOPS_PER_KSTEP = {"fp64": 880.8}
 
 
 def wannier_workload(precision: str = "fp64"):
@@ -352,7 +353,7 @@ def bench_serving(args) -> int:
 # counters SQ_INSTS_VALU_{FMA,MUL,ADD}_F64 (FMA = 2, x 64 lanes) on this workload's
 # generator: per RK4 step for the plain kernel, per accepted step for the adaptive one
 # (rejected attempts and the per-wave laser, controller and reduction work included).
-BATCH_FLOPS = {"plain_fp64_rk4": 392.6, "adaptive_fp64": ADAPT_FLOPS_PER_KSTEP["fp64"]}
+BATCH_FLOPS = {"plain_fp64_rk4": 340.3, "adaptive_fp64": ADAPT_FLOPS_PER_KSTEP["fp64"]}
 BATCH_KERNEL = {"plain_fp64_rk4": "haldane_batch_kernel<double, 4, false, true>",
                 "plain_fp32_rk4": "haldane_batch_kernel<float, 4, false, true>",
                 "adaptive_fp64": "haldane_adaptive_kernel<double, true, 1>",
