@@ -26,7 +26,7 @@
 // FP64 chain at 4 cycles an instruction, about 240 of them for an RK4 step of a k point
 // (316 before the k sums moved to the matrix pipe and the sample and the right-hand side
 // were factored; 465 for RK5 with T1), so fewer instructions are what there is to gain.
-#include "haldane_dev.hpp"
+#include "haldane_setup.hpp"
 
 namespace sbe {
 namespace {
@@ -287,55 +287,10 @@ __global__ __launch_bounds__(kBlock) void haldane_batch_kernel(const HaldaneArgs
                                      static_cast<int64_t>(blockIdx.x) - block_first[inst]);
 }
 
-// Initial state (SBEs.h:284-364): rho_H = diag(occupations) at k, rho = U rho_H U^dag
-// -> n = f0 + f1, s = (f1 - f0) dh(k). Padding points get a zero state.
 template <typename R>
 __global__ __launch_bounds__(kBlock) void haldane_init_kernel(HaldaneArgs a, int nval, int fermi, double ef)
 {
-    const int64_t k = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-    const int64_t ks = a.nk_stride;
-    R *st = static_cast<R *>(a.state);
-    double n = 0, sx = 0, sy = 0, sz = 0;
-    if (k < a.nk) {
-        const double kx = a.kpts[k], ky = a.kpts[ks + k];
-        double er[6], ei[6];
-        for (int j = 0; j < 3; ++j) {
-            sincos(kx * a.va[j][0] + ky * a.va[j][1], &ei[j], &er[j]);
-            sincos(kx * a.vb[j][0] + ky * a.vb[j][1], &ei[j + 3], &er[j + 3]);
-        }
-        const Vec3<double> d = dvec<double>(er, ei, a.t1, a.c3, a.M0);
-        const double d0 = a.c0 * (er[3] + er[4] + er[5]);
-        const double dn = sqrt(d.x * d.x + d.y * d.y + d.z * d.z);
-        double hx = 0, hy = 0, hz = -1;  // degenerate point: eigenbasis = orbital basis
-        if (dn > 0) { hx = d.x / dn; hy = d.y / dn; hz = d.z / dn; }
-        double f0, f1;
-        if (fermi) {
-            const double kT = 300.0 / 3.15775024804e5;
-            f0 = 1.0 / (exp((d0 - dn - ef) / kT) + 1.0);
-            f1 = 1.0 / (exp((d0 + dn - ef) / kT) + 1.0);
-            const double sum = f0 + f1;
-            f0 /= sum;
-            f1 /= sum;
-        } else {
-            f0 = nval > 0 ? 1.0 : 0.0;
-            f1 = nval > 1 ? 1.0 : 0.0;
-        }
-        n = f0 + f1;
-        sx = (f1 - f0) * hx;
-        sy = (f1 - f0) * hy;
-        sz = (f1 - f0) * hz;
-    }
-    st[k] = static_cast<R>(n);
-    st[ks + k] = static_cast<R>(sx);
-    st[2 * ks + k] = static_cast<R>(sy);
-    st[3 * ks + k] = static_cast<R>(sz);
-    if (StateT<R>::kComp) {
-        // compensation = -(low part) so that value = hi - c is exact in FP64
-        st[4 * ks + k] = static_cast<R>(static_cast<double>(static_cast<R>(n)) - n);
-        st[5 * ks + k] = static_cast<R>(static_cast<double>(static_cast<R>(sx)) - sx);
-        st[6 * ks + k] = static_cast<R>(static_cast<double>(static_cast<R>(sy)) - sy);
-        st[7 * ks + k] = static_cast<R>(static_cast<double>(static_cast<R>(sz)) - sz);
-    }
+    init_point<R>(a, static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x, nval, fermi, ef);
 }
 
 // Orbital-basis AoS export: rho[k][2][2][re,im] (the reference dmatrix).

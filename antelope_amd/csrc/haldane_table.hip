@@ -6,64 +6,32 @@
 // over; 300 x 300 k, 86,168 rows: create 10.9 ms that way, 0.30 ms here.
 #include <cstring>
 
-#include "sbe_internal.hpp"
+#include "haldane_setup.hpp"
 
 namespace sbe {
 namespace {
 
-// A(t) less its value at atmin, the sum of the pulses in order
-__device__ void field_at(const TableArgs &a, double t, double A[3])
-{
-    A[0] = A[1] = A[2] = 0.0;
-    for (int p = 0; p < a.npulses; ++p) {
-        double pa[3], pe[3];
-        pulse_field(a.pulses[p], t, a.consistent != 0, pa, pe);
-        for (int j = 0; j < 3; ++j) A[j] += pa[j];
-    }
-    for (int j = 0; j < 3; ++j) A[j] -= a.A_at_min[j];
-}
+using namespace dev;
 
 __global__ __launch_bounds__(256) void haldane_table_kernel(const TableArgs a, double *__restrict__ tab,
                                                             float *__restrict__ tab32)
 {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= a.nsteps * a.nstage) return;
-    const int64_t n = a.step0 + i / a.nstage;
-    const int s = static_cast<int>(i % a.nstage);
-    const double tn = a.atmin + a.dt * static_cast<double>(n);
-    const double tn1 = a.atmin + a.dt * static_cast<double>(n + 1);
-    // the stage at c = 1 is taken at t_{n+1} itself, so its row is the next step's first row bit
-    // for bit (the step kernels carry it across steps)
-    double A[3];
-    field_at(a, a.c[s] == 1.0 ? tn1 : tn + a.c[s] * a.dt, A);
-    if (a.plain) {
-        tab[2 * i] = A[0];
-        tab[2 * i + 1] = A[1];
-        if (tab32) {
-            tab32[2 * i] = static_cast<float>(A[0]);
-            tab32[2 * i + 1] = static_cast<float>(A[1]);
-        }
+    table_row(a, static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x, tab, tab32);
+}
+
+// the initial state (blocks below nstate) and the laser rows (the others) of an FP64 solve in one
+// launch: neither needs the other, and at 5 and 6 us each they would wait in turn (40 x 40 k points,
+// 64 steps without allocation: 55.7 -> 52.2 us the call)
+__global__ __launch_bounds__(256) void haldane_begin_kernel(const HaldaneArgs h, int fermi, double ef, int nstate,
+                                                            const TableArgs a, double *__restrict__ tab)
+{
+    const int b = static_cast<int>(blockIdx.x);
+    if (b < nstate) {
+        const int64_t k = static_cast<int64_t>(b) * 256 + threadIdx.x;
+        if (k < h.nk_stride) init_point<double>(h, k, h.nval, fermi, ef);
         return;
     }
-    double *row = tab + i * 12;
-    for (int j = 0; j < 3; ++j) {
-        const double pa = A[0] * a.va[j][0] + A[1] * a.va[j][1];
-        const double pb = A[0] * a.vb[j][0] + A[1] * a.vb[j][1];
-        double sa, ca, sb, cb;
-        sincos(pa, &sa, &ca);
-        sincos(pb, &sb, &cb);
-        row[2 * j] = a.t1 * ca;  // NN part carries t1
-        row[2 * j + 1] = a.t1 * sa;
-        row[6 + 2 * j] = cb;
-        row[7 + 2 * j] = sb;
-        if (tab32) {
-            float *r32 = tab32 + i * 12;
-            r32[2 * j] = static_cast<float>(a.t1 * ca);
-            r32[2 * j + 1] = static_cast<float>(a.t1 * sa);
-            r32[6 + 2 * j] = static_cast<float>(cb);
-            r32[7 + 2 * j] = static_cast<float>(sb);
-        }
-    }
+    table_row(a, static_cast<int64_t>(b - nstate) * 256 + threadIdx.x, tab, nullptr);
 }
 
 // A - A(t_min) and the consistent dA/dt = -E at t_n, summed in pulse order
@@ -125,6 +93,18 @@ hipError_t launch_haldane_table(const TableArgs &a, double *tab, float *tab32, h
     if (a.npulses > kMaxDevicePulses || a.nstage < 1 || a.nstage > 7) return hipErrorInvalidValue;
     if (a.nsteps <= 0) return hipSuccess;
     haldane_table_kernel<<<blocks(a.nsteps * a.nstage), 256, 0, s>>>(a, tab, tab32);
+    return hipGetLastError();
+}
+
+hipError_t launch_haldane_begin(const HaldaneArgs &h, int init_type, double ef, const TableArgs &a, double *tab,
+                                hipStream_t s)
+{
+    if (h.precision != SBE_PREC_FP64 || a.plain || a.npulses > kMaxDevicePulses || a.nstage < 1 || a.nstage > 7 ||
+        a.nsteps < 1)
+        return hipErrorInvalidValue;
+    const unsigned nstate = blocks(h.nk_stride);
+    haldane_begin_kernel<<<nstate + blocks(a.nsteps * a.nstage), 256, 0, s>>>(
+        h, init_type == SBE_INIT_FERMI_DIRAC, ef, static_cast<int>(nstate), a, tab);
     return hipGetLastError();
 }
 

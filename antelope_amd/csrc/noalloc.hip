@@ -138,7 +138,7 @@ extern "C" int sbe_run_haldane_noalloc(const sbe_config *cfg, const sbe_model *m
     h.kpts = kpts;
     h.weight = kpts + 3 * nk_stride;
     h.state = state;
-    if (init_state) {
+    if (init_state && step_begin == step_end) {
         e = launch_haldane_init(h, cfg->init_type, cfg->fermi_energy, s);
         if (e != hipSuccess) return hip_fail(e, "init kernel");
     }
@@ -153,7 +153,9 @@ extern "C" int sbe_run_haldane_noalloc(const sbe_config *cfg, const sbe_model *m
         const int64_t n = std::min<int64_t>(chunk, step_end - s0);
         ta.step0 = s0;
         ta.nsteps = n;
-        if ((e = launch_haldane_table(ta, d_tab, nullptr, s)) != hipSuccess) return hip_fail(e, "table kernel");
+        if (init_state && s0 == step_begin) e = launch_haldane_begin(h, cfg->init_type, cfg->fermi_energy, ta, d_tab, s);
+        else e = launch_haldane_table(ta, d_tab, nullptr, s);
+        if (e != hipSuccess) return hip_fail(e, "table kernel");
         HaldaneArgs a = h;
         a.phase_tab = d_tab;
         a.step0 = 0;  // the table starts at this launch's first step

@@ -274,6 +274,9 @@ namespace sbe {
 // points and weights of a block, SoA [4][nk_stride] (zeros past nk)
 TableArgs table_args(const Laser &L, const Tableau &t, int nstage, double t1, const double va[3][2], const double vb[3][2]);
 hipError_t launch_haldane_table(const TableArgs &a, double *tab, float *tab32, hipStream_t s);
+// launch_haldane_init and launch_haldane_table of an FP64 solve in one launch
+hipError_t launch_haldane_begin(const HaldaneArgs &h, int init_type, double ef, const TableArgs &a, double *tab,
+                                hipStream_t s);
 hipError_t launch_field_table(const TableArgs &a, int64_t rows, double *at, hipStream_t s);
 hipError_t launch_kgrid(const GridArgs &g, int64_t k_begin, int64_t nk, int64_t nk_stride, double *kpts, hipStream_t s);
 // Launchers (haldane.hip, series.hip).

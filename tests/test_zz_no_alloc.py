@@ -140,3 +140,18 @@ def test_noalloc_rejects_what_it_does_not_run():
     rc = lib.sbe_run_haldane_noalloc(C.byref(c), C.byref(m), dummy, dummy, n, n, 0, 10, 1, dummy, None)
     assert rc == A.SBE_ERR_RANGE
     assert b"scratch" in lib.sbe_last_error(None)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,steps,rk", [((1, 1), 1, 4), ((16, 16), 64, 4), ((23, 23), 65, 4), ((16, 16), 43, 5)])
+def test_noalloc_first_launch(n, steps, rk):
+    """The initial state and the laser rows in one launch (haldane_begin_kernel), at the edges of its blocks."""
+    model = haldane_cfg1_model()
+    cfg = small_config(n=n, ncycles=1.0, ellip=0.3, rk=rk, grid="mp")
+    ref = _rows_from_solver(cfg, model, steps)
+    p = Problem(cfg, model)
+    print("noalloc:", n, steps, rk, flush=True)
+    got = p.run(0, steps, init=True)
+    p.free()
+    assert np.isfinite(got).all()
+    assert np.abs(got - ref).max() <= 1e-12 * np.abs(ref).max()
