@@ -91,11 +91,49 @@ __device__ __forceinline__ void occupations(const HaldaneArgs &a, double e0, dou
 
 constexpr int kTile = 64;  // time steps per LDS tile of the A(t) table
 
+// Sum each of v[0..7] over the 64 lanes of the wave (reduce-scatter):
+// lane l ends with the total of v[(l >> 3) & 7]. Requires all 64 lanes.
+__device__ __forceinline__ double wave_reduce8(double v[8])
+{
+    const int lane = __lane_id();
+    // lane bit 5: permlane32 swap + add
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        double a = v[j], b = v[j + 4];
+        swap32(a, b);
+        v[j] = a + b;  // lanes 0-31: v[j], lanes 32-63: v[j+4]
+    }
+    // lane bit 4: permlane16 swap + add
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        double a = v[j], b = v[j + 2];
+        swap16(a, b);
+        v[j] = a + b;  // even rows: v[j], odd rows: v[j+2]
+    }
+    // lane bit 3: rotate by 8 inside each 16-lane row (= lane ^ 8)
+    const bool hi = (lane & 8) != 0;
+    const double keep = hi ? v[1] : v[0];
+    const double send = hi ? v[0] : v[1];
+    double x = keep + dpp_f64<0x128>(send);  // row_ror:8
+    // lanes 8q..8q+7 now share value index q: all-reduce over the low 3 bits
+    x += dpp_f64<0x141>(x);  // row_half_mirror (i <-> 7-i)
+    x += dpp_f64<0x4E>(x);   // quad_perm [2,3,0,1]
+    x += dpp_f64<0xB1>(x);   // quad_perm [1,0,3,2]
+    return x;
+}
+
+// The k sums of a step: on the matrix pipe (wave_sum8), which saves issue slots, from this many
+// waves up; below, by swaps and DPP (wave_reduce8), whose chain is shorter: this gauge's step has
+// little else to put beside it. RK4, us a step, swaps against matrix pipe: 48x48 k points 0.300
+// and 0.332, 200x200 0.332 and 0.346, 300x300 (1408 waves) 0.510 and 0.522, 800x800 (10000
+// waves) 2.71 and 2.45.
+constexpr int kMatrixSumWaves = 4096;
+
 // Step kernel body; R, RK, T1ON, DEPH, KPT as in the length-gauge kernel.
 // The stage right-hand side is evaluated as half of the reference RHS with
 // the factor 2 folded into the RK coefficients:
 //   f/2 = h x y - (g2/2)(y_x, y_y, 0) - (g1/2)(0, 0, y_z - s0_z).
-template <typename R, int RK, bool T1ON, bool DEPH, int KPT>
+template <typename R, int RK, bool T1ON, bool DEPH, int KPT, bool MSUM>
 __device__ __forceinline__ void vel_body(const HaldaneArgs &a, const R *__restrict__ tabr, R *__restrict__ st,
                                          double *__restrict__ partials, int64_t blk)
 {
@@ -195,7 +233,9 @@ __device__ __forceinline__ void vel_body(const HaldaneArgs &a, const R *__restri
             v[6] += static_cast<double>(z) * w;
             v[7] -= static_cast<double>(z) * w;  // band populations (n -+ v7)/2 as in the length gauge
         }
-        partials[(static_cast<int64_t>(step) * a.nwaves + wave) * kHaldaneNV + sum8_value(lane)] = wave_sum8(v);
+        double *row = partials + (static_cast<int64_t>(step) * a.nwaves + wave) * kHaldaneNV;
+        if (MSUM) row[sum8_value(lane)] = wave_sum8(v);
+        else row[lane >> 3] = wave_reduce8(v);
 
         // ---- one RK step (SBEs.h:596-624)
 #pragma unroll
@@ -279,11 +319,11 @@ __device__ __forceinline__ void vel_body(const HaldaneArgs &a, const R *__restri
     }
 }
 
-template <typename R, int RK, bool T1ON, bool DEPH, int KPT>
+template <typename R, int RK, bool T1ON, bool DEPH, int KPT, bool MSUM>
 __global__ __launch_bounds__(kBlock) void haldane_vel_kernel(const HaldaneArgs a, const R *__restrict__ tabr,
                                                              R *__restrict__ st, double *__restrict__ partials)
 {
-    vel_body<R, RK, T1ON, DEPH, KPT>(a, tabr, st, partials, blockIdx.x);
+    vel_body<R, RK, T1ON, DEPH, KPT, MSUM>(a, tabr, st, partials, blockIdx.x);
 }
 
 // Initial state: rho_H = diag(f0, f1) -> n = f0 + f1, s = (0, 0, f0 - f1).
@@ -315,22 +355,23 @@ __global__ __launch_bounds__(kBlock) void haldane_vel_init_kernel(HaldaneArgs a)
     }
 }
 
-template <typename R, int RK, int KPT>
+template <typename R, int RK, int KPT, bool MSUM>
 void launch_vel(const HaldaneArgs &a, const R *tab, bool t1_on, hipStream_t s)
 {
     const dim3 grid(static_cast<unsigned>(a.nk_stride / (kBlock * KPT)));
     R *st = static_cast<R *>(a.state);
     const bool deph = a.gam1 != 0.0 || a.gam2 != 0.0;
-    if (t1_on) haldane_vel_kernel<R, RK, true, true, KPT><<<grid, kBlock, 0, s>>>(a, tab, st, a.partials);
-    else if (deph) haldane_vel_kernel<R, RK, false, true, KPT><<<grid, kBlock, 0, s>>>(a, tab, st, a.partials);
-    else haldane_vel_kernel<R, RK, false, false, KPT><<<grid, kBlock, 0, s>>>(a, tab, st, a.partials);
+    if (t1_on) haldane_vel_kernel<R, RK, true, true, KPT, MSUM><<<grid, kBlock, 0, s>>>(a, tab, st, a.partials);
+    else if (deph) haldane_vel_kernel<R, RK, false, true, KPT, MSUM><<<grid, kBlock, 0, s>>>(a, tab, st, a.partials);
+    else haldane_vel_kernel<R, RK, false, false, KPT, MSUM><<<grid, kBlock, 0, s>>>(a, tab, st, a.partials);
 }
 
 template <typename R, int RK>
 void launch_vel_kpt(const HaldaneArgs &a, const R *tab, bool t1_on, hipStream_t s)
 {
-    if (a.kpt == 2) launch_vel<R, RK, 2>(a, tab, t1_on, s);
-    else launch_vel<R, RK, 1>(a, tab, t1_on, s);
+    const bool msum = a.nwaves >= kMatrixSumWaves;
+    if (a.kpt == 2) msum ? launch_vel<R, RK, 2, true>(a, tab, t1_on, s) : launch_vel<R, RK, 2, false>(a, tab, t1_on, s);
+    else msum ? launch_vel<R, RK, 1, true>(a, tab, t1_on, s) : launch_vel<R, RK, 1, false>(a, tab, t1_on, s);
 }
 
 }  // namespace

@@ -30,3 +30,20 @@ def test_wave_sums(oracle, n, gauge, rk, inter_intra):
             assert rel_l2(got[key], ref[key]) < 1e-10, key
         else:
             assert not np.any(got[key]), key
+
+
+def test_velocity_sums_by_matrix_pipe():
+    """The velocity gauge's sums change route at 4096 waves (262144 k points): k blocks below it against the
+    whole grid above, the same sums to rounding."""
+    cfg = small_config(n=(520, 505), ncycles=0.02, rk=4, ellip=0.4, grid="mp", T1=300.0, gauge="VelocityHamiltonian")
+    model = haldane_cfg1_model()
+    nk, cut = 520 * 505, 100000
+
+    def run(a, b):
+        with SBESolver(cfg, model, a, b) as s:
+            s.run()
+            return s.series()
+
+    whole, parts = run(-1, -1), [run(0, cut), run(cut, nk)]
+    for key in ("j_inter", "j_intra", "band_pop", "rho_bar"):
+        assert rel_l2(parts[0][key] + parts[1][key], whole[key]) < 1e-10, key
