@@ -124,9 +124,9 @@ __device__ __forceinline__ double wave_reduce8(double v[8])
 
 // The k sums of a step: on the matrix pipe (wave_sum8), which saves issue slots, from this many
 // waves up; below, by swaps and DPP (wave_reduce8), whose chain is shorter: this gauge's step has
-// little else to put beside it. RK4, us a step, swaps against matrix pipe: 48x48 k points 0.300
-// and 0.332, 200x200 0.332 and 0.346, 300x300 (1408 waves) 0.510 and 0.522, 800x800 (10000
-// waves) 2.71 and 2.45.
+// little else to put beside it. RK4, us a step, swaps against matrix pipe: 48x48 k points 0.301
+// and 0.332, 200x200 0.313 and 0.346, 300x300 (1408 waves) 0.476 and 0.522; before any change
+// 800x800 (10000 waves) 2.71, with the matrix pipe 2.40.
 constexpr int kMatrixSumWaves = 4096;
 
 // Step kernel body; R, RK, T1ON, DEPH, KPT as in the length-gauge kernel.
