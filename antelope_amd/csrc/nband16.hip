@@ -45,9 +45,11 @@ using namespace tile;
 // Stage i: y = rho + sum_j dt a_ij k_j; k_i = f(y); after the last stage
 // rho += sum_i dt b_i k_i. PAIR: stage sg and the next stage sg2 at the same
 // time (RK4's c = 1/2, 1/2) in one pass, sharing H~, U and rho in registers;
-// sg2's input takes sg's derivative from registers.
+// sg2's input takes sg's derivative from registers. Two waves a SIMD: at three (168 registers) the
+// refinement spills 46 to 58 of them to scratch (SPLIT16, 16 bands, 48x48x8 k points, 16 RK5 steps: 41.6 ms
+// at three, 38.0 at two, and 39.3 before the refinement was second order).
 template <bool PAIR>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(PAIR ? 2 : 3))) void nb16_rhs_kernel(
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void nb16_rhs_kernel(
     const NbArgs a, const NbStage sg, const NbStage sg2, const cd *__restrict__ mats, cd *__restrict__ rho,
     cd *__restrict__ kbuf, cd *__restrict__ Ust)
 {
