@@ -30,6 +30,7 @@ struct NbArgs {
     const double *rweight; // [nr] 1/degeneracy
     const double2 *ham;    // [nr][N][N]
     const double2 *pos;    // [nr][3][N][N]
+    int herm;              // ham and pos are Hermitian, X(-R) = X(R)^dag: H and H~ are too (to rounding)
     // FP16-split Fourier sums (SBE_PREC_SPLIT16): halves as raw 16-bit words
     int split16;
     int nr_pad;            // nr rounded up to the MFMA K (32)

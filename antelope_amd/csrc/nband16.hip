@@ -435,7 +435,8 @@ __device__ __forceinline__ double lane_value(double x, int j)
     return __hiloint2double(hi, lo);
 }
 
-template <int RK>
+// HERM: H~ and H are Hermitian to rounding (NbArgs::herm), so a tile's conjugate is its transpose's tile
+template <int RK, bool HERM>
 __global__ __launch_bounds__(64 * kFusedW) __attribute__((amdgpu_waves_per_eu(RK == 4 ? 2 : 1))) void nb16_step_kernel(
     const NbArgs a, const NbFused f, cd *__restrict__ rho, cd *__restrict__ Ust, double *__restrict__ partials)
 {
@@ -461,11 +462,9 @@ __global__ __launch_bounds__(64 * kFusedW) __attribute__((amdgpu_waves_per_eu(RK
     cd *e1 = fused_slot(step_lds, 2) + w * kNbFusedMaxM1;
     if (lane < M1) e1[lane] = a.boxE[0][static_cast<int64_t>(active ? k1 : 0) * M1 + lane];
 
-    // RK4: H~ is Hermitian (its conjugate is H~^T's tile); RK5 takes it as a general matrix
-    constexpr bool kHerm = RK == 4;
     auto form_ht = [&](int slot) {
         const Tile T = form_tile(fused_slot(step_lds, slot), e1, M1, N);
-        return kHerm ? T : transpose(T, buf);
+        return HERM ? T : transpose(T, buf);
     };
     Tile R, U, Ut, Y, Acc, Ht, X;
     double lam = 0.0, p = 0.0;
@@ -566,7 +565,7 @@ __global__ __launch_bounds__(64 * kFusedW) __attribute__((amdgpu_waves_per_eu(RK
         __syncthreads();  // sums read: the transpose buffers are free
     }
     // ---- stage 1 at t_n
-    if (active) X = stage_derivative_m<kHerm>(a, R, Ht, M, buf);
+    if (active) X = stage_derivative_m<HERM>(a, R, Ht, M, buf);
     if constexpr (RK == 4) {
     if (active) {
         axpy_tile(Acc, X, dt / 6.0, R);
@@ -576,18 +575,18 @@ __global__ __launch_bounds__(64 * kFusedW) __attribute__((amdgpu_waves_per_eu(RK
     fused_wait();  // [H~ H at t + dt/2]
     Tile H;
     if (active) {
-        Ht = form_tile(fused_slot(step_lds, 0), e1, M1, N);
+        Ht = form_ht(0);
         if (a.deph) H = form_tile(fused_slot(step_lds, 1), e1, M1, N);
     }
     __syncthreads();  // slots read
     stage_async(a, step_lds, f.t2_end, 0, f.t2_end, 1, col, w, lane);
     if (active) {
         // (within the step only: the columns' unitarity is left to the refinement at its end)
-        if (a.deph) eig_refine(H, U, Ut, N, buf, false, true);
+        if (a.deph) eig_refine(H, U, Ut, N, buf, false, HERM);
         Tile Mh{};
         double dd;
         if (a.deph) Mh = band_diag(Y, U, Ut, dd);
-        X = stage_derivative_m<true>(a, Y, Ht, Mh, buf);
+        X = stage_derivative_m<HERM>(a, Y, Ht, Mh, buf);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             Acc.re[r] = fma(dt / 3.0, X.re[r], Acc.re[r]);
@@ -595,7 +594,7 @@ __global__ __launch_bounds__(64 * kFusedW) __attribute__((amdgpu_waves_per_eu(RK
         }
         axpy_tile(Y, X, 0.5 * dt, R);
         if (a.deph) Mh = band_diag(Y, U, Ut, dd);
-        X = stage_derivative_m<true>(a, Y, Ht, Mh, buf);
+        X = stage_derivative_m<HERM>(a, Y, Ht, Mh, buf);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             Acc.re[r] = fma(dt / 3.0, X.re[r], Acc.re[r]);
@@ -606,13 +605,13 @@ __global__ __launch_bounds__(64 * kFusedW) __attribute__((amdgpu_waves_per_eu(RK
     // ---- stage 4 at t_n + dt; eigenvectors and energies for the next sample
     fused_wait();  // [H~ H at t + dt]
     if (active) {
-        Ht = form_tile(fused_slot(step_lds, 0), e1, M1, N);
+        Ht = form_ht(0);
         H = form_tile(fused_slot(step_lds, 1), e1, M1, N);
-        eig_refine(H, U, Ut, N, buf, true, true, &lam);
+        eig_refine(H, U, Ut, N, buf, true, HERM, &lam);
         Tile Me{};
         double dd;
         if (a.deph) Me = band_diag(Y, U, Ut, dd);
-        X = stage_derivative_m<true>(a, Y, Ht, Me, buf);
+        X = stage_derivative_m<HERM>(a, Y, Ht, Me, buf);
         axpy_tile(R, X, dt / 6.0, Acc);
     }
     } else {
@@ -643,14 +642,14 @@ __global__ __launch_bounds__(64 * kFusedW) __attribute__((amdgpu_waves_per_eu(RK
             Tile Md{};
             double dd;
             if (a.deph) Md = band_diag(Yi, V, Vt, dd);
-            Kd[st] = stage_derivative_m<false>(a, Yi, Ht, Md, buf);
+            Kd[st] = stage_derivative_m<HERM>(a, Yi, Ht, Md, buf);
         };
         const cd *mid = f.t2_half;
 #pragma unroll
         for (int st = 1; st <= 3; ++st) {  // 1/4, 3/8, 12/13
             pair(st < 3 ? mid + st * f.mid_stride : f.t2_end);
             if (active) {
-                if (a.deph) eig_refine(H, U, Ut, N, buf, true, false);
+                if (a.deph) eig_refine(H, U, Ut, N, buf, true, HERM);
                 deriv(st, U, Ut);
                 if (st == 2) {
                     Vm = U;
@@ -660,12 +659,12 @@ __global__ __launch_bounds__(64 * kFusedW) __attribute__((amdgpu_waves_per_eu(RK
         }
         pair(mid + 3 * f.mid_stride);
         if (active) {
-            eig_refine(H, U, Ut, N, buf, true, false, &lam);
+            eig_refine(H, U, Ut, N, buf, true, HERM, &lam);
             deriv(4, U, Ut);
         }
         pair(nullptr);
         if (active) {
-            if (a.deph) eig_refine(H, Vm, Vmt, N, buf, true, false);
+            if (a.deph) eig_refine(H, Vm, Vmt, N, buf, true, HERM);
             deriv(5, Vm, Vmt);
 #pragma unroll
             for (int j = 0; j < 6; ++j)
@@ -737,15 +736,15 @@ static hipError_t allow_lds(const void *kernel, size_t lds)
     return hipSuccess;
 }
 
-template <int RK>
+template <int RK, bool HERM>
 static hipError_t launch_step(const NbArgs &a, const NbFused &f, double2 *rho, double2 *U, double *partials,
                               hipStream_t s)
 {
     constexpr size_t lds = sizeof(double2) * static_cast<size_t>(
         kFusedW * kFusedBuf + 2 * kNbFusedMaxM1 * kFusedPitch + kFusedW * kNbFusedMaxM1);
-    const hipError_t e = allow_lds(reinterpret_cast<const void *>(&nb16_step_kernel<RK>), lds);
+    const hipError_t e = allow_lds(reinterpret_cast<const void *>(&nb16_step_kernel<RK, HERM>), lds);
     if (e != hipSuccess) return e;
-    nb16_step_kernel<RK><<<dim3(static_cast<unsigned>(f.nblocks)), 64 * kFusedW, lds, s>>>(a, f, rho, U, partials);
+    nb16_step_kernel<RK, HERM><<<dim3(static_cast<unsigned>(f.nblocks)), 64 * kFusedW, lds, s>>>(a, f, rho, U, partials);
     return hipGetLastError();
 }
 
@@ -753,8 +752,10 @@ hipError_t nb16_launch_step(const NbArgs &a, const NbFused &f, int rk_order, dou
                             hipStream_t s)
 {
     if (a.N > 16 || !a.box || a.boxM[0] < 1 || a.boxM[0] > kNbFusedMaxM1 || f.nblocks < 1) return hipErrorInvalidValue;
-    if (rk_order == SBE_RK4) return launch_step<4>(a, f, rho, U, partials, s);
-    if (rk_order == SBE_RK5_FEHLBERG) return launch_step<5>(a, f, rho, U, partials, s);
+    if (rk_order == SBE_RK4)
+        return a.herm ? launch_step<4, true>(a, f, rho, U, partials, s) : launch_step<4, false>(a, f, rho, U, partials, s);
+    if (rk_order == SBE_RK5_FEHLBERG)
+        return a.herm ? launch_step<5, true>(a, f, rho, U, partials, s) : launch_step<5, false>(a, f, rho, U, partials, s);
     return hipErrorInvalidValue;
 }
 

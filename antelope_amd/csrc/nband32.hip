@@ -34,6 +34,7 @@ struct Q {
     double *sc;    // [2][128]
     int p, q, ph;  // quadrant; exchange phase (pair 0 or 1)
     int N;
+    bool herm = true;  // H is Hermitian to rounding
 
     __device__ cd *s(int i) const { return slot + (2 * ph + i) * kQSlot; }
     __device__ double *scal() const { return sc + ph * 128; }
@@ -218,7 +219,23 @@ __device__ double q_orthonormalize(Q &L, Tile &U)
     return q_max(L, e);
 }
 
-// Warm-started eigenvectors of H = Hk (Hermitian to rounding, FP64 sums; read again where
+// this wave's quadrant of the Hermitian part of H
+__device__ __forceinline__ Tile q_load_herm(const Q &L, const cd *H)
+{
+    Tile T = q_load(L, H, false);
+    if (!L.herm) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if (!q_valid(L, r)) continue;
+            const cd t = H[(16 * L.q + lane_c()) * L.N + 16 * L.p + lane_g() + 4 * r];
+            T.re[r] = 0.5 * (T.re[r] + t.x);
+            T.im[r] = 0.5 * (T.im[r] - t.y);
+        }
+    }
+    return T;
+}
+
+// Warm-started eigenvectors of the Hermitian part of H = Hk (read again where
 // needed rather than held in registers): simultaneous Jacobi rotations written as
 // products, the last round U (I + K) once max|K| < small_tol, then (ortho) a
 // Newton-Schulz step; lam_out: this lane's column of diag(U^dag H U) before the last
@@ -228,7 +245,7 @@ __device__ double q_orthonormalize(Q &L, Tile &U)
 __device__ void q_refine(Q &L, const cd *Hk, Tile &U, double small_tol, bool ortho, double &lam_out)
 {
     const int N = L.N;
-    Tile W = q_prod(L, U, true, q_prod(L, q_load(L, Hk, false), false, U, false), false);  // U^dag (H U)
+    Tile W = q_prod(L, U, true, q_prod(L, q_load_herm(L, Hk), false, U, false), false);  // U^dag (H U)
     double lam_last = 0.0;
     for (int it = 0; it < 30; ++it) {
         double lam_r[4], lam_c;
@@ -283,7 +300,7 @@ __device__ void q_refine(Q &L, const cd *Hk, Tile &U, double small_tol, bool ort
         if (kmax > 1e-3) {  // V far from unitary: restore U fully, then W from H itself
             for (int n = 0; n < 8; ++n)
                 if (q_orthonormalize(L, U) < 1e-8) break;
-            W = q_prod(L, U, true, q_prod(L, q_load(L, Hk, false), false, U, false), false);
+            W = q_prod(L, U, true, q_prod(L, q_load_herm(L, Hk), false, U, false), false);
         } else {
             W = q_prod(L, V, true, q_prod(L, W, false, V, false), false);  // V^dag (W V)
         }
@@ -306,10 +323,10 @@ __device__ Tile q_band_diag(Q &L, const Tile &Y, const Tile &U, double &d)
     return q_prod(L, Ud, false, U, true);
 }
 
-// -i(H~ y - (H~ y)^dag) - g2 y - (g1 - g2) M (H~ Hermitian)
+// -i(H~ y - (H~ y)^dag) - g2 y - (g1 - g2) M, H~ a general matrix (its positions need not be Hermitian)
 __device__ Tile q_stage(Q &L, const NbArgs &a, const Tile &Y, const Tile &Ht, const Tile &M)
 {
-    const Tile T = q_prod(L, Ht, true, Y, false);  // H~ y
+    const Tile T = q_prod(L, Ht, false, Y, false);  // H~ y
     const Tile Td = q_adjoint(L, T);
     Tile X;
 #pragma unroll
@@ -366,7 +383,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1))) void n
     __shared__ double rsum[2 * kQStage];  // the block's sum_k w rho (each element owned by one lane)
     __shared__ double scal[2 * 128];
     const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-    Q L{slots, scal, w >> 1, w & 1, 0, a.N};
+    Q L{slots, scal, w >> 1, w & 1, 0, a.N, a.herm != 0};
     const int N = a.N, nn = N * N;
     const int c = lane_c(), g = lane_g(), lane = threadIdx.x & 63;
     const int64_t slot = a.nk_stride * nn;

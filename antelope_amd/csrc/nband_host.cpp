@@ -4,9 +4,11 @@
 //   stage i: Fourier sums {H + E.D, H} at t_n + c_i dt -> nb_rhs_kernel
 // (antelope.cpp:297-338 with SBEs.h:596-624).
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <map>
 #include <string>
 #include <vector>
 
@@ -446,6 +448,35 @@ bool box_tables(const sbe_model &m, const std::vector<double> &hk, int64_t nk, c
     return true;
 }
 
+// Every lattice sum of the model is Hermitian at real k: w X(-R) = (w X(R))^dag for H and the
+// positions, to rounding. Files need not be (positions above all); the kernels that take a matrix's
+// conjugate for its transpose then form the transpose instead.
+bool hermitian_model(const sbe_model &m)
+{
+    if (am::is_analytic(m.kind) || m.nrpts < 1) return true;
+    const size_t N = static_cast<size_t>(m.nband), nn = N * N;
+    std::map<std::array<int32_t, 3>, int> at;
+    for (int r = 0; r < m.nrpts; ++r)
+        if (!at.insert({{m.rvec[3 * r], m.rvec[3 * r + 1], m.rvec[3 * r + 2]}, r}).second) return false;  // R twice
+    auto holds = [&](const double *x, int mats) {
+        double big = 0.0, off = 0.0;
+        for (int r = 0; r < m.nrpts; ++r) {
+            const auto it = at.find({-m.rvec[3 * r], -m.rvec[3 * r + 1], -m.rvec[3 * r + 2]});
+            const double w = m.rweight[r], v = it == at.end() ? 0.0 : m.rweight[it->second];
+            const double *a = x + 2 * nn * mats * r, *b = it == at.end() ? a : x + 2 * nn * mats * it->second;
+            for (int c = 0; c < mats; ++c, a += 2 * nn, b += 2 * nn)
+                for (size_t i = 0; i < N; ++i)
+                    for (size_t j = 0; j < N; ++j) {
+                        const double *p = a + 2 * (i * N + j), *q = b + 2 * (j * N + i);
+                        big = std::max(big, std::max(std::fabs(w * p[0]), std::fabs(w * p[1])));
+                        off = std::max(off, std::max(std::fabs(w * p[0] - v * q[0]), std::fabs(w * p[1] + v * q[1])));
+                    }
+        }
+        return off <= 0x1p-50 * big;
+    };
+    return holds(m.ham, 1) && (m.is_dipole_zero || !m.pos || holds(m.pos, 3));
+}
+
 // Device tables of the time-fused analytic steps: the class's coefficients, the energies, A at
 // the distinct times of every step and the table of phases formed from it
 int setup_evolve(sbe_ctx *ctx, const AnalyticTerms &t, char *buf, int nblocks)
@@ -655,6 +686,7 @@ int nb_setup(sbe_ctx *ctx)
         a.tile16 = N <= 16 && !(tuned && tu.nb_kernels == 2);
         if (const char *e = std::getenv("ANTELOPE_NB_LDS")) a.tile16 = N <= 16 && std::atoi(e) != 1;
     }
+    a.herm = hermitian_model(m) ? 1 : 0;
     a.kpts = dk;
     a.weight = dk + 3 * p.nk_stride;
     a.rcart = dr;

@@ -194,6 +194,33 @@ def test_step_rk5(oracle, monkeypatch, N, nmax, npts, T1, T2, ii):
         assert s.info.device_bytes == query_footprint(cfg, m)
 
 
+@pytest.mark.parametrize("what", ["positions", "both"])
+@pytest.mark.parametrize("N,nmax,npts", [(9, (0, 2, 0), (5, 9, 1)), (12, (1, 1, 0), (7, 7, 1)), (16, (3, 1, 0), (9, 3, 1)),
+                                         (17, (1, 1, 0), (4, 4, 1)), (32, (1, 1, 1), (3, 3, 3))])
+def test_matrices_not_hermitian(oracle, monkeypatch, N, nmax, npts, what):
+    """RK4 steps of 9 to 32 bands (nb16_step_kernel<4>, nb32_step_kernel) with matrices r(-R) != r(R)^dag, and H
+    too by a thousandth (its Hermitian part has the eigenvectors, the commutator takes all of it): the oracle's and the
+    separate kernels' results, as every other route gives them."""
+    m = synthetic_wannier(N, nmax=nmax, seed=130 + N)
+    m.pos = m.pos * (1.0 + 0.3j)
+    if what == "both":
+        rng = np.random.default_rng(N)
+        m.ham = m.ham + 1e-3 * np.abs(m.ham).max() * rng.normal(size=m.ham.shape)
+    cfg = RunConfig(npoints=list(npts), pulses=[Pulse(E0=0.01, w0=0.05, ncycles=0.25, ellip=0.4, envelope="sin2")],
+                    dt=0.5, T1=150.0, T2=80.0, rk_order=4, inter_intra=True)
+    print(N, nmax, npts, what, flush=True)
+    got, foot = _run(cfg, m), query_footprint(cfg, m)
+    with monkeypatch.context() as mp:
+        mp.setenv("ANTELOPE_NB_FUSED", "0")
+        sep = _run(cfg, m)
+        assert foot != query_footprint(cfg, m)  # the fused step's plan was the one that ran
+    ref = oracle.run(cfg, m, nthreads=8, want_state=True) if what == "positions" else sep
+    for key in ("j_inter", "j_intra", "band_pop", "rho_bar", "state"):
+        if np.linalg.norm(ref[key]) > 0.0:
+            print(f"  {key}: {rel_l2(got[key], ref[key]):.1e} {rel_l2(got[key], sep[key]):.1e}", flush=True)
+            assert rel_l2(got[key], ref[key]) < 1e-10 and rel_l2(got[key], sep[key]) < 1e-10, key
+
+
 @pytest.mark.parametrize("N,npts,nmax", [(8, (5, 5, 3), (1, 1, 1)), (16, (6, 5, 1), (2, 2, 0))])
 def test_refined_eigenvectors_hold_rounding(oracle, N, npts, nmax):
     """The refinement may end only where what it leaves off the diagonal is below rounding also between
