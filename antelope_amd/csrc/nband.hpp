@@ -191,9 +191,9 @@ struct EvolveTerms {  // analytic_terms.hpp
 struct NbEvolve {
     EvolveTerms terms;
     const double2 *coef;   // [1 + 2 T + 1][N][N]: m0, (p_t, q_t) per term, the current's element factors
-    const double *table;   // [nt + 1][row]: cos / sin(A.v_t) at the step's distinct times
+    const double *table;   // [s1 - s0 + 1][row]: cos / sin(A.v_t) at the distinct times of step s0 on
     int jz;                // any z current
-    int64_t nt, s0, s1;
+    int64_t s0, s1;
     double dt;
     int nblocks;
     double *lam;           // [nk_stride][8] band energies at the stored eigenvectors' time
@@ -205,8 +205,10 @@ inline int evolve_times(int rk_order) { return rk_order == 4 ? 2 : 5; }
 inline int evolve_padded_terms(int T) { return T <= 3 ? 3 : (T <= 6 ? 6 : 9); }
 inline int evolve_row_len(int rk_order, int T) { return (6 + 2 * evolve_times(rk_order)) * evolve_padded_terms(T); }
 int evolve_blocks(int N, int64_t nk);
-// the table of rows n in [0, rows) from A at the distinct times, [rows][times][3]
-hipError_t launch_evolve_table(const double *A, const EvolveTerms &t, int rk_order, int64_t rows, double *tab, hipStream_t s);
+// the table of rows n in [step0, step0 + nsteps) of the laser at its times t_n + c_u dt, or (A
+// not null) from A of the whole pulse at them, [n][times][3]
+struct TableArgs;
+hipError_t launch_evolve_table(const TableArgs &laser, const double *A, const EvolveTerms &t, int rk_order, double *tab, hipStream_t s);
 hipError_t launch_evolve(const NbArgs &a, const NbEvolve &e, int rk_order, double2 *rho, double2 *U, double *partials,
                          hipStream_t s);
 

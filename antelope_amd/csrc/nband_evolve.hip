@@ -22,7 +22,7 @@
 // sample and model kernels; MoS2 (3 bands), 72 x 72 k, RK4: 4.6 ms against 103 ms.
 #include <cmath>
 
-#include "haldane_dev.hpp"
+#include "haldane_setup.hpp"
 #include "tile_eig.hpp"
 
 namespace sbe {
@@ -49,17 +49,23 @@ constexpr int mid_times() { return RK == 4 ? 1 : 4; }
 template <int RK, int NT>
 constexpr int row_len() { return (8 + 2 * mid_times<RK>()) * NT; }
 
-// table[n][...] for n in [0, nt]: A [nt + 1][1 + mids][3]
-__global__ __launch_bounds__(256) void evolve_table_kernel(const double *__restrict__ A, const EvolveTerms w, int mids,
-                                                           int nt_pad, int64_t rows, double *__restrict__ tab)
+// table[n - step0][...]
+__global__ __launch_bounds__(256) void evolve_table_kernel(const TableArgs laser, const double *__restrict__ A, const EvolveTerms w,
+                                                           int mids, int nt_pad, double *__restrict__ tab)
 {
     const int64_t id = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
     const int t = static_cast<int>(id % nt_pad);
     const int64_t q = id / nt_pad;
     const int u = static_cast<int>(q % (1 + mids));
     const int64_t n = q / (1 + mids);
-    if (n >= rows) return;
-    const double *a = A + (n * (1 + mids) + u) * 3;
+    if (n >= laser.nsteps) return;
+    const int64_t step = laser.step0 + n;
+    double a[3];
+    if (A) {
+        for (int i = 0; i < 3; ++i) a[i] = A[(step * (1 + mids) + u) * 3 + i];
+    } else {
+        dev::field_at(laser, laser.atmin + laser.dt * static_cast<double>(step) + laser.c[u] * laser.dt, a);
+    }
     double s = 0.0, c = 0.0;
     if (t < w.T) sincos(a[0] * w.vec[t][0] + a[1] * w.vec[t][1] + a[2] * w.vec[t][2], &s, &c);
     double *row = tab + n * (8 + 2 * mids) * nt_pad;
@@ -159,7 +165,7 @@ struct AnalyticSource {
         m0 = in ? e.coef[el] : zero;
         sc = in ? e.coef[(1 + 2 * e.terms.T) * nn + el] : zero;
         for (int x = threadIdx.x; x < 2 * R; x += 64 * kWaves)
-            rows[((e.s0 + x / R) % 3) * R + x % R] = e.table[e.s0 * R + x];
+            rows[((e.s0 + x / R) % 3) * R + x % R] = e.table[x];
         __syncthreads();
         sl = static_cast<int>(e.s0 % 3);
         sn = sl == 2 ? 0 : sl + 1;
@@ -182,8 +188,8 @@ struct AnalyticSource {
     __device__ void start(T &Ht, T &H) { Ht = H = hmat(rows + sl * R); }
     __device__ void begin(int64_t step)
     {
-        fetch = threadIdx.x < R && step + 2 <= e.nt;
-        ahead = fetch ? e.table[(step + 2) * R + threadIdx.x] : 0.0;
+        fetch = threadIdx.x < R && step + 2 <= e.s1;
+        ahead = fetch ? e.table[(step + 2 - e.s0) * R + threadIdx.x] : 0.0;
     }
     __device__ void current(int ax, double &jr, double &ji) const
     {
@@ -567,11 +573,12 @@ int evolve_blocks(int N, int64_t nk)
     return static_cast<int>((nk + per - 1) / per);
 }
 
-hipError_t launch_evolve_table(const double *A, const EvolveTerms &t, int rk_order, int64_t rows, double *tab, hipStream_t s)
+hipError_t launch_evolve_table(const TableArgs &laser, const double *A, const EvolveTerms &t, int rk_order, double *tab, hipStream_t s)
 {
     const int mids = evolve_times(rk_order) - 1, ntp = evolve_padded_terms(t.T);
-    const int64_t n = rows * (1 + mids) * ntp;
-    evolve_table_kernel<<<dim3(static_cast<unsigned>((n + 255) / 256)), 256, 0, s>>>(A, t, mids, ntp, rows, tab);
+    if (laser.nsteps < 1 || laser.nstage != 1 + mids || (!A && laser.npulses > kMaxDevicePulses)) return hipErrorInvalidValue;
+    const int64_t n = laser.nsteps * (1 + mids) * ntp;
+    evolve_table_kernel<<<dim3(static_cast<unsigned>((n + 255) / 256)), 256, 0, s>>>(laser, A, t, mids, ntp, tab);
     return hipGetLastError();
 }
 

@@ -302,16 +302,46 @@ struct NbPlan {
     size_t bytes_fused;  // fused steps: second-pass outputs, scratch, band energies, A and E
     FusedEval fe;
     size_t bytes_vel;    // time-fused velocity steps: A at the stage times of the whole pulse
-    size_t bytes_evolve; // time-fused analytic steps: coefficients, energies, A and the table of the pulse
+    size_t bytes_evolve; // time-fused analytic steps: coefficients, energies, a launch's phase table (and A)
     // offsets inside the box buffer: B, T1, T2, E_1..E_3, R map, k map
     size_t off_t1, off_t2, off_e[3], off_r, off_kinv;
+
+    size_t total() const
+    {
+        return bytes_evolve + bytes_P + bytes_rho + bytes_mats + bytes_k + bytes_tab + bytes_partials + bytes_series +
+               bytes_split + bytes_b64 + bytes_box + bytes_fused + bytes_vel;
+    }
 };
 
 size_t align256(size_t x) { return (x + 255) / 256 * 256; }
 
-NbPlan nb_plan(int N, int nr, int64_t nk, int64_t nt, int nstage, bool split16, const BoxShape &bx, bool fused,
-               bool vel_fused = false, bool nb32 = false, int evolve_terms = -1)
+// Which kernels a solve takes. lean: the routes whose scratch is not in the separate kernels' plan
+// (time-fused RK5 and analytic steps) are left, and rows of partial sums take no more than the
+// separate kernels' would: for a solve that does not fit otherwise.
+struct NbRoutes {
+    BoxShape bx;
+    bool split16, lean, fused, vel_fused, nb32, evolve;
+    AnalyticTerms terms;
+    NbRoutes(const sbe_config &cfg, const sbe_model &m, int64_t nk, bool lean_) : split16(cfg.precision == SBE_PREC_SPLIT16), lean(lean_)
+    {
+        bx = box_shape(cfg, m, nk, split16);
+        fused = fused_eligible(cfg, m, nk, bx) || (!lean && rk5_eligible(cfg, m, nk, bx));
+        vel_fused = vel_fused_eligible(cfg, m, nk) && !(lean && cfg.rk_order != SBE_RK4);
+        nb32 = nb32_eligible(cfg, m);
+        evolve = !lean && evolve_eligible(cfg, m, nk, terms);
+    }
+};
+
+// The phase table of the time-fused analytic steps covers one launch: as many steps as fit the
+// matrix and stage slots that this route does without, and no fewer than kEvolveTableSteps
+// (0.3 MB at most; a launch of fewer steps of a small grid would be no longer than its overhead).
+constexpr int64_t kEvolveTableSteps = 256;
+
+NbPlan nb_plan(const sbe_config &cfg, const sbe_model &m, int64_t nk, int64_t nt, int nstage, const NbRoutes &rt)
 {
+    const int N = m.nband, nr = am::is_analytic(m.kind) ? 0 : m.nrpts;
+    const bool split16 = rt.split16, fused = rt.fused, vel_fused = rt.vel_fused, nb32 = rt.nb32;
+    const BoxShape &bx = rt.bx;
     NbPlan p{};
     p.nk_stride = (nk + 63) / 64 * 64;
     p.sample_waves = static_cast<int>(std::min<int64_t>(nk, 2048));
@@ -322,24 +352,35 @@ NbPlan nb_plan(int N, int nr, int64_t nk, int64_t nt, int nstage, bool split16, 
     if (fused && N <= 8) rows = std::max<int64_t>(p.sample_waves, box_evolve_blocks(N, bx.K));
     if (vel_fused) rows = std::max<int64_t>(rows, N > 16 ? nk : vel_fused_blocks(N, nk));
     p.bytes_vel = vel_fused ? align256(static_cast<size_t>(nt) * nstage * 3 * sizeof(double)) : 0;
-    p.bytes_evolve = 0;
-    if (evolve_terms >= 0) {
-        rows = evolve_blocks(N, nk);
-        const int rk = nstage == 4 ? SBE_RK4 : SBE_RK5_FEHLBERG;
-        p.bytes_evolve = align256((2 + 2 * static_cast<size_t>(evolve_terms)) * nn * sizeof(double2)) +
-                         align256(static_cast<size_t>(p.nk_stride) * 8 * sizeof(double)) +
-                         align256(static_cast<size_t>(nt + 1) * evolve_times(rk) * 3 * sizeof(double)) +
-                         align256(static_cast<size_t>(nt + 1) * evolve_row_len(rk, evolve_terms) * sizeof(double));
-    }
+    if (rt.evolve) rows = evolve_blocks(N, nk);
+    p.bytes_rho = static_cast<size_t>(p.nk_stride) * nn * sizeof(double2);
     const size_t row = static_cast<size_t>(rows) * p.nv * sizeof(double);
-    p.chunk = std::max<int64_t>(1, std::min<int64_t>(nt, static_cast<int64_t>(kNbPartialBytes / row)));
+    auto chunk_of = [&](size_t bytes, size_t r) { return std::max<int64_t>(1, std::min<int64_t>(nt, static_cast<int64_t>(bytes / r))); };
+    p.chunk = chunk_of(kNbPartialBytes, row);
+    if (rt.lean) {
+        const size_t sep = static_cast<size_t>(p.sample_waves) * p.nv * sizeof(double);
+        p.chunk = chunk_of(static_cast<size_t>(chunk_of(kNbPartialBytes, sep)) * sep, row);
+    }
+    p.bytes_evolve = 0;
+    if (rt.evolve) {
+        const int rk = nstage == 4 ? SBE_RK4 : SBE_RK5_FEHLBERG;
+        const size_t tab_row = static_cast<size_t>(evolve_row_len(rk, rt.terms.T)) * sizeof(double);
+        const size_t spare = static_cast<size_t>(3 + nstage) * p.bytes_rho;
+        p.chunk = std::min(p.chunk, std::max<int64_t>(kEvolveTableSteps, static_cast<int64_t>(spare / tab_row)));
+        p.bytes_evolve = align256((2 + 2 * static_cast<size_t>(rt.terms.T)) * nn * sizeof(double2)) +
+                         align256(static_cast<size_t>(p.nk_stride) * 8 * sizeof(double)) +
+                         align256(static_cast<size_t>(p.chunk + 1) * tab_row);
+        if (cfg.npulses > kMaxDevicePulses)  // A from the host
+            p.bytes_evolve += align256(static_cast<size_t>(nt + 1) * evolve_times(rk) * 3 * sizeof(double));
+    }
     // e^{ik.R} for the dense sums (also the N <= 32 fused step's one-launch sums); the
     // separable form does not read it
     const bool dm32 = nb32 && nb32_dense_multi_n(nr, nk);
     p.bytes_P = bx.ok && !dm32 ? 0 : static_cast<size_t>(p.nk_stride) * nr * sizeof(double2);
-    p.bytes_rho = static_cast<size_t>(p.nk_stride) * nn * sizeof(double2);
-    p.bytes_mats = 5 * p.bytes_rho;  // H~, H, J_x, J_y, J_z
-    p.bytes_k = static_cast<size_t>(nstage + 1) * p.bytes_rho;  // stage derivatives + eigenvectors
+    // H~, H, J_x, J_y, J_z; stage derivatives and eigenvectors. The time-fused analytic steps read
+    // only the eigenvectors; the initial state and the band-basis export take two matrices
+    p.bytes_mats = (rt.evolve ? 2 : 5) * p.bytes_rho;
+    p.bytes_k = static_cast<size_t>(rt.evolve ? 1 : nstage + 1) * p.bytes_rho;
     p.bytes_tab = static_cast<size_t>(p.nk_stride) * 4 * sizeof(double) + static_cast<size_t>(nr) * 4 * sizeof(double) +
                   static_cast<size_t>(nr) * 4 * nn * sizeof(double2);
     p.bytes_partials = static_cast<size_t>(p.chunk) * row;
@@ -477,9 +518,10 @@ bool hermitian_model(const sbe_model &m)
     return holds(m.ham, 1) && (m.is_dipole_zero || !m.pos || holds(m.pos, 3));
 }
 
-// Device tables of the time-fused analytic steps: the class's coefficients, the energies, A at
-// the distinct times of every step and the table of phases formed from it
-int setup_evolve(sbe_ctx *ctx, const AnalyticTerms &t, char *buf, int nblocks)
+// Device buffers of the time-fused analytic steps: the class's coefficients, the energies, a
+// launch's table of phases, and for more pulses than the table kernel takes A at the distinct
+// times of every step
+int setup_evolve(sbe_ctx *ctx, const AnalyticTerms &t, char *buf, int64_t chunk, int nblocks)
 {
     const NbArgs &a = ctx->nargs;
     const size_t nn = static_cast<size_t>(a.N) * a.N;
@@ -497,28 +539,33 @@ int setup_evolve(sbe_ctx *ctx, const AnalyticTerms &t, char *buf, int nblocks)
         c.insert(c.end(), t.q.begin() + 2 * nn * i, t.q.begin() + 2 * nn * (i + 1));
     }
     c.insert(c.end(), t.scale.begin(), t.scale.end());
-    const double mid[2][4] = {{ctx->tab.c[1]}, {ctx->tab.c[1], ctx->tab.c[2], ctx->tab.c[3], ctx->tab.c[5]}};
-    std::vector<double> A(static_cast<size_t>(nt + 1) * times * 3);
-    for (int64_t n = 0; n <= nt; ++n) {
-        const double tn = ctx->laser.atmin + ctx->laser.dt * static_cast<double>(n);  // antelope.cpp:299
-        for (int u = 0; u < times; ++u) {
-            double E[3];
-            ctx->laser.eval(u == 0 ? tn : tn + mid[rk == SBE_RK4 ? 0 : 1][u - 1] * ctx->laser.dt,
-                            A.data() + (static_cast<size_t>(n) * times + u) * 3, E);
-        }
-    }
+    const Tableau &tb = ctx->tab;
+    const double mid[2][4] = {{tb.c[1]}, {tb.c[1], tb.c[2], tb.c[3], tb.c[5]}};
     char *q = buf;
     auto take = [&](size_t bytes) { char *r = q; q += align256(bytes); return r; };
     char *dc = take(c.size() * sizeof(double));
     e.lam = reinterpret_cast<double *>(take(static_cast<size_t>(a.nk_stride) * 8 * sizeof(double)));
-    double *dA = reinterpret_cast<double *>(take(A.size() * sizeof(double)));
-    double *dtab = reinterpret_cast<double *>(take(static_cast<size_t>(nt + 1) * evolve_row_len(rk, t.T) * sizeof(double)));
+    ctx->evolve_tab = reinterpret_cast<double *>(take(static_cast<size_t>(chunk + 1) * evolve_row_len(rk, t.T) * sizeof(double)));
     int rc = hipc(ctx, hipMemcpy(dc, c.data(), c.size() * sizeof(double), hipMemcpyHostToDevice), "upload terms");
-    if (!rc) rc = hipc(ctx, hipMemcpy(dA, A.data(), A.size() * sizeof(double), hipMemcpyHostToDevice), "upload A");
-    if (!rc) rc = hipc(ctx, launch_evolve_table(dA, e.terms, rk, nt + 1, dtab, ctx->stream), "phase table kernel");
+    const double none[3][2] = {};
+    ctx->evolve_laser = table_args(ctx->laser, tb, times, 0.0, none, none);
+    ctx->evolve_laser.c[0] = 0.0;
+    for (int u = 1; u < times; ++u) ctx->evolve_laser.c[u] = mid[rk == SBE_RK4 ? 0 : 1][u - 1];
+    ctx->evolve_A = nullptr;
+    if (ctx->evolve_laser.npulses > kMaxDevicePulses) {
+        std::vector<double> A(static_cast<size_t>(nt + 1) * times * 3);
+        for (int64_t n = 0; n <= nt; ++n) {
+            const double tn = ctx->laser.atmin + ctx->laser.dt * static_cast<double>(n);  // antelope.cpp:299
+            for (int u = 0; u < times; ++u) {
+                double E[3];
+                ctx->laser.eval(tn + ctx->evolve_laser.c[u] * ctx->laser.dt, A.data() + (static_cast<size_t>(n) * times + u) * 3, E);
+            }
+        }
+        ctx->evolve_A = reinterpret_cast<double *>(take(A.size() * sizeof(double)));
+        if (!rc) rc = hipc(ctx, hipMemcpy(ctx->evolve_A, A.data(), A.size() * sizeof(double), hipMemcpyHostToDevice), "upload A");
+    }
     e.coef = reinterpret_cast<const double2 *>(dc);
-    e.table = dtab;
-    e.nt = nt;
+    e.table = ctx->evolve_tab;
     e.dt = ctx->laser.dt;
     e.nblocks = nblocks;
     ctx->nbe = rc == SBE_OK;
@@ -527,19 +574,9 @@ int setup_evolve(sbe_ctx *ctx, const AnalyticTerms &t, char *buf, int nblocks)
 
 }  // namespace
 
-size_t nb_footprint(const sbe_config &cfg, const sbe_model &m, int64_t nk, int64_t nt, int nstage)
+size_t nb_footprint(const sbe_config &cfg, const sbe_model &m, int64_t nk, int64_t nt, int nstage, bool lean)
 {
-    const bool split16 = cfg.precision == SBE_PREC_SPLIT16;
-    const BoxShape bx = box_shape(cfg, m, nk, split16);
-    const bool fused = fused_eligible(cfg, m, nk, bx) || rk5_eligible(cfg, m, nk, bx);
-    const bool vfused = vel_fused_eligible(cfg, m, nk);
-    const bool f32 = nb32_eligible(cfg, m);
-    AnalyticTerms terms;
-    const int nterms = evolve_eligible(cfg, m, nk, terms) ? terms.T : -1;
-    const NbPlan p =
-        nb_plan(m.nband, am::is_analytic(m.kind) ? 0 : m.nrpts, nk, nt, nstage, split16, bx, fused, vfused, f32, nterms);
-    return p.bytes_evolve + p.bytes_P + p.bytes_rho + p.bytes_mats + p.bytes_k + p.bytes_tab + p.bytes_partials + p.bytes_series +
-           p.bytes_split + p.bytes_b64 + p.bytes_box + p.bytes_fused + p.bytes_vel;
+    return nb_plan(cfg, m, nk, nt, nstage, NbRoutes(cfg, m, nk, lean)).total();
 }
 
 int nb_validate(const sbe_model &m, std::string &err)
@@ -606,15 +643,10 @@ int nb_setup(sbe_ctx *ctx)
     const bool analytic = am::is_analytic(m.kind);
     const int N = m.nband, nr = analytic ? 0 : m.nrpts;
     const int64_t nk = ctx->grid.k_end - ctx->grid.k_begin;
-    const bool split16 = ctx->cfg.precision == SBE_PREC_SPLIT16;
-    const BoxShape bx = box_shape(ctx->cfg, m, nk, split16);
-    const bool fused = fused_eligible(ctx->cfg, m, nk, bx) || rk5_eligible(ctx->cfg, m, nk, bx);
-    const bool vfused = vel_fused_eligible(ctx->cfg, m, nk);
-    const bool f32 = nb32_eligible(ctx->cfg, m);
-    AnalyticTerms terms;
-    const bool evolve = evolve_eligible(ctx->cfg, m, nk, terms);
-    const NbPlan p =
-        nb_plan(N, nr, nk, ctx->laser.nt, ctx->tab.nstage, split16, bx, fused, vfused, f32, evolve ? terms.T : -1);
+    const NbRoutes rt(ctx->cfg, m, nk, ctx->lean);
+    const bool split16 = rt.split16, fused = rt.fused;
+    const BoxShape &bx = rt.bx;
+    const NbPlan p = nb_plan(ctx->cfg, m, nk, ctx->laser.nt, ctx->tab.nstage, rt);
     const size_t nn = static_cast<size_t>(N) * N;
     ctx->nk = nk;
     ctx->nk_stride = p.nk_stride;
@@ -626,7 +658,7 @@ int nb_setup(sbe_ctx *ctx)
     ctx->nb_rho = nalloc<double2>(ctx, p.bytes_rho, rc);
     ctx->nb_mats = nalloc<double2>(ctx, p.bytes_mats, rc);
     ctx->nb_k = nalloc<double2>(ctx, p.bytes_k, rc);
-    if (!rc) ctx->nb_U = ctx->nb_k + static_cast<size_t>(ctx->tab.nstage) * p.nk_stride * nn;
+    if (!rc) ctx->nb_U = ctx->nb_k + (p.bytes_k - p.bytes_rho) / sizeof(double2);
     char *tab = nalloc<char>(ctx, p.bytes_tab, rc);
     ctx->d_partials = nalloc<double>(ctx, p.bytes_partials, rc);
     ctx->d_series = nalloc<double>(ctx, p.bytes_series, rc);
@@ -797,7 +829,7 @@ int nb_setup(sbe_ctx *ctx)
     // fused RK4 steps for 16 < N <= 32: H~ H pairs in mats slots 0-1 and stage-derivative
     // slots 0-1, 2-3 (J in mats slots 2-4); with the separable sums, per evaluation scratch
     ctx->nb32 = false;
-    if (f32 && fbuf && ctx->tab.nstage == 4) {
+    if (rt.nb32 && fbuf && ctx->tab.nstage == 4) {
         const size_t slot = static_cast<size_t>(p.nk_stride) * nn;
         ctx->nb32_pair[0] = ctx->nb_mats;
         ctx->nb32_pair[1] = ctx->nb_k;
@@ -841,7 +873,7 @@ int nb_setup(sbe_ctx *ctx)
     }
 
     ctx->nbe = false;
-    if (ebuf) rc = setup_evolve(ctx, terms, ebuf, evolve_blocks(N, nk));
+    if (ebuf) rc = setup_evolve(ctx, rt.terms, ebuf, p.chunk, evolve_blocks(N, nk));
     if (rc) return rc;
 
     a.velocity = ctx->velocity ? 1 : 0;
@@ -1228,7 +1260,11 @@ static int nb_run_evolve(sbe_ctx *ctx, int64_t step_begin, int64_t step_end)
         const int64_t n = std::min<int64_t>(ctx->chunk_steps, step_end - c0);
         e.s0 = c0;
         e.s1 = c0 + n;
-        rc = hipc(ctx, launch_evolve(a, e, ctx->cfg.rk_order, ctx->nb_rho, ctx->nb_U, ctx->d_partials, ctx->stream),
+        ctx->evolve_laser.step0 = c0;
+        ctx->evolve_laser.nsteps = n + 1;
+        rc = hipc(ctx, launch_evolve_table(ctx->evolve_laser, ctx->evolve_A, e.terms, ctx->cfg.rk_order, ctx->evolve_tab, ctx->stream),
+                  "phase table kernel");
+        if (!rc) rc = hipc(ctx, launch_evolve(a, e, ctx->cfg.rk_order, ctx->nb_rho, ctx->nb_U, ctx->d_partials, ctx->stream),
                   "step kernel");
         e.lam_valid = 1;  // the launch leaves the eigenvectors and energies at t_{s1}
         if (!rc)

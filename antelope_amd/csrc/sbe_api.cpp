@@ -60,6 +60,8 @@ thread_local size_t t_partial_bytes = kPartialBytes;
 // set while a batch creates its members: the batch step kernel runs one k point
 // per lane for every member, so a member's rows and block count must be planned so
 thread_local bool t_batch_member = false;
+// set for a solve that has to take the lean N-band plan (NbRoutes in nband_host.cpp)
+thread_local bool t_lean = false;
 
 struct Plan {
     int kpt = 1;
@@ -320,6 +322,22 @@ int create_batch_member(const sbe_config *cfg, const sbe_model *model, sbe_ctx *
     return rc;
 }
 
+int create_lean(const sbe_config *cfg, const sbe_model *model, sbe_ctx **out)
+{
+    t_lean = true;
+    const int rc = sbe_create(cfg, model, -1, -1, out);
+    t_lean = false;
+    return rc;
+}
+
+int query_footprint(const sbe_config *cfg, const sbe_model *model, bool lean, size_t *bytes)
+{
+    t_lean = lean;
+    const int rc = sbe_query_footprint(cfg, model, -1, -1, bytes);
+    t_lean = false;
+    return rc;
+}
+
 bool shared_eligible(const sbe_ctx *c)
 {
     return c->path == PathKind::Haldane2 && !c->adaptive && !c->velocity && c->hargs.kpt == 1;
@@ -492,7 +510,7 @@ int sbe_query_footprint(const sbe_config *cfg, const sbe_model *model, int64_t k
     }
     if (k_begin < 0 || k_end > ntot || k_begin >= k_end) return set_error(nullptr, SBE_ERR_RANGE, "bad k range");
     if (model->kind != SBE_MODEL_HALDANE) {
-        if (bytes) *bytes = sbe::nb_footprint(*cfg, *model, k_end - k_begin, L.nt, tab.nstage);
+        if (bytes) *bytes = sbe::nb_footprint(*cfg, *model, k_end - k_begin, L.nt, tab.nstage, t_lean);
         return SBE_OK;
     }
     Plan p;
@@ -562,7 +580,16 @@ int sbe_create(const sbe_config *cfg, const sbe_model *model, int64_t k_begin, i
     if (model->kind != SBE_MODEL_HALDANE) {
         ctx->path = sbe::PathKind::NBand;
         rc = hip_check(ctx, hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking), "hipStreamCreate");
+        ctx->lean = t_lean;
         if (!rc) rc = sbe::nb_setup(ctx);
+        if (rc == SBE_ERR_OOM && !ctx->lean) {  // once more with the scratch of the separate kernels alone
+            (void)hipGetLastError();
+            for (auto &b : ctx->owned) (void)hipFree(b.ptr);
+            ctx->owned.clear();
+            ctx->device_bytes = 0;
+            ctx->lean = true;
+            rc = sbe::nb_setup(ctx);
+        }
         if (rc) {
             set_error(nullptr, rc, ctx->err);
             sbe_destroy(ctx);

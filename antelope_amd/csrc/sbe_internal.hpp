@@ -261,6 +261,9 @@ struct sbe_ctx {
     // time-fused length-gauge steps of the analytic classes (nb_evolve_kernel)
     bool nbe = false;
     sbe::NbEvolve evolve{};
+    sbe::TableArgs evolve_laser{};
+    double *evolve_tab = nullptr, *evolve_A = nullptr;
+    bool lean = false;  // N-band: the plan without the scratch of the newer routes (NbRoutes)
     std::string err;
 
     // optional kernel timing: (start, stop) event pairs per kernel class
@@ -317,7 +320,8 @@ hipError_t launch_adaptive_advance(const AdaptiveArgs *d_insts, int n, int64_t n
 int haldane_waves(int64_t nk);
 // N-band host side (nband_host.cpp)
 int nb_validate(const sbe_model &m, std::string &err);
-size_t nb_footprint(const sbe_config &cfg, const sbe_model &m, int64_t nk, int64_t nt, int nstage);
+// lean: the plan of a solve that does not fit otherwise (NbRoutes)
+size_t nb_footprint(const sbe_config &cfg, const sbe_model &m, int64_t nk, int64_t nt, int nstage, bool lean = false);
 int nb_setup(sbe_ctx *ctx);
 int nb_run(sbe_ctx *ctx, int64_t step_begin, int64_t step_end);
 int nb_series(sbe_ctx *ctx, double *j_inter, double *j_intra, double *rho_bar, double *band_pop);
@@ -341,6 +345,9 @@ struct SharedLaunch {
     int cap_insts = 0, cap_map = 0;
 };
 int create_batch_member(const sbe_config *cfg, const sbe_model *model, sbe_ctx **out);
+// sbe_query_footprint and sbe_create of the whole grid, with the lean plan of an N-band solve
+int query_footprint(const sbe_config *cfg, const sbe_model *model, bool lean, size_t *bytes);
+int create_lean(const sbe_config *cfg, const sbe_model *model, sbe_ctx **out);
 bool shared_eligible(const sbe_ctx *c);
 int shared_key(const sbe_ctx *c);  // members of one launch share it (tableau, precision)
 int launch_shared(sbe_ctx *const *cs, const int64_t *nsteps, int n, SharedLaunch &buf, hipStream_t s, std::string &err);

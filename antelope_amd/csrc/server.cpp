@@ -61,6 +61,7 @@ struct Request {
     std::vector<int32_t> rvec;
     std::vector<double> rweight, ham, pos;
     size_t footprint = 0;
+    bool lean = false;  // the plan without the scratch of the faster routes: the other exceeds the budget
     sbe_ctx *ctx = nullptr;
     int lane = -1;                 // shared lane key, or -1: own stream
     int64_t last_seq = 0;          // lane launch that carries this request's last enqueued slice
@@ -262,7 +263,13 @@ int sbe_server_submit(sbe_server *s, const sbe_config *cfg, const sbe_model *mod
         r->model.ham = r->ham.data();
         r->model.pos = model->pos ? r->pos.data() : nullptr;
     }
-    const int rc = sbe_query_footprint(&r->cfg, &r->model, -1, -1, &r->footprint);
+    int rc = sbe::query_footprint(&r->cfg, &r->model, false, &r->footprint);
+    if (rc == SBE_OK && r->footprint > s->budget) {
+        size_t lean = 0;
+        rc = sbe::query_footprint(&r->cfg, &r->model, true, &lean);
+        r->lean = lean < r->footprint;
+        r->footprint = std::min(lean, r->footprint);
+    }
     if (rc != SBE_OK) return srv_fail(s, rc, sbe_last_error(nullptr));
     if (r->footprint > s->budget)
         return srv_fail(s, SBE_ERR_OOM, "request needs " + std::to_string(r->footprint) + " bytes, budget is " +
@@ -334,6 +341,7 @@ int sbe_server_step(sbe_server *s)
         const bool lane_kind = r.model.kind == SBE_MODEL_HALDANE && r.cfg.gauge == SBE_GAUGE_LENGTH_WANNIER &&
                                (r.cfg.rk_order == SBE_RK4 || r.cfg.rk_order == SBE_RK5_FEHLBERG);
         const int rc = lane_kind ? sbe::create_batch_member(&r.cfg, &r.model, &r.ctx)
+                       : r.lean  ? sbe::create_lean(&r.cfg, &r.model, &r.ctx)
                                  : sbe_create(&r.cfg, &r.model, -1, -1, &r.ctx);
         if (rc != SBE_OK) {
             r.err = sbe_last_error(nullptr);

@@ -265,7 +265,8 @@ int sbe_get_state(sbe_ctx *ctx, int32_t basis, double *rho);
 
 int sbe_get_info(const sbe_ctx *ctx, sbe_info *info);
 
-/* Device bytes a context for this problem would allocate. */
+/* Device bytes a context for this problem would allocate (an N-band context that does not get them is
+ * planned once more without the scratch of the time-fused RK5 and analytic steps). */
 int sbe_query_footprint(const sbe_config *cfg, const sbe_model *model,
                         int64_t k_begin, int64_t k_end, size_t *bytes);
 
