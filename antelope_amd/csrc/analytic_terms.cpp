@@ -14,6 +14,14 @@ namespace {
 using cplx = std::complex<double>;
 constexpr double kTwoPi = 6.28318530717958647692;
 
+// products and sizes without std::complex's care for infinities and overflow (ten times the time,
+// at every footprint query); a NaN stays one
+cplx mul(const cplx &a, const cplx &b)
+{
+    return cplx(a.real() * b.real() - a.imag() * b.imag(), a.real() * b.imag() + a.imag() * b.real());
+}
+double size(const cplx &a) { return std::fabs(a.real()) + std::fabs(a.imag()); }
+
 // Per class: the spacings u of its bond components (k.v_t = sum_i n_i u_i k_i
 // with integers n_i, |n_i| <= reach), the sign of J against dH/dk, and which
 // component of v each current slot differentiates (-1: the slot is zero).
@@ -84,7 +92,7 @@ bool analytic_terms(int kind, int N, const double *params, AnalyticTerms &out)
                                      Ld[2] > 1 ? kTwoPi * z / Ld[2] / lay.u[2] : 0.0};
                 std::vector<cplx> H;
                 eval(kind, N, params, k, H, nullptr);
-                for (const cplx &v : H) hmax = std::max(hmax, std::abs(v));
+                for (const cplx &v : H) hmax = std::max(hmax, size(v));
                 smp.push_back(std::move(H));
             }
     if (!std::isfinite(hmax)) return false;
@@ -93,16 +101,35 @@ bool analytic_terms(int kind, int N, const double *params, AnalyticTerms &out)
     for (int d = 0; d < 3; ++d)
         for (int m = 0; m < Ld[d]; ++m)
             root[d].push_back(std::polar(1.0, -kTwoPi * m / Ld[d]));
-    auto coef = [&](int nx, int ny, int nz, int e) {
-        cplx s = 0.0;
-        size_t q = 0;
-        auto at = [&](int d, int n, int x) { return root[d][((n * x) % Ld[d] + Ld[d]) % Ld[d]]; };
-        for (int x = 0; x < Ld[0]; ++x)
-            for (int y = 0; y < Ld[1]; ++y) {
-                const cplx xy = at(0, nx, x) * at(1, ny, y);
-                for (int z = 0; z < Ld[2]; ++z, ++q) s += smp[q][e] * (xy * at(2, nz, z));
+    // the transform of every element, one axis at a time (elements that are zero throughout stay so)
+    const size_t stride[3] = {static_cast<size_t>(Ld[1]) * Ld[2], static_cast<size_t>(Ld[2]), 1};
+    std::vector<std::vector<cplx>> tr(nn);
+    for (int e = 0; e < nn; ++e) {
+        std::vector<cplx> &f = tr[e];
+        f.reserve(smp.size());
+        bool any = false;
+        for (const std::vector<cplx> &H : smp) {
+            f.push_back(H[e]);
+            any = any || H[e] != cplx(0.0);
+        }
+        for (int d = 0; d < 3 && any; ++d) {
+            if (Ld[d] == 1) continue;
+            cplx line[2][9];
+            for (size_t q = 0; q < f.size(); ++q) {
+                if ((q / stride[d]) % Ld[d] != 0) continue;  // the first point of each line
+                for (int x = 0; x < Ld[d]; ++x) line[0][x] = f[q + x * stride[d]];
+                for (int n = 0; n < Ld[d]; ++n) {
+                    line[1][n] = 0.0;
+                    for (int x = 0; x < Ld[d]; ++x) line[1][n] += mul(line[0][x], root[d][(n * x) % Ld[d]]);
+                }
+                for (int n = 0; n < Ld[d]; ++n) f[q + n * stride[d]] = line[1][n];
             }
-        return s / static_cast<double>(smp.size());
+        }
+        for (cplx &v : f) v /= static_cast<double>(smp.size());
+    }
+    auto coef = [&](int nx, int ny, int nz, int e) {
+        auto wrap = [&](int d, int n) { return static_cast<size_t>((n % Ld[d] + Ld[d]) % Ld[d]); };
+        return tr[e][wrap(0, nx) * stride[0] + wrap(1, ny) * stride[1] + wrap(2, nz)];
     };
     auto clean = [&](cplx v) {  // rounding residue of the transform
         return cplx(std::fabs(v.real()) < 1e-15 * hmax ? 0.0 : v.real(), std::fabs(v.imag()) < 1e-15 * hmax ? 0.0 : v.imag());
@@ -127,8 +154,8 @@ bool analytic_terms(int kind, int N, const double *params, AnalyticTerms &out)
                 for (int e = 0; e < nn; ++e) {
                     const cplx a = coef(nx, ny, nz, e), b = coef(-nx, -ny, -nz, e);
                     P[e] = clean(a + b);
-                    Q[e] = clean(cplx(0.0, 1.0) * (a - b));
-                    big = std::max({big, std::abs(P[e]), std::abs(Q[e])});
+                    Q[e] = clean(cplx(b.imag() - a.imag(), a.real() - b.real()));  // i (a - b)
+                    big = std::max({big, size(P[e]), size(Q[e])});
                 }
                 if (big < 1e-13 * hmax) continue;
                 if (out.T == kMaxTerms) return false;
@@ -163,21 +190,28 @@ bool analytic_terms(int kind, int N, const double *params, AnalyticTerms &out)
         std::vector<cplx> H, J;
         eval(kind, N, params, k, H, &J);
         double jmax = 0.0;
-        for (const cplx &v : J) jmax = std::max(jmax, std::abs(v));
+        for (const cplx &v : J) jmax = std::max(jmax, size(v));
+        double cs[kMaxTerms], sn[kMaxTerms];
+        for (int t = 0; t < out.T; ++t) {
+            const double th = k[0] * out.vec[t][0] + k[1] * out.vec[t][1] + k[2] * out.vec[t][2];
+            cs[t] = std::cos(th);
+            sn[t] = std::sin(th);
+        }
         for (int e = 0; e < nn; ++e) {
+            const cplx scale(out.scale[2 * e], out.scale[2 * e + 1]);
             cplx h(out.m0[2 * e], out.m0[2 * e + 1]), g[3] = {0.0, 0.0, 0.0};
             for (int t = 0; t < out.T; ++t) {
-                const double th = k[0] * out.vec[t][0] + k[1] * out.vec[t][1] + k[2] * out.vec[t][2];
                 const size_t o = 2 * (static_cast<size_t>(t) * nn + e);
                 const cplx p(out.p[o], out.p[o + 1]), q(out.q[o], out.q[o + 1]);
-                h += p * std::cos(th) + q * std::sin(th);
-                for (int c = 0; c < 3; ++c) g[c] += cplx(out.scale[2 * e], out.scale[2 * e + 1]) * out.grad[t][c] * (q * std::cos(th) - p * std::sin(th));
+                h += p * cs[t] + q * sn[t];
+                const cplx dh = mul(scale, q * cs[t] - p * sn[t]);
+                for (int c = 0; c < 3; ++c) g[c] += out.grad[t][c] * dh;
             }
-            if (!(std::abs(h - H[e]) <= 1e-12 * hmax)) return false;
+            if (!(size(h - H[e]) <= 1e-12 * hmax)) return false;
             const int tr = (e % N) * N + e / N;
             for (int c = 0; c < 3; ++c) {
                 const cplx jh = 0.5 * (J[static_cast<size_t>(c) * nn + e] + std::conj(J[static_cast<size_t>(c) * nn + tr]));
-                if (!(std::abs(g[c] - jh) <= 1e-12 * std::max(jmax, hmax))) return false;
+                if (!(size(g[c] - jh) <= 1e-12 * std::max(jmax, hmax))) return false;
             }
         }
     }
