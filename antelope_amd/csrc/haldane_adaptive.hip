@@ -500,6 +500,11 @@ __device__ __forceinline__ void kahan(R &sum, R &c, R inc)
 // and the oldest node drops out of the stencil by itself. The node times are
 // uniform (in the wave's LDS slice); each lane keeps the differences of its
 // wave-summed observable (sum8_value).
+// SWAPS: the sums come from wave_reduce8, whose lane l holds value l >> 3, member l & 7. The FP32-state
+// stepper takes it: its chain waits for each step's sums, and there the matrix pipe's longer way is not
+// made up by the issue slots it saves (64 solves of 200x200: 173.8 ms a pass against 180.6; the FP64 stepper,
+// 141.5 with the matrix pipe, was at 145.8 with swaps).
+template <bool SWAPS>
 struct SampleRing {
     double D[6];  // divided differences of this lane's value, newest node first
     double *t;    // [6] node times, newest first (LDS)
@@ -555,14 +560,14 @@ struct SampleRing {
         double tk[6];  // the node times, from LDS once per call
 #pragma unroll
         for (int k = 0; k < 6; ++k) tk[k] = t[k];
-        const int j = sum8_member(__lane_id());
+        const int j = SWAPS ? (__lane_id() & 7) : sum8_member(__lane_id());
         while (mi < mend) {
             const bool in = j < mend - mi;
             const int mj = in ? mi + j : mi;
             const double tm = atmin + dt_out * static_cast<double>(mj);
             const bool ok = in && !(tm > t_hi);
             // the times grow with j, so the members that write are a prefix of each value's
-            const int n = __popcll(__ballot(ok) & kSum8First);
+            const int n = __popcll(__ballot(ok) & (SWAPS ? 0xffull : kSum8First));
             if (ok) part[(static_cast<int64_t>(mj) - out0) * row_stride] = at(tm, tk);
             mi += n;
             if (n < 8) break;
@@ -635,8 +640,8 @@ __device__ void adaptive_body(const AdaptiveArgs &A, int64_t blk, const int64_t 
     // T1 is off on this path (the host rejects it): g1 = 0
     const R gh2 = static_cast<R>(0.5 * a.gam2), gh12 = static_cast<R>(-0.5 * a.gam2);
     const R ii = a.inter_intra ? R(1) : R(0);
-    // this lane writes value sum8_value of the wave's partial row of each sample
-    double *part = a.partials + static_cast<int64_t>(wave) * kHaldaneNV + sum8_value(lane);
+    // this lane writes value lane >> 3 of the wave's partial row of each sample
+    double *part = a.partials + static_cast<int64_t>(wave) * kHaldaneNV + (lane >> 3);
     const int64_t row_stride = static_cast<int64_t>(a.nwaves) * kHaldaneNV;
 
     __shared__ R lds_rows[kAdaptiveBlock / 64][6 * kRow];
@@ -700,13 +705,13 @@ __device__ void adaptive_body(const AdaptiveArgs &A, int64_t blk, const int64_t 
     bool failed = false;
 
     // Step ends carry the wave sums of the observables (this lane: value
-    // sum8_value) into the six-node ring; samples are its Lagrange
+    // lane >> 3) into the six-node ring; samples are its Lagrange
     // interpolants. At the window start: the sample itself, and the first
     // stage.
     Vec3<R> k1[KPT];
     Vec3<R> dh0[KPT];  // delta form: dh at the current step start (error scale)
     __shared__ double lds_ring[kAdaptiveBlock / 64][6];
-    SampleRing ring;
+    SampleRing<true> ring;
     ring.cnt = 0;
     ring.t = lds_ring[threadIdx.x >> 6];
 #pragma unroll
@@ -736,7 +741,7 @@ __device__ void adaptive_body(const AdaptiveArgs &A, int64_t blk, const int64_t 
                            Vec3<R>{2 * k1[q].x, 2 * k1[q].y, 2 * k1[q].z}, row, a, ii, o, od);
             }
         }
-        const double O0 = wave_sum8(o);
+        const double O0 = wave_reduce8(o);
         part[(m - out0) * row_stride] = O0;
         ring.push(t, O0);
         ++m;
@@ -836,7 +841,7 @@ __device__ void adaptive_body(const AdaptiveArgs &A, int64_t blk, const int64_t 
                 else observe<R>(p[q], p[q].n - p[q].cn, Vec3<R>{p[q].sx - p[q].cx, p[q].sy - p[q].cy, p[q].sz - p[q].cz},
                                 Vec3<R>{2 * k1[q].x, 2 * k1[q].y, 2 * k1[q].z}, row7, a, ii, o, od);
             }
-            ring.push(tn, wave_sum8(o));
+            ring.push(tn, wave_reduce8(o));
             if (ring.cnt >= 6) emit(ring.t[2]);  // samples up to node c - 2
             t = tn;
             ++nacc;
@@ -971,7 +976,7 @@ __device__ void adaptive_body64(const AdaptiveArgs &A, int64_t blk, const int64_
     int64_t nacc = 0, nrej = 0;
     bool failed = false;
     __shared__ double lds_ring[kAdaptiveBlock / 64][6];
-    SampleRing ring;
+    SampleRing<false> ring;
     ring.cnt = 0;
     ring.t = lds_ring[threadIdx.x >> 6];
 #pragma unroll

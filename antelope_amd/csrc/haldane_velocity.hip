@@ -91,37 +91,6 @@ __device__ __forceinline__ void occupations(const HaldaneArgs &a, double e0, dou
 
 constexpr int kTile = 64;  // time steps per LDS tile of the A(t) table
 
-// Sum each of v[0..7] over the 64 lanes of the wave (reduce-scatter):
-// lane l ends with the total of v[(l >> 3) & 7]. Requires all 64 lanes.
-__device__ __forceinline__ double wave_reduce8(double v[8])
-{
-    const int lane = __lane_id();
-    // lane bit 5: permlane32 swap + add
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        double a = v[j], b = v[j + 4];
-        swap32(a, b);
-        v[j] = a + b;  // lanes 0-31: v[j], lanes 32-63: v[j+4]
-    }
-    // lane bit 4: permlane16 swap + add
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        double a = v[j], b = v[j + 2];
-        swap16(a, b);
-        v[j] = a + b;  // even rows: v[j], odd rows: v[j+2]
-    }
-    // lane bit 3: rotate by 8 inside each 16-lane row (= lane ^ 8)
-    const bool hi = (lane & 8) != 0;
-    const double keep = hi ? v[1] : v[0];
-    const double send = hi ? v[0] : v[1];
-    double x = keep + dpp_f64<0x128>(send);  // row_ror:8
-    // lanes 8q..8q+7 now share value index q: all-reduce over the low 3 bits
-    x += dpp_f64<0x141>(x);  // row_half_mirror (i <-> 7-i)
-    x += dpp_f64<0x4E>(x);   // quad_perm [2,3,0,1]
-    x += dpp_f64<0xB1>(x);   // quad_perm [1,0,3,2]
-    return x;
-}
-
 // The k sums of a step: on the matrix pipe (wave_sum8), which saves issue slots, from this many
 // waves up; below, by swaps and DPP (wave_reduce8), whose chain is shorter: this gauge's step has
 // little else to put beside it. RK4, us a step, swaps against matrix pipe: 48x48 k points 0.301
