@@ -374,14 +374,16 @@ int sbe_batch_autotune(int32_t n, const sbe_config *cfgs, const sbe_model *model
  *           before the step, sum_k w (j_inter_x, j_inter_y, j_intra_x,
  *           j_intra_y, s_x, s_y, s_z, s.d/|d|) at k + A(t_n); sbe_get_series
  *           forms j_inter, j_intra, rho_bar and band_pop from the same values.
+ *           The call returns before they exist, so nothing checks them: a
+ *           value that is not finite (a state or weight that is not) makes
+ *           all eight of its step NaN, whichever it was.
  * The laser rows and the partial sums of the k reduction use one static
  * device array of SBE_NOALLOC_SCRATCH_BYTES per device (held until the
  * process ends); k sets whose partial rows of one step exceed it are
  * rejected with SBE_ERR_RANGE (about 16 M k points). The call only enqueues
  * kernels on `stream` (a hipStream_t; NULL = the default stream) and returns;
  * the caller synchronizes. Calls that overlap on one GPU race on the shared
- * array. Results equal sbe_run's to rounding (the laser rows are evaluated
- * on the device instead of the host). */
+ * array. Results equal sbe_run's to rounding. */
 #define SBE_NOALLOC_SCRATCH_BYTES (16u << 20)
 #define SBE_NOALLOC_K_ALIGN 512
 int sbe_run_haldane_noalloc(const sbe_config *cfg, const sbe_model *model, const double *kpts, double *state,
