@@ -91,12 +91,14 @@ __device__ __forceinline__ void occupations(const HaldaneArgs &a, double e0, dou
 
 constexpr int kTile = 64;  // time steps per LDS tile of the A(t) table
 
-// The k sums of a step: on the matrix pipe (wave_sum8), which saves issue slots, from this many
-// waves up; below, by swaps and DPP (wave_reduce8), whose chain is shorter: this gauge's step has
-// little else to put beside it. RK4, us a step, swaps against matrix pipe: 48x48 k points 0.301
-// and 0.332, 200x200 0.313 and 0.346, 300x300 (1408 waves) 0.476 and 0.522; before any change
-// 800x800 (10000 waves) 2.71, with the matrix pipe 2.40.
-constexpr int kMatrixSumWaves = 4096;
+// The k sums of a step by swaps and DPP (wave_reduce8), whose chain is short: this gauge's step has little
+// else to put beside it. With FP32 state, whose step issues more instructions for its compensation, on the
+// matrix pipe (wave_sum8: fewer issue slots) from this many waves up. us a step, swaps and matrix pipe:
+//   FP64 RK4  48^2 k points (36 waves) 0.312 and 0.346, 300^2 (704) 0.509 and 0.546, 720^2 (4052) 1.92 and 2.02,
+//             1000^2 (7816) 3.86 and 4.00, 2000^2 (31252) 15.8 and 16.4
+//   FP32 RK4  48^2 (36) 0.342 and 0.374, 300^2 (1408) 0.604 and 0.627, 400^2 (2504) 0.902 and 0.898, 1000^2 (15628) 4.62 and 4.50
+//   FP32 RK5  300^2 0.825 and 0.858, 400^2 1.228 and 1.210, 1000^2 6.37 and 6.00
+constexpr int kMatrixSumWaves = 2560;
 
 // Step kernel body; R, RK, T1ON, DEPH, KPT as in the length-gauge kernel.
 // The stage right-hand side is evaluated as half of the reference RHS with
@@ -338,9 +340,10 @@ void launch_vel(const HaldaneArgs &a, const R *tab, bool t1_on, hipStream_t s)
 template <typename R, int RK>
 void launch_vel_kpt(const HaldaneArgs &a, const R *tab, bool t1_on, hipStream_t s)
 {
-    const bool msum = a.nwaves >= kMatrixSumWaves;
-    if (a.kpt == 2) msum ? launch_vel<R, RK, 2, true>(a, tab, t1_on, s) : launch_vel<R, RK, 2, false>(a, tab, t1_on, s);
-    else msum ? launch_vel<R, RK, 1, true>(a, tab, t1_on, s) : launch_vel<R, RK, 1, false>(a, tab, t1_on, s);
+    constexpr bool kMay = StateT<R>::kComp;  // FP32 state
+    const bool msum = kMay && a.nwaves >= kMatrixSumWaves;
+    if (a.kpt == 2) msum ? launch_vel<R, RK, 2, kMay>(a, tab, t1_on, s) : launch_vel<R, RK, 2, false>(a, tab, t1_on, s);
+    else msum ? launch_vel<R, RK, 1, kMay>(a, tab, t1_on, s) : launch_vel<R, RK, 1, false>(a, tab, t1_on, s);
 }
 
 }  // namespace

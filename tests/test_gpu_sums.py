@@ -33,8 +33,8 @@ def test_wave_sums(oracle, n, gauge, rk, inter_intra):
 
 
 def test_velocity_sums_by_matrix_pipe():
-    """The velocity gauge's sums change route at 4096 waves (262144 k points): k blocks below it against the
-    whole grid above, the same sums to rounding."""
+    """k blocks of a grid against the whole of it, the same sums to rounding. (FP64 sums by swaps at any size; the FP32
+    state's change of route is tested below.)"""
     cfg = small_config(n=(520, 505), ncycles=0.02, rk=4, ellip=0.4, grid="mp", T1=300.0, gauge="VelocityHamiltonian")
     model = haldane_cfg1_model()
     nk, cut = 520 * 505, 100000
@@ -47,3 +47,28 @@ def test_velocity_sums_by_matrix_pipe():
     whole, parts = run(-1, -1), [run(0, cut), run(cut, nk)]
     for key in ("j_inter", "j_intra", "band_pop", "rho_bar"):
         assert rel_l2(parts[0][key] + parts[1][key], whole[key]) < 1e-10, key
+
+
+@pytest.mark.parametrize("rk,T1", [(4, 0.0), (5, 300.0)])
+@pytest.mark.parametrize("kpt", [1, 2])
+def test_velocity_fp32_sums_by_matrix_pipe(monkeypatch, rk, T1, kpt):
+    """With FP32 state the velocity gauge's sums take the matrix pipe from 2560 waves up: a whole grid above it against
+    its k blocks below, which use swaps. Both add the same FP64 values, in another order: 1e-12 of the largest."""
+    n = (500, 440) if kpt == 1 else (800, 550)
+    nk, cut = n[0] * n[1], 160000 if kpt == 1 else 315000
+    waves = lambda k: -(-k // (256 * kpt)) * 4  # noqa: E731  (blocks of four waves, kpt k points per lane)
+    assert waves(nk) >= 2560 > max(waves(cut), waves(nk - cut))
+    monkeypatch.setenv("ANTELOPE_HALDANE_KPT", str(kpt))
+    cfg = small_config(n=n, ncycles=0.02, rk=rk, ellip=0.4, grid="mp", T1=T1, gauge="VelocityHamiltonian", precision="fp32")
+    model = haldane_cfg1_model()
+    print("fp32 velocity sums:", rk, T1, kpt, flush=True)
+
+    def run(a, b):
+        with SBESolver(cfg, model, a, b) as s:
+            s.run()
+            return s.series()
+
+    whole, parts = run(-1, -1), [run(0, cut), run(cut, nk)]
+    for key in ("j_inter", "j_intra", "band_pop", "rho_bar"):
+        a, b = parts[0][key] + parts[1][key], whole[key]
+        assert np.abs(a - b).max() <= 1e-12 * np.abs(b).max(), key
