@@ -18,13 +18,13 @@
 // chunk. H(k+A) uses e^{i(k+A).v} = e^{ik.v} e^{iA.v}: the six e^{ik.v} are
 // computed once per launch, the k-independent e^{iA(t).v} come from a
 // per-stage table staged in LDS. Every time sample is reduced over the 64
-// lanes of a wave on the matrix pipe, and one row of 8 FP64 partial sums per
+// lanes of a wave by swaps and DPP, and one row of 8 FP64 partial sums per
 // wave and step goes to HBM; a second kernel (series.hip) sums the rows in a
 // fixed order.
 //
 // Bound by the VALU: a wave alone on its SIMD (fewer than 65536 k points) issues its
 // FP64 chain at 4 cycles an instruction, about 240 of them for an RK4 step of a k point
-// (316 before the k sums moved to the matrix pipe and the sample and the right-hand side
+// (316 before the sample and the right-hand side
 // were factored; 465 for RK5 with T1), so fewer instructions are what there is to gain.
 #include "haldane_setup.hpp"
 
@@ -99,7 +99,7 @@ __device__ __forceinline__ void steps_body(const HaldaneArgs &a, const R *__rest
     const R gh1 = static_cast<R>(0.5 * a.gam1), gh2 = static_cast<R>(0.5 * a.gam2);
     const R gh12 = static_cast<R>(0.5 * (a.gam1 - a.gam2));
     const int lane = __lane_id();
-    const double scale = sum8_scale(a, lane);
+    const double scale = sum8_scale<true>(a, lane);
     const bool ii = a.inter_intra != 0;
 
     // The k-independent phase rows of kTile steps are staged in LDS (double
@@ -154,8 +154,8 @@ __device__ __forceinline__ void steps_body(const HaldaneArgs &a, const R *__rest
 #pragma unroll
         for (int q = 0; q < KPT; ++q) time_sample<R>(p[q], ph[q], a, v);
         // eight lanes hold each value: duplicate stores of equal data keep the step branch-free
-        partials[(static_cast<int64_t>(step) * a.nwaves + wave) * kHaldaneNV + sum8_value(lane)] =
-            sample_sums(v, scale, ii, lane);
+        partials[(static_cast<int64_t>(step) * a.nwaves + wave) * kHaldaneNV + Sum8<true>::value(lane)] =
+            sample_sums<true>(v, scale, ii, lane);
 
         // ---- one RK step (SBEs.h:596-624), stage RHS halved (see above)
 #pragma unroll

@@ -499,7 +499,7 @@ __device__ __forceinline__ void kahan(R &sum, R &c, R inc)
 // updates them in place, D'_0 = f_new, D'_k = (D'_k-1 - D_k-1) / (t_new - t_n+1-k),
 // and the oldest node drops out of the stencil by itself. The node times are
 // uniform (in the wave's LDS slice); each lane keeps the differences of its
-// wave-summed observable (sum8_value).
+// wave-summed observable (Sum8::value).
 // SWAPS: the sums come from wave_reduce8, whose lane l holds value l >> 3, member l & 7. The FP32-state
 // stepper takes it: its chain waits for each step's sums, and there the matrix pipe's longer way is not
 // made up by the issue slots it saves (64 solves of 200x200: 173.8 ms a pass against 180.6; the FP64 stepper,
@@ -551,7 +551,7 @@ struct SampleRing {
     // Writes the samples mi, mi + 1, ... (below mend) whose times
     // atmin + n dt_out do not exceed t_hi, and returns the next one. The eight
     // lanes of a value hold the same ring, so a lane evaluates sample
-    // mi + sum8_member of it: eight samples per pass, each with the
+    // mi + Sum8::member of it: eight samples per pass, each with the
     // arithmetic of a single evaluation. part points at this lane's value
     // column of sample row out0.
     __device__ __forceinline__ int emit(int mi, int mend, double atmin, double dt_out, double t_hi, double *part,
@@ -560,14 +560,14 @@ struct SampleRing {
         double tk[6];  // the node times, from LDS once per call
 #pragma unroll
         for (int k = 0; k < 6; ++k) tk[k] = t[k];
-        const int j = SWAPS ? (__lane_id() & 7) : sum8_member(__lane_id());
+        const int j = Sum8<SWAPS>::member(__lane_id());
         while (mi < mend) {
             const bool in = j < mend - mi;
             const int mj = in ? mi + j : mi;
             const double tm = atmin + dt_out * static_cast<double>(mj);
             const bool ok = in && !(tm > t_hi);
             // the times grow with j, so the members that write are a prefix of each value's
-            const int n = __popcll(__ballot(ok) & (SWAPS ? 0xffull : kSum8First));
+            const int n = __popcll(__ballot(ok) & Sum8<SWAPS>::kFirst);
             if (ok) part[(static_cast<int64_t>(mj) - out0) * row_stride] = at(tm, tk);
             mi += n;
             if (n < 8) break;
@@ -640,8 +640,8 @@ __device__ void adaptive_body(const AdaptiveArgs &A, int64_t blk, const int64_t 
     // T1 is off on this path (the host rejects it): g1 = 0
     const R gh2 = static_cast<R>(0.5 * a.gam2), gh12 = static_cast<R>(-0.5 * a.gam2);
     const R ii = a.inter_intra ? R(1) : R(0);
-    // this lane writes value lane >> 3 of the wave's partial row of each sample
-    double *part = a.partials + static_cast<int64_t>(wave) * kHaldaneNV + (lane >> 3);
+    // this lane writes value Sum8::value of the wave's partial row of each sample
+    double *part = a.partials + static_cast<int64_t>(wave) * kHaldaneNV + Sum8<true>::value(lane);
     const int64_t row_stride = static_cast<int64_t>(a.nwaves) * kHaldaneNV;
 
     __shared__ R lds_rows[kAdaptiveBlock / 64][6 * kRow];
@@ -705,7 +705,7 @@ __device__ void adaptive_body(const AdaptiveArgs &A, int64_t blk, const int64_t 
     bool failed = false;
 
     // Step ends carry the wave sums of the observables (this lane: value
-    // lane >> 3) into the six-node ring; samples are its Lagrange
+    // Sum8::value) into the six-node ring; samples are its Lagrange
     // interpolants. At the window start: the sample itself, and the first
     // stage.
     Vec3<R> k1[KPT];
@@ -741,7 +741,7 @@ __device__ void adaptive_body(const AdaptiveArgs &A, int64_t blk, const int64_t 
                            Vec3<R>{2 * k1[q].x, 2 * k1[q].y, 2 * k1[q].z}, row, a, ii, o, od);
             }
         }
-        const double O0 = wave_reduce8(o);
+        const double O0 = Sum8<true>::total(o);
         part[(m - out0) * row_stride] = O0;
         ring.push(t, O0);
         ++m;
@@ -841,7 +841,7 @@ __device__ void adaptive_body(const AdaptiveArgs &A, int64_t blk, const int64_t 
                 else observe<R>(p[q], p[q].n - p[q].cn, Vec3<R>{p[q].sx - p[q].cx, p[q].sy - p[q].cy, p[q].sz - p[q].cz},
                                 Vec3<R>{2 * k1[q].x, 2 * k1[q].y, 2 * k1[q].z}, row7, a, ii, o, od);
             }
-            ring.push(tn, wave_reduce8(o));
+            ring.push(tn, Sum8<true>::total(o));
             if (ring.cnt >= 6) emit(ring.t[2]);  // samples up to node c - 2
             t = tn;
             ++nacc;
@@ -959,8 +959,8 @@ __device__ void adaptive_body64(const AdaptiveArgs &A, int64_t blk, const int64_
     const double c3 = a.c3, M0 = a.M0;
     const double gh2 = 0.5 * a.gam2, gh12 = -0.5 * a.gam2;  // T1 off on this path
     const bool ii = a.inter_intra != 0;
-    const double scale = sum8_scale(a, lane);
-    double *part = a.partials + static_cast<int64_t>(wave) * kHaldaneNV + sum8_value(lane);
+    const double scale = sum8_scale<false>(a, lane);
+    double *part = a.partials + static_cast<int64_t>(wave) * kHaldaneNV + Sum8<false>::value(lane);
     const int64_t row_stride = static_cast<int64_t>(a.nwaves) * kHaldaneNV;
     __shared__ double lds_rows[kAdaptiveBlock / 64][6 * kRow];
     double *rows = lds_rows[threadIdx.x >> 6];
@@ -998,7 +998,7 @@ __device__ void adaptive_body64(const AdaptiveArgs &A, int64_t blk, const int64_
             k1[q] = half_rhs<DEPH>(e.d, -gh12 * e.inv, y, gh2);
             sample_state(e, p[q].w, p[q].n, y.x, y.y, y.z, a, v);
         }
-        const double val = sample_sums(v, scale, ii, lane);
+        const double val = sample_sums<false>(v, scale, ii, lane);
         part[0] = val;
         ring.push(t, val);
         ++m;
@@ -1103,7 +1103,7 @@ __device__ void adaptive_body64(const AdaptiveArgs &A, int64_t blk, const int64_
                 k1[q] = half_rhs<DEPH>(e1.d, -gh12 * e1.inv, y, gh2);  // f(t + h, y5)
                 sample_state(e1, p[q].w, p[q].n, y.x, y.y, y.z, a, v);
             }
-            ring.push(tn, sample_sums(v, scale, ii, lane));
+            ring.push(tn, sample_sums<false>(v, scale, ii, lane));
             if (ring.cnt >= 6) emit(ring.t[2]);  // samples up to node c - 2
             t = tn;
             ++nacc;

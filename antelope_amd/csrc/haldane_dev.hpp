@@ -85,10 +85,8 @@ constexpr unsigned long long kSum8First = 0x0000111100001111ull;  // the lanes o
 // lanes into column q, so four values share one accumulator; a second one with A = ones
 // adds the rows of that. The four blocks of a row are added with DPP. 10 MFMAs and 8 VALU
 // additions and moves, against 45 VALU instructions of a reduce-scatter by permlane swaps
-// and DPP (316 -> 280 instructions of an RK4 step of the 2-band kernel). A value that is not
-// finite meets the others' zeros and makes all eight NaN; every reader of the sums refuses such a row or
-// says so. (An accumulator and a select per value would keep them apart: 40x40 k points, 64 steps without
-// allocation, 64.3 us against 52.3.)
+// and DPP, but a longer way to the sums. A value that is not
+// finite meets the others' zeros and makes all eight NaN: only for sums whose reader refuses such a row.
 __device__ __forceinline__ double wave_sum8(const double v[8])
 {
     const int lane = __lane_id();
@@ -108,7 +106,10 @@ __device__ __forceinline__ double wave_sum8(const double v[8])
 }
 
 // Sum each of v[0..7] over the 64 lanes of the wave by swaps and DPP (reduce-scatter):
-// lane l ends with the total of v[(l >> 3) & 7]. Requires all 64 lanes.
+// lane l ends with the total of v[(l >> 3) & 7]. Requires all 64 lanes. The faster of the two in the
+// fixed-step length-gauge kernels, us a step, swaps and matrix pipe: FP64 RK4 40^2 k points 0.634 and 0.649,
+// 300^2 1.10 and 1.12, 1000^2 8.7 and 9.9; FP32 300^2 0.99 and 1.03; 64 solves of 200^2 408 and 421 ms (FP64),
+// 291 and 307 (FP32).
 __device__ __forceinline__ double wave_reduce8(double v[8])
 {
     const int lane = __lane_id();
@@ -311,22 +312,41 @@ __device__ __forceinline__ void sample_state(const Phases<R> &e, double wk, R n,
     v[7] += static_cast<double>(e.dd > R(0) ? sd * e.q : -s_z);
 }
 
+// Which of the two a kernel takes, and the lanes of a value
+template <bool SWAPS>
+struct Sum8 {
+    static constexpr unsigned long long kFirst = SWAPS ? 0xffull : kSum8First;  // the lanes of value 0
+    static __device__ __forceinline__ int value(int lane) { return SWAPS ? lane >> 3 : sum8_value(lane); }
+    static __device__ __forceinline__ int member(int lane) { return SWAPS ? lane & 7 : sum8_member(lane); }
+    static __device__ __forceinline__ double total(double v[8]) { return SWAPS ? wave_reduce8(v) : wave_sum8(v); }
+    // of value q the total of value q ^ 2
+    static __device__ __forceinline__ double other_pair(double x, int lane)
+    {
+        if (!SWAPS) return dpp_f64<0x4E>(x);
+        double a = x, b = x;
+        swap16(a, b);  // even rows hold (own, other), odd rows (other, own)
+        return (lane & 16) != 0 ? a : b;
+    }
+};
+
 // the factor of this lane's value in the k sums of sample_state
+template <bool SWAPS>
 __device__ __forceinline__ double sum8_scale(const HaldaneArgs &a, int lane)
 {
-    const int v = sum8_value(lane);
+    const int v = Sum8<SWAPS>::value(lane);
     if (v > 3) return 1.0;
     return (v & 1 ? -0.5 : -0.86602540378443864676) * a.va[0][1];  // va[0] = (0, a0)
 }
 
 // The k sums of a sample in this lane's value: inter and intra as they are, or (GenCurrent) the
 // total current in the first pair and nothing in the second.
-__device__ __forceinline__ double sample_sums(const double v[8], double scale, bool inter_intra, int lane)
+template <bool SWAPS>
+__device__ __forceinline__ double sample_sums(double v[8], double scale, bool inter_intra, int lane)
 {
-    double r = wave_sum8(v) * scale;
+    double r = Sum8<SWAPS>::total(v) * scale;
     if (!inter_intra) {  // uniform
-        const double o = dpp_f64<0x4E>(r);  // values 0 <-> 2, 1 <-> 3
-        const int q = sum8_value(lane);
+        const double o = Sum8<SWAPS>::other_pair(r, lane);  // values 0 <-> 2, 1 <-> 3
+        const int q = Sum8<SWAPS>::value(lane);
         r = q > 3 ? r : (q < 2 ? r + o : 0.0);
     }
     return r;

@@ -205,8 +205,7 @@ __device__ __forceinline__ void vel_body(const HaldaneArgs &a, const R *__restri
             v[7] -= static_cast<double>(z) * w;  // band populations (n -+ v7)/2 as in the length gauge
         }
         double *row = partials + (static_cast<int64_t>(step) * a.nwaves + wave) * kHaldaneNV;
-        if (MSUM) row[sum8_value(lane)] = wave_sum8(v);
-        else row[lane >> 3] = wave_reduce8(v);
+        row[Sum8<!MSUM>::value(lane)] = Sum8<!MSUM>::total(v);
 
         // ---- one RK step (SBEs.h:596-624)
 #pragma unroll

@@ -374,9 +374,6 @@ int sbe_batch_autotune(int32_t n, const sbe_config *cfgs, const sbe_model *model
  *           before the step, sum_k w (j_inter_x, j_inter_y, j_intra_x,
  *           j_intra_y, s_x, s_y, s_z, s.d/|d|) at k + A(t_n); sbe_get_series
  *           forms j_inter, j_intra, rho_bar and band_pop from the same values.
- *           The call returns before they exist, so nothing checks them: a
- *           value that is not finite (a state or weight that is not) makes
- *           all eight of its step NaN, whichever it was.
  * The laser rows and the partial sums of the k reduction use one static
  * device array of SBE_NOALLOC_SCRATCH_BYTES per device (held until the
  * process ends); k sets whose partial rows of one step exceed it are
