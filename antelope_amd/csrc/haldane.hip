@@ -100,6 +100,7 @@ __device__ __forceinline__ void steps_body(const HaldaneArgs &a, const R *__rest
     const R gh12 = static_cast<R>(0.5 * (a.gam1 - a.gam2));
     const int lane = __lane_id();
     const double scale = sum8_scale<true>(a, lane);
+    double *const mine = partials + wave * kHaldaneNV + Sum8<true>::value(lane);  // this lane's value of a row
     const bool ii = a.inter_intra != 0;
 
     // The k-independent phase rows of kTile steps are staged in LDS (double
@@ -154,8 +155,7 @@ __device__ __forceinline__ void steps_body(const HaldaneArgs &a, const R *__rest
 #pragma unroll
         for (int q = 0; q < KPT; ++q) time_sample<R>(p[q], ph[q], a, v);
         // eight lanes hold each value: duplicate stores of equal data keep the step branch-free
-        partials[(static_cast<int64_t>(step) * a.nwaves + wave) * kHaldaneNV + Sum8<true>::value(lane)] =
-            sample_sums<true>(v, scale, ii, lane);
+        mine[static_cast<int64_t>(step) * a.nwaves * kHaldaneNV] = sample_sums<true>(v, scale, ii, lane);
 
         // ---- one RK step (SBEs.h:596-624), stage RHS halved (see above)
 #pragma unroll

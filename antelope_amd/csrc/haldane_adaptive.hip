@@ -500,7 +500,7 @@ __device__ __forceinline__ void kahan(R &sum, R &c, R inc)
 // and the oldest node drops out of the stencil by itself. The node times are
 // uniform (in the wave's LDS slice); each lane keeps the differences of its
 // wave-summed observable (Sum8::value).
-// SWAPS: the sums come from wave_reduce8, whose lane l holds value l >> 3, member l & 7. The FP32-state
+// SWAPS: the sums come from wave_reduce8 (Sum8). The FP32-state
 // stepper takes it: its chain waits for each step's sums, and there the matrix pipe's longer way is not
 // made up by the issue slots it saves (64 solves of 200x200: 173.8 ms a pass against 180.6; the FP64 stepper,
 // 141.5 with the matrix pipe, was at 145.8 with swaps).

@@ -106,10 +106,12 @@ __device__ __forceinline__ double wave_sum8(const double v[8])
 }
 
 // Sum each of v[0..7] over the 64 lanes of the wave by swaps and DPP (reduce-scatter):
-// lane l ends with the total of v[(l >> 3) & 7]. Requires all 64 lanes. The faster of the two in the
+// lane l ends with the total of v[reduce8_value(l)] (value q ^ 2 eight lanes away, in DPP's reach). Requires
+// all 64 lanes. The faster of the two in the
 // fixed-step length-gauge kernels, us a step, swaps and matrix pipe: FP64 RK4 40^2 k points 0.634 and 0.649,
 // 300^2 1.10 and 1.12, 1000^2 8.7 and 9.9; FP32 300^2 0.99 and 1.03; 64 solves of 200^2 408 and 421 ms (FP64),
 // 291 and 307 (FP32).
+__device__ __forceinline__ int reduce8_value(int lane) { return ((lane >> 3) & 4) | ((lane >> 2) & 2) | ((lane >> 4) & 1); }
 __device__ __forceinline__ double wave_reduce8(double v[8])
 {
     const int lane = __lane_id();
@@ -123,16 +125,16 @@ __device__ __forceinline__ double wave_reduce8(double v[8])
     // lane bit 4: permlane16 swap + add
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-        double a = v[j], b = v[j + 2];
+        double a = v[2 * j], b = v[2 * j + 1];
         swap16(a, b);
-        v[j] = a + b;  // even rows: v[j], odd rows: v[j+2]
+        v[j] = a + b;  // even rows: v[2j], odd rows: v[2j+1]
     }
     // lane bit 3: rotate by 8 inside each 16-lane row (= lane ^ 8)
     const bool hi = (lane & 8) != 0;
     const double keep = hi ? v[1] : v[0];
     const double send = hi ? v[0] : v[1];
     double x = keep + dpp_f64<0x128>(send);  // row_ror:8
-    // lanes 8q..8q+7 now share value index q: all-reduce over the low 3 bits
+    // eight consecutive lanes now share a value: all-reduce over the low 3 bits
     x += dpp_f64<0x141>(x);  // row_half_mirror (i <-> 7-i)
     x += dpp_f64<0x4E>(x);   // quad_perm [2,3,0,1]
     x += dpp_f64<0xB1>(x);   // quad_perm [1,0,3,2]
@@ -316,17 +318,11 @@ __device__ __forceinline__ void sample_state(const Phases<R> &e, double wk, R n,
 template <bool SWAPS>
 struct Sum8 {
     static constexpr unsigned long long kFirst = SWAPS ? 0xffull : kSum8First;  // the lanes of value 0
-    static __device__ __forceinline__ int value(int lane) { return SWAPS ? lane >> 3 : sum8_value(lane); }
+    static __device__ __forceinline__ int value(int lane) { return SWAPS ? reduce8_value(lane) : sum8_value(lane); }
     static __device__ __forceinline__ int member(int lane) { return SWAPS ? lane & 7 : sum8_member(lane); }
     static __device__ __forceinline__ double total(double v[8]) { return SWAPS ? wave_reduce8(v) : wave_sum8(v); }
-    // of value q the total of value q ^ 2
-    static __device__ __forceinline__ double other_pair(double x, int lane)
-    {
-        if (!SWAPS) return dpp_f64<0x4E>(x);
-        double a = x, b = x;
-        swap16(a, b);  // even rows hold (own, other), odd rows (other, own)
-        return (lane & 16) != 0 ? a : b;
-    }
+    // of value q the total of value q ^ 2 (row_ror:8, quad_perm [2,3,0,1])
+    static __device__ __forceinline__ double other_pair(double x) { return dpp_f64<SWAPS ? 0x128 : 0x4E>(x); }
 };
 
 // the factor of this lane's value in the k sums of sample_state
@@ -345,7 +341,7 @@ __device__ __forceinline__ double sample_sums(double v[8], double scale, bool in
 {
     double r = Sum8<SWAPS>::total(v) * scale;
     if (!inter_intra) {  // uniform
-        const double o = Sum8<SWAPS>::other_pair(r, lane);  // values 0 <-> 2, 1 <-> 3
+        const double o = Sum8<SWAPS>::other_pair(r);  // values 0 <-> 2, 1 <-> 3
         const int q = Sum8<SWAPS>::value(lane);
         r = q > 3 ? r : (q < 2 ? r + o : 0.0);
     }
