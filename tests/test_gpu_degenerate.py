@@ -32,7 +32,7 @@ def _run(cfg, m):
 
 
 @pytest.mark.parametrize("fused", [True, False])
-@pytest.mark.parametrize("n,npts,rk", [(1, (6, 6, 1), 4), (2, (7, 6, 1), 5), (2, (9, 8, 1), 4), (4, (7, 6, 1), 4), (4, (7, 6, 1), 5),
+@pytest.mark.parametrize("n,npts,rk", [(1, (9, 8, 1), 4), (2, (7, 6, 1), 5), (2, (9, 8, 1), 4), (4, (7, 6, 1), 4), (4, (7, 6, 1), 5),
                                        (5, (7, 6, 1), 5), (8, (8, 7, 1), 4), (8, (8, 7, 1), 5)])
 def test_spin_doubled_wannier(monkeypatch, n, npts, rk, fused):
     single = synthetic_wannier(n, nmax=(1, 1, 0), seed=300 + n, onsite=0.3 if n > 1 else 0.0)

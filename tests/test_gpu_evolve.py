@@ -5,6 +5,8 @@ N-band paths) and the same against the separate kernels; split runs give the sam
 off points where two bands meet exactly (Gamma for the transition-metal and Kane-Mele classes, the line k_x = 0 with
 spin-orbit, planes through Gamma for WDSM_TaAs): there the band basis, and so the dephasing and the band populations,
 is the eigensolver's choice and the two paths differ with rounding / gap."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -132,8 +134,10 @@ def test_box_evolve(oracle, monkeypatch, N, nmax, npts, rk, T1, T2, ii):
 
 
 @pytest.mark.parametrize("N,nmax,npts,T2,ii", [
-    (9, (0, 1, 0), (3, 5, 1), 80.0, True),     # one lattice vector along a1, a block not full
-    (12, (1, 1, 0), (4, 4, 1), 80.0, False),
+    (9, (0, 1, 0), (3, 5, 1), 80.0, True),     # too few k points for the separable sums: the separate kernels
+    (12, (1, 1, 0), (4, 4, 1), 80.0, False),   # (these two against the oracle)
+    (9, (0, 2, 0), (5, 9, 1), 80.0, True),     # one lattice vector along a1, a block not full
+    (12, (1, 1, 0), (7, 7, 1), 80.0, False),
     (13, (2, 0, 1), (5, 2, 2), 0.0, True),     # three chunks of a staged row
     (16, (3, 1, 0), (9, 3, 1), 80.0, True),    # seven lattice vectors, three blocks a column
 ])
@@ -145,18 +149,21 @@ def test_step_blocks(oracle, monkeypatch, N, nmax, npts, T2, ii):
                     dt=0.5, T2=T2, rk_order=4, inter_intra=ii)
     print(N, nmax, npts, flush=True)
     ref = oracle.run(cfg, m, nthreads=8, want_state=True)
-    got = _run(cfg, m)
+    got, foot = _run(cfg, m), query_footprint(cfg, m)
     with monkeypatch.context() as mp:
         mp.setenv("ANTELOPE_NB_FUSED", "0")
         sep = _run(cfg, m)
+        assert (foot != query_footprint(cfg, m)) == (npts not in ((3, 5, 1), (4, 4, 1)))  # the plan that ran
     for key in ("j_inter", "j_intra", "band_pop", "rho_bar", "state"):
         if np.linalg.norm(ref[key]) > 0.0:
             assert rel_l2(got[key], ref[key]) < 1e-10 and rel_l2(got[key], sep[key]) < 1e-10, key
 
 
 @pytest.mark.parametrize("N,nmax,npts,T1,T2,ii", [
-    (9, (0, 1, 0), (3, 5, 1), 0.0, 80.0, True),
+    (9, (0, 1, 0), (3, 5, 1), 0.0, 80.0, True),      # as above: the separate kernels
     (12, (1, 1, 0), (4, 4, 1), 120.0, 80.0, False),
+    (9, (0, 2, 0), (5, 9, 1), 0.0, 80.0, True),
+    (12, (1, 1, 0), (7, 7, 1), 120.0, 80.0, False),
     (13, (2, 0, 1), (5, 2, 2), 0.0, 0.0, True),
     (16, (3, 1, 0), (9, 3, 1), 150.0, 80.0, True),
     (16, (1, 1, 0), (64, 8, 1), 0.0, 80.0, True),  # scratch in the stage-derivative slots
@@ -263,3 +270,49 @@ def test_velocity_evolve(oracle, monkeypatch, N, npts, rk, T1, T2, ii):
         assert rel_l2(got[key], sep[key]) < 1e-12, key
         if key != "state":
             assert rel_l2(got[key], ref[key]) < 1e-10, key
+
+
+@pytest.mark.parametrize("N,rk", [(9, 4), (9, 5), (16, 4), (16, 5)])
+def test_velocity_eight_wave_blocks(monkeypatch, N, rk):
+    """Blocks of eight waves (9 to 16 bands from 2041 k points), the last one not full, against one launch per step.
+    At 16 bands they take more LDS than a kernel gets unasked."""
+    npts = (409, 5, 1)  # 2045
+    assert (2045 + 7) // 8 >= 256 and 2045 % 8
+    m = synthetic_wannier(N, nmax=(1, 1, 0), seed=150 + N)
+    cfg = RunConfig(npoints=list(npts), pulses=[Pulse(E0=0.01, w0=0.05, ncycles=0.0625, ellip=0.4, envelope="sin2")],
+                    dt=0.5, T1=120.0, T2=80.0, rk_order=rk, inter_intra=True, gauge="VelocityHamiltonian")
+    print(N, rk, flush=True)
+    got, foot = _run(cfg, m), query_footprint(cfg, m)
+    with monkeypatch.context() as mp:
+        mp.setenv("ANTELOPE_NB_FUSED", "0")
+        sep = _run(cfg, m)
+        assert foot != query_footprint(cfg, m)
+    for key in ("j_inter", "j_intra", "band_pop", "rho_bar", "state"):
+        assert rel_l2(got[key], sep[key]) < 1e-12, key
+
+
+@pytest.mark.parametrize("gauge,rk", [("LengthWannier", 4), ("VelocityHamiltonian", 5)])
+def test_parted_series(oracle, gauge, rk):
+    """Series from 1 MiB on come parted: rho's sums straight into the caller's array, the rest beside them, through the
+    buffer of the partial sums. Read half way and at the end, and without rho's sums (whole rows)."""
+    m = synthetic_wannier(8, nmax=(1, 1, 0), seed=160)
+    cfg = RunConfig(npoints=[3, 3, 1], pulses=[Pulse(E0=0.01, w0=0.05, ncycles=4.0, ellip=0.4, envelope="sin2")],
+                    dt=0.5, T2=80.0, rk_order=rk, inter_intra=True, gauge=gauge)
+    print(gauge, rk, flush=True)
+    ref = oracle.run(cfg, m, nthreads=8)
+    with SBESolver(cfg, m) as s:
+        nt = s.nt
+        assert nt * (6 + 8 + 2 * 64) * 8 >= 1 << 20
+        s.run(0, nt // 2)
+        half = s.series()
+        s.run()
+        got, again = s.series(), s.series()
+        rows = {"j_inter": np.zeros((nt, 3)), "j_intra": np.zeros((nt, 3)), "band_pop": np.zeros((nt, 8))}
+        p = {k: v.ctypes.data_as(C.POINTER(C.c_double)) for k, v in rows.items()}
+        assert s._lib.sbe_get_series(s._ctx, p["j_inter"], p["j_intra"], None, p["band_pop"]) == 0
+    for key in ("j_inter", "j_intra", "band_pop", "rho_bar"):
+        assert rel_l2(got[key], ref[key]) < 1e-10, key
+        assert np.array_equal(got[key], again[key]), key
+        assert np.array_equal(half[key][: nt // 2], got[key][: nt // 2]), key
+    for key in rows:
+        assert np.array_equal(rows[key], got[key]), key

@@ -98,7 +98,7 @@ def test_fused_split_runs_and_state_reads_are_bitwise(monkeypatch):
 
 
 def test_fused_rk5_keeps_separate_kernels(oracle, monkeypatch):
-    """The fused step is the classical RK4 tableau; RK5 plans the separate kernels."""
+    """RK5: one plan whether its time-fused kernels or the separate ones run, and the oracle's results."""
     model = synthetic_wannier(6, nmax=(2, 2, 1), seed=12)
     cfg = _cfg((6, 5, 2), rk=5, ncycles=0.25)
     print("case: rk5", flush=True)
@@ -114,16 +114,16 @@ def test_fused_rk5_keeps_separate_kernels(oracle, monkeypatch):
     ("n16_velocity_t1t2_total_current", 16, dict(T2=60.0, inter_intra=False)),
     ("n24_velocity_t2_four_waves_per_k", 24, dict()),
     ("n32_velocity_t1t2_total_current", 32, dict(T1=150.0, T2=60.0, inter_intra=False)),
-    ("n8_velocity_2048k_eight_waves_per_block", 8, dict(npts=(16, 16, 8), ncycles=0.25)),
+    ("n8_velocity_2048k", 8, dict(npts=(16, 16, 8), ncycles=0.25)),
 ])
 def test_time_fused_velocity_gauge(oracle, monkeypatch, label, N, kw):
     """The time-fused velocity-gauge kernels (all steps of a chunk in one launch; one wave
-    per k point for N <= 16, a block of four waves per k point above) against the oracle
+    per k point for N <= 16 or four k points, a block of four waves per k point above) against the oracle
     and the one-launch-per-step kernel, and split runs."""
     import dataclasses
     model = synthetic_wannier(N, nmax=(1, 1, 1), seed=70 + N)
     T1 = kw.pop("T1", 150.0 if N == 16 else -1.0)
-    npts = kw.pop("npts", (5, 4, 2))  # blocks of 4 waves for N <= 16 below 2048 k points, of 8 above
+    npts = kw.pop("npts", (5, 4, 2))  # (blocks of eight waves, 9 to 16 bands: test_gpu_evolve.py)
     cfg = dataclasses.replace(_cfg(npts, **kw), gauge="VelocityHamiltonian", T1=T1)
     print(f"case: {label}", flush=True)
     ref = oracle.run(cfg, model, nthreads=8, want_state=False)

@@ -5,7 +5,7 @@ sums over whole grids have their own tests."""
 import numpy as np
 import pytest
 
-from antelope_amd import SBESolver
+from antelope_amd import Pulse, SBESolver
 from tests.cases import haldane_cfg1_model, rel_l2, small_config
 
 pytestmark = pytest.mark.gpu
@@ -72,3 +72,23 @@ def test_velocity_fp32_sums_by_matrix_pipe(monkeypatch, rk, T1, kpt):
     for key in ("j_inter", "j_intra", "band_pop", "rho_bar"):
         a, b = parts[0][key] + parts[1][key], whole[key]
         assert np.abs(a - b).max() <= 1e-12 * np.abs(b).max(), key
+
+
+@pytest.mark.parametrize("gauge,rk,precision", [("LengthWannier", 4, "fp64"), ("LengthWannier", 5, "fp32"),
+                                                ("VelocityHamiltonian", 5, "fp64"), ("VelocityHamiltonian", 4, "fp32")])
+def test_nine_pulses(oracle, gauge, rk, precision):
+    """More pulses than the laser-row kernel's arguments hold: the rows come from the host. FP64 against the oracle
+    (1e-10), FP32 state within 6e-5 of it (the bar of the FP32 forms)."""
+    cfg = small_config(n=(9, 8), ncycles=1.0, rk=rk, inter_intra=True, ellip=0.4, grid="mp", T1=300.0, gauge=gauge,
+                       precision=precision)
+    one = cfg.pulses[0]
+    cfg.pulses = [Pulse(E0=one.E0 / (1 + i), w0=one.w0 * (1 + 0.05 * i), ncycles=1.0, ellip=0.1 * i, cep=0.2 * i, envelope="sin2")
+                  for i in range(9)]
+    model = haldane_cfg1_model()
+    print("nine pulses:", gauge, rk, precision, flush=True)
+    ref = oracle.run(cfg, model, nthreads=4)
+    with SBESolver(cfg, model) as s:
+        s.run()
+        got = s.series()
+    for key in ("j_inter", "j_intra", "band_pop", "rho_bar"):
+        assert rel_l2(got[key], ref[key]) < (1e-10 if precision == "fp64" else 6e-5), key
