@@ -97,6 +97,8 @@ struct NbFused {
     int g1;                  // blocks per (k2, k3) column: ceil(K1 / kNbFusedWaves)
     int nblocks;             // g1 K2 K3: partial rows per step
 };
+// dynamic LDS beyond the default limit: raises the kernel's limit, once per device and kernel (nband16.hip)
+hipError_t allow_lds(const void *kernel, size_t lds);
 hipError_t nb16_launch_step(const NbArgs &a, const NbFused &f, int rk_order, double2 *rho, double2 *U, double *partials,
                             hipStream_t s);
 // the separable sums of one evaluation up to the second pass: t2 [M1][K2][K3][bcols]

@@ -718,7 +718,7 @@ hipError_t nb16_launch_sample(const NbArgs &a, const double2 *mats, const double
 }
 
 // dynamic LDS beyond the default limit: raise the kernel's limit, once per device and kernel
-static hipError_t allow_lds(const void *kernel, size_t lds)
+hipError_t allow_lds(const void *kernel, size_t lds)
 {
     if (lds <= (size_t(64) << 10)) return hipSuccess;
     static std::mutex mu;

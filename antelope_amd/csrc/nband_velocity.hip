@@ -14,9 +14,6 @@
 // Wannier N = 12, 16 x 15 x 4 k, RK5: 6.4 us per step against 14.4 us with one
 // launch per step (12.1 us of kernel), which also wrote and read rho and pMatrix
 // every step.
-#include <map>
-#include <mutex>
-
 #include "haldane_dev.hpp"
 #include "tile_eig.hpp"
 
@@ -173,25 +170,6 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) voi
             if (i < N && c < N) rho[k * nn + i * N + c] = make_double2(R.re[r], R.im[r]);
         }
     }
-}
-
-// dynamic LDS beyond the default limit: raise the kernel's limit, once per device and kernel
-hipError_t allow_lds(const void *kernel, size_t lds)
-{
-    if (lds <= (size_t(64) << 10)) return hipSuccess;
-    static std::mutex mu;
-    static std::map<std::pair<int, const void *>, size_t> raised;
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return e;
-    std::lock_guard<std::mutex> lk(mu);
-    size_t &have = raised[{dev, kernel}];
-    if (have < lds) {
-        e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-        if (e != hipSuccess) return e;
-        have = lds;
-    }
-    return hipSuccess;
 }
 
 template <class T, int RK, int W>

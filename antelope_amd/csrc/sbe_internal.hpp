@@ -225,15 +225,15 @@ struct sbe_ctx {
     bool nbf_small = false;  // N <= 8: nb_box_evolve_kernel
     bool nbf_jz = false;     // any lattice vector with a z component
     int nbf_mids = 1;        // evaluation times between t_n and t_n + dt
-    // second-pass outputs of up to nbf_S steps: J at t_n and H~ H at t_n + dt/2 per step, the
-    // end pairs H~ H at t_n + dt in a ring of nbf_S + 1 (step mod ring)
+    // second-pass outputs of up to nbf_S steps: J at t_n and H~ H at the nbf_mids times between per
+    // step, the end pairs H~ H at t_n + dt in a ring of nbf_S + 1 (step mod ring)
     int nbf_S = 0;
     double2 *nbf_tj = nullptr, *nbf_th = nullptr, *nbf_ring = nullptr;
     int64_t nbf_t2_stride = 0;
     double *nbf_lam = nullptr;   // [nk_stride][16] band energies at the stored eigenvectors' time
     double2 *nbf_bs = nullptr, *nbf_t1s = nullptr;  // per evaluation: B on the box, first-pass output
     int64_t nbf_b_stride = 0, nbf_t1_stride = 0;
-    const double *nbf_laser = nullptr;  // [nt][3][6] A, E at t_n, t_n + dt/2, t_n + dt
+    const double *nbf_laser = nullptr;  // [nt][nbf_mids + 2][6] A, E at t_n, the times between, t_n + dt
     int nbf_g1 = 0, nbf_nblocks = 0;
     bool nbf_prev_valid = false;  // the ring holds H~, H at nbf_prev_time for the step that starts there
     double nbf_prev_time = 0;
