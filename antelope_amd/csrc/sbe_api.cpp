@@ -1069,17 +1069,21 @@ int sbe_batch_create(int32_t n, const sbe_config *cfgs, const sbe_model *models,
     sbe_batch *b = new (std::nothrow) sbe_batch();
     if (!b) return batch_fail(nullptr, SBE_ERR_OOM, "host allocation failed");
     b->adaptive = cfgs[0].rk_order == SBE_RK_CASH_KARP;
-    // The groups' streams come before the members' own (idle while the batch runs) and the step streams
-    // before the reductions': streams share the process's four hardware queues in the order of their
-    // creation, and a step stream behind another group's reductions, which wait for that group's steps, runs
-    // after them instead of beside them (2 solves of 60x60, the first batch of a process: 7.5 ms against 5.0).
+    // Streams share the process's four hardware queues in the order of their creation. Fixed steps: the groups'
+    // come before the members' own (idle while the batch runs) and the step streams before the reductions': a
+    // step stream behind another group's reductions, which wait for that group's steps, runs after them instead
+    // of beside them (2 solves of 60x60, the first batch of a process: 7.5 ms against 5.0). The adaptive stepper's
+    // long windows don't meet that and take another place on the queues better: after the members', each group's
+    // reductions behind its steps, 64 solves of 200x200 take 132.5 ms (FP32) and 141.6 (FP64), in the fixed steps'
+    // order 138.3 and 142.5, the first batch of 2 solves 9.9 ms in both.
     const int ng = n >= 2 ? 2 : 1;
     b->groups.resize(ng);
     hipError_t e = hipSuccess;
-    for (BatchGroup &g : b->groups)
-        if (e == hipSuccess) e = hipStreamCreateWithFlags(&g.stream, hipStreamNonBlocking);
-    for (BatchGroup &g : b->groups)
-        if (e == hipSuccess) e = hipStreamCreateWithFlags(&g.rstream, hipStreamNonBlocking);
+    auto create = [&](hipStream_t &s) { if (e == hipSuccess) e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking); };
+    if (!b->adaptive) {
+        for (BatchGroup &g : b->groups) create(g.stream);
+        for (BatchGroup &g : b->groups) create(g.rstream);
+    }
     if (e != hipSuccess) {
         const std::string m = std::string("batch streams: ") + hipGetErrorString(e);
         sbe_batch_destroy(b);
@@ -1135,7 +1139,12 @@ int sbe_batch_create(int32_t n, const sbe_config *cfgs, const sbe_model *models,
         for (BatchGroup &g : b->groups)
             std::stable_sort(g.solves.begin(), g.solves.end(), [&](int x, int y) { return field(x) > field(y); });
     }
-    e = hipEventCreateWithFlags(&b->run_start, hipEventDisableTiming);
+    if (b->adaptive)
+        for (BatchGroup &g : b->groups) {
+            create(g.stream);
+            create(g.rstream);
+        }
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&b->run_start, hipEventDisableTiming);
     int arg0 = 0;
     for (BatchGroup &g : b->groups) {
         g.arg0 = arg0;
