@@ -969,6 +969,13 @@ int sbe_get_info(const sbe_ctx *ctx, sbe_info *info)
 
 }  // extern "C"
 
+// The steps of a solve that a launch window has put into its partial rows.
+struct BatchSum {
+    int solve = 0;
+    int64_t first = 0;
+    int32_t nsteps = 0;
+};
+
 // A group of a batch's solves with its own streams: its launch windows follow
 // each other on `stream`, its k-sum reductions run on `rstream` while its next
 // window steps, and the windows alternate between two partial-row buffers per
@@ -989,6 +996,7 @@ struct BatchGroup {
     hipEvent_t win_done[2] = {nullptr, nullptr}, red_done[2] = {nullptr, nullptr};
     bool red_pending[2] = {false, false};
     int64_t windows = 0;                 // windows launched (parity = windows & 1)
+    std::vector<BatchSum> sums[2];       // by parity: the window's k sums, still to be enqueued
     sbe::SeriesJob *h_jobs = nullptr;    // [2][n_g] pinned job lists of the reductions
     sbe::SeriesJob *d_jobs = nullptr;    // [2][n_g]
 };
@@ -1069,26 +1077,6 @@ int sbe_batch_create(int32_t n, const sbe_config *cfgs, const sbe_model *models,
     sbe_batch *b = new (std::nothrow) sbe_batch();
     if (!b) return batch_fail(nullptr, SBE_ERR_OOM, "host allocation failed");
     b->adaptive = cfgs[0].rk_order == SBE_RK_CASH_KARP;
-    // Streams share the process's four hardware queues in the order of their creation. Fixed steps: the groups'
-    // come before the members' own (idle while the batch runs) and the step streams before the reductions': a
-    // step stream behind another group's reductions, which wait for that group's steps, runs after them instead
-    // of beside them (2 solves of 60x60, the first batch of a process: 7.5 ms against 5.0). The adaptive stepper's
-    // long windows don't meet that and take another place on the queues better: after the members', each group's
-    // reductions behind its steps, 64 solves of 200x200 take 132.5 ms (FP32) and 141.6 (FP64), in the fixed steps'
-    // order 138.3 and 142.5, the first batch of 2 solves 9.9 ms in both.
-    const int ng = n >= 2 ? 2 : 1;
-    b->groups.resize(ng);
-    hipError_t e = hipSuccess;
-    auto create = [&](hipStream_t &s) { if (e == hipSuccess) e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking); };
-    if (!b->adaptive) {
-        for (BatchGroup &g : b->groups) create(g.stream);
-        for (BatchGroup &g : b->groups) create(g.rstream);
-    }
-    if (e != hipSuccess) {
-        const std::string m = std::string("batch streams: ") + hipGetErrorString(e);
-        sbe_batch_destroy(b);
-        return batch_fail(nullptr, SBE_ERR_HIP, m);
-    }
     t_partial_bytes = kBatchPartialBytes;
     t_batch_member = !b->adaptive;  // the adaptive batch takes each member's kpt
     for (int i = 0; i < n; ++i) {
@@ -1114,6 +1102,8 @@ int sbe_batch_create(int32_t n, const sbe_config *cfgs, const sbe_model *models,
     b->prec = cfgs[0].precision;
     // groups of about equal work (k points x samples): longest first, each solve to the lighter
     // group (one group for a single solve)
+    const int ng = n >= 2 ? 2 : 1;
+    b->groups.resize(ng);
     {
         std::vector<int> order(n);
         std::vector<double> work(n);
@@ -1139,17 +1129,14 @@ int sbe_batch_create(int32_t n, const sbe_config *cfgs, const sbe_model *models,
         for (BatchGroup &g : b->groups)
             std::stable_sort(g.solves.begin(), g.solves.end(), [&](int x, int y) { return field(x) > field(y); });
     }
-    if (b->adaptive)
-        for (BatchGroup &g : b->groups) {
-            create(g.stream);
-            create(g.rstream);
-        }
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&b->run_start, hipEventDisableTiming);
+    hipError_t e = hipEventCreateWithFlags(&b->run_start, hipEventDisableTiming);
     int arg0 = 0;
     for (BatchGroup &g : b->groups) {
         g.arg0 = arg0;
         arg0 += static_cast<int>(g.solves.size());
         const size_t nj = 2 * g.solves.size();
+        if (e == hipSuccess) e = hipStreamCreateWithFlags(&g.stream, hipStreamNonBlocking);
+        if (e == hipSuccess) e = hipStreamCreateWithFlags(&g.rstream, hipStreamNonBlocking);
         for (int p = 0; p < 2 && e == hipSuccess; ++p) {
             e = hipEventCreateWithFlags(&g.win_done[p], hipEventDisableTiming);
             if (e == hipSuccess) e = hipEventCreateWithFlags(&g.red_done[p], hipEventDisableTiming);
@@ -1207,8 +1194,8 @@ int sbe_batch_create(int32_t n, const sbe_config *cfgs, const sbe_model *models,
 }
 
 namespace {
-// One launch window of group g: the step launch on g.stream (its partial rows in
-// this window's parity buffers), then the group's k sums on g.rstream.
+// One launch window of group g: the step launch on g.stream (its partial rows in this window's parity
+// buffers). Its k sums are enqueued by batch_sums.
 hipError_t batch_window(sbe_batch *b, BatchGroup &g, int64_t launch, std::vector<sbe::HaldaneArgs> &args)
 {
     const int n = static_cast<int>(b->ctx.size());
@@ -1258,39 +1245,48 @@ hipError_t batch_window(sbe_batch *b, BatchGroup &g, int64_t launch, std::vector
         if (eb) (void)hipEventDestroy(eb);
     }
     if (e == hipSuccess) e = hipEventRecord(g.win_done[par], g.stream);
-    // the k sums of this window: one launch for the group when each member fits one pass (the
-    // same per-step arithmetic as a member's own reduction, so the same bits)
-    if (e == hipSuccess) e = hipStreamWaitEvent(g.rstream, g.win_done[par], 0);
+    if (e != hipSuccess) return e;
+    for (int i : g.solves) {
+        if (insts[i].nsteps <= 0) continue;
+        g.sums[par].push_back({i, b->ctx[i]->steps_done, insts[i].nsteps});
+        b->ctx[i]->steps_done += insts[i].nsteps;
+    }
+    ++g.windows;
+    return hipSuccess;
+}
+
+// The k sums of group g's window of parity par on g.rstream, if they are still to be enqueued: one launch for the
+// group when each member fits one pass (the same per-step arithmetic as a member's own reduction, so the same bits)
+hipError_t batch_sums(sbe_batch *b, BatchGroup &g, int par)
+{
+    if (g.sums[par].empty()) return hipSuccess;
+    hipError_t e = hipStreamWaitEvent(g.rstream, g.win_done[par], 0);
     // the pinned job list of this parity was last read by the reduction two windows back
     if (e == hipSuccess && g.red_pending[par]) e = hipEventSynchronize(g.red_done[par]);
+    const int ngs = static_cast<int>(g.solves.size());
     sbe::SeriesJob *h_jobs = g.h_jobs + static_cast<int64_t>(par) * ngs;
     sbe::SeriesJob *d_jobs = g.d_jobs + static_cast<int64_t>(par) * ngs;
     int njobs = 0;
     int64_t total = 0;
-    for (int i : g.solves) {
+    for (const BatchSum &w : g.sums[par]) {
         if (e != hipSuccess) break;
-        sbe_ctx *c = b->ctx[i];
-        if (insts[i].nsteps <= 0) continue;
-        double *rows = par ? b->part2[i] : c->d_partials;
+        sbe_ctx *c = b->ctx[w.solve];
+        double *rows = par ? b->part2[w.solve] : c->d_partials;
         if (b->multi) {
-            h_jobs[njobs++] = {rows, c->d_series + c->steps_done * c->nv, c->nwaves, insts[i].nsteps, total,
-                               c->nonfinite_d};
-            total += insts[i].nsteps;
+            h_jobs[njobs++] = {rows, c->d_series + w.first * c->nv, c->nwaves, w.nsteps, total, c->nonfinite_d};
+            total += w.nsteps;
         } else {
-            e = sbe::launch_series_reduce(rows, insts[i].nsteps, c->nwaves, c->nv, c->d_series + c->steps_done * c->nv,
-                                          g.rstream, c->nonfinite_d);
+            e = sbe::launch_series_reduce(rows, w.nsteps, c->nwaves, c->nv, c->d_series + w.first * c->nv, g.rstream,
+                                          c->nonfinite_d);
         }
-        c->steps_done += insts[i].nsteps;
     }
     if (e == hipSuccess && njobs > 0) {
         e = hipMemcpyAsync(d_jobs, h_jobs, sizeof(sbe::SeriesJob) * njobs, hipMemcpyHostToDevice, g.rstream);
         if (e == hipSuccess) e = sbe::launch_series_reduce_multi(d_jobs, njobs, total, sbe::kHaldaneNV, g.rstream);
     }
     if (e == hipSuccess) e = hipEventRecord(g.red_done[par], g.rstream);
-    if (e == hipSuccess) {
-        g.red_pending[par] = true;
-        ++g.windows;
-    }
+    g.red_pending[par] = g.red_pending[par] || e == hipSuccess;
+    g.sums[par].clear();
     return e;
 }
 }  // namespace
@@ -1317,15 +1313,27 @@ int sbe_batch_run(sbe_batch *b, int64_t max_steps)
             for (int i : g.solves) active = active || b->ctx[i]->steps_done < b->ctx[i]->laser.nt;
             if (active && e == hipSuccess) e = batch_window(b, g, launch, insts);
         }
+        // The sums one window late: streams share the process's four hardware queues, and where a group's
+        // reductions, which wait for its steps, stood before the other group's steps in one queue, the groups ran
+        // one after the other (2 solves of 60x60, the first batch of a process: 29.8 ms, 20.1 in this order).
+        for (BatchGroup &g : b->groups)
+            if (e == hipSuccess) e = batch_sums(b, g, static_cast<int>(g.windows & 1));
         budget -= launch;
     }
+    for (BatchGroup &g : b->groups)
+        for (const int64_t w : {g.windows, g.windows + 1})
+            if (e == hipSuccess) e = batch_sums(b, g, static_cast<int>(w & 1));
     // the first stream completes no earlier than every group's last reduction (synchronize and
     // reset wait on it)
     for (BatchGroup &g : b->groups) {
         if (e != hipSuccess || g.windows == 0) continue;
         e = hipStreamWaitEvent(b->stream, g.red_done[(g.windows + 1) & 1], 0);
     }
-    if (e != hipSuccess) return batch_fail(b, SBE_ERR_HIP, std::string("batch launch: ") + hipGetErrorString(e));
+    if (e != hipSuccess) {
+        for (BatchGroup &g : b->groups)
+            for (std::vector<BatchSum> &w : g.sums) w.clear();
+        return batch_fail(b, SBE_ERR_HIP, std::string("batch launch: ") + hipGetErrorString(e));
+    }
     return SBE_OK;
 }
 
