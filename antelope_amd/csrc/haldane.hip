@@ -23,9 +23,9 @@
 // fixed order.
 //
 // Bound by the VALU: a wave alone on its SIMD (fewer than 65536 k points) issues its
-// FP64 chain at 4 cycles an instruction, about 240 of them for an RK4 step of a k point
-// (316 before the sample and the right-hand side
-// were factored; 465 for RK5 with T1), so fewer instructions are what there is to gain.
+// FP64 chain at 4 cycles an instruction, 273 of them for an RK4 step of a k point with one
+// point per lane (316 before the sample and the right-hand side were factored), 247 with two;
+// about 480 for RK5 with T1. Fewer instructions are what there is to gain.
 #include "haldane_setup.hpp"
 
 namespace sbe {

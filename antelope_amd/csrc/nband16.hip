@@ -325,14 +325,14 @@ __global__ __launch_bounds__(64) void nb16_vel_step_kernel(const NbArgs a, const
 // HBM traffic. The waves' sample sums are added in LDS in wave order into
 // one partial row per block.
 //
-// Bound by the FP64 pipe, which MFMA and VALU share: per k point 31 thousand cycles of
-// MFMA (30 products), about 16 of VALU, and 30 of waits for LDS, barriers and MFMA results
-// that the second wave of the SIMD covers in part. Two staging slots instead of four let two
+// Bound by the FP64 pipe, which MFMA and VALU share: of the 64 thousand cycles that a SIMD spends
+// on a k point 32 are MFMA (32 products) and about 15 VALU; the rest are waits for LDS, barriers and MFMA
+// results that the second wave of the SIMD does not cover. Two staging slots instead of four let two
 // blocks of four waves share a CU (one of eight before): while one waits at a barrier the
 // other has products to do. That and one fixed chunk of every staged row per wave, in place
 // of a chunk list with a division per load (3800 scalar instructions per k point), took
 // 48x48x8 with 16 bands from 371 to 329 ms, 628 steps; six wave sums in one (wave_sum8) are
-// part of it.
+// part of it. (In kernel time 308 ms then and 317 since the refinement ends degenerate bands in a unitary basis.)
 //
 // RK5 (Fehlberg): the same blocks and staging over five later times; the six stage
 // derivatives stay in registers, so one wave has a SIMD to itself (512 registers). One launch

@@ -51,9 +51,8 @@ PEAK_HBM_GBS = 8000.0
 ALGO_BYTES_PER_KSTEP = {"fp64": 128.0, "fp32": 64.0, "adaptive_fp64": 128.0}
 # Executed flops per k-point RK4 step of the step kernel, from the rocprofv3
 # counters SQ_INSTS_VALU_{FMA,MUL,ADD}_{F64,F32} (FMA = 2) on this workload:
-# FP64 337; FP32 state 326 FP32 + 11 FP64 (the k sums run on the matrix pipe and are not
-# counted).
-FLOPS_PER_KSTEP = {"fp64": 337.2, "fp32": 336.8}
+# FP64 341; FP32 state 325 FP32 + 19 FP64 (the k sums).
+FLOPS_PER_KSTEP = {"fp64": 341.2, "fp32": 344.8}
 KERNEL_NAME = {"fp64": "haldane_steps_kernel<double, 4, false, true, 2>",
                "fp32": "haldane_steps_kernel<float, 4, false, true, 1>",
                "adaptive_fp64": "haldane_adaptive_kernel<double, true, 1>"}
@@ -201,10 +200,9 @@ def bench_wannier(args) -> int:
     r = res["fp64"]
     ks = forms["fp64"]["k_steps_per_s"]
     # flops per k-point RK4 step of the fused step (nb16_step_kernel, one launch per step):
-    # 20 complex 16 x 16 products (8 N^3 each; rocprofv3 SQ_INSTS_MFMA = 320 per wave and
-    # step, 16 MFMAs a product: 2 for the sample's band-diagonal part, 3 per stage
-    # (H~ y and the band-diagonal part of y) past the first's 1, 3 per eigen refinement,
-    # 2 for the last Newton-Schulz step), the separable Fourier sums' passes along a3 and
+    # 19.3 complex 16 x 16 products (8 N^3 each; rocprofv3 SQ_INSTS_VALU_MFMA_MOPS_F64 x 512
+    # over the first steps of the pulse: 634 kflop per k point; over a whole pulse of 628 steps 31.6
+    # products, the eigen refinements taking more rounds in its field), the separable Fourier sums' passes along a3 and
     # a2 for 7 matrices (M1 M2 K3 M3 + M1 K2 K3 M2 complex multiply-adds per column for the
     # whole grid) and their pass along a1 inside the step kernel (8 tiles of M1 terms per
     # k point: J_x, J_y, J_z and H~ at t, H~ and H at t + dt/2 and at t + dt). The
@@ -219,9 +217,9 @@ def bench_wannier(args) -> int:
     Mb = [int(rv[:, i].max() - rv[:, i].min() + 1) for i in range(3)]
     if box:
         pass23 = Mb[0] * Mb[1] * 8 * Mb[2] + Mb[0] * 48 * 8 * Mb[1]
-        flops = 20 * 8 * N ** 3 + 7 * 8 * N * N * pass23 / nk + 8 * 8 * N * N * Mb[0]
+        flops = 19.3 * 8 * N ** 3 + 7 * 8 * N * N * pass23 / nk + 8 * 8 * N * N * Mb[0]
     else:
-        flops = 7 * fsum + 20 * 8 * N ** 3
+        flops = 7 * fsum + 19.3 * 8 * N ** 3
     flops_ref = 4 * (4 * fsum + 8 * N ** 3) + 4 * fsum + 8 * 8 * N ** 3
     line = {"metric": METRIC, "value": ks, "unit": "k-point·RK-steps/s", "n_gpus": 1,
             "steps": r["steps"], "warmup": min(args.warmup, 5), "ms_per_step": r["wall_s"] * 1e3 / r["steps"],
@@ -353,7 +351,7 @@ def bench_serving(args) -> int:
 # counters SQ_INSTS_VALU_{FMA,MUL,ADD}_F64 (FMA = 2, x 64 lanes) on this workload's
 # generator: per RK4 step for the plain kernel, per accepted step for the adaptive one
 # (rejected attempts and the per-wave laser, controller and reduction work included).
-BATCH_FLOPS = {"plain_fp64_rk4": 340.3, "adaptive_fp64": ADAPT_FLOPS_PER_KSTEP["fp64"]}
+BATCH_FLOPS = {"plain_fp64_rk4": 348.4, "adaptive_fp64": ADAPT_FLOPS_PER_KSTEP["fp64"]}
 BATCH_KERNEL = {"plain_fp64_rk4": "haldane_batch_kernel<double, 4, false, true>",
                 "plain_fp32_rk4": "haldane_batch_kernel<float, 4, false, true>",
                 "adaptive_fp64": "haldane_adaptive_kernel<double, true, 1>",
